@@ -65,6 +65,22 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* problem
 int32_t nav_ba_cost_eval(nav_ba_cost_handle* h, int32_t dtype, const void* T_cw, const void* X, const void* intr,
                          void* cost, void* g_pose, void* g_X, void* g_intr, void* stream);
 
+/* The same evaluation at the poses T = exp(xi) T_cw, xi [n_cam][6] pose
+ * tangents (omega, upsilon):
+ *   T       [n_cam][12]  out: the poses the cost was evaluated at
+ *   total   [1]          out: the sum of the problems' costs (FP64 sum, rounded once)
+ * and the rest as nav_ba_cost_eval (g_pose is the left-tangent gradient at T). */
+int32_t nav_ba_cost_eval_tangent(nav_ba_cost_handle* h, int32_t dtype, const void* xi, const void* T_cw,
+                                 const void* X, const void* intr, void* T, void* total, void* cost, void* g_pose,
+                                 void* g_X, void* g_intr, void* stream);
+
+/* g_xi [n][6] = J_l(xi)^T g_pose, J_l the left Jacobian of SE3: the gradient
+ * with respect to xi from the left-tangent gradient at exp(xi) T_cw.  Needs no
+ * handle; runs on `device`, arrays in its memory, and leaves the caller's
+ * current device as it was. */
+int32_t nav_ba_cost_tangent_grad(int32_t device, int32_t dtype, int32_t n, const void* xi, const void* g_pose,
+                                 void* g_xi, void* stream);
+
 /* Sizes of the prepared batch. */
 int32_t nav_ba_cost_sizes(const nav_ba_cost_handle* h, int32_t* n_cam, int32_t* n_pt, int32_t* n_obs,
                           int32_t* n_problems);

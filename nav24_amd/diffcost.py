@@ -49,6 +49,10 @@ def lib() -> C.CDLL:
         L.nav_ba_cost_prepare.restype = C.c_int32
         L.nav_ba_cost_eval.argtypes = [H, C.c_int32, vp, vp, vp, vp, vp, vp, vp, vp]
         L.nav_ba_cost_eval.restype = C.c_int32
+        L.nav_ba_cost_eval_tangent.argtypes = [H, C.c_int32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+        L.nav_ba_cost_eval_tangent.restype = C.c_int32
+        L.nav_ba_cost_tangent_grad.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
+        L.nav_ba_cost_tangent_grad.restype = C.c_int32
         L.nav_ba_cost_sizes.argtypes = [H, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32),
                                         C.POINTER(C.c_int32)]
         L.nav_ba_cost_sizes.restype = C.c_int32
@@ -124,6 +128,51 @@ class CostBatch:
                                            C.c_void_p(stream)))
         return CostResult(cost, gp, gx, gi)
 
+    def _eval_tangent(self, xi, X, intr, T_cw, grad: bool):
+        """(total cost, T = exp(xi) T_cw, CostResult at T) for inputs that
+        `_poses_on_device` accepts, on torch's current stream."""
+        import torch
+        dt, dev = xi.dtype, xi.device
+        xi, X, intr, T_cw = (t.contiguous() for t in (xi, X, intr, T_cw))
+        T = torch.empty_like(T_cw)
+        total = torch.empty((), dtype=dt, device=dev)
+        cost = torch.empty(self.n_problems, dtype=dt, device=dev)
+        gp = torch.empty((self.n_cam, 6), dtype=dt, device=dev) if grad else None
+        gx = torch.empty((self.n_pt, 3), dtype=dt, device=dev) if grad else None
+        gi = torch.empty(8, dtype=dt, device=dev) if grad else None
+        ptr = (lambda t: t.data_ptr() if t is not None else None)
+        self._check(lib().nav_ba_cost_eval_tangent(
+            self._h, NAV_BA_COST_F64 if dt == torch.float64 else NAV_BA_COST_F32, ptr(xi), ptr(T_cw), ptr(X), ptr(intr),
+            ptr(T), ptr(total), ptr(cost), ptr(gp), ptr(gx), ptr(gi), torch.cuda.current_stream(dev).cuda_stream))
+        return total, T, CostResult(cost, gp, gx, gi)
+
+
+def _poses_on_device(batch, xi, X, intr, T_cw) -> bool:
+    """Whether the pose map and its adjoint can run in the device kernels: one
+    type and one device for all four tensors, and the batch's shapes.  Anything
+    else (mixed types, broadcast poses, another evaluator) goes through
+    `se3_left` and the batch's `eval`."""
+    import torch
+    dt, dev = xi.dtype, xi.device
+    return (getattr(type(batch), "eval", None) is CostBatch.eval and dt in (torch.float64, torch.float32) and xi.is_cuda
+            and all(t.dtype == dt and t.device == dev for t in (X, intr, T_cw))
+            and tuple(xi.shape) == (batch.n_cam, 6) and tuple(T_cw.shape) == (batch.n_cam, 12)
+            and tuple(X.shape) == (batch.n_pt, 3) and tuple(intr.shape) == (8,))
+
+
+def _tangent_grad(xi, g_pose):
+    """J_l(xi)^T g_pose in one kernel, for xi and g_pose as `_eval_tangent` took
+    and returned them."""
+    import torch
+    xi = xi.contiguous()
+    out = torch.empty_like(g_pose)
+    st = lib().nav_ba_cost_tangent_grad(
+        xi.device.index, NAV_BA_COST_F64 if xi.dtype == torch.float64 else NAV_BA_COST_F32, xi.shape[0], xi.data_ptr(),
+        g_pose.data_ptr(), out.data_ptr(), torch.cuda.current_stream(xi.device).cuda_stream)
+    if st != NAV_BA_OK:
+        raise CostError(st, "nav_ba_cost_tangent_grad")
+    return out
+
 
 def se3_left(xi, T_cw):
     """exp(xi) T_cw for every pose row [R (9) | t (3)], xi = (omega, upsilon), in torch.
@@ -180,26 +229,36 @@ try:
 
         @staticmethod
         def forward(ctx, xi, X, intr, T_cw, batch):
+            need = any(ctx.needs_input_grad[:3])
             with torch.no_grad():
-                T = se3_left(xi, T_cw)
-                need = any(ctx.needs_input_grad[:3])
-                r = batch.eval(T, X.contiguous(), intr.contiguous(), grad=need)
+                kernels = _poses_on_device(batch, xi, X, intr, T_cw)
+                if kernels:
+                    cost, T, r = batch._eval_tangent(xi, X, intr, T_cw, need)
+                else:
+                    T = se3_left(xi, T_cw)
+                    r = batch.eval(T, X.contiguous(), intr.contiguous(), grad=need)
+                    cost = r.cost.sum()
             if need:
                 ctx.save_for_backward(r.g_pose, r.g_X, r.g_intr, xi.detach(), T_cw.detach(), T)
+            ctx.kernels = kernels
             ctx.need = need
-            return r.cost.sum()
+            return cost
 
         @staticmethod
         def backward(ctx, g):
             gp, gx, gi, xi, T_cw, T = ctx.saved_tensors
             g_xi = None
             if ctx.needs_input_grad[0]:
-                # d cost / d xi = (d T / d xi)^T G_T, G_T the entry gradient of the
-                # left-tangent gradient gp at T: J_l(xi)^T gp
-                with torch.enable_grad():
-                    x = xi.clone().requires_grad_(True)
-                    Tx = se3_left(x, T_cw)
-                    (g_xi,) = torch.autograd.grad(Tx, x, tangent_to_entry_grad(gp, T))
+                # d cost / d xi = J_l(xi)^T gp, gp the left-tangent gradient at T
+                # (a saved-tensor hook may have moved or converted them)
+                if ctx.kernels and xi.is_cuda and (gp.device, gp.dtype) == (xi.device, xi.dtype):
+                    g_xi = _tangent_grad(xi, gp.contiguous())
+                else:
+                    # (d T / d xi)^T G_T, G_T the entry gradient of gp at T
+                    with torch.enable_grad():
+                        x = xi.clone().requires_grad_(True)
+                        Tx = se3_left(x, T_cw)
+                        (g_xi,) = torch.autograd.grad(Tx, x, tangent_to_entry_grad(gp, T))
                 g_xi = g * g_xi
             return g_xi, g * gx, g * gi, None, None
 except ImportError:  # torch is optional for the C ABI users

@@ -134,3 +134,50 @@ def test_autograd_gradcheck_fp64(dev, xi_scale):
     f = lambda a, x, k: BACost.apply(a, x, k, Tt, b)
     assert torch.autograd.gradcheck(f, (xi, Xt, it), eps=1e-6, atol=1e-4, rtol=1e-5)
     b.close()
+
+
+@pytest.mark.parametrize("scale", [0.0, 1e-4, 0.05, 0.28, 0.3, 2.0])
+@pytest.mark.parametrize("n_cam", [2, 64, 65])
+def test_pose_tangent_kernels_match_torch(dev, n_cam, scale):
+    """exp(xi) T_cw and J_l(xi)^T g of the device kernels against `se3_left` and
+    its autograd in double: one pose to one more than a workgroup's, angles on
+    both sides of the series' end (theta = 0.5).  A result is a few dozen FP64
+    operations on terms of order |t| (here below 10), so 1e-12 relative to the
+    largest entry; the reference's own closed forms cancel to about 1e-13 at
+    theta = 0.05.  FP32: one rounding of the FP64 result at its inputs."""
+    from nav24_amd.diffcost import CostBatch, _tangent_grad, se3_left, tangent_to_entry_grad
+    probs = batch_problems(n=1, n_pt=60, n_cam=n_cam)
+    T, X, intr = concat(probs)
+    g = torch.Generator().manual_seed(n_cam)
+    xi = scale * torch.randn(n_cam, 6, generator=g, dtype=torch.float64)
+    gp = torch.randn(n_cam, 6, generator=g, dtype=torch.float64)
+    b = CostBatch(probs)
+    for dt, tol in ((torch.float64, 1e-12), (torch.float32, 2.0 ** -23)):
+        x, t, v = (a.to(dt).double() for a in (xi, torch.tensor(T), gp))  # the inputs the kernel sees
+        args = [a.to(dt).to(dev) for a in (xi, torch.tensor(X), torch.tensor(intr), torch.tensor(T))]
+        total, Td, r = b._eval_tangent(*args, True)
+        ref = se3_left(x, t)
+        assert (Td.double().cpu() - ref).abs().max() <= tol * ref.abs().max()
+        assert abs(total.double().item() - r.cost.double().sum().item()) <= 2.0 ** -22 * total.double().item()
+        y = x.clone().requires_grad_(True)
+        Ty = se3_left(y, t)
+        (want,) = torch.autograd.grad(Ty, y, tangent_to_entry_grad(v, Ty.detach()))
+        got = _tangent_grad(args[0], gp.to(dt).to(dev))
+        assert (got.double().cpu() - want).abs().max() <= 10 * tol * want.abs().max()
+    b.close()
+
+
+def test_backward_after_the_batch_is_closed(dev):
+    """Backward needs nothing of the batch: it may be closed after forward."""
+    from nav24_amd.diffcost import BACost, CostBatch
+    probs = batch_problems(n=1, n_pt=60, n_cam=4)
+    T, X, intr = concat(probs)
+    xi = torch.full((4, 6), 0.01, dtype=torch.float64, device=dev, requires_grad=True)
+    Xt = torch.tensor(X, device=dev, requires_grad=True)
+    it = torch.tensor(intr, device=dev, requires_grad=True)
+    b = CostBatch(probs)
+    (want,) = torch.autograd.grad(BACost.apply(xi, Xt, it, torch.tensor(T, device=dev), b), xi)
+    cost = BACost.apply(xi, Xt, it, torch.tensor(T, device=dev), b)
+    b.close()
+    (got,) = torch.autograd.grad(cost, xi)
+    assert torch.equal(got, want)
