@@ -685,29 +685,36 @@ __global__ __launch_bounds__(256) void k_chol_back_tile(const double* __restrict
 
 // ---------------------------------------------------------------- per-window systems
 // One workgroup (512 threads) per running window, and for a single problem of
-// at most 30 free cameras.  The window's reduced system (n = 6 nb unknowns)
-// is summed from the Schur rows' partials straight into LDS, as a packed lower
-// triangle of 6x6 camera blocks (block (I, J), J <= I, at (I(I+1)/2 + J) * kBS
-// doubles, row-major inside; the odd stride kBS = 37 spreads neighbouring
-// blocks over LDS banks).  Right-looking block Cholesky, per block column K:
-//   panel  L_IK = A_IK M_K^T and y_I -= L_IK y_K, one thread per row of a
-//          block (block row K+1 in the first lanes of wave 0);
-//   next   wave 0: A_{K+1,K+1} -= L_{K+1,K} L_{K+1,K}^T, one entry per lane,
-//          then L = chol(A_{K+1,K+1}), M_{K+1} = L^-1 and y_{K+1} = M_{K+1}
-//          y_{K+1} in registers of lane 0 (1/sqrt by rsq + two Newton steps;
-//          six lanes with a row each measured no faster);
-//   update meanwhile, waves 1..7: A_IJ -= L_IK L_JK^T for the other blocks,
-//          K < J <= I, one thread per 6x6 block (36 register accumulators).
-// Two barriers per block column; the chain through the columns is wave 0's
-// panel rows, its diagonal update and the 6x6 factor.  Backward substitution
-// x_K = M_K^T (y_K - sum_{I>K} L_IK^T x_I) runs block by block in wave 0, with
-// no workgroup barrier; then the window's candidate poses are formed from the
-// step in LDS (the camera update, fused).  A pivot that is not positive and
-// finite marks the window failed (dp = 0, lm.fail = 1), as the tiled path does.
-constexpr int kBS = 37;
+// at most 30 free cameras: the window's reduced system (n = 6 nb unknowns) is
+// summed from the Schur rows' partials straight into LDS, factored there as
+// S = L D L^T (L unit lower, no square roots: a reciprocal's chain is shorter)
+// and solved.  The system lies in LDS as 16x16 tiles of the lower triangle,
+// the operand size of the FP64 matrix instruction; the right-hand side is row n
+// below the matrix, so the forward step is part of the panel solve.
+// Per tile column k, with M_k the inverse of the diagonal tile's unit factor:
+//   solve    W_ik = A_ik M_k^T (= L_ik D_k) for the rows i > k, one tile per
+//            wave at a time;
+//   chain    wave 0: A_{k+1,k+1} -= W D^-1 W^T, then the tile's LDL^T and
+//            M_{k+1} in registers (tile16_ldl);
+//   update   meanwhile, waves 1..7: A_ij -= W_ik D_k^-1 W_jk^T for the other
+//            tiles, k < j <= i.
+// Two barriers per tile column.  The backward step x_k = M_k^T D_k^-1 (z_k -
+// sum_{i>k} W_ik^T x_i) runs over the waves with one barrier per tile column;
+// then the window's candidate poses are formed from the step in LDS (the
+// camera update, fused).  Bound by the chain through the diagonal tiles (four
+// pivots at a time, about 3.3 k cycles per tile) and, in the first columns of
+// a large window, by the updates' matrix instructions.  A pivot that is not
+// positive and finite marks the window failed (dp = 0, lm.fail = 1), as the
+// tiled path does.
+// Measured (rocprofv3, average per launch): one 30-camera window 82 -> 48 us, one
+// 8-camera window 16.4 -> 13.5, 24 windows 80 -> 47, 512 windows 84 -> 51,
+// against a right-looking form in 6x6 blocks on the vector units, one wave
+// factoring a block column per barrier.  Of the 120 k cycles of a 28-camera
+// window the load takes 32 k (one round trip to memory a chunk of the rows), the
+// eleven columns 60 k, the backward step 13 k.
+constexpr int kBS = 37;  // stride of a 6x6 block in LDS (k_chol_blocks)
 constexpr int kSmallThreads = 512;
-
-__device__ __forceinline__ int blk_off(int I, int J) { return (I * (I + 1) / 2 + J) * kBS; }
+constexpr int kSmallWaves = kSmallThreads / kWave;
 
 // Lower-triangular 6x6 Cholesky and inverse of the block at a (row-major 6x6,
 // lower part read), result L written back to a (lower part) and M = L^-1 to m
@@ -770,201 +777,207 @@ __device__ __forceinline__ bool diag_factor(double* a, double* m, double* y) {
     return ok_all;
 }
 
-// Block column C of a window's system in LDS, by one wave: first the update
-// by panel K (A_IC -= L_IK L_CK^T for I >= C; none when K < 0), then its
-// factorisation in registers, one row per lane and slot (rows 6C + lane +
-// 64 q): for each of its six columns j, the pivot l_jj = sqrt(d_j) (1/sqrt by
-// rsq and two Newton steps, kept in dinv), the rows below scaled by 1/l_jj,
-// the forward step y_j = y_j / l_jj and y_r -= l_rj y_j below, and the rank-1
-// update of the column block's later columns; the pivots and multipliers come
-// from lanes 0..5 as wave-uniform values.  The factor L_IC overwrites the
-// column block and y its rows.  Returns false on a pivot that is not
-// positive and finite (replaced by 1), the same in every lane.
-template <int kQ>
-__device__ __forceinline__ bool win_panel_q(double* Lb, double* yv, double* dinv, int n, int C, int K, int lane) {
-    const int r0 = 6 * C;
-    double v[kQ][6], yq[kQ];
-    double u[6][6];  // L_CK, wave-uniform
-    if (K >= 0) {
-#pragma unroll
-        for (int e = 0; e < 36; ++e) u[e / 6][e % 6] = Lb[blk_off(C, K) + e];
+// LDS of one window's system: n rows of the matrix and the right-hand side as
+// row n, in tiles of the lower triangle row by row, the last tile row with
+// only the rows it has; then the reciprocal pivots, the solution and a row of
+// 16 per wave.  Tile rows are 17 doubles apart: 16 lanes reading one row or
+// one column touch 16 bank pairs, and an element's offset stays linear in its
+// indices, so a lane keeps one offset per operand layout and the four elements
+// are immediate offsets (with an exclusive-or swizzle instead, the address
+// arithmetic cost more than the products).  The last tile row is read as if it
+// had 16 rows: what lies behind it belongs to the same buffer, and results of
+// those rows are never stored.
+constexpr int kTileStride = 17;
+constexpr int kTileSize = 16 * kTileStride;
+struct WinTiles {
+    int nt, nc, last, tail;        // tile rows, tile columns, rows of the last tile row, columns of the last tile column
+    int dinv, x, xw, total;        // offsets in doubles
+    __host__ __device__ explicit WinTiles(int n) {
+        nt = (n >> 4) + 1;
+        nc = (n + 15) >> 4;
+        last = (n & 15) + 1;
+        tail = n - 16 * (nc - 1);
+        dinv = kTileSize * (nt * (nt - 1) / 2) + kTileStride * last * nc;
+        dinv += dinv & 1;
+        x = dinv + 16 * nc;
+        xw = x + 16 * nc;
+        total = xw + 16 * kSmallWaves + kTileSize;  // a whole tile may be read from the last one's place
     }
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int r = r0 + lane + 64 * q;
-        yq[q] = 0.0;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) v[q][c] = 0.0;
-        if (r < n) {
-            const int I = r / 6, i = r - 6 * (r / 6);
-            const double* a = Lb + blk_off(I, C) + 6 * i;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) v[q][c] = a[c];
-            yq[q] = yv[r];
-            if (K >= 0) {
-                const double* l = Lb + blk_off(I, K) + 6 * i;
-                double lk[6];
-#pragma unroll
-                for (int m = 0; m < 6; ++m) lk[m] = l[m];
-#pragma unroll
-                for (int c = 0; c < 6; ++c) {
-                    double w = v[q][c];
-#pragma unroll
-                    for (int m = 0; m < 6; ++m) w -= lk[m] * u[c][m];
-                    v[q][c] = w;
-                }
-            }
-        }
+    __device__ __forceinline__ int tile(int i, int j) const {
+        return (kTileSize / 2) * (i * (i + 1)) + (i == nt - 1 ? kTileStride * last : kTileSize) * j;
     }
-    bool ok_all = true;
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        double d = lane_value(v[0][j], j);
-        const bool ok = (d > 0.0) && isfinite(d);
-        ok_all = ok_all && ok;
-        d = ok ? d : 1.0;
-        double rs = __builtin_amdgcn_rsq(d);
-        rs = rs * (1.5 - 0.5 * d * rs * rs);
-        rs = rs * (1.5 - 0.5 * d * rs * rs);
-        const double yj = lane_value(yq[0], j) * rs;
-        // unmasked: a row past n (zero) is never written back, and the diagonal
-        // block's rows (lanes 0..5 of slot 0) take extra operations only above
-        // the diagonal, which nothing reads; only their right-hand side, final
-        // once their own pivot is passed, is masked
-#pragma unroll
-        for (int q = 0; q < kQ; ++q) {
-            v[q][j] *= rs;
-            if (q > 0 || lane > j) yq[q] -= v[q][j] * yj;
-        }
-        if (lane == j) {
-            v[0][j] = d * rs;
-            yq[0] = yj;
-        }
-#pragma unroll
-        for (int c = j + 1; c < 6; ++c) {
-            const double lcj = lane_value(v[0][j], c);
-#pragma unroll
-            for (int q = 0; q < kQ; ++q) v[q][c] -= v[q][j] * lcj;
-        }
-        if (lane == 0) dinv[r0 + j] = rs;
-    }
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) {
-        const int r = r0 + lane + 64 * q;
-        if (r < n) {
-            const int I = r / 6, i = r - 6 * (r / 6);
-            double* a = Lb + blk_off(I, C) + 6 * i;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) a[c] = v[q][c];
-            yv[r] = yq[q];
-        }
-    }
-    return ok_all;
+};
+
+// Reciprocal: the hardware's estimate (relative error e below 2^-24) and one
+// step of third order, r (1 + e + e^2).
+__device__ __forceinline__ double fast_rcp(double d) {
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
-// win_panel_q with as many row slots as block column C has rows (n - 6C).
-__device__ __forceinline__ bool win_panel(double* Lb, double* yv, double* dinv, int n, int C, int K, int lane) {
-    static_assert(kSmallMaxN <= 192, "three row slots of 64 lanes");
-    const int rows = n - 6 * C;
-    if (rows > 128) return win_panel_q<3>(Lb, yv, dinv, n, C, K, lane);
-    if (rows > 64) return win_panel_q<2>(Lb, yv, dinv, n, C, K, lane);
-    return win_panel_q<1>(Lb, yv, dinv, n, C, K, lane);
+// Four products of 4x4 blocks, D_b = A_b B_b (b = 0..3), with A[i][k] in lane
+// i + 4b + 16k, B[k][j] in lane j + 4b + 16k and D[i][j] in lane j + 4b + 16i
+// (checked on gfx950 against a host product).
+__device__ __forceinline__ double mfma4x4x4(double a, double b) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, 0.0, 0, 0, 0);
 }
 
-// Part of one (row, slot) block of a window's reduced system from the Schur
-// rows' partials: NE = 36 entries (the whole block, 16-byte loads chunk by
-// chunk) or NE = 6 (one row of the block, the loads of up to seven chunks in
-// flight at once).  Task index q: block q / (36 / NE), part q % (36 / NE).
-// The chunks of an entry are added in the one-problem reduction's order
-// (k_schur_reduce): in groups of eight into eight partial sums, the rest into
-// the first, combined pairwise.
-template <int NE>
-__device__ __forceinline__ void sum_block_part(const DevProblem& P, const double* __restrict__ spart,
-                                               const double* __restrict__ Hc, double* Lb, const int* srow,
-                                               const int* rcol, const int* rns, const int* rnch,
-                                               const long long* rp0, int nb, int fc0, double lambda, int q) {
-    constexpr int kParts = 36 / NE;
-    const int b = q / kParts, part = q - kParts * (q / kParts);
-    int lo = 0, hi = nb - 1;  // the row: largest lf with srow[lf] <= b
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (srow[mid] <= b) lo = mid; else hi = mid - 1;
-    }
-    const int lf = lo, f = fc0 + lf, s = b - srow[lf];
-    const int nch = rnch[lf];
-    const long long stride = 36LL * rns[lf] + 6;  // doubles; even, so every item is 16-byte aligned
-    const int e0 = NE * part;
-    const double* sp = spart + rp0[lf] + 36 * s + e0;
-    const int lg = s == 0 ? lf : P.colcam[rcol[lf] + s] - fc0;
-    double a[NE];
-    double h[NE];  // the diagonal block's Hpp + lambda I entries, loaded ahead
-    if (nch < 8) {
+// LDL^T of a symmetric 16x16 tile and the inverse of its unit factor, by one
+// wave in registers.  acc holds the tile in the matrix instruction's result
+// layout (element v of lane (i, k) = l & 15, l >> 4: row 4 v + k, column i);
+// by symmetry acc[p] is then the column panel 4p..4p+3 in the layout of an
+// operand (lane (i, k): row i, column 4p + k), so a panel needs no data
+// movement.  Per panel p of four columns:
+//   the 4x4 diagonal block's LDL^T and the inverse N of its unit factor, the
+//     same in every lane from ten lane reads;
+//   W = A_p N^T as four 4x4 blocks, L_p = W D^-1, acc -= W L_p^T;
+//   Z, which starts as the identity and ends as the inverse: Z_p = N Z_p,
+//     Z -= L_p Z_p for the rows below.
+// dv[p] = the reciprocal pivot of column 4p + k in lane (i, k).  Returns false
+// if a pivot was not positive and finite (its values are then arbitrary), the
+// same in every lane.
+// A solve by substitution in 4x4 blocks instead of the inverse was no more
+// accurate over 512 ill-conditioned windows (the same quantiles of the pose and
+// cost errors against the oracle) and 4 us slower on the largest window.
+__device__ __forceinline__ bool tile16_ldl(dbl4 acc, dbl4& Z, double dv[4]) {
+    const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4, i4 = lane & 3;
 #pragma unroll
-        for (int k = 0; k < NE; ++k) {
-            const int i = (e0 + k) / 6, c = (e0 + k) % 6;
-            h[k] = s == 0 ? Hc[28 * (size_t)f + sym6(i, c)] + (i == c ? lambda : 0.0) : 0.0;
-        }
-        // fewer than eight chunks: one partial sum in chunk order, then the
-        // seven empty ones added pairwise
-        const double z = 0.0;
+    for (int v = 0; v < 4; ++v) Z[v] = (4 * v + k == i) ? 1.0 : 0.0;
 #pragma unroll
-        for (int e = 0; e < NE; ++e) a[e] = 0.0;
-        if constexpr (NE == 36) {
-            for (int ch = 0; ch < nch; ++ch) {
-                const double2* p2 = reinterpret_cast<const double2*>(sp + ch * stride);
-                double2 v[18];
-#pragma unroll
-                for (int k = 0; k < 18; ++k) v[k] = p2[k];
-#pragma unroll
-                for (int k = 0; k < 18; ++k) {
-                    a[2 * k] += v[k].x;
-                    a[2 * k + 1] += v[k].y;
-                }
-            }
+    for (int p = 0; p < 4; ++p) {
+        const double a = acc[p];
+        const int q = 4 * p;
+        const double a00 = lane_value(a, q), a10 = lane_value(a, q + 1), a11 = lane_value(a, q + 17),
+                     a20 = lane_value(a, q + 2), a21 = lane_value(a, q + 18), a30 = lane_value(a, q + 3),
+                     a31 = lane_value(a, q + 19), a22 = lane_value(a, q + 34), a32 = lane_value(a, q + 35),
+                     a33 = lane_value(a, q + 51);
+        const double i0 = fast_rcp(a00);
+        const double l10 = a10 * i0, l20 = a20 * i0, l30 = a30 * i0;
+        const double d1 = fma(-l10, a10, a11), t21 = fma(-l20, a10, a21), t31 = fma(-l30, a10, a31);
+        const double i1 = fast_rcp(d1);
+        const double l21 = t21 * i1, l31 = t31 * i1;
+        const double d2 = fma(-l21, t21, fma(-l20, a20, a22)), t32 = fma(-l31, t21, fma(-l30, a20, a32));
+        const double i2 = fast_rcp(d2);
+        const double l32 = t32 * i2;
+        const double d3 = fma(-l32, t32, fma(-l31, t31, fma(-l30, a30, a33)));
+        const double i3 = fast_rcp(d3);
+        // N, unit lower, element (i & 3, k) in lane (i, k)
+        const double n20 = fma(l21, l10, -l20), n31 = fma(l32, l21, -l31);
+        const double n30 = fma(-l32, n20, fma(l31, l10, -l30));
+        double nv = i4 == k ? 1.0 : 0.0;
+        if (i4 == 1 && k == 0) nv = -l10;
+        if (i4 == 2 && k == 0) nv = n20;
+        if (i4 == 2 && k == 1) nv = -l21;
+        if (i4 == 3 && k == 2) nv = -l32;
+        if (i4 == 3 && k == 1) nv = n31;
+        if (i4 == 3 && k == 0) nv = n30;
+        dv[p] = k == 0 ? i0 : k == 1 ? i1 : k == 2 ? i2 : i3;
+        if (p < 3) {
+            const double w = mfma4x4x4(nv, a);  // W[i][k]
+            const double zp = mfma4x4x4(nv, Z[p]);  // row 4p + k, column i of N Z_p
+            const double lp = w * dv[p];
+            acc = mfma16x16x4(-w, lp, acc);
+            Z = mfma16x16x4(i >= q + 4 ? -lp : 0.0, zp, Z);
+            Z[p] = zp;
         } else {
-            double2 v[7][3];
-#pragma unroll
-            for (int ch = 0; ch < 7; ++ch) {
-                const double2* p2 = reinterpret_cast<const double2*>(sp + min(ch, nch - 1) * stride);
-#pragma unroll
-                for (int k = 0; k < 3; ++k) v[ch][k] = p2[k];
-            }
-#pragma unroll
-            for (int ch = 0; ch < 7; ++ch)
-                if (ch < nch)
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        a[2 * k] += v[ch][k].x;
-                        a[2 * k + 1] += v[ch][k].y;
-                    }
+            Z[p] = mfma4x4x4(nv, Z[p]);
         }
-#pragma unroll
-        for (int e = 0; e < NE; ++e) a[e] = ((a[e] + z) + (z + z)) + ((z + z) + (z + z));
-    } else {
-        // eight chunks or more (small chunks of long camera rows): entry by
-        // entry, written as it is summed
-        for (int k = 0; k < NE; ++k) {
-            double w[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) w[u] = 0.0;
-            int ch = 0;
-            for (; ch + 8 <= nch; ch += 8) {
-#pragma unroll
-                for (int u = 0; u < 8; ++u) w[u] += sp[(ch + u) * stride + k];
-            }
-            for (; ch < nch; ++ch) w[0] += sp[ch * stride + k];
-            const double sum = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
-            const int i = (e0 + k) / 6, c = (e0 + k) % 6;
-            if (s == 0) Lb[blk_off(lf, lf) + 6 * i + c] = Hc[28 * (size_t)f + sym6(i, c)] + (i == c ? lambda : 0.0) - sum;
-            else Lb[blk_off(lg, lf) + 6 * c + i] = -sum;
-        }
-        return;
     }
+    bool good = true;
 #pragma unroll
-    for (int k = 0; k < NE; ++k) {
-        const int i = (e0 + k) / 6, c = (e0 + k) % 6;
-        if (s == 0) Lb[blk_off(lf, lf) + 6 * i + c] = h[k] - a[k];
-        else Lb[blk_off(lg, lf) + 6 * c + i] = -a[k];
+    for (int p = 0; p < 4; ++p) good = good && dv[p] > 0.0 && isfinite(dv[p]);
+    return __all(good);
+}
+
+// Sum over the four lanes (i, 0..3), in each of them: row pairs, then halves.
+__device__ __forceinline__ double sum_over_k(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    const auto l1 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h1 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    const double s = __longlong_as_double(((long long)h1[0] << 32) | l1[0]) +
+                     __longlong_as_double(((long long)h1[1] << 32) | l1[1]);
+    const long long c = __double_as_longlong(s);
+    const unsigned lo2 = (unsigned)c, hi2 = (unsigned)(c >> 32);
+    const auto l2 = __builtin_amdgcn_permlane32_swap(lo2, lo2, false, false);
+    const auto h2 = __builtin_amdgcn_permlane32_swap(hi2, hi2, false, false);
+    return __longlong_as_double(((long long)h2[0] << 32) | l2[0]) +
+           __longlong_as_double(((long long)h2[1] << 32) | l2[1]);
+}
+
+// One S row f of the window, by one wave.  Lanes 0..53 take three slots of 18
+// 16-byte pairs at a time, so a lane's entry (i, c), (i, c + 1) of the 6x6
+// block is the same in every step; lanes 54..56 take the three pairs of the
+// right-hand side's coefficient in the first.  NP = steps for the row's slots.
+struct SRow {
+    int lf, ns, nch, cols;  // row, slots, chunks; lane s: window camera of slot s
+    const double* item;     // partial sums of its first chunk; the chunks lie 36 ns + 6 apart
+};
+
+template <int NP>
+__device__ __forceinline__ void row_load(double2 v[NP], const SRow& r, int ch, int lane) {
+    const double2* p = reinterpret_cast<const double2*>(r.item + (size_t)ch * (36 * r.ns + 6));
+    const int i0 = lane < 54 ? lane : 18 * r.ns + min(lane - 54, 2), end = 18 * r.ns + 2;
+    const int step = lane < 54 ? 54 : 0;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) v[u] = p[min(i0 + step * u, end)];
+}
+
+// This lane's two values of the row's Hpp (packed) and b: of its entries of
+// the diagonal block, or of its pair of the coefficient.
+__device__ __forceinline__ double2 row_h(const double* __restrict__ hc, int lane) {
+    const int i = lane / 3, c = 2 * (lane - 3 * i);
+    const int e = lane < 18 ? sym6(i, c) : 21 + 2 * min(max(lane - 54, 0), 2);
+    return double2{hc[e], hc[lane < 18 ? sym6(i, c + 1) : e + 1]};
+}
+
+template <int NP>
+__device__ __forceinline__ void row_add(double2 v[NP], const double2 x[NP]) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        v[u].x += x[u].x;
+        v[u].y += x[u].y;
+    }
+}
+
+// The row's entries of the system's lower triangle from its sums: S_ff = Hpp +
+// lambda I - sum on the diagonal block (slot 0), S_gf = -sum^T below it, g_f =
+// b_f - coefficient in row n.  rowat[3 g + c / 2]: byte offset of row 6 g + c
+// of the system in its first tile, the top bit set in the last tile row (whose
+// tiles are shorter) and kNoRow for the slots that are not stored here: three
+// integer operations a pair find its place, where a closed form took thirty.
+constexpr unsigned kNoRow = 0x40000000u;
+
+template <int NP>
+__device__ __forceinline__ void row_store(const double2 v[NP], const SRow& r, double2 hh, double lambda,
+                                          const WinTiles& L, double* sm, const unsigned* rowat, int n, int lane) {
+    const int so = lane / 18, pr = lane - 18 * so;
+    const int i = pr / 3, c = 2 * (pr - 3 * i);
+    const int C = 6 * r.lf + i, ic = C >> 4, cc = C & 15;
+    const bool diag = lane < 18;
+    if (diag || (lane >= 54 && lane < 57)) {
+        // two neighbours (row, D), (row, D + 1), D even: of the diagonal block, or of row n
+        const int row = diag ? C : n, D = 6 * r.lf + (diag ? c : 2 * (lane - 54)), ir = row >> 4;
+        const int T = (kTileSize / 2) * (ir * (ir + 1)) + (ir == L.nt - 1 ? kTileStride * L.last : kTileSize) * (D >> 4);
+        double* d = sm + T + kTileStride * (row & 15) + (D & 15);
+        if (row >= D) d[0] = hh.x + (row == D ? lambda : 0.0) - v[0].x;
+        if (row > D) d[1] = hh.y + (row == D + 1 ? lambda : 0.0) - v[0].y;
+    }
+    const unsigned full = 8u * (kTileSize * ic + cc), cut = 8u * (kTileStride * L.last * ic + cc) - 0x80000000u;
+    const unsigned spare = 8u * L.xw;  // where the pairs that are not stored go
+    // lane s: the byte offset in rowat of slot s's camera; lanes without a slot, and
+    // slot 0, name the camera past the last one, whose rows are not stored
+    const int g = 12 * ((lane > 0 && lane < r.ns) ? r.cols : kSmallMaxN / 6);
+    const int from = 4 * (lane < 54 ? so : kSmallMaxN / 6), half = 2 * c;
+    const char* at0 = reinterpret_cast<const char*>(rowat);
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        const unsigned at = *reinterpret_cast<const unsigned*>(at0 + (__builtin_amdgcn_ds_bpermute(from + 12 * u, g) + half));
+        const unsigned o = min(at + ((int)at < 0 ? cut : full), spare);
+        double* d = reinterpret_cast<double*>(reinterpret_cast<char*>(sm) + o);
+        d[0] = -v[u].x;
+        d[kTileStride] = -v[u].y;  // the row is even: the next one is in the tile
     }
 }
 
@@ -973,215 +986,335 @@ __global__ __launch_bounds__(kSmallThreads) void k_chol_small(DevProblem P, cons
                                                               double* __restrict__ dp, LMDev* lm,
                                                               const PoseQT* __restrict__ pose, PoseQT* __restrict__ pn,
                                                               CamRT* __restrict__ cn, double* __restrict__ red_scale) {
-    constexpr int kRows = kSmallMaxN / 6;
-    extern __shared__ double sm[];
-    __shared__ double xk[6];
-    __shared__ double ssum[kSmallThreads / 64];
+    static_assert(kSmallMaxN <= 180, "four S rows per wave, of at most 30, 22, 14 and 6 slots");
+    extern __shared__ __align__(16) double sm[];
+    __shared__ double ssum[kSmallWaves];
+    __shared__ unsigned rowat[3 * (kSmallMaxN / 6 + 1)];
     __shared__ int bad;
-    __shared__ int srow[kRows + 1];
-    __shared__ int rcol[kRows], rns[kRows], rnch[kRows];
-    __shared__ long long rp0[kRows];
     const int win = P.win_chol_order[blockIdx.x];
     if (!running(lm, win)) return;
     const int fc0 = P.win_fc0[win];
     const int nb = P.win_fc0[win + 1] - fc0;
     const int n = 6 * nb;
-    const int nblk = nb * (nb + 1) / 2;
-    double* Lb = sm;                      // nblk * kBS
-    double* yv = sm + (size_t)nblk * kBS;  // n: right-hand side, then the step
-    double* dinv = yv + n;                 // n: 1 / l_jj
+    const WinTiles L(n);
     const int g0 = 6 * fc0;
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const int lane = tid & 63, i16 = lane & 15, k4 = lane >> 4;
     const int wid = wave_id();
     const double lambda = lm[win].lambda;
     const int fail0 = lm[win].fail;
+    const int cam0 = P.win_cam0[win], cam1 = P.win_cam0[win + 1];
+    CamIn cin;  // the inputs of this thread's first camera, loaded while the system is solved
     if (nb > 0) {
-    // ---- the window's reduced system, summed from the Schur rows' partials
-    // straight into LDS: per S row f, S_ff = Hpp + lambda I - sum and S_gf =
-    // -sum^T over the row's chunk items, and g_f = bp_f - coefficient, the
-    // same sums in the same order as the one-problem reduction
-    // (k_schur_reduce), so both give the same bits; blocks without
-    // co-visibility stay zero.  A row of at most 30 slots is one column group,
-    // whose chunk items lie back to back (36 doubles per slot, then 6 of the
-    // coefficient).  One thread per block, or per row of a block, sums its
-    // entries (sum_block_part), and one more per row the row's coefficient.
-    for (int i = tid; i < nblk * kBS; i += kSmallThreads) Lb[i] = 0.0;
-    if (wid == 0) {
-        int v = 0;
-        if (lane < nb) {
-            const int f = fc0 + lane;
-            const int c0 = P.colptr[f];
-            v = P.colptr[f + 1] - c0;
-            rcol[lane] = c0;
-            rns[lane] = v;
-            rnch[lane] = P.row_nchunks[f];
-            rp0[lane] = P.row_pofs0[f];
-        }
-        int incl = v;  // slots before each row: a wave prefix sum (nb <= 30 lanes)
+    // ---- the system, summed from the Schur rows' partials.  A row of at most 30
+    // slots is one column group, whose chunk items lie back to back (36 doubles
+    // per slot, then 6).  Wave w takes the rows w, 15 - w, 16 + w and 31 - w
+    // (about the same number of slots for every wave), all four rows' first
+    // chunks in flight at once.  Blocks without co-visibility stay zero.
+    SRow row[4];
 #pragma unroll
-        for (int d = 1; d < 32; d <<= 1) {
-            const int o = __shfl_up(incl, d);
-            if (lane >= d) incl += o;
+    for (int q = 0; q < 4; ++q) {
+        const int lf = q == 0 ? wid : q == 1 ? 15 - wid : q == 2 ? 16 + wid : 31 - wid;
+        row[q] = SRow{lf, 0, 0, 0, spart};
+        if (lf < nb) {
+            const int f = fc0 + lf;
+            const int c0 = P.colptr[f];
+            row[q].ns = P.colptr[f + 1] - c0;
+            row[q].nch = P.row_nchunks[f];
+            row[q].item = spart + P.row_pofs0[f];
+            if (lane < row[q].ns) row[q].cols = P.colcam[c0 + lane] - fc0;
         }
-        if (lane < nb) srow[lane] = incl - v;
-        if (lane == nb - 1) srow[nb] = incl;
-        if (lane == 0) bad = 0;
+    }
+    auto clear = [&]() {  // while the loads are in flight
+        double2* z = reinterpret_cast<double2*>(sm);
+        for (int q = tid; q < L.total / 2; q += kSmallThreads) z[q] = double2{0.0, 0.0};
+        if (tid < 3 * (kSmallMaxN / 6 + 1)) {
+            const int R = 2 * tid, ir = R >> 4;  // row 6 g + c = 2 (3 g + c / 2)
+            const unsigned o = 8u * ((kTileSize / 2) * ir * (ir + 1) + kTileStride * (R & 15));
+            rowat[tid] = R < n ? o | (ir == L.nt - 1 ? 0x80000000u : 0u) : kNoRow;
+        }
+        if (tid == 0) bad = 0;
+        __syncthreads();
+    };
+    const double* hc = Hc + 28 * (size_t)fc0;
+    if (nb <= kSmallWaves) {
+        // one row of at most eight slots per wave: its chunks six at a time
+        constexpr int kCh = 6;
+        double2 v[3], x[kCh][3], h0;
+        if (row[0].ns) {
+            h0 = row_h(hc + 28 * row[0].lf, lane);
+            row_load<3>(v, row[0], 0, lane);
+#pragma unroll
+            for (int u = 0; u < kCh; ++u) row_load<3>(x[u], row[0], min(1 + u, row[0].nch - 1), lane);
+        }
+        clear();
+        if (row[0].ns) {
+            for (int ch = 1; ch < row[0].nch; ch += kCh) {
+#pragma unroll
+                for (int u = 0; u < kCh; ++u)
+                    if (ch + u < row[0].nch) row_add<3>(v, x[u]);
+                if (ch + kCh < row[0].nch)
+#pragma unroll
+                    for (int u = 0; u < kCh; ++u) row_load<3>(x[u], row[0], min(ch + kCh + u, row[0].nch - 1), lane);
+            }
+            row_store<3>(v, row[0], h0, lambda, L, sm, rowat, n, lane);
+        }
+    } else {
+        double2 v0[10], v1[8], v2[5], v3[2], h[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[q] = row_h(hc + 28 * min(row[q].lf, nb - 1), lane);
+        row_load<10>(v0, row[0], 0, lane);  // nb > 8: every wave has this row
+        if (row[1].ns) row_load<8>(v1, row[1], 0, lane);
+        if (row[2].ns) row_load<5>(v2, row[2], 0, lane);
+        if (row[3].ns) row_load<2>(v3, row[3], 0, lane);
+        clear();
+        const int most = max(max(row[0].nch, row[1].nch), max(row[2].nch, row[3].nch));
+        for (int ch = 1; ch < most; ++ch) {
+            {
+                double2 x0[10];
+                if (ch < row[0].nch) {
+                    row_load<10>(x0, row[0], ch, lane);
+                    row_add<10>(v0, x0);
+                }
+            }
+            double2 x1[8], x2[5], x3[2];
+            if (ch < row[1].nch) row_load<8>(x1, row[1], ch, lane);
+            if (ch < row[2].nch) row_load<5>(x2, row[2], ch, lane);
+            if (ch < row[3].nch) row_load<2>(x3, row[3], ch, lane);
+            if (ch < row[1].nch) row_add<8>(v1, x1);
+            if (ch < row[2].nch) row_add<5>(v2, x2);
+            if (ch < row[3].nch) row_add<2>(v3, x3);
+        }
+        row_store<10>(v0, row[0], h[0], lambda, L, sm, rowat, n, lane);
+        if (row[1].ns) row_store<8>(v1, row[1], h[1], lambda, L, sm, rowat, n, lane);
+        if (row[2].ns) row_store<5>(v2, row[2], h[2], lambda, L, sm, rowat, n, lane);
+        if (row[3].ns) row_store<2>(v3, row[3], h[3], lambda, L, sm, rowat, n, lane);
     }
     __syncthreads();
-    const int nslots = srow[nb];
-    // blocks in six row tasks (all chunk loads of a task in flight at once)
-    // where they fit one pass, whole blocks otherwise
-    const bool rows6 = 6 * nslots + nb <= kSmallThreads;
-    const int ntask = rows6 ? 6 * nslots : nslots;
-    if (tid < ntask) {
-        if (rows6) sum_block_part<6>(P, spart, Hc, Lb, srow, rcol, rns, rnch, rp0, nb, fc0, lambda, tid);
-        else sum_block_part<36>(P, spart, Hc, Lb, srow, rcol, rns, rnch, rp0, nb, fc0, lambda, tid);
-    } else if (tid < ntask + nb) {
-        // right-hand side of row lf: g = bp - coefficient, the coefficient of the
-        // row's chunks in four partial sums (chunks congruent mod 4), as the reduction
-        const int lf = tid - ntask, f = fc0 + lf;
-        const int nch = rnch[lf];
-        const long long stride = 36LL * rns[lf] + 6;
-        const double* cq = spart + rp0[lf] + 36 * rns[lf];
-        double bp[6];
+    // the diagonal tiles' upper halves
+    for (int d = wid; d < L.nc; d += kSmallWaves) {
+        double* T = sm + L.tile(d, d);
+        const int rows = d == L.nc - 1 ? L.tail : 16;
 #pragma unroll
-        for (int e = 0; e < 6; ++e) bp[e] = Hc[28 * (size_t)f + 21 + e];
-        double cp[4][6];
+        for (int v = 0; v < 4; ++v) {
+            const int r = 4 * v + k4;
+            if (r > i16 && r < rows) T[kTileStride * i16 + r] = T[kTileStride * r + i16];
+        }
+    }
+    __syncthreads();
+    // ---- factorisation and forward step
+    double* dinv = sm + L.dinv;
+    double* x = sm + L.x;
+    const int nt = L.nt, nc = L.nc, last = L.last;
+    const bool split = nt > nc;  // the right-hand side has a tile row of its own
+    // this lane's places in a tile: operand element (i, 4t + k) at oop + 4t,
+    // result element (4v + k, i) at ores + 4v rows
+    const int oop = kTileStride * i16 + k4, ores = kTileStride * k4 + i16;
+    constexpr int kV = 4 * kTileStride;
+    // a tile row's result; the last one has fewer rows
+    auto put = [&](double* T, const dbl4& r, bool full) {
+        if (full) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+            for (int v = 0; v < 4; ++v) T[v * kV] = r[v];
+        } else {
 #pragma unroll
-            for (int e = 0; e < 6; ++e) cp[q][e] = 0.0;
-        for (int c0 = 0; c0 < nch; c0 += 4) {
-            double w[4][6];
+            for (int v = 0; v < 4; ++v)
+                if (4 * v + k4 < last) T[v * kV] = r[v];
+        }
+    };
+    // wave 0's part of column k: the diagonal tile (updated by column k - 1),
+    // its factor and inverse; M_k takes the tile's place
+    auto chain = [&](int k) {
+        double* T = sm + L.tile(k, k) + ores;
+        dbl4 acc, Z;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const double* p = cq + min(c0 + q, nch - 1) * stride;
+        for (int v = 0; v < 4; ++v) acc[v] = T[v * kV];
+        if (k > 0) {
+            const double* w = sm + L.tile(k, k - 1) + oop;
+            const double* d = dinv + 16 * (k - 1) + k4;
+            double wv[4], dk[4];
 #pragma unroll
-                for (int e = 0; e < 6; ++e) w[q][e] = p[e];
+            for (int t = 0; t < 4; ++t) {
+                wv[t] = w[4 * t];
+                dk[t] = d[4 * t];
             }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (c0 + q < nch)
-#pragma unroll
-                    for (int e = 0; e < 6; ++e) cp[q][e] += w[q][e];
+            for (int t = 0; t < 4; ++t) acc = mfma16x16x4(wv[t] * -dk[t], wv[t], acc);
         }
+        const int rows = k == nc - 1 ? L.tail : 16;
+        if (rows < 16) {
 #pragma unroll
-        for (int e = 0; e < 6; ++e) yv[6 * lf + e] = bp[e] - ((cp[0][e] + cp[1][e]) + (cp[2][e] + cp[3][e]));
-    }
+            for (int v = 0; v < 4; ++v) {
+                const int r = 4 * v + k4;
+                if (r == rows) T[v * kV] = acc[v];  // the right-hand side's row
+                acc[v] = (r < rows && i16 < rows) ? acc[v] : (r == i16 ? 1.0 : 0.0);  // identity past the end
+            }
+        }
+        double dv[4];
+        if (!tile16_ldl(acc, Z, dv) && lane == 0) bad = 1;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (4 * v + k4 < rows) T[v * kV] = Z[v];
+            if (i16 == 0) dinv[16 * k + 4 * v + k4] = dv[v];
+        }
+    };
+    if (wid == 0) chain(0);
     __syncthreads();
-    // ---- factorisation, right-looking by block columns of six.  Wave 0 keeps
-    // the chain: it updates block column C = K+1 with panel K and factors it
-    // in registers (win_panel), while waves 1..7 apply panel K to the block
-    // columns beyond C; one barrier per block column.
-    if (wid == 0 && !win_panel(Lb, yv, dinv, n, 0, -1, lane) && lane == 0) bad = 1;
-    __syncthreads();
-    for (int K = 0; K + 1 < nb; ++K) {
+    for (int k = 0; k < nc; ++k) {
+        // solve: W_ik = A_ik M_k^T in place for the tile rows i > k
+        if (k + 1 + wid < nt) {
+            double m[4];
+            const double* M = sm + L.tile(k, k) + oop;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) m[t] = M[4 * t];
+            for (int i = k + 1 + wid; i < nt; i += kSmallWaves) {
+                double* A = sm + L.tile(i, k);
+                double a[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) a[t] = A[oop + 4 * t];
+                dbl4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc = mfma16x16x4(a[t], m[t], acc);
+                wave_sync();
+                put(A + ores, acc, i < nt - 1);
+            }
+        }
+        __syncthreads();
+        if (k + 1 >= nc) break;
         if (wid == 0) {
-            if (!win_panel(Lb, yv, dinv, n, K + 1, K, lane) && lane == 0) bad = 1;
+            __builtin_amdgcn_s_setprio(3);
+            chain(k + 1);
+            __builtin_amdgcn_s_setprio(0);
         } else {
-            // A_IJ -= L_IK L_JK^T for K+2 <= J <= I by waves 1..7: one 6x6 block
-            // per thread (36 register accumulators) while the blocks outnumber
-            // the threads' sixths, else one block row per thread, so that the
-            // last columns' few blocks do not hold the barrier for a whole
-            // block's 216 products.  Either way each entry subtracts its six
-            // products in the same order.
-            const int rem = nb - K - 2;
-            const int nupd = rem * (rem + 1) / 2;
-            if (6 * nupd > kSmallThreads - 64) {
-                for (int q = tid - 64; q < nupd; q += kSmallThreads - 64) {
-                    // q -> (I, J), column-major from the diagonal
-                    int jj = 0, qq = q, len = rem;
-                    while (qq >= len) { qq -= len; ++jj; --len; }
-                    const int J = K + 2 + jj, I = J + qq;
-                    const double* A = Lb + blk_off(I, K);
-                    const double* B = Lb + blk_off(J, K);
-                    double* C = Lb + blk_off(I, J);
-                    double acc[36];
+            // update of the tiles (i, j), k < j <= i, beyond the chain's: whole tile
+            // rows, the longest first, wave w the rows nt - w and nt - 15 + w; two
+            // tiles at a time
+            double dk[4];
 #pragma unroll
-                    for (int e = 0; e < 36; ++e) acc[e] = C[e];
-                    double bm[36];
+            for (int t = 0; t < 4; ++t) dk[t] = -dinv[16 * k + 4 * t + k4];
+#pragma unroll 1
+            for (int h = 0; h < 2; ++h) {
+                const int i = h ? nt - 15 + wid : nt - wid;
+                if (i < k + 2) continue;
+                const bool full = i < nt - 1;
+                const int jend = min(i, nc - 1), step = full ? kTileSize : kTileStride * last;
+                double a[4];
+                const double* W = sm + L.tile(i, k) + oop;
+                double* C = sm + L.tile(i, k + 1) + ores;
 #pragma unroll
-                    for (int e = 0; e < 36; ++e) bm[e] = B[e];
+                for (int t = 0; t < 4; ++t) a[t] = W[4 * t] * dk[t];
+                int j = k + 1;
+                for (; j < jend; j += 2) {
+                    const double* B0 = sm + L.tile(j, k) + oop;
+                    const double* B1 = sm + L.tile(j + 1, k) + oop;
+                    double b0[4], b1[4];
+                    dbl4 c0, c1;
 #pragma unroll
-                    for (int r = 0; r < 6; ++r) {
-                        double ar[6];
+                    for (int t = 0; t < 4; ++t) b0[t] = B0[4 * t];
 #pragma unroll
-                        for (int m = 0; m < 6; ++m) ar[m] = A[6 * r + m];
+                    for (int v = 0; v < 4; ++v) c0[v] = C[v * kV];
 #pragma unroll
-                        for (int c = 0; c < 6; ++c) {
-                            double v = acc[6 * r + c];
+                    for (int t = 0; t < 4; ++t) b1[t] = B1[4 * t];
 #pragma unroll
-                            for (int m = 0; m < 6; ++m) v -= ar[m] * bm[6 * c + m];
-                            acc[6 * r + c] = v;
-                        }
+                    for (int v = 0; v < 4; ++v) c1[v] = C[step + v * kV];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        c0 = mfma16x16x4(a[t], b0[t], c0);
+                        c1 = mfma16x16x4(a[t], b1[t], c1);
                     }
-#pragma unroll
-                    for (int e = 0; e < 36; ++e) C[e] = acc[e];
+                    put(C, c0, full);
+                    put(C + step, c1, full);
+                    C += 2 * step;
                 }
-            } else if (tid - 64 < 6 * nupd) {
-                const int q = (tid - 64) / 6, r = (tid - 64) - 6 * ((tid - 64) / 6);
-                int jj = 0, qq = q, len = rem;
-                while (qq >= len) { qq -= len; ++jj; --len; }
-                const int J = K + 2 + jj, I = J + qq;
-                const double* A = Lb + blk_off(I, K) + 6 * r;
-                const double* B = Lb + blk_off(J, K);
-                double* C = Lb + blk_off(I, J) + 6 * r;
-                double ar[6], acc[6];
+                if (j == jend) {
+                    const double* B0 = sm + L.tile(j, k) + oop;
+                    double b0[4];
+                    dbl4 c0;
 #pragma unroll
-                for (int m = 0; m < 6; ++m) ar[m] = A[m];
+                    for (int t = 0; t < 4; ++t) b0[t] = B0[4 * t];
 #pragma unroll
-                for (int c = 0; c < 6; ++c) acc[c] = C[c];
+                    for (int v = 0; v < 4; ++v) c0[v] = C[v * kV];
 #pragma unroll
-                for (int c = 0; c < 6; ++c) {
-                    double v = acc[c];
-#pragma unroll
-                    for (int m = 0; m < 6; ++m) v -= ar[m] * B[6 * c + m];
-                    acc[c] = v;
+                    for (int t = 0; t < 4; ++t) c0 = mfma16x16x4(a[t], b0[t], c0);
+                    put(C, c0, full);
                 }
-#pragma unroll
-                for (int c = 0; c < 6; ++c) C[c] = acc[c];
             }
         }
         __syncthreads();
     }
+    if (cam0 + tid < cam1) cin = camera_inputs(P, pose, Hc, cam0 + tid);
     if (bad) {
-        for (int i = tid; i < n; i += kSmallThreads) dp[g0 + i] = 0.0;
+        for (int q = tid; q < n; q += kSmallThreads) dp[g0 + q] = 0.0;
         if (tid == 0) lm[win].fail = 1;
-    } else if (wid == 0) {
-        // backward, by wave 0 alone: x_K = L_KK^-T (y_K - sum_{I>K} L_IK^T x_I),
-        // the 6x6 solve in lane 0; y holds the updated right-hand sides, then the step
-        for (int K = nb - 1; K >= 0; --K) {
-            if (lane == 0) {
-                const double* L = Lb + blk_off(K, K);
-                double x[6];
+    } else {
+        // ---- backward step.  The solved right-hand side z = D^-1 of row n; its part
+        // in the last diagonal tile (whose inverse lies above it) is solved here.
+        const double* yrow = sm + L.tile(nt - 1, 0) + kTileStride * (last - 1);
+        const int ystep = kTileStride * last;
+        for (int q = tid; q < 16 * (split ? nc : nc - 1); q += kSmallThreads)
+            x[q] = yrow[(q >> 4) * ystep + (q & 15)] * dinv[q];
+        if (!split && wid == kSmallWaves - 1) {
+            const double* M = sm + L.tile(nc - 1, nc - 1) + oop;
+            const double* y = yrow + (nc - 1) * ystep + k4;
+            double p = 0.0;
 #pragma unroll
-                for (int i = 5; i >= 0; --i) {
-                    double v = yv[6 * K + i];
+            for (int t = 0; t < 4; ++t) p = fma(M[4 * t], 4 * t + k4 < L.tail ? y[4 * t] : 0.0, p);
+            p = sum_over_k(p);
+            if (k4 == 0) x[16 * (nc - 1) + i16] = i16 < L.tail ? p * dinv[16 * (nc - 1) + i16] : 0.0;
+        }
+        __syncthreads();
+        // Every wave forms x_k = M_k^T s_k (the same values) and then updates its
+        // share to the left, s_j -= D_j^-1 W_kj^T x_k: four products per lane, summed
+        // over the lanes of a column.  At most two tiles a wave; everything but s_k is
+        // loaded ahead of x_k.
+        static_assert(kSmallMaxN <= 16 * (2 * kSmallWaves + 1), "two tiles to the left per wave");
+        double* xk = sm + L.xw + 16 * wid;
+        double m[4];
 #pragma unroll
-                    for (int k = i + 1; k < 6; ++k) v -= L[6 * k + i] * x[k];
-                    x[i] = v * dinv[6 * K + i];
-                }
+        for (int t = 0; t < 4; ++t) m[t] = 4 * t + k4 < L.tail ? sm[L.tile(nc - 1, nc - 1) + ores + t * kV] : 0.0;
+        for (int k = nc - 1; k >= 0; --k) {
+            const int rows = k == nc - 1 ? L.tail : 16;
+            double s4[4], w[2][4], xd[2], dd[2];
 #pragma unroll
-                for (int i = 0; i < 6; ++i) {
-                    xk[i] = x[i];
-                    yv[6 * K + i] = x[i];
-                    dp[g0 + 6 * K + i] = x[i];
-                }
+            for (int t = 0; t < 4; ++t) s4[t] = x[16 * k + 4 * t + k4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int j = min(wid + kSmallWaves * h, k);
+                const double* W = sm + L.tile(k, j) + ores;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) w[h][t] = 4 * t + k4 < rows ? W[t * kV] : 0.0;
+                xd[h] = x[16 * j + i16];
+                dd[h] = dinv[16 * j + i16];
+            }
+            double p = sum_over_k(fma(s4[0], m[0], s4[1] * m[1]) + fma(s4[2], m[2], s4[3] * m[3]));
+            p = i16 < rows ? p : 0.0;
+            if (k4 == 0) xk[i16] = p;
+            if (k > 0) {  // the next step's inverse
+                const double* M = sm + L.tile(k - 1, k - 1) + ores;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) m[t] = M[t * kV];
             }
             wave_sync();
-            for (int t = lane; t < 6 * K; t += 64) {
-                const int J = t / 6, c = t - 6 * (t / 6);
-                const double* L = Lb + blk_off(K, J);
-                double v = 0.0;
+            double xs[4];
 #pragma unroll
-                for (int r = 0; r < 6; ++r) v += L[6 * r + c] * xk[r];
-                yv[t] -= v;
+            for (int t = 0; t < 4; ++t) xs[t] = xk[4 * t + k4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int j = wid + kSmallWaves * h;
+                if (j >= k) continue;
+                const double u = sum_over_k(fma(xs[0], w[h][0], xs[1] * w[h][1]) + fma(xs[2], w[h][2], xs[3] * w[h][3]));
+                if (k4 == 0) x[16 * j + i16] = fma(-u, dd[h], xd[h]);
             }
-            wave_sync();
+            __syncthreads();  // s_k has been read by every wave, s_j (j < k) updated
+            if (wid == 0 && k4 == 0 && i16 < rows) {
+                x[16 * k + i16] = p;
+                dp[g0 + 16 * k + i16] = p;
+            }
         }
     }
-    }  // nb > 0
+    } else if (cam0 + tid < cam1) {
+        cin = camera_inputs(P, pose, Hc, cam0 + tid);
+    }
     __syncthreads();
     // candidate poses of the window's cameras from the step in LDS, and their
     // part of x'(lambda x + b): the camera update (k_update_cam), with the same
@@ -1189,16 +1322,15 @@ __global__ __launch_bounds__(kSmallThreads) void k_chol_small(DevProblem P, cons
     const int fail = (nb > 0 && bad) ? 1 : fail0;
     double sc = 0.0;
     if (tid < 256)
-        for (int c = P.win_cam0[win] + tid; c < P.win_cam0[win + 1]; c += 256)
-            sc += camera_candidate(camera_inputs(P, pose, Hc, c), lambda, fail, c,
-                                   [&](int f, int i) { return yv[6 * (f - fc0) + i]; }, pn, cn);
+        for (int c = cam0 + tid; c < cam1; c += 256)
+            sc += camera_candidate(c == cam0 + tid ? cin : camera_inputs(P, pose, Hc, c), lambda, fail, c,
+                                   [&](int f, int i) { return sm[L.x + 6 * (f - fc0) + i]; }, pn, cn);
     const double s = block_sum<double, 256>(sc, ssum);
     if (tid == 0) red_scale[win] = s;
 }
 
 size_t cholesky_small_smem(const DevProblem& P) {
-    const size_t nb = (size_t)P.max_win_fc;
-    return sizeof(double) * (nb * (nb + 1) / 2 * kBS + 12 * nb);
+    return sizeof(double) * (size_t)WinTiles(std::max(6 * P.max_win_fc, 6)).total;
 }
 
 // One workgroup per window, largest windows first: with the largest window's
