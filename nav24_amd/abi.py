@@ -213,3 +213,46 @@ class ResultBuffers:
         return Result(self.T_cw, self.X, self.outlier, self.cost_history[: c.iterations + 1],
                       c.iterations, c.trials, c.stop_reason, c.n_outliers, c.initial_cost,
                       c.final_cost, c.final_lambda, c.solve_ms, status)
+
+
+# nav_ba_result as a numpy record (its pointers as integers)
+_RESULT_RECORD = np.dtype({
+    "names": [n for n, _ in NavBaResult._fields_],
+    "formats": [{C.c_int32: np.int32, C.c_double: np.float64}.get(t, np.uint64) for _, t in NavBaResult._fields_],
+    "offsets": [getattr(NavBaResult, n).offset for n, _ in NavBaResult._fields_],
+    "itemsize": C.sizeof(NavBaResult)})
+
+
+class BatchResultBuffers:
+    """Output arrays for the nav_ba_results of a batch: one allocation per kind
+    of output, of which every window's result holds its part."""
+
+    def __init__(self, windows, n_iter: int):
+        n = len(windows)
+        first = np.zeros((n + 1, 3), np.int64)
+        if n:
+            np.cumsum([(w.n_cam, w.n_pt, w.n_obs) for w in windows], axis=0, out=first[1:])
+        self._first = first
+        n_cam, n_pt, n_obs = (int(v) for v in first[-1])
+        self.T_cw = np.empty((n_cam, 12), np.float64)
+        self.X = np.empty((n_pt, 3), np.float64)
+        self.outlier = np.empty(n_obs, np.uint8)
+        self.cost_history = np.full((n, max(n_iter, 0) + 1), np.nan, np.float64)
+        self._rec = np.zeros(n, _RESULT_RECORD)
+        self._rec["T_cw"] = self.T_cw.ctypes.data + 96 * first[:-1, 0]
+        self._rec["X"] = self.X.ctypes.data + 24 * first[:-1, 1]
+        self._rec["outlier"] = self.outlier.ctypes.data + first[:-1, 2]
+        self._rec["cost_history"] = self.cost_history.ctypes.data + self.cost_history.strides[0] * np.arange(n)
+        self.c = (NavBaResult * n).from_buffer(self._rec)
+
+    def results(self):
+        """One Result per window."""
+        first = self._first.tolist()
+        stats = self._rec[["iterations", "trials", "stop_reason", "n_outliers", "initial_cost", "final_cost",
+                           "final_lambda", "solve_ms"]].tolist()
+        out = []
+        for w, s in enumerate(stats):
+            (c0, p0, o0), (c1, p1, o1) = first[w], first[w + 1]
+            out.append(Result(self.T_cw[c0:c1], self.X[p0:p1], self.outlier[o0:o1], self.cost_history[w, :s[0] + 1], *s,
+                              NAV_BA_EMPTY if s[2] == NAV_BA_STOP_EMPTY else NAV_BA_OK))
+        return out

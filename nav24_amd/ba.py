@@ -16,7 +16,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 
 from ._loader import load_library
-from .abi import (NAV_BA_EMPTY, NAV_BA_OK, NAV_BA_STOP_EMPTY, STATUS_NAMES, NavBaOptions, NavBaProblem, NavBaResult,
+from .abi import (NAV_BA_EMPTY, NAV_BA_OK, STATUS_NAMES, BatchResultBuffers, NavBaOptions, NavBaProblem, NavBaResult,
                   Options, Problem, Result, ResultBuffers)
 
 _dp = C.POINTER(C.c_double)
@@ -177,17 +177,13 @@ class GraphOptimHip:
         arr = (NavBaProblem * len(windows))(*[w.c_struct() for w in windows])
         return arr, opts.c_struct()
 
-    def _results(self, windows: Sequence[Problem], n_iter: int):
-        bufs = [ResultBuffers(w, n_iter) for w in windows]
-        return bufs, (NavBaResult * len(windows))(*[b.c for b in bufs])
-
     def solve_batched(self, windows: Sequence[Problem], opts: Options) -> List[Result]:
         """One GraphOptim::solve per window, all windows in one device solve."""
         arr, os_ = self._batch(windows, opts)
-        bufs, res = self._results(windows, opts.n_iter)
-        st = lib().nav_ba_solve_batched(self._h, arr, len(windows), C.byref(os_), res)
+        bufs = BatchResultBuffers(windows, opts.n_iter)
+        st = lib().nav_ba_solve_batched(self._h, arr, len(windows), C.byref(os_), bufs.c)
         self._check(st, allow_empty=True)
-        return [self._window_result(b, res[i]) for i, b in enumerate(bufs)]
+        return bufs.results()
 
     def prepare_batched(self, windows: Sequence[Problem], opts: Options) -> None:
         arr, os_ = self._batch(windows, opts)
@@ -197,16 +193,10 @@ class GraphOptimHip:
 
     def fetch_batched(self) -> List[Result]:
         windows = self._prob
-        bufs, res = self._results(windows, self._opts.n_iter)
-        st = lib().nav_ba_fetch_batched(self._h, res, len(windows))
+        bufs = BatchResultBuffers(windows, self._opts.n_iter)
+        st = lib().nav_ba_fetch_batched(self._h, bufs.c, len(windows))
         self._check(st, allow_empty=True)
-        return [self._window_result(b, res[i]) for i, b in enumerate(bufs)]
-
-    @staticmethod
-    def _window_result(b: ResultBuffers, c: NavBaResult) -> Result:
-        b.c = c
-        st = NAV_BA_EMPTY if c.stop_reason == NAV_BA_STOP_EMPTY else NAV_BA_OK
-        return b.result(st)
+        return bufs.results()
 
     def set_timing(self, enable: bool) -> None:
         """Stage-by-stage launches with HIP events around each stage (no graphs)."""

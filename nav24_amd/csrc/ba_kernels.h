@@ -192,6 +192,19 @@ struct DevWork {
     PcgState* pcg_st;
 };
 
+// Offsets in bytes of a solve's results in one buffer: poses [n_cam][12],
+// points [n_pt][3] and flags [n_obs], all windows' in caller order end to end.
+struct ResultPlaces {
+    size_t T, X, flags, total;
+    long long n_cam, n_pt, n_obs;
+    ResultPlaces(size_t cams, size_t pts, size_t obs) : n_cam(cams), n_pt(pts), n_obs(obs) {
+        T = 0;
+        X = T + sizeof(double) * 12 * cams;
+        flags = (X + sizeof(double) * 3 * pts + 15) & ~(size_t)15;
+        total = flags + ((obs + 15) & ~(size_t)15);
+    }
+};
+
 __device__ __forceinline__ bool needs_lin(const LMDev* lm, int w) { return lm[w].phase == kPhaseLin; }
 __device__ __forceinline__ bool running(const LMDev* lm, int w) { return lm[w].phase != kPhaseDone; }
 
@@ -310,5 +323,10 @@ void launch_lm_set_chi(const DevProblem& P, const DevWork& W, hipStream_t st);
 void launch_commit(const DevProblem& P, const DevState& cur, const DevState& cand, const DevWork& W, hipStream_t st);
 void launch_flags(const DevProblem& P, const DevState& s, const DevWork& W, double thr, hipStream_t st);
 void launch_final(const DevProblem& P, const DevWork& W, hipStream_t st);
+// The results in caller order into `out` (device-visible host memory): pt_src
+// the local point of each caller point, or -1 (then the caller's own, from x_in);
+// compat rounds the points to float.
+void launch_results(const DevProblem& P, const DevState& cur, const DevWork& W, const int* pt_src, const double* x_in,
+                    const ResultPlaces& at, bool compat, char* out, hipStream_t st);
 
 }  // namespace navba

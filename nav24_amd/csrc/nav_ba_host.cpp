@@ -22,6 +22,7 @@
 #include <mutex>
 #include <queue>
 #include <string>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -53,6 +54,12 @@ constexpr int kTuneChunks[] = {128, 256, 512, 1024, 2048, 4096};
 constexpr int kTuneReps = 3;
 constexpr float kTuneNear = 1.05f;
 constexpr float kTuneMargin = 0.95f;
+
+// fetch: result bytes from which a few host threads copy to the caller's arrays
+// (below, the copy takes less than the threads' start; 512 windows, 40 MB, are
+// fetched in 2.7 ms, against 28.8 with copies in device order and one thread)
+constexpr size_t kFetchThreadBytes = 4 << 20;
+constexpr int kFetchThreads = 8;
 
 struct DevBuf {
     void* p = nullptr;
@@ -102,8 +109,9 @@ struct StageTimer {
 struct WinHost {
     int n_cam = 0, n_pt = 0, n_obs = 0;
     int cam0 = 0, pt_local0 = 0, pt_local1 = 0, obs0 = 0;  // ranges in the concatenated problem
+    size_t pt0 = 0;                // first of this window's caller points in the concatenated caller order
     std::vector<int> pt_orig;      // local point -> caller point index of this window
-    std::vector<double> X_in, T_in;
+    std::vector<double> X_in, T_in;  // an empty window's state, returned as it came
     bool empty = false;
 };
 
@@ -134,6 +142,7 @@ struct HostLayout {
     std::vector<WinHost> win;
     std::vector<int> cam_off, obs_off, pt_first, cam_win, pt_win;
     std::vector<int> o_cam, o_pt, o_orig, pt_ptr;
+    std::vector<int> pt_src;   // concatenated caller point -> local point, or -1 without observations
     std::vector<double> o_uv;
     std::vector<uint8_t> pt_free;
     std::vector<int> cam_free, free_cam, win_fc0, win_cam0;
@@ -201,6 +210,12 @@ struct nav_ba_handle {
     // prepare; a prepare with the same key only uploads the new state
     std::vector<char> prep_key;
     bool prep_cached = false;  // the last prepare took the cached index
+    // results: the points' sources and, where some have no observation, the
+    // caller's points; a pinned buffer that fetch's kernel writes in caller order
+    const int* pt_src = nullptr;
+    double* x_in = nullptr;
+    char* rbuf = nullptr;
+    size_t rbuf_cap = 0;
     // results of the last run
     bool ran = false;
     std::vector<LMDev> lm_out;
@@ -315,16 +330,6 @@ void host_quat_from_R(const double* R, double q[4]) {
     if (q[3] < 0) { q[0] = -q[0]; q[1] = -q[1]; q[2] = -q[2]; q[3] = -q[3]; }
     const double n = std::sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
     q[0] /= n; q[1] /= n; q[2] /= n; q[3] /= n;
-}
-
-void host_R_from_quat(const double q[4], double R[9]) {
-    const double tx = 2 * q[0], ty = 2 * q[1], tz = 2 * q[2];
-    const double twx = tx * q[3], twy = ty * q[3], twz = tz * q[3];
-    const double txx = tx * q[0], txy = ty * q[0], txz = tz * q[0];
-    const double tyy = ty * q[1], tyz = tz * q[1], tzz = tz * q[2];
-    R[0] = 1 - (tyy + tzz); R[1] = txy - twz;       R[2] = txz + twy;
-    R[3] = txy + twz;       R[4] = 1 - (txx + tzz); R[5] = tyz - twx;
-    R[6] = txz - twy;       R[7] = tyz + twx;       R[8] = 1 - (txx + tyy);
 }
 
 inline double rf32(double v) { return (double)(float)v; }
@@ -906,6 +911,22 @@ int check_args(const nav_ba_problem* probs, int n_win, const nav_ba_options* o, 
     return NAV_BA_OK;
 }
 
+// An empty window's state, which fetch returns unchanged.
+void keep_input(WinHost& wh, const nav_ba_problem& p) {
+    wh.T_in.assign(p.T_cw, p.T_cw + 12 * (size_t)p.n_cam);
+    wh.X_in.assign(p.X, p.X + 3 * (size_t)p.n_pt);
+}
+
+// The caller's points end to end, where some of them have no observation (they
+// are returned as they came); nothing otherwise.
+std::vector<double> unobserved_input(const HostLayout& L, const nav_ba_problem* probs) {
+    std::vector<double> x;
+    if (L.pt_src.size() == (size_t)L.np) return x;
+    x.reserve(3 * L.pt_src.size());
+    for (int w = 0; w < L.n_win; ++w) x.insert(x.end(), probs[w].X, probs[w].X + 3 * (size_t)probs[w].n_pt);
+    return x;
+}
+
 // The graph build of BE_GraphOptim.cpp:79-211 as flat arrays (arguments
 // already checked).  NAV_BA_OK or NAV_BA_TOO_LARGE with its message.
 int build_layout(const nav_ba_problem* probs, int n_win, const nav_ba_options* o, bool batched, HostLayout& L,
@@ -935,8 +956,7 @@ int build_layout(const nav_ba_problem* probs, int n_win, const nav_ba_options* o
         WinHost& wh = L.win[w];
         wh.n_cam = p.n_cam; wh.n_pt = p.n_pt; wh.n_obs = p.n_obs;
         wh.cam0 = L.cam_off[w]; wh.obs0 = L.obs_off[w];
-        wh.T_in.assign(p.T_cw, p.T_cw + 12 * (size_t)p.n_cam);
-        wh.X_in.assign(p.X, p.X + 3 * (size_t)p.n_pt);
+        wh.pt0 = L.pt_src.size();
         for (int c = 0; c < p.n_cam; ++c) L.cam_win[L.cam_off[w] + c] = w;
         std::vector<int> cnt(p.n_pt, 0), loc(p.n_pt, -1);
         for (int i = 0; i < p.n_obs; ++i) cnt[p.obs_pt[i]]++;
@@ -945,6 +965,8 @@ int build_layout(const nav_ba_problem* probs, int n_win, const nav_ba_options* o
             if (cnt[i] > 0) { loc[i] = np++; wh.pt_orig.push_back(i); L.pt_win.push_back(w); }
         wh.pt_local1 = np;
         wh.empty = (p.n_cam == 0 || wh.pt_orig.empty());
+        L.pt_src.insert(L.pt_src.end(), loc.begin(), loc.end());
+        if (wh.empty) keep_input(wh, p);
         any = any || !wh.empty;
         for (int i = 0; i < p.n_obs; ++i) {
             g_cam[L.obs_off[w] + i] = L.cam_off[w] + p.obs_cam[i];
@@ -1329,8 +1351,7 @@ int refresh_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     const bool compat = o->compat_fp32_io != 0;
     for (int w = 0; w < n_win; ++w) {
         const nav_ba_problem& p = probs[w];
-        L.win[w].T_in.assign(p.T_cw, p.T_cw + 12 * (size_t)p.n_cam);
-        L.win[w].X_in.assign(p.X, p.X + 3 * (size_t)p.n_pt);
+        if (L.win[w].empty) keep_input(L.win[w], p);
         // a window's observations are contiguous in point-major order
         for (int k = L.pt_ptr[L.pt_first[w]]; k < L.pt_ptr[L.pt_first[w + 1]]; ++k) {
             const double* uv = p.obs_uv + 2 * (size_t)(L.o_orig[k] - L.obs_off[w]);
@@ -1356,7 +1377,9 @@ int refresh_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     // through the pinned staging of the first prepare (it held these arrays and more)
     const size_t b_ouv = sizeof(double) * L.o_uv.size(), b_cuv = sizeof(double) * L.c_uv.size();
     const size_t b_pose = sizeof(PoseQT) * L.pose0.size(), b_x = sizeof(D4) * L.X0.size();
-    const size_t need = b_ouv + b_cuv + b_pose + b_x;
+    const std::vector<double> xin = unobserved_input(L, probs);
+    const size_t b_xin = sizeof(double) * xin.size();
+    const size_t need = b_ouv + b_cuv + b_pose + b_x + b_xin;
     if (h->stage_cap < need) {
         if (h->stage) (void)hipHostFree(h->stage);
         h->stage = nullptr;
@@ -1374,6 +1397,10 @@ int refresh_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     if (b_cuv) HIPTRY(h, hipMemcpyAsync((void*)h->P.c_uv, sp + b_ouv, b_cuv, hipMemcpyHostToDevice, s));
     HIPTRY(h, hipMemcpyAsync(h->init.pose, sp + b_ouv + b_cuv, b_pose, hipMemcpyHostToDevice, s));
     HIPTRY(h, hipMemcpyAsync(h->init.X, sp + b_ouv + b_cuv + b_pose, b_x, hipMemcpyHostToDevice, s));
+    if (b_xin) {
+        std::memcpy(sp + b_ouv + b_cuv + b_pose + b_x, xin.data(), b_xin);
+        HIPTRY(h, hipMemcpyAsync(h->x_in, sp + b_ouv + b_cuv + b_pose + b_x, b_xin, hipMemcpyHostToDevice, s));
+    }
     HIPTRY(h, hipStreamSynchronize(s));
     h->ran = false;
     h->prepared = true;
@@ -1460,8 +1487,13 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     UP(P.win_pt0, L.win_pt0); UP(P.win_S, L.win_S); UP(P.win_lda, L.win_lda);
     UP(P.cblk_o0, L.cblk_o0); UP(P.cblk_win, L.cblk_win); UP(P.win_cblk0, L.win_cblk0);
     UP(P.win_tile0, L.win_tile0); UP(P.win_chol_order, L.win_chol_order);
+    UP(h->pt_src, L.pt_src);
+    const std::vector<double> xin = unobserved_input(L, probs);
+    const double* xin_dev = nullptr;
+    UP(xin_dev, xin);
 #undef UP
     if ((st = pk.flush(h)) != NAV_BA_OK) return st;
+    h->x_in = const_cast<double*>(xin_dev);
     P.n_tiles = (int)L.tile_win.size();
     P.n_hitems = (int)L.hf.size();
     P.n_win = n_win;
@@ -1539,8 +1571,8 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     return NAV_BA_OK;
 }
 
-int fetch_window(nav_ba_handle* h, int w, const std::vector<PoseQT>& pose, const std::vector<D4>& X,
-                 const std::vector<uint8_t>& flags, nav_ba_result* r) {
+// Window w's statistics (its arrays are copied by copy_window).
+int fetch_window(nav_ba_handle* h, int w, nav_ba_result* r) {
     const WinHost& wh = h->layout.win[w];
     r->solve_ms = h->solve_ms;
     if (wh.empty || h->all_empty) {
@@ -1562,55 +1594,57 @@ int fetch_window(nav_ba_handle* h, int w, const std::vector<PoseQT>& pose, const
     r->final_lambda = L.lambda;
     if (r->cost_history)
         for (int i = 0; i <= L.iter; ++i) r->cost_history[i] = hist[i];
-    if (r->T_cw)
-        for (int c = 0; c < wh.n_cam; ++c) {
-            const PoseQT& q = pose[wh.cam0 + c];
-            double* T = r->T_cw + 12 * (size_t)c;
-            host_R_from_quat(q.q, T);  // BE_GraphOptim.cpp:220-223
-            T[9] = q.t[0]; T[10] = q.t[1]; T[11] = q.t[2];
-        }
-    if (r->X) {
-        std::memcpy(r->X, wh.X_in.data(), sizeof(double) * 3 * (size_t)wh.n_pt);
-        const bool compat = h->opt.compat_fp32_io != 0;
-        for (int q = wh.pt_local0; q < wh.pt_local1; ++q) {
-            double* o = r->X + 3 * (size_t)wh.pt_orig[q - wh.pt_local0];
-            o[0] = compat ? rf32(X[q].x) : X[q].x;  // estimate().cast<float>() (BE_GraphOptim.cpp:239)
-            o[1] = compat ? rf32(X[q].y) : X[q].y;
-            o[2] = compat ? rf32(X[q].z) : X[q].z;
-        }
-    }
-    if (r->outlier && wh.n_obs > 0) std::memcpy(r->outlier, flags.data() + wh.obs0, (size_t)wh.n_obs);
     return NAV_BA_OK;
+}
+
+// Window w's poses, points and flags from the pinned result buffer.
+void copy_window(const nav_ba_handle* h, int w, const ResultPlaces& at, const nav_ba_result& r) {
+    const WinHost& wh = h->layout.win[w];
+    if (wh.empty) return;
+    if (r.T_cw) std::memcpy(r.T_cw, (const double*)(h->rbuf + at.T) + 12 * (size_t)wh.cam0, sizeof(double) * 12 * wh.n_cam);
+    if (r.X) std::memcpy(r.X, (const double*)(h->rbuf + at.X) + 3 * wh.pt0, sizeof(double) * 3 * (size_t)wh.n_pt);
+    if (r.outlier && wh.n_obs > 0) std::memcpy(r.outlier, h->rbuf + at.flags + wh.obs0, (size_t)wh.n_obs);
 }
 
 int fetch_all(nav_ba_handle* h, nav_ba_result* results, int n) {
     if (!h || !results) return NAV_BA_BAD_ARG;
     if (!h->prepared || !h->ran) return fail(h, NAV_BA_NOT_PREPARED, "fetch before nav_ba_run");
     if (n != (int)h->layout.win.size()) return fail(h, NAV_BA_BAD_ARG, "result count differs from the prepared window count");
-    std::vector<PoseQT> pose;
-    std::vector<D4> X, X1;
-    std::vector<uint8_t> flags;
-    if (!h->all_empty) {
-        HIPTRY(h, hipSetDevice(h->device));
-        pose.resize(h->P.n_cam);
-        X.resize(h->P.n_pt);
-        X1.resize(h->P.n_pt);
-        flags.resize(h->P.n_obs);
-        HIPTRY(h, hipMemcpyAsync(pose.data(), h->cur.pose, sizeof(PoseQT) * pose.size(), hipMemcpyDeviceToHost, h->stream));
-        HIPTRY(h, hipMemcpyAsync(X.data(), h->P.xb0, sizeof(D4) * X.size(), hipMemcpyDeviceToHost, h->stream));
-        HIPTRY(h, hipMemcpyAsync(X1.data(), h->P.xb1, sizeof(D4) * X1.size(), hipMemcpyDeviceToHost, h->stream));
-        if (!flags.empty())
-            HIPTRY(h, hipMemcpyAsync(flags.data(), h->W.outlier, flags.size(), hipMemcpyDeviceToHost, h->stream));
-        HIPTRY(h, hipStreamSynchronize(h->stream));
-        // each window's current points from the state buffer its LM state names
-        for (int q = 0; q < h->P.n_pt; ++q)
-            if (h->lm_out[h->layout.pt_win[q]].xsel) X[q] = X1[q];
-    }
     int worst = NAV_BA_OK;
     for (int w = 0; w < n; ++w) {
-        const int st = fetch_window(h, w, pose, X, flags, &results[w]);
+        const int st = fetch_window(h, w, &results[w]);
         if (st != NAV_BA_OK) worst = st;
     }
+    if (h->all_empty) return worst;
+    // poses, points and flags in caller order, written by one kernel straight into
+    // pinned memory: no copies in device order (each through a staging buffer of
+    // the runtime) and no reordering on the host
+    HIPTRY(h, hipSetDevice(h->device));
+    const ResultPlaces at(h->P.n_cam, h->layout.pt_src.size(), h->P.n_obs);
+    if (h->rbuf_cap < at.total) {
+        if (h->rbuf) (void)hipHostFree(h->rbuf);
+        h->rbuf = nullptr;
+        h->rbuf_cap = 0;
+        HIPTRY(h, hipHostMalloc((void**)&h->rbuf, at.total, hipHostMallocDefault));
+        h->rbuf_cap = at.total;
+    }
+    launch_results(h->P, h->cur, h->W, h->pt_src, h->x_in, at, h->opt.compat_fp32_io != 0, h->rbuf, h->stream);
+    HIPTRY(h, hipGetLastError());
+    HIPTRY(h, hipStreamSynchronize(h->stream));
+    // the copies to the caller's arrays fault their pages in: a few threads where
+    // that is megabytes
+    const int nth = at.total >= kFetchThreadBytes ? std::min(kFetchThreads, n) : 1;
+    std::vector<std::thread> pool;
+    try {
+        pool.reserve(nth);
+        for (int t = 1; t < nth; ++t)
+            pool.emplace_back([=] { for (int w = t; w < n; w += nth) copy_window(h, w, at, results[w]); });
+    } catch (...) {  // no more threads: the ones that run do their share, this one the others'
+    }
+    for (int t = 0; t < nth; ++t)
+        if (t == 0 || t > (int)pool.size())
+            for (int w = t; w < n; w += nth) copy_window(h, w, at, results[w]);
+    for (auto& t : pool) t.join();
     return worst;
 }
 
@@ -1667,6 +1701,7 @@ void nav_ba_destroy(nav_ba_handle* h) {
     if (h->hpcg) (void)hipHostFree(h->hpcg);
     if (h->stage) (void)hipHostFree(h->stage);
     if (h->stage_s) (void)hipHostFree(h->stage_s);
+    if (h->rbuf) (void)hipHostFree(h->rbuf);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
