@@ -177,7 +177,7 @@ struct DevWork {
     double* y;
     double* dp;
     double* Lm;         // one problem: Cholesky factor (tiled: n_pad^2; blocks: packed 6x6 blocks)
-    double* Li;         // tiled path: inverses of the diagonal factor tiles [nt][64][64]
+    double* Li;         // tiled path: inverses of the diagonal factor tiles [nt][kInvTile]
     double* fpart;      // tiled path: forward-step products L_ij y_j [nt][nt][64]
     double* red_cost;   // [n_cblk] the cost at the current state (start of a solve, flags)
     double* red_tcost;  // [n_tiles] the trial cost at the candidate state, per linearisation tile
@@ -289,6 +289,7 @@ template <typename T> void launch_schur_reduce(const DevProblem& P, const DevWor
 // also form the candidate poses (cholesky_updates_cameras); otherwise launch_update_cam does.
 void launch_cholesky_solve(const DevProblem& P, const DevState& cur, const DevState& cand, const DevWork& W,
                            hipStream_t st);
+constexpr int kInvTile = 4096 + 2560;  // doubles of a diagonal tile's inverse: row-major, then packed blocks
 constexpr int kBackSingleMax = 10;  // tiles up to which the backward step runs in one workgroup
 inline bool cholesky_updates_cameras(const DevProblem& P) {
     return P.n_fc > 0 && (P.use_win || (!P.batched && !P.use_blocks && !P.use_pcg && P.nt <= kBackSingleMax));

@@ -18,52 +18,17 @@
 // tile, inverts it and runs that tile's forward step.  The factor goes to a
 // separate buffer, so no workgroup overwrites a tile another one still reads;
 // the diagonal factors L_kk themselves are never stored (only M_k is used).
-// The tile products run on FP64 MFMA (v_mfma_f64_16x16x4); the chain through
-// the pivots runs in registers.  The backward step is a single launch.
+// All products run on FP64 MFMA (v_mfma_f64_16x16x4).
+// Measured (rocprofv3, average per launch, launch included): 28 tiles, step
+// 23.8 -> 16.8 us, first tile 18 -> 12.9 us, backward 28 launches of 4.2 -> 7 of
+// 9.5 us; 6 tiles, step 21.6 -> 14.6 us, against a factorisation of the diagonal
+// tile by pivots (31 k cycles of the step's 55 k; square roots, a column per
+// pivot through LDS), operands staged through LDS and a launch per tile in the
+// backward step.  A step's floor is its launch (about 2 us), one round trip to
+// memory and the chain of the diagonal tile.
 #include "ba_kernels.h"
 
 namespace navba {
-
-typedef double TileLds[64][65];
-
-// A 64x64 tile through registers, 16 elements per thread: fetch issues the
-// global loads, put writes LDS (several fetches can be in flight before the
-// first put).
-__device__ __forceinline__ void tile_fetch(double v[16], const double* __restrict__ src, int lda) {
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int idx = threadIdx.x + 256 * s;
-        v[s] = src[(size_t)(idx >> 6) * lda + (idx & 63)];
-    }
-}
-
-__device__ __forceinline__ void tile_put(TileLds& T, const double v[16]) {
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int idx = threadIdx.x + 256 * s;
-        T[idx >> 6][idx & 63] = v[s];
-    }
-}
-
-__device__ __forceinline__ void tile_load(TileLds& T, const double* __restrict__ src, int lda) {
-    double v[16];
-    tile_fetch(v, src, lda);
-    tile_put(T, v);
-}
-
-__device__ __forceinline__ void tile_store(const TileLds& T, double* __restrict__ dst, int lda) {
-    double v[16];
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int idx = threadIdx.x + 256 * s;
-        v[s] = T[idx >> 6][idx & 63];
-    }
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int idx = threadIdx.x + 256 * s;
-        dst[(size_t)(idx >> 6) * lda + (idx & 63)] = v[s];
-    }
-}
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
@@ -85,103 +50,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// M[C..C+15][C..C+15] = L^-1 of the 16x16 diagonal block of the factor in A
-// (lower triangle, rpiv = 1 / diag), by one wave: its two 8x8 diagonal blocks
-// by substitution (one lane per column), then M21 = -M22 (L21 M11) on FP64
-// MFMA (8x8 products, zero padded to 16x16).  The block's upper right 8x8
-// quarter is not written (it must already hold zeros).
-__device__ __forceinline__ void wave_inv16(const TileLds& A, const double* rpiv, TileLds& M, int C) {
-    const int lane = threadIdx.x & 63;
-    const int r16 = lane & 15, kq = lane >> 4, r8 = lane & 7;
-    const int R = C + 8;
-    if (lane < 16) {
-        const int b = C + 8 * (lane >> 3), j = lane & 7;
-        double d[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) d[i] = (i == j) ? rpiv[b + j] : 0.0;
-#pragma unroll
-        for (int i = 1; i < 8; ++i) {
-            double s = 0.0;
-#pragma unroll
-            for (int k = 0; k < i; ++k) s += A[b + i][b + k] * d[k];  // d[k] = 0 for k < j
-            if (i > j) d[i] = -s * rpiv[b + i];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) M[b + i][b + j] = d[i];
-    }
-    wave_sync();
-    // T = L21 M11 (8x8): rows i = 4v + kq < 8, columns r16 < 8 of the 16x16
-    // product (operand rows and columns 8..15 zero; row 8 + r8 read instead)
-    const bool in = r16 < 8;
-    dbl4 t = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int m0 = 0; m0 < 8; m0 += 4) {
-        const double va = A[R + r8][C + m0 + kq], vb = M[C + m0 + kq][C + r16];
-        t = mfma16x16x4(in ? va : 0.0, in ? vb : 0.0, t);
-    }
-    if (in) {
-        M[R + kq][C + r16] = t[0];
-        M[R + 4 + kq][C + r16] = t[1];
-    }
-    wave_sync();
-    dbl4 u = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int m0 = 0; m0 < 8; m0 += 4) {
-        const double va = M[R + r8][R + m0 + kq], vb = M[R + m0 + kq][C + r16];
-        u = mfma16x16x4(in ? va : 0.0, in ? vb : 0.0, u);
-    }
-    wave_sync();
-    if (in) {
-        M[R + kq][C + r16] = -u[0];
-        M[R + 4 + kq][C + r16] = -u[1];
-    }
-    wave_sync();
-}
-
-// 16x16 block product of one wave, acc += X[xr.., xc..] Y[yr.., yc..]; the
-// result's element v in lane (r16, kq) is row 4v + kq, column r16.
-__device__ __forceinline__ dbl4 blk_mul(const TileLds& X, int xr, int xc, const TileLds& Y, int yr, int yc, dbl4 acc) {
-    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-    double a[4], b[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-        a[kk] = X[xr + r16][xc + 4 * kk + kq];
-        b[kk] = Y[yr + 4 * kk + kq][yc + r16];
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) acc = mfma16x16x4(a[kk], b[kk], acc);
-    return acc;
-}
-
-// Block (r, c) of M (16x16) <- sign * acc, in the layout of blk_mul.
-__device__ __forceinline__ void blk_put(TileLds& M, int r, int c, dbl4 acc, double sign) {
-    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) M[16 * r + 4 * v + kq][16 * c + r16] = sign * acc[v];
-}
-
-// Block (i, j) of the tile inverse, M_ij = -M_ii T_ij, where block (i, j) of M
-// holds T_ij = sum_{j<=k<i} L_ik M_kj (one wave; in place).
-__device__ __forceinline__ void blk_finish(TileLds& M, int i, int j) {
-    const dbl4 z = {0.0, 0.0, 0.0, 0.0};
-    const dbl4 t = blk_mul(M, 16 * i, 16 * i, M, 16 * i, 16 * j, z);
-    wave_sync();
-    blk_put(M, i, j, t, -1.0);
-}
-
-// Block (i, j) of M += L_ik M_kj (or = when first), one wave.
-__device__ __forceinline__ void blk_term(const TileLds& A, TileLds& M, int i, int k, int j, bool first) {
-    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (!first) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[v] = M[16 * i + 4 * v + kq][16 * j + r16];
-    }
-    acc = blk_mul(A, 16 * i, 16 * k, M, 16 * k, 16 * j, acc);
-    wave_sync();
-    blk_put(M, i, j, acc, 1.0);
-}
-
 // The value of v in lane l (l wave-uniform), as a uniform double.
 __device__ __forceinline__ double lane_value(double v, int l) {
     const long long b = __double_as_longlong(v);
@@ -190,304 +58,431 @@ __device__ __forceinline__ double lane_value(double v, int l) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// In-LDS Cholesky of the SPD tile A (64x64, 256 threads) and the inverse of
-// its factor: the lower triangle of A becomes L, rpiv[j] = 1 / L_jj and
-// M = L^-1 (upper triangle zero).  The strict upper triangle of A's four
-// 16x16 diagonal blocks is left with scratch values, the rest of A's upper
-// triangle is unchanged.  Wave w owns columns 16w..16w+15, lane l row l.
-// Four stages, one barrier between stages; in stage s:
-//   waves w >= s apply panel s-1 (final since the last barrier) to their
-//     columns, rows 16w.., on FP64 MFMA (16x16 blocks, K = 16, in place);
-//   wave s then factors its 16 columns in registers.  Pivot j: 1/sqrt(d_j)
-//     by rsq and two Goldschmidt steps; the next pivot is formed from
-//     wave-uniform values read before this pivot's column update,
-//     d_{j+1} = a_{j+1,j+1} - (a_{j+1,j} / sqrt(d_j))^2, so that the chain
-//     through the pivots holds no cross-lane step; columns j+1 and j+2 are
-//     updated with uniform multipliers, the others with the scaled column
-//     broadcast through `scratch` (16 x 64 doubles of LDS, not M);
-//   wave s-1, whose panel is final, forms the inverse's block row s-1 in 16x16
-//     blocks, M_ii = L_ii^-1 and M_ij = -M_ii T_ij, and adds its terms to
-//     the sums T_mj = sum_{j<=k<m} L_mk M_kj of the rows below (kept in M's
-//     blocks (m, j)); stage 0's idle waves clear M's upper triangle.
-// After the last stage wave 3 forms block row 3.  A pivot that is not
-// positive and finite is replaced by 1 (the values stay finite); the return
-// value, the same in every thread, says whether one was.
-__device__ __forceinline__ bool tile_potrf_inv(TileLds& A, double* rpiv, double* scratch, TileLds& M, int nst) {
-    const int lane = threadIdx.x & 63, w = wave_id();
-    const int r16 = lane & 15, kq = lane >> 4;
-    const int c0 = 16 * w;
-    double (*cb)[64] = reinterpret_cast<double (*)[64]>(scratch);
-    bool bad = false;
-    for (int s = 0; s < nst; ++s) {
-        if (s == 0 && w > 0) {
-            for (int idx = (int)threadIdx.x - 64; idx < 4096; idx += 192) {
-                const int i = idx >> 6, j = idx & 63;
-                if ((j >> 3) > (i >> 3)) M[i][j] = 0.0;
-            }
-        }
-        if (s == 0 && w >= nst) {
-            // identity padding rows (the last tile of the system): their part of
-            // the factor is the identity already in A; M's rows are the identity
-            for (int idx = lane; idx < 16 * 64; idx += kWave) {
-                const int i = c0 + (idx >> 6), j = idx & 63;
-                if ((j >> 3) <= (i >> 3)) M[i][j] = (i == j) ? 1.0 : 0.0;
-            }
-            if (lane < 16) rpiv[c0 + lane] = 1.0;
-        }
-        if (s > 0 && w == s - 1) {
-            // block row s-1 of the inverse and its terms of the rows below
-            wave_inv16(A, rpiv, M, 16 * w);
-            for (int j = 0; j < w; ++j) blk_finish(M, w, j);
-            for (int m = w + 1; m < nst; ++m)
-                for (int j = 0; j <= w; ++j) blk_term(A, M, m, w, j, j == w);
-        }
-        if (s > 0 && w >= s && w < nst) {
-            const int p = 16 * (s - 1);
-            double bv[4], av[4][4];
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) bv[kk] = A[c0 + r16][p + 4 * kk + kq];
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-                if (bi >= w)
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) av[bi][kk] = A[16 * bi + r16][p + 4 * kk + kq];
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi) {
-                if (bi >= w) {
-                    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) acc = mfma16x16x4(av[bi][kk], bv[kk], acc);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) A[16 * bi + 4 * v + kq][c0 + r16] -= acc[v];
-                }
-            }
-        }
-        if (w == s) {
-            wave_sync();
-            double x[16];
-#pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = A[lane][c0 + c];
-            double rp[16];
-            double d = lane_value(x[0], c0);
-            double a1 = lane_value(x[0], c0 + 1), a2 = lane_value(x[0], c0 + 2), ad = lane_value(x[1], c0 + 1);
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const bool ok = (d > 0.0) && isfinite(d);
-                bad |= !ok;
-                d = ok ? d : 1.0;
-                double H = __builtin_amdgcn_rsq(d);
-                double g = d * H;
-#pragma unroll
-                for (int it = 0; it < 2; ++it) {
-                    const double e = fma(-g, H, 1.0);
-                    const double gh = 0.5 * g, Hh = 0.5 * H;
-                    g = fma(gh, e, g);
-                    H = fma(Hh, e, H);
-                }
-                rp[j] = H;
-                const double l1 = a1 * H, l2 = a2 * H;
-                const double dn = fma(-l1, l1, ad);
-                x[j] = (lane == c0 + j) ? g : x[j] * H;
-                if (j + 3 < 16) cb[j][lane] = x[j];
-                if (j + 1 < 16) x[j + 1] = fma(-x[j], l1, x[j + 1]);
-                if (j + 2 < 16) x[j + 2] = fma(-x[j], l2, x[j + 2]);
-                if (j + 1 < 16) {
-                    d = dn;
-                    a1 = (j + 2 < 16) ? lane_value(x[j + 1], c0 + j + 2) : 0.0;
-                    a2 = (j + 3 < 16) ? lane_value(x[j + 1], c0 + j + 3) : 0.0;
-                    ad = (j + 2 < 16) ? lane_value(x[j + 2], c0 + j + 2) : 0.0;
-                }
-                if (j + 3 < 16) {
-                    wave_sync();
-#pragma unroll
-                    for (int c = j + 3; c < 16; ++c) x[c] = fma(-x[j], cb[j][c0 + c], x[c]);
-                }
-            }
-            if (lane >= c0) {
-#pragma unroll
-                for (int c = 0; c < 16; ++c) A[lane][c0 + c] = x[c];
-            }
-            if (lane == 0) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) rpiv[c0 + j] = rp[j];
-            }
-        }
-        if (s < nst - 1) __syncthreads();
-    }
-    bad = __syncthreads_or(bad);
-    if (w == nst - 1) {
-        wave_inv16(A, rpiv, M, 16 * w);
-        for (int j = 0; j < w; ++j) blk_finish(M, w, j);
-    }
-    __syncthreads();
-    return bad;
+// Reciprocal: the hardware's estimate (relative error e below 2^-24) and one
+// step of third order, r (1 + e + e^2).
+__device__ __forceinline__ double fast_rcp(double d) {
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
-// acc[b] = block (wave, b) of X Y^T in 16x16 blocks; with kTriY, Y is lower
-// triangular and the zero part of the sum is skipped.
-template <bool kTriY>
-__device__ __forceinline__ void tile_mfma_nt(const TileLds& X, const TileLds& Y, dbl4 acc[4]) {
-    const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int m0 = 0; m0 < 64; m0 += 4) {
-        const double a = X[16 * w + r16][m0 + kq];
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-            if (!kTriY || m0 < 16 * b + 16) acc[b] = mfma16x16x4(a, Y[16 * b + r16][m0 + kq], acc[b]);
-    }
+// Four products of 4x4 blocks, D_b = A_b B_b (b = 0..3), with A[i][k] in lane
+// i + 4b + 16k, B[k][j] in lane j + 4b + 16k and D[i][j] in lane j + 4b + 16i
+// (checked on gfx950 against a host product).
+__device__ __forceinline__ double mfma4x4x4(double a, double b) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, 0.0, 0, 0, 0);
 }
 
-// B <- B M^T (the panel solve B L^-T with M = L^-1 lower triangular, in LDS).
-__device__ __forceinline__ void tile_right_mul_t(TileLds& B, const TileLds& M) {
-    dbl4 acc[4];
-    tile_mfma_nt<true>(B, M, acc);
-    const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
-    __syncthreads();
+// LDL^T of a symmetric 16x16 tile and the inverse of its unit factor, by one
+// wave in registers.  acc holds the tile in the matrix instruction's result
+// layout (element v of lane (i, k) = l & 15, l >> 4: row 4 v + k, column i);
+// by symmetry acc[p] is then the column panel 4p..4p+3 in the layout of an
+// operand (lane (i, k): row i, column 4p + k), so a panel needs no data
+// movement.  Per panel p of four columns:
+//   the 4x4 diagonal block's LDL^T and the inverse N of its unit factor, the
+//     same in every lane from ten lane reads;
+//   W = A_p N^T as four 4x4 blocks, L_p = W D^-1, acc -= W L_p^T;
+//   Z, which starts as the identity and ends as the inverse: Z_p = N Z_p,
+//     Z -= L_p Z_p for the rows below.
+// dv[p] = the reciprocal pivot of column 4p + k in lane (i, k).  Returns false
+// if a pivot was not positive and finite (its values are then arbitrary), the
+// same in every lane.
+// A solve by substitution in 4x4 blocks instead of the inverse was no more
+// accurate over 512 ill-conditioned windows (the same quantiles of the pose and
+// cost errors against the oracle) and 4 us slower on the largest window.
+__device__ __forceinline__ bool tile16_ldl(dbl4 acc, dbl4& Z, double dv[4]) {
+    const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4, i4 = lane & 3;
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int v = 0; v < 4; ++v) Z[v] = (4 * v + k == i) ? 1.0 : 0.0;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) B[16 * w + 4 * v + kq][16 * b + r16] = acc[b][v];
-    __syncthreads();
-}
-
-// out = B v for a 64x64 tile B in LDS and a 64-vector v in global memory
-// (four threads per row, summed by DPP in a fixed order).
-__device__ __forceinline__ void tile_gemv(const TileLds& B, const double* __restrict__ v, double* __restrict__ out) {
-    const int tid = threadIdx.x;
-    const int r = tid >> 2, q = tid & 3;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll
-    for (int m = q; m < 64; m += 16) {
-        s0 += B[r][m] * v[m];
-        s1 += B[r][m + 4] * v[m + 4];
-        s2 += B[r][m + 8] * v[m + 8];
-        s3 += B[r][m + 12] * v[m + 12];
-    }
-    double s = (s0 + s1) + (s2 + s3);
-    s += dpp_move<0xB1>(s);
-    s += dpp_move<0x4E>(s);
-    if (q == 0) out[r] = s;
-}
-
-// y_k = M_k (g_k - sum_{j<=k-1} L_kj y_j).  The products L_kj y_j were formed
-// by the workgroups that computed L_kj (tile_gemv into fpart[k][j], 64 values
-// each); the nterms of them are summed here in a fixed order, so the row block
-// of the factor is not read again.  M_k is in LDS.
-__device__ __forceinline__ void tile_forward(const TileLds& M, const double* __restrict__ fpart, int nterms,
-                                             const double* __restrict__ g, double* __restrict__ y, double* rv) {
-    const int tid = threadIdx.x;
-    const int r = tid >> 2, q = tid & 3;
-    {
-        double s0 = 0.0, s1 = 0.0;
-        int j = q;
-        for (; j + 4 < nterms; j += 8) {
-            s0 += fpart[64 * j + r];
-            s1 += fpart[64 * (j + 4) + r];
+    for (int p = 0; p < 4; ++p) {
+        const double a = acc[p];
+        const int q = 4 * p;
+        const double a00 = lane_value(a, q), a10 = lane_value(a, q + 1), a11 = lane_value(a, q + 17),
+                     a20 = lane_value(a, q + 2), a21 = lane_value(a, q + 18), a30 = lane_value(a, q + 3),
+                     a31 = lane_value(a, q + 19), a22 = lane_value(a, q + 34), a32 = lane_value(a, q + 35),
+                     a33 = lane_value(a, q + 51);
+        const double i0 = fast_rcp(a00);
+        const double l10 = a10 * i0, l20 = a20 * i0, l30 = a30 * i0;
+        const double d1 = fma(-l10, a10, a11), t21 = fma(-l20, a10, a21), t31 = fma(-l30, a10, a31);
+        const double i1 = fast_rcp(d1);
+        const double l21 = t21 * i1, l31 = t31 * i1;
+        const double d2 = fma(-l21, t21, fma(-l20, a20, a22)), t32 = fma(-l31, t21, fma(-l30, a20, a32));
+        const double i2 = fast_rcp(d2);
+        const double l32 = t32 * i2;
+        const double d3 = fma(-l32, t32, fma(-l31, t31, fma(-l30, a30, a33)));
+        const double i3 = fast_rcp(d3);
+        // N, unit lower, element (i & 3, k) in lane (i, k)
+        const double n20 = fma(l21, l10, -l20), n31 = fma(l32, l21, -l31);
+        const double n30 = fma(-l32, n20, fma(l31, l10, -l30));
+        double nv = i4 == k ? 1.0 : 0.0;
+        if (i4 == 1 && k == 0) nv = -l10;
+        if (i4 == 2 && k == 0) nv = n20;
+        if (i4 == 2 && k == 1) nv = -l21;
+        if (i4 == 3 && k == 2) nv = -l32;
+        if (i4 == 3 && k == 1) nv = n31;
+        if (i4 == 3 && k == 0) nv = n30;
+        dv[p] = k == 0 ? i0 : k == 1 ? i1 : k == 2 ? i2 : i3;
+        if (p < 3) {
+            const double w = mfma4x4x4(nv, a);  // W[i][k]
+            const double zp = mfma4x4x4(nv, Z[p]);  // row 4p + k, column i of N Z_p
+            const double lp = w * dv[p];
+            acc = mfma16x16x4(-w, lp, acc);
+            Z = mfma16x16x4(i >= q + 4 ? -lp : 0.0, zp, Z);
+            Z[p] = zp;
+        } else {
+            Z[p] = mfma4x4x4(nv, Z[p]);
         }
-        if (j < nterms) s0 += fpart[64 * j + r];
-        double s = s0 + s1;
-        s += dpp_move<0xB1>(s);
-        s += dpp_move<0x4E>(s);
-        if (q == 0) rv[r] = g[r] - s;
     }
-    __syncthreads();
-    double s0 = 0.0, s1 = 0.0;
-    for (int m = q; m < 64; m += 8) {  // M[r][m] = 0 for m > r
-        s0 += M[r][m] * rv[m];
-        s1 += M[r][m + 4] * rv[m + 4];
-    }
-    double s = s0 + s1;
-    s += dpp_move<0xB1>(s);
-    s += dpp_move<0x4E>(s);
-    if (q == 0) y[r] = s;
-    __syncthreads();
+    bool good = true;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) good = good && dv[p] > 0.0 && isfinite(dv[p]);
+    return __all(good);
+}
+
+// Sum over the four lanes (i, 0..3), in each of them: row pairs, then halves.
+__device__ __forceinline__ double sum_over_k(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    const auto l1 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h1 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    const double s = __longlong_as_double(((long long)h1[0] << 32) | l1[0]) +
+                     __longlong_as_double(((long long)h1[1] << 32) | l1[1]);
+    const long long c = __double_as_longlong(s);
+    const unsigned lo2 = (unsigned)c, hi2 = (unsigned)(c >> 32);
+    const auto l2 = __builtin_amdgcn_permlane32_swap(lo2, lo2, false, false);
+    const auto h2 = __builtin_amdgcn_permlane32_swap(hi2, hi2, false, false);
+    return __longlong_as_double(((long long)h2[0] << 32) | l2[0]) +
+           __longlong_as_double(((long long)h2[1] << 32) | l2[1]);
 }
 
 // 16-column stages of diagonal tile i that hold rows of the n-row system (the
 // last tile's padding rows beyond are the identity and are not factored).
 __device__ __forceinline__ int tile_stages(int n, int i) { return min(4, (n - 64 * i + 15) >> 4); }
 
-__global__ __launch_bounds__(256) void k_chol_first(const double* __restrict__ S, double* __restrict__ Lm,
-                                                    double* __restrict__ Li, int lda, int n, const double* __restrict__ g,
-                                                    double* __restrict__ y, LMDev* lm) {
-    __shared__ TileLds A;
-    __shared__ TileLds M;
-    __shared__ double scratch[16 * 64];
-    __shared__ double rv[64];
-    __shared__ double rpiv[64];
-    tile_load(A, S, lda);
-    if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished
-    __syncthreads();
-    if (tile_potrf_inv(A, rpiv, scratch, M, tile_stages(n, 0)) && threadIdx.x == 0) atomicOr(&lm->fail, 1);
-    tile_store(M, Li, 64);
-    tile_forward(M, nullptr, 0, g, y, rv);
+// ---------------------------------------------------------------- diagonal tiles
+// A diagonal tile is factored by one workgroup of four waves, its 16x16 blocks
+// in registers: wave w holds the blocks (w, 0..w), block (w, j) in operand
+// layout (element p of lane (i, k): row i, column 4 p + k).  With A and B
+// swapped, the matrix instruction returns a product's transpose, which is that
+// same layout, so a block goes through solve and update without data movement.
+// Stage s (two barriers):
+//   wave s    LDL^T of block (s, s) and the inverse Z_s of its unit factor
+//             (tile16_ldl); the other waves, whose blocks are done, meanwhile
+//             form R_sw = sum_{w<=k<s} L_sk M_kw, wave w owning block column w
+//             of the inverse, which needs only its own blocks M_kw;
+//   barrier   Z_s, the reciprocal pivots;
+//   wave i>s  W_is = A_is Z_s^T (= L_is D_s), shared through LDS; barrier;
+//             A_ij -= W_is D_s^-1 W_js^T, s < j <= i: wave s + 1 needs one block
+//             before it goes on;
+//   wave w<s  M_sw = -Z_s R_sw;
+//   wave 0    the right-hand side, carried like a block row whose 16 rows are
+//             all g: z_s = Z_s g_s, g_j -= W_js D_s^-1 z_s.
+// The tile's factor in LL^T form is L D^1/2, its inverse M = D^-1/2 (unit
+// inverse), its forward result y = D^-1/2 z; M and y are scaled on the way out.
+// Bound by the chain through the four blocks (about 3 k cycles each).
+struct DiagLds {
+    double Z[4][16 * 17];  // [row][17]: read along rows and columns without bank conflicts
+    double W[6][256];      // W_is in lane order, block i (i - 1) / 2 + s
+    double dinv[64];       // reciprocal pivots
+    double sd[64];         // their square roots
+    double g[64];          // right-hand side
+};
+
+// Inverse tiles: M row-major (64x64, for the backward step), then its lower
+// 16x16 blocks (b, c) at kInvPack + 256 (b (b + 1) / 2 + c) in the order in
+// which k_chol_step's lanes read them: entry (j, 4 k + e) at 4 (j + 16 k) + e.
+constexpr int kInvPack = 4096;
+static_assert(kInvTile == kInvPack + 10 * 256, "inverse tile size");
+
+__device__ __forceinline__ double fast_sqrt(double d) {  // by rsq and two Goldschmidt steps; d > 0
+    double H = __builtin_amdgcn_rsq(d), g = d * H;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const double e = fma(-g, H, 1.0);
+        g = fma(0.5 * g, e, g);
+        H = fma(0.5 * H, e, H);
+    }
+    return g;
 }
 
-__global__ __launch_bounds__(256) void k_chol_step(double* __restrict__ S, double* __restrict__ Lm,
-                                                   double* __restrict__ Li, int lda, int n, int k,
-                                                   const double* __restrict__ g, double* __restrict__ y,
-                                                   double* __restrict__ fpart, int nt, LMDev* lm) {
-    __shared__ TileLds Mk;
-    __shared__ TileLds Bi;
-    __shared__ TileLds Bj;
-    __shared__ double rv[64];
-    __shared__ double rpiv[64];
+// Block (b, c) of the inverse, m in result layout, its rows scaled by sd.
+__device__ __forceinline__ void inv_store(double* __restrict__ Li, int b, int c, dbl4 m, const double* sd) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+    double* pk = Li + kInvPack + 256 * (b * (b + 1) / 2 + c) + 64 * (r16 >> 2) + (r16 & 3);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int r = 4 * v + kq;
+        const double x = m[v] * sd[16 * b + r];
+        Li[(16 * b + r) * 64 + 16 * c + r16] = x;
+        pk[4 * r] = x;
+    }
+}
+
+// a: the calling wave's blocks; D.g is written (a barrier follows before it is
+// read); nst: stages that hold rows of the system.  Li and y receive the
+// tile's inverse and forward result.  Returns false in the wave that met a
+// pivot which is not positive and finite.
+__device__ __forceinline__ bool diag_factor(dbl4 a[4], DiagLds& D, int nst, double* __restrict__ Li,
+                                            double* __restrict__ y) {
+    const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
+    const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
+    bool good = true;
+    dbl4 m[4], gt[4], zs = zero;  // m[i]: block (i, w) of the unit inverse, result layout
+    for (int b = 0; b < w; ++b)  // the blocks above the diagonal
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Li[(16 * b + 4 * v + kq) * 64 + 16 * w + r16] = 0.0;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        dbl4 R = zero;
+        if (w == s) {
+            double dv[4] = {1.0, 1.0, 1.0, 1.0};
+            if (s < nst) {
+                good = tile16_ldl(a[s], m[s], dv);
+            } else {  // padding rows: the identity
+#pragma unroll
+                for (int v = 0; v < 4; ++v) m[s][v] = (4 * v + kq == r16) ? 1.0 : 0.0;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) D.Z[s][17 * (4 * v + kq) + r16] = m[s][v];
+            if (r16 < 4) {
+                const double d = r16 == 0 ? dv[0] : r16 == 1 ? dv[1] : r16 == 2 ? dv[2] : dv[3];
+                D.dinv[16 * s + 4 * r16 + kq] = d;
+                D.sd[16 * s + 4 * r16 + kq] = fast_sqrt(d);
+            }
+        } else if (w < s) {
+            inv_store(Li, s - 1, w, m[s - 1], D.sd);
+#pragma unroll
+            for (int k = 0; k < s; ++k)
+                if (k >= w) {
+                    const double* W = D.W[s * (s - 1) / 2 + k];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+                        R = mfma16x16x4(W[64 * p + lane] * D.dinv[16 * k + 4 * p + kq], m[k][p], R);
+                }
+        }
+        if (w == 0 && s > 0) {
+            if (r16 == 0)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) y[16 * (s - 1) + 4 * v + kq] = zs[v] * D.sd[16 * (s - 1) + 4 * v + kq];
+        }
+        __syncthreads();
+        if (w == 0 && s == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) gt[j][p] = D.g[16 * j + 4 * p + kq];
+        }
+        double zt[4], dk[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            zt[p] = D.Z[s][17 * r16 + 4 * p + kq];
+            dk[p] = D.dinv[16 * s + 4 * p + kq];
+        }
+        dbl4 wv = zero;
+        if (w > s) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) wv = mfma16x16x4(zt[p], a[s][p], wv);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) D.W[w * (w - 1) / 2 + s][64 * p + lane] = wv[p];
+        }
+        if (s < 3) __syncthreads();
+        if (w > s) {
+#pragma unroll
+            for (int j = s + 1; j < 4; ++j)
+                if (j <= w) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        const double x = j == w ? wv[p] : D.W[j * (j - 1) / 2 + s][64 * p + lane];
+                        a[j] = mfma16x16x4(-x, wv[p] * dk[p], a[j]);
+                    }
+                }
+        }
+        if (w == 0) {
+            zs = zero;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) zs = mfma16x16x4(zt[p], gt[s][p], zs);
+#pragma unroll
+            for (int j = s + 1; j < 4; ++j)
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    gt[j] = mfma16x16x4(-D.W[j * (j - 1) / 2 + s][64 * p + lane], zs[p] * dk[p], gt[j]);
+        }
+        if (w < s) {
+            m[s] = zero;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) m[s] = mfma16x16x4(-zt[p], R[p], m[s]);
+        }
+    }
+    inv_store(Li, 3, w, m[3], D.sd);
+    if (w == 0 && r16 == 0)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[48 + 4 * v + kq] = zs[v] * D.sd[48 + 4 * v + kq];
+    return good;
+}
+
+__global__ __launch_bounds__(256) void k_chol_first(const double* __restrict__ S, double* __restrict__ Li, int lda, int n,
+                                                    const double* __restrict__ g, double* __restrict__ y, LMDev* lm) {
+    __shared__ DiagLds D;
+    const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
+    dbl4 a[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (j <= w)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) a[j][p] = S[(size_t)(16 * w + r16) * lda + 16 * j + 4 * p + kq];
+    if (threadIdx.x < 64) D.g[threadIdx.x] = g[threadIdx.x];
+    if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished
+    if (!diag_factor(a, D, tile_stages(n, 0), Li, y) && lane == 0) atomicOr(&lm->fail, 1);
+}
+
+// Four consecutive doubles of a row.
+__device__ __forceinline__ void load4(double v[4], const double* __restrict__ p) {
+    const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
+// W = A_k M_k^T for the calling wave's 16 rows: va[4 g + e] of lane (i, k) is
+// entry (i, 16 g + 4 k + e) of the rows (the order of a product's terms is
+// free, so each lane takes 32 contiguous bytes), vm the blocks of M_k in the
+// same order.  W in operand layout: element 4 b + v, column 16 b + 4 v + k.
+__device__ __forceinline__ void panel_rows(const double va[16], const double vm[40], dbl4 W[4]) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        W[b] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int g = 0; g <= b; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                W[b] = mfma16x16x4(vm[4 * (b * (b + 1) / 2 + g) + e], va[4 * g + e], W[b]);
+    }
+}
+
+// One launch per tile column k; workgroup (i, j), k < j <= i, four waves, wave w
+// the rows 16 w.. of the tile.  Operands come from memory straight into
+// registers in the order the matrix instructions take them, L_ik stays there
+// (panel_rows), and only L_jk, which every wave needs, goes through LDS: one
+// barrier.  Workgroup (k+1, k+1) goes on to factor its tile, its wave 0 as soon
+// as it has the first block; it is the launch's critical path, so its waves take
+// priority over those that share its compute unit.
+__global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, double* __restrict__ Lm,
+                                                      double* __restrict__ Li, int lda, int n, int k,
+                                                      const double* __restrict__ g, double* __restrict__ y,
+                                                      double* __restrict__ fpart, int nt, LMDev* lm) {
+    __shared__ double Wj[4][16][64];  // [rows 16 b][element][lane]
+    __shared__ double ys[64];
+    __shared__ DiagLds D;
     const int idx = blockIdx.x;
     int ii = (int)((sqrt(8.0 * idx + 1.0) - 1.0) * 0.5);
     while ((ii + 1) * (ii + 2) / 2 <= idx) ++ii;
     while (ii * (ii + 1) / 2 > idx) --ii;
     const int jj = idx - ii * (ii + 1) / 2;
     const int i = k + 1 + ii, j = k + 1 + jj;
-    const bool same = (i == j);
-    // every global load of the launch in flight at once: M_k, A_ik, A_jk and
-    // the tile A_ij to update (no other workgroup writes any of them)
+    const bool same = (i == j), diag = idx == 0;
+    if (diag) __builtin_amdgcn_s_setprio(3);
+    // every global load of the launch in flight at once (no other workgroup
+    // writes any of them)
     const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
-    double* Aij = S + (size_t)(64 * i) * lda + 64 * j;
-    double vm[16], vi[16], vj[16], cur[4][4];
-    tile_fetch(vm, Li + (size_t)4096 * k, 64);
-    tile_fetch(vi, S + (size_t)(64 * i) * lda + 64 * k, lda);
-    if (!same) tile_fetch(vj, S + (size_t)(64 * j) * lda + 64 * k, lda);
+    double vm[40], vi[16], vj[16];
+    const double* Ai = S + (size_t)(64 * i + 16 * w + r16) * lda + 64 * k + 4 * kq;
+    const double* Aj = S + (size_t)(64 * j + 16 * w + r16) * lda + 64 * k + 4 * kq;
+    const double* Mk = Li + (size_t)kInvTile * k + kInvPack + 4 * lane;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) load4(vi + 4 * q, Ai + 16 * q);
+#pragma unroll
+    for (int q = 0; q < 10; ++q) load4(vm + 4 * q, Mk + 256 * q);
+    if (!same) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load4(vj + 4 * q, Aj + 16 * q);
+    }
+    dbl4 cur[4];
+    const double yk = j == k + 1 && w == 1 ? y[64 * k + lane] : 0.0;
+    double* Aij = S + (size_t)(64 * i + 16 * w) * lda + 64 * j;
+    if (diag) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b <= w)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) cur[b][v] = Aij[(size_t)r16 * lda + 16 * b + 4 * v + kq];
+    } else {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) cur[b][v] = Aij[(size_t)(4 * v + kq) * lda + 16 * b + r16];
+    }
+    if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished (loads in flight meanwhile)
+    dbl4 Wi[4], Wr[4];
+    panel_rows(vi, vm, Wi);  // L_ik
+    if (same) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) Wr[b] = Wi[b];
+    } else {
+        panel_rows(vj, vm, Wr);  // L_jk
+    }
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) cur[b][v] = Aij[(size_t)(16 * w + 4 * v + kq) * lda + 16 * b + r16];
-    if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished (loads in flight meanwhile)
-    tile_put(Mk, vm);
-    tile_put(Bi, vi);
-    if (!same) tile_put(Bj, vj);
+        for (int v = 0; v < 4; ++v) Wj[w][4 * b + v][lane] = Wr[b][v];
+    if (w == 1) ys[lane] = yk;
     __syncthreads();
-    tile_right_mul_t(Bi, Mk);  // L_ik
-    if (!same) tile_right_mul_t(Bj, Mk);  // L_jk
+    if (diag) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b <= w)
+#pragma unroll
+                for (int p = 0; p < 16; ++p) cur[b] = mfma16x16x4(-Wj[b][p][lane], Wi[p >> 2][p & 3], cur[b]);
+    }
+    if (diag) {
+        // right-hand side of the tile, by wave 1, a row per lane: the terms
+        // L_it y_t of the earlier launches and this one's L_ik y_k
+        if (w == 1) {
+            const double* fp = fpart + (size_t)i * nt * 64 + lane;
+            double f[4] = {g[64 * i + lane], 0.0, 0.0, 0.0};
+            int t = 0;
+            for (; t + 4 <= k; t += 4)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) f[u] -= fp[64 * (t + u)];
+            for (; t < k; ++t) f[0] -= fp[64 * t];
+#pragma unroll
+            for (int p = 0; p < 16; ++p)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) f[q] = fma(-Wj[kq][p][r16 + 16 * q], ys[4 * p + q], f[q]);
+            D.g[lane] = (f[0] + f[1]) + (f[2] + f[3]);
+        }
+    } else if (j == k + 1) {
+        // L_ik y_k, for the forward step of tile i
+        double f = 0.0;
+#pragma unroll
+        for (int p = 0; p < 16; ++p) f = fma(Wi[p >> 2][p & 3], ys[4 * p + kq], f);
+        f = sum_over_k(f);
+        if (kq == 0) fpart[((size_t)i * nt + k) * 64 + 16 * w + r16] = f;
+    }
     if (j == k + 1) {
-        tile_store(Bi, Lm + (size_t)(64 * i) * lda + 64 * k, lda);
-        tile_gemv(Bi, y + 64 * k, fpart + ((size_t)i * nt + k) * 64);  // L_ik y_k for the forward step of tile i
+        double* L = Lm + (size_t)(64 * i + 16 * w + r16) * lda + 64 * k + kq;
+#pragma unroll
+        for (int p = 0; p < 16; ++p) L[4 * p] = Wi[p >> 2][p & 3];
     }
-    dbl4 acc[4];
-    tile_mfma_nt<false>(Bi, same ? Bi : Bj, acc);
-    if (same && i == k + 1) {
-        // Mk is free (the last product that read it ended with a barrier): it
-        // takes the updated tile to factor, Bj its inverse
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Mk[16 * w + 4 * v + kq][16 * b + r16] = cur[b][v] - acc[b][v];
-        __syncthreads();
-        if (tile_potrf_inv(Mk, rpiv, &Bi[0][0], Bj, tile_stages(n, i)) && threadIdx.x == 0) atomicOr(&lm->fail, 1);
-        tile_store(Bj, Li + (size_t)4096 * i, 64);
-        __syncthreads();  // fpart[i][k] (written above by this workgroup) is read back by the forward step
-        tile_forward(Bj, fpart + (size_t)i * nt * 64, k + 1, g + 64 * i, y + 64 * i, rv);
-    } else {
-        // a diagonal tile keeps its upper triangle (never read; left unchanged
-        // so that it does not drift over the trials of a solve)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if (!same || 16 * w + 4 * v + kq >= 16 * b + r16)
-                    Aij[(size_t)(16 * w + 4 * v + kq) * lda + 16 * b + r16] = cur[b][v] - acc[b][v];
+    if (diag) {
+        if (!diag_factor(cur, D, tile_stages(n, i), Li + (size_t)kInvTile * i, y + 64 * i) && lane == 0)
+            atomicOr(&lm->fail, 1);
+        return;
     }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int p = 0; p < 16; ++p) cur[b] = mfma16x16x4(-Wi[p >> 2][p & 3], Wj[b][p][lane], cur[b]);
+    // a diagonal tile keeps its upper triangle (never used; left unchanged so
+    // that it does not drift over the trials of a solve)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * w + 4 * v + kq;
+            if (!same || r >= 16 * b + r16) Aij[(size_t)(4 * v + kq) * lda + 16 * b + r16] = cur[b][v];
+        }
 }
 
 // Backward step x = L^-T y for up to kBackSingleMax tiles in one workgroup of
@@ -535,7 +530,7 @@ __global__ __launch_bounds__(kBackThreads) void k_chol_back(DevProblem P, const 
     // M_k of the next step is loaded during the current one
     double mv[8];
     {
-        const double* Mk = Li + (size_t)4096 * (nt - 1);
+        const double* Mk = Li + (size_t)kInvTile * (nt - 1);
 #pragma unroll
         for (int u = 0; u < 8; ++u) mv[u] = Mk[(grp + 8 * u) * 64 + c];
     }
@@ -566,7 +561,7 @@ __global__ __launch_bounds__(kBackThreads) void k_chol_back(DevProblem P, const 
             part[grp][c] = (s0 + s1) + (s2 + s3);
         }
         if (k > 0) {
-            const double* Mk = Li + (size_t)4096 * (k - 1);
+            const double* Mk = Li + (size_t)kInvTile * (k - 1);
 #pragma unroll
             for (int u = 0; u < 8; ++u) mv[u] = Mk[(grp + 8 * u) * 64 + c];
         }
@@ -609,78 +604,118 @@ __global__ __launch_bounds__(kBackThreads) void k_chol_back(DevProblem P, const 
     if (tid == 0) red_scale[0] = s;
 }
 
-// Backward step for many tiles (more than kBackSingleMax): one launch per tile
-// k from the last, so the reads of the factor spread over k + 1 CUs.  The
-// right-hand sides r of the tiles still to solve live in y (the forward
-// result) and are updated in place: every workgroup of launch k forms
-// x_k = M_k^T r_k (a 64x64 product, recomputed by each workgroup instead of
-// waiting for one); workgroup k writes it to dp, workgroup i < k subtracts
-// L_ki^T x_k from r_i.  r_k is only read during launch k, and final when it
-// starts (launches j > k subtracted their terms).  dp = 0 when the
-// factorisation failed.
-__global__ __launch_bounds__(256) void k_chol_back_tile(const double* __restrict__ Lm, const double* __restrict__ Li,
-                                                   int lda, int nt, int k, double* __restrict__ y,
-                                                   double* __restrict__ dp, const LMDev* lm) {
-    __shared__ double part[4][64];
-    __shared__ double xk[64];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int i = blockIdx.x;  // 0..k: i == k writes x_k, i < k updates r_i
-    // every global load of the launch is issued before the first use: the
-    // L_ki column slice (independent of x_k), M_k, r_k and the failure flag
-    double lv[16];
-    if (i < k) {
-        const double* L = Lm + (size_t)(64 * k) * lda + 64 * i + lane;
+// Backward step for many tiles (more than kBackSingleMax): one launch per group
+// of up to kBackGroup tiles k1, k1 - 1, .., from the last, so the reads of the
+// factor spread over the chip.  The right-hand sides r of the tiles still to
+// solve live in y (the forward result) and are updated in place: every
+// workgroup of a launch forms the group's x (M_k^T r_k and the updates within
+// the group, recomputed by each workgroup instead of waiting for one); the last
+// workgroup writes them to dp, workgroup i below the group subtracts their terms
+// L_ki^T x_k from r_i.  The group's r are only read during its launch, and final
+// when it starts.  dp = 0 when the factorisation failed.
+constexpr int kBackGroup = 4;
+
+__global__ __launch_bounds__(kBackThreads) void k_chol_back_group(const double* __restrict__ Lm,
+                                                                  const double* __restrict__ Li, int lda, int nt,
+                                                                  int k1, int cnt, double* __restrict__ y,
+                                                                  double* __restrict__ dp, const LMDev* lm) {
+    __shared__ double part[kBackGroup - 1][8][64];
+    __shared__ double xs[kBackGroup][64];
+    __shared__ double rs[kBackGroup][64];
+    const int tid = threadIdx.x, c = tid & 63, grp = tid >> 6;  // column c, rows grp + 8 u of every tile
+    const int k0 = k1 - cnt + 1, i = blockIdx.x;  // i == k0 writes the group's x, i < k0 updates r_i
+    // every load before its first use: M_k, r_k and the group's own tiles L_kh, h < k
+    double mv[kBackGroup][8], gv[kBackGroup][kBackGroup][8];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) lv[t] = L[(size_t)(wid + 4 * t) * lda];
-    }
-    double mv[16], rv[16];
-    {
-        const double* Mk = Li + (size_t)4096 * k;
-        const double* rk = y + 64 * k;
+    for (int q = 0; q < kBackGroup; ++q) {
+        if (q >= cnt) continue;
+        const double* M = Li + (size_t)kInvTile * (k1 - q) + grp * 64 + c;
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {  // rows r = wid + 4t; M_k[r][c] = 0 for r < c
-            mv[t] = Mk[(wid + 4 * t) * 64 + lane];
-            rv[t] = rk[wid + 4 * t];
+        for (int u = 0; u < 8; ++u) mv[q][u] = M[512 * u];
+#pragma unroll
+        for (int h = q + 1; h < kBackGroup; ++h) {
+            if (h >= cnt) continue;
+            const double* L = Lm + (size_t)(64 * (k1 - q) + grp) * lda + 64 * (k1 - h) + c;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) gv[q][h][u] = L[(size_t)(8 * u) * lda];
         }
     }
+    if (grp < cnt) rs[grp][c] = y[64 * (k1 - grp) + c];
     if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished
-    const int fail = lm->fail;
-    if (fail) {
-        if (k == nt - 1 && tid < 64) dp[64 * i + tid] = 0.0;  // launch nt-1 has one workgroup per tile
-        return;
-    }
-    // x_k[c] = sum_r M_k[r][c] r_k[r]: lanes over c, waves over r
-    {
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-#pragma unroll
-        for (int t = 0; t < 16; t += 4) {
-            t0 += mv[t] * rv[t];
-            t1 += mv[t + 1] * rv[t + 1];
-            t2 += mv[t + 2] * rv[t + 2];
-            t3 += mv[t + 3] * rv[t + 3];
+    if (lm->fail) {
+        if (k1 == nt - 1) {  // this launch has a workgroup for every tile
+            if (i < k0) {
+                if (tid < 64) dp[64 * i + tid] = 0.0;
+            } else if (grp < cnt) {
+                dp[64 * (k1 - grp) + c] = 0.0;
+            }
         }
-        part[wid][lane] = (t0 + t1) + (t2 + t3);
-    }
-    __syncthreads();
-    if (wid == 0) xk[lane] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-    __syncthreads();
-    if (i == k) {
-        if (tid < 64) dp[64 * k + tid] = xk[tid];
         return;
     }
-    // r_i[c] -= sum_m L[64k + m][64i + c] x_k[m]: lanes over c, waves over m = wid + 4t
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    double lv[kBackGroup][8];
+    __syncthreads();
 #pragma unroll
-    for (int t = 0; t < 16; t += 4) {
-        s0 += lv[t] * xk[wid + 4 * t];
-        s1 += lv[t + 1] * xk[wid + 4 * t + 4];
-        s2 += lv[t + 2] * xk[wid + 4 * t + 8];
-        s3 += lv[t + 3] * xk[wid + 4 * t + 12];
+    for (int q = 0; q < kBackGroup; ++q) {
+        if (q < cnt) {
+            double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                s0 = fma(mv[q][u], rs[q][grp + 8 * u], s0);
+                s1 = fma(mv[q][u + 1], rs[q][grp + 8 * u + 8], s1);
+            }
+            part[0][grp][c] = s0 + s1;
+            if (i < k0) {  // the tile L_ki of the update, while the chain goes on
+                const double* L = Lm + (size_t)(64 * (k1 - q) + grp) * lda + 64 * i + c;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) lv[q][u] = L[(size_t)(8 * u) * lda];
+            }
+            __syncthreads();
+            if (tid < 64) {
+                const double x = ((part[0][0][tid] + part[0][1][tid]) + (part[0][2][tid] + part[0][3][tid])) +
+                                 ((part[0][4][tid] + part[0][5][tid]) + (part[0][6][tid] + part[0][7][tid]));
+                xs[q][tid] = x;
+                if (i == k0) dp[64 * (k1 - q) + tid] = x;
+            }
+            __syncthreads();
+            if (q + 1 < cnt) {
+#pragma unroll
+                for (int h = q + 1; h < kBackGroup; ++h) {
+                    if (h >= cnt) continue;
+                    double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+                    for (int u = 0; u < 8; u += 2) {
+                        t0 = fma(gv[q][h][u], xs[q][grp + 8 * u], t0);
+                        t1 = fma(gv[q][h][u + 1], xs[q][grp + 8 * u + 8], t1);
+                    }
+                    part[h - 1][grp][c] = t0 + t1;
+                }
+                __syncthreads();
+                if (grp > q && grp < cnt) {
+                    const double (*pt)[64] = part[grp - 1];
+                    rs[grp][c] -= ((pt[0][c] + pt[1][c]) + (pt[2][c] + pt[3][c])) +
+                                  ((pt[4][c] + pt[5][c]) + (pt[6][c] + pt[7][c]));
+                }
+                __syncthreads();
+            }
+        }
     }
+    if (i == k0) return;
+    double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < kBackGroup; ++q) {
+        if (q >= cnt) continue;
+#pragma unroll
+        for (int u = 0; u < 8; u += 2) {
+            s0 = fma(lv[q][u], xs[q][grp + 8 * u], s0);
+            s1 = fma(lv[q][u + 1], xs[q][grp + 8 * u + 8], s1);
+        }
+    }
+    __syncthreads();  // part is free (the last step's sums are read)
+    part[0][grp][c] = s0 + s1;
     __syncthreads();
-    part[wid][lane] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    if (wid == 0) y[64 * i + lane] -= (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (tid < 64)
+        y[64 * i + tid] -= ((part[0][0][tid] + part[0][1][tid]) + (part[0][2][tid] + part[0][3][tid])) +
+                           ((part[0][4][tid] + part[0][5][tid]) + (part[0][6][tid] + part[0][7][tid]));
 }
 
 // ---------------------------------------------------------------- per-window systems
@@ -807,104 +842,6 @@ struct WinTiles {
         return (kTileSize / 2) * (i * (i + 1)) + (i == nt - 1 ? kTileStride * last : kTileSize) * j;
     }
 };
-
-// Reciprocal: the hardware's estimate (relative error e below 2^-24) and one
-// step of third order, r (1 + e + e^2).
-__device__ __forceinline__ double fast_rcp(double d) {
-    const double r = __builtin_amdgcn_rcp(d);
-    const double e = fma(-d, r, 1.0);
-    return fma(r, fma(e, e, e), r);
-}
-
-// Four products of 4x4 blocks, D_b = A_b B_b (b = 0..3), with A[i][k] in lane
-// i + 4b + 16k, B[k][j] in lane j + 4b + 16k and D[i][j] in lane j + 4b + 16i
-// (checked on gfx950 against a host product).
-__device__ __forceinline__ double mfma4x4x4(double a, double b) {
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, 0.0, 0, 0, 0);
-}
-
-// LDL^T of a symmetric 16x16 tile and the inverse of its unit factor, by one
-// wave in registers.  acc holds the tile in the matrix instruction's result
-// layout (element v of lane (i, k) = l & 15, l >> 4: row 4 v + k, column i);
-// by symmetry acc[p] is then the column panel 4p..4p+3 in the layout of an
-// operand (lane (i, k): row i, column 4p + k), so a panel needs no data
-// movement.  Per panel p of four columns:
-//   the 4x4 diagonal block's LDL^T and the inverse N of its unit factor, the
-//     same in every lane from ten lane reads;
-//   W = A_p N^T as four 4x4 blocks, L_p = W D^-1, acc -= W L_p^T;
-//   Z, which starts as the identity and ends as the inverse: Z_p = N Z_p,
-//     Z -= L_p Z_p for the rows below.
-// dv[p] = the reciprocal pivot of column 4p + k in lane (i, k).  Returns false
-// if a pivot was not positive and finite (its values are then arbitrary), the
-// same in every lane.
-// A solve by substitution in 4x4 blocks instead of the inverse was no more
-// accurate over 512 ill-conditioned windows (the same quantiles of the pose and
-// cost errors against the oracle) and 4 us slower on the largest window.
-__device__ __forceinline__ bool tile16_ldl(dbl4 acc, dbl4& Z, double dv[4]) {
-    const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4, i4 = lane & 3;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Z[v] = (4 * v + k == i) ? 1.0 : 0.0;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const double a = acc[p];
-        const int q = 4 * p;
-        const double a00 = lane_value(a, q), a10 = lane_value(a, q + 1), a11 = lane_value(a, q + 17),
-                     a20 = lane_value(a, q + 2), a21 = lane_value(a, q + 18), a30 = lane_value(a, q + 3),
-                     a31 = lane_value(a, q + 19), a22 = lane_value(a, q + 34), a32 = lane_value(a, q + 35),
-                     a33 = lane_value(a, q + 51);
-        const double i0 = fast_rcp(a00);
-        const double l10 = a10 * i0, l20 = a20 * i0, l30 = a30 * i0;
-        const double d1 = fma(-l10, a10, a11), t21 = fma(-l20, a10, a21), t31 = fma(-l30, a10, a31);
-        const double i1 = fast_rcp(d1);
-        const double l21 = t21 * i1, l31 = t31 * i1;
-        const double d2 = fma(-l21, t21, fma(-l20, a20, a22)), t32 = fma(-l31, t21, fma(-l30, a20, a32));
-        const double i2 = fast_rcp(d2);
-        const double l32 = t32 * i2;
-        const double d3 = fma(-l32, t32, fma(-l31, t31, fma(-l30, a30, a33)));
-        const double i3 = fast_rcp(d3);
-        // N, unit lower, element (i & 3, k) in lane (i, k)
-        const double n20 = fma(l21, l10, -l20), n31 = fma(l32, l21, -l31);
-        const double n30 = fma(-l32, n20, fma(l31, l10, -l30));
-        double nv = i4 == k ? 1.0 : 0.0;
-        if (i4 == 1 && k == 0) nv = -l10;
-        if (i4 == 2 && k == 0) nv = n20;
-        if (i4 == 2 && k == 1) nv = -l21;
-        if (i4 == 3 && k == 2) nv = -l32;
-        if (i4 == 3 && k == 1) nv = n31;
-        if (i4 == 3 && k == 0) nv = n30;
-        dv[p] = k == 0 ? i0 : k == 1 ? i1 : k == 2 ? i2 : i3;
-        if (p < 3) {
-            const double w = mfma4x4x4(nv, a);  // W[i][k]
-            const double zp = mfma4x4x4(nv, Z[p]);  // row 4p + k, column i of N Z_p
-            const double lp = w * dv[p];
-            acc = mfma16x16x4(-w, lp, acc);
-            Z = mfma16x16x4(i >= q + 4 ? -lp : 0.0, zp, Z);
-            Z[p] = zp;
-        } else {
-            Z[p] = mfma4x4x4(nv, Z[p]);
-        }
-    }
-    bool good = true;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) good = good && dv[p] > 0.0 && isfinite(dv[p]);
-    return __all(good);
-}
-
-// Sum over the four lanes (i, 0..3), in each of them: row pairs, then halves.
-__device__ __forceinline__ double sum_over_k(double v) {
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
-    const auto l1 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-    const auto h1 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-    const double s = __longlong_as_double(((long long)h1[0] << 32) | l1[0]) +
-                     __longlong_as_double(((long long)h1[1] << 32) | l1[1]);
-    const long long c = __double_as_longlong(s);
-    const unsigned lo2 = (unsigned)c, hi2 = (unsigned)(c >> 32);
-    const auto l2 = __builtin_amdgcn_permlane32_swap(lo2, lo2, false, false);
-    const auto h2 = __builtin_amdgcn_permlane32_swap(hi2, hi2, false, false);
-    return __longlong_as_double(((long long)h2[0] << 32) | l2[0]) +
-           __longlong_as_double(((long long)h2[1] << 32) | l2[1]);
-}
 
 // One S row f of the window, by one wave.  Lanes 0..53 take three slots of 18
 // 16-byte pairs at a time, so a lane's entry (i, c), (i, c + 1) of the 6x6
@@ -1546,7 +1483,7 @@ void launch_cholesky_solve(const DevProblem& P, const DevState& cur, const DevSt
                            (const double*)W.S, lda, P.n_fc, (const double*)W.g, W.Lm, W.dp, W.lm);
         return;
     }
-    hipLaunchKernelGGL(k_chol_first, dim3(1), dim3(256), 0, st, (const double*)W.S, W.Lm, W.Li, lda, P.n,
+    hipLaunchKernelGGL(k_chol_first, dim3(1), dim3(256), 0, st, (const double*)W.S, W.Li, lda, P.n,
                        (const double*)W.g, W.y, W.lm);
     for (int k = 0; k + 1 < nt; ++k) {
         const int rem = nt - k - 1;
@@ -1562,9 +1499,11 @@ void launch_cholesky_solve(const DevProblem& P, const DevState& cur, const DevSt
                            (const LMDev*)W.lm, (const PoseQT*)cur.pose, (const double*)W.Hc, cand.pose, cand.cam,
                            W.red_scale);
     } else {
-        for (int k = nt - 1; k >= 0; --k)
-            hipLaunchKernelGGL(k_chol_back_tile, dim3(k + 1), dim3(256), 0, st, (const double*)W.Lm,
-                               (const double*)W.Li, lda, nt, k, W.y, W.dp, (const LMDev*)W.lm);
+        for (int k1 = nt - 1; k1 >= 0; k1 -= kBackGroup) {
+            const int cnt = std::min(kBackGroup, k1 + 1);
+            hipLaunchKernelGGL(k_chol_back_group, dim3(k1 - cnt + 2), dim3(kBackThreads), 0, st, (const double*)W.Lm,
+                               (const double*)W.Li, lda, nt, k1, cnt, W.y, W.dp, (const LMDev*)W.lm);
+        }
     }
 }
 

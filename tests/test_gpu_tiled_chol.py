@@ -1,0 +1,40 @@
+"""The tiled factorisation of one problem (64x64 tiles of 16x16 blocks) at the
+sizes where its tiling can go wrong, against the FP64 oracle: less than a block,
+one to four stages of the last tile, a tile's end and one camera past it, and
+from eleven tiles on (the backward step in groups of four tiles) each remainder
+of the groups."""
+import numpy as np
+import pytest
+
+from nav24_amd import problems
+from nav24_amd.abi import NAV_BA_FP64, workload_options
+from oracle import oracle
+from parity_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+# 6 n_free unknowns: 6, 18, 48 and 60 (one tile, 1 to 4 stages), 66 (two unknowns in
+# the second tile), 192 (three whole tiles), 258, 276 (1 and 2 stages of the fifth), 600
+# (ten tiles), 642, 708, 774, 846 (11 to 14 tiles: groups 4+4+3, 4+4+4, 4+4+4+1, 4+4+4+2)
+@pytest.mark.parametrize("n_free", [1, 3, 8, 10, 11, 32, 43, 46, 100, 107, 118, 129, 141])
+def test_tiled_sizes_match_oracle(n_free):
+    """Three LM iterations.  The two solves differ by the order of their FP64
+    sums only; the scene is well conditioned (three views, a few mrad), where the
+    repository's parity bars hold: 1e-9 on costs, 1e-6 on poses."""
+    from nav24_amd.ba import GraphOptimHip
+    p = problems.workload(3, seed=n_free, n_cam=n_free + 2, n_pt=400 + 8 * n_free, obs_min=3, rot_sigma=0.005,
+                          trans_sigma=0.01, point_sigma=0.02)
+    o = workload_options(3)
+    o.precision, o.n_iter = NAV_BA_FP64, 3
+    ref = oracle.solve(p, o)
+    s = GraphOptimHip(0)
+    s.set_solver(1)
+    r, again = s.solve(p, o), s.solve(p, o)
+    s.close()
+    assert (r.iterations, r.trials, r.stop_reason) == (ref.iterations, ref.trials, ref.stop_reason)
+    rel = np.abs(r.cost_history - ref.cost_history).max() / ref.cost_history.max()
+    dT = np.abs(r.T_cw - ref.T_cw).max()
+    say(f"free cameras {n_free}: cost {rel:.1e}, pose {dT:.1e}")
+    assert rel <= 1e-9 and dT <= 1e-6
+    assert np.array_equal(r.T_cw, again.T_cw)
