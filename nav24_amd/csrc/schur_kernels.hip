@@ -7,24 +7,34 @@
 // One workgroup owns one work item: block row f of S, restricted to one group
 // of column cameras (the slots) and one chunk of camera f's observations,
 // taken in rounds:
-//   phase A  one lane per observation a of camera f on a free point p:
-//            W_a = Hpl_a Dinv_p (FP64) and the point go to the lane's row of
-//            an LDS buffer; the diagonal pair (a, a) adds W_a Hpl_a^T
-//            (symmetric, 21 values) and Hpl_a Dinv_p bl_p (6) to the lane's
+//   phase A  one lane per observation a of camera f on a free point p: with
+//            Hpl_a = J_xi,a^T w_a J_X,a, the factor E_a = w_a J_X,a Dinv_p (2x3,
+//            FP64), J_xi,a and the point go to the lane's row of an LDS buffer;
+//            the diagonal pair (a, a) adds J_xi,a^T (E_a w_a J_X,a^T) J_xi,a
+//            (symmetric, 21 values) and J_xi,a^T E_a bl_p (6) to the lane's
 //            registers;
 //   phase B  every lane is bound to one slot (column camera) for the round:
 //            the host split each slot's pairs (a, b) — b a later observation
 //            of a's point on that camera — evenly over the lanes it gave the
 //            slot.  A lane walks its pairs (8-byte entries {b, a's row in the
 //            buffer}, read coalesced, one row per step; its camera, the first
-//            two entries and their weights are loaded before phase A, so their
-//            latency hides behind it), forms W_a Hpl_b^T = (W_a (w_b J_X,b)^T)
-//            J_xi,b from recomputed Jacobians and sums the 6x6 blocks in
-//            registers;
+//            two entries and their weights are loaded during the previous
+//            round's flush), forms Hpl_a Dinv_p Hpl_b^T = J_xi,a^T (E_a (w_b
+//            J_X,b)^T) J_xi,b, whose middle factor is 2x2, from recomputed
+//            Jacobians and sums the 6x6 blocks in registers;
 //   flush    a slot's lanes come in aligned groups of 2 or 4 (per round);
 //            each group adds its sums by DPP swaps, one lane per group stages
 //            them in LDS, and each slot's groups are added in a fixed order to
 //            the slot's accumulator (one writer per entry).
+// Bound by latency and FP64 issue together: two or three waves per SIMD keep the
+// vector units busy for under half of a launch, so registers and LDS per
+// workgroup count as much as operations.  With the 2x2 middle factor a row of the
+// LDS buffer is 14 doubles instead of 22 (W_a, 6x3, and the point), a pair reads 6
+// instead of 11 16-byte words, and the producer/consumer kernel fits three
+// workgroups on a CU: 512 windows 352 -> 280 us per launch, 24 windows 28 -> 24
+// (FP32 Jacobians), 300-keyframe loop 212 -> 197, 60 keyframes 145 -> 137 (per round
+// form, limited by its registers to two workgroups).  Two pairs per step in the
+// consumers, which needs 200 registers, was slower than the third workgroup.
 // A round is 256 observations for the whole workgroup: its 256 lanes share
 // the slots (balance over many lanes), with workgroup barriers between the
 // phases.  (Rounds of 64 observations per wave, each wave with its own
@@ -32,7 +42,7 @@
 // windows, whose rows have under 30 slots.)
 // Every sum has a fixed order: no atomics, so the rows are the same bits on
 // every run.  Work items are dispatched heaviest first (a host-side permutation).
-// T is the type of the Jacobian entries only.  Cameras, points, W, the pair
+// T is the type of the Jacobian entries only.  Cameras, points, E, the pair
 // products and the S-row slots are FP64 for both compute types: the point
 // elimination cancels Hpp against Hpl Dinv Hpl^T, and with a few-view point's
 // Dinv rounded to FP32 the final cost of an uneven window moved by 1e-3
@@ -41,23 +51,40 @@
 
 namespace navba {
 
-constexpr int kWbuf = 22;        // per observation row: W (18), point (3), padding (16-byte rows)
 constexpr int kStageStride = 37; // odd stride of the staged rows (one per lane group, 36 entries)
 
+// An observation a's row in LDS: what a pair (a, b) needs of a.
+//   E_a (6 doubles), the point (3) and the entries of J_xi,a (type T; a pinhole's
+//   two structural zeros left out); or, for the FP64 pinhole, the normalised
+//   image point (x / z, y / z) and 1 / z in place of J_xi,a, whose entries are
+//   products of these, with the focal lengths folded into E_a: 12 doubles.
+// A row is a whole number of 16-byte reads, and its stride in banks is 4 times an
+// odd number, so that the lanes' rows start in all sixteen 16-byte columns.
+template <typename T, int CM>
+struct RowA {
+    static constexpr bool normalised = CM == kCamPinhole && sizeof(T) == 8;
+    static constexpr int stride = normalised || CM == kCamPinhole ? 14 : sizeof(T) == 8 ? 22 : 18;
+    static constexpr int n_xi = CM == kCamPinhole ? 10 : 12;
+    static_assert(normalised || 9 * sizeof(double) + n_xi * sizeof(T) <= stride * sizeof(double), "row size");
+    static_assert(stride % 2 == 0 && (stride / 2) % 2 == 1, "row stride");
+};
+
 // LDS of one work item.
+template <typename T, int CM>
 struct SchurLayout {
-    size_t acc, wbuf, lslot, lrange, red, total;
+    static constexpr int rows = RowA<T, CM>::stride * kBlock, staged = kStageStride * (kBlock / 2);
+    size_t acc, wbuf, lslot, lcam, lrange, red, total;
     __host__ __device__ SchurLayout(int ns) {
         size_t o = 0;
         acc = o;    o += sizeof(double) * 36 * (size_t)ns;            // [slot][36]
-        wbuf = o;   o += sizeof(double) * kWbuf * kBlock;             // also the flush staging
+        wbuf = o;   o += sizeof(double) * (rows > staged ? rows : staged);  // also the flush staging
         lslot = o;  o += sizeof(int) * kBlock;                        // slot of each lane this round
+        lcam = o;   o += sizeof(int) * (size_t)ns;                    // camera per slot
         lrange = o; o += sizeof(int) * 2 * (size_t)ns;                // first lane, lane count per slot
-        red = o;    o += sizeof(double) * (kBlock / kWave) * 27;      // diagonal block and coefficient per wave
-        total = (o + 15) & ~(size_t)15;
+        red = (o + 7) & ~(size_t)7;
+        total = (red + sizeof(double) * (kBlock / kWave) * 27 + 15) & ~(size_t)15;  // diagonal block and coefficient per wave
     }
 };
-static_assert(kStageStride * (kBlock / 2) <= kWbuf * kBlock, "flush staging fits in the observation buffer");
 
 // Inputs of phase A for one observation: its point's state and Hll / bl and
 // its measurement, loaded ahead of use (every load needs only the point index).
@@ -97,58 +124,123 @@ __device__ __forceinline__ void pa_load(const DevProblem& P, const D4* __restric
     for (int i = 0; i < 9; ++i) in.h[i] = Hl[9 * (size_t)p + i];
 }
 
-// Phase A for one observation of camera (Rf, tf): W and the point into row
-// wb, diagonal pair and coefficient into the registers.
+// C = [C00 C01; C10 C11] = E (2x3) J (2x3)^T
+__device__ __forceinline__ void mul_et(const double E[6], const double J[6], double C[4]) {
+    C[0] = E[0] * J[0] + E[1] * J[1] + E[2] * J[2];
+    C[1] = E[0] * J[3] + E[1] * J[4] + E[2] * J[5];
+    C[2] = E[3] * J[0] + E[4] * J[1] + E[5] * J[2];
+    C[3] = E[3] * J[3] + E[4] * J[4] + E[5] * J[5];
+}
+
+// [M0 M1] = J_xi^T C (6x2), J_xi = [A0; A1], skipping the pinhole zeros of J_xi
+// at (0, 4) and (1, 3).
+template <int CM>
+__device__ __forceinline__ void mul_xi_c(const double A0[6], const double A1[6], const double C[4], double M0[6],
+                                         double M1[6]) {
+    constexpr bool zx = CamTraits<CM>::xi_zeros;
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+        if (zx && r == 4) {
+            M0[r] = A1[r] * C[2];
+            M1[r] = A1[r] * C[3];
+        } else if (zx && r == 3) {
+            M0[r] = A0[r] * C[0];
+            M1[r] = A0[r] * C[1];
+        } else {
+            M0[r] = A0[r] * C[0] + A1[r] * C[2];
+            M1[r] = A0[r] * C[1] + A1[r] * C[3];
+        }
+    }
+}
+
+// The rows of a pinhole's J_xi over fx and fy, from the normalised point (a, b) and 1 / z.
+__device__ __forceinline__ void unit_xi(double a, double b, double iz, double A0[6], double A1[6]) {
+    const double ab = a * b;
+    A0[0] = ab;
+    A0[1] = -fma(a, a, 1.0);
+    A0[2] = b;
+    A0[3] = -iz;
+    A0[4] = 0.0;
+    A0[5] = a * iz;
+    A1[0] = fma(b, b, 1.0);
+    A1[1] = -ab;
+    A1[2] = -a;
+    A1[3] = 0.0;
+    A1[4] = -iz;
+    A1[5] = b * iz;
+}
+
+// Phase A for one observation of camera (Rf, tf): E, J_xi and the point into
+// row wb, diagonal pair and coefficient into the registers.
 template <typename T, int CM, typename In>
 __device__ __forceinline__ void schur_phase_a(const DevProblem& P, const double Rf[9], const double tf[3],
                                               const In& in, double lambda, bool g0, double* wb, double coef[6],
                                               double dsum[21]) {
     if (!in.live) return;
+    constexpr bool zx = CamTraits<CM>::xi_zeros;
     EdgeLin<T> La;
     const double sa = edge_linearize_m<CM>(P, Rf, tf, in.x, in.y, in.z, in.u, in.v, La);
     const double wa = (double)huber_weight<T>(sa, P);  // as k_lin_pt, without a gather of w
-    double JXa[6];
+    double JXa[6], E[6];
 #pragma unroll
     for (int j = 0; j < 6; ++j) JXa[j] = (double)La.JX[j];
-    double Ha[18];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        const double A0 = (double)La.Jxi[i] * wa, A1 = (double)La.Jxi[6 + i] * wa;
-#pragma unroll
-        for (int j = 0; j < 3; ++j)  // a pinhole J_xi is zero at (0, 4) and (1, 3)
-            Ha[3 * i + j] = (CamTraits<CM>::xi_zeros && i == 4) ? A1 * JXa[3 + j]
-                          : (CamTraits<CM>::xi_zeros && i == 3) ? A0 * JXa[j] : A0 * JXa[j] + A1 * JXa[3 + j];
-    }
     double Dp[6];
     const double* hp = in.hl();
     point_dinv(hp, lambda, Dp);
     const double d00 = Dp[0], d01 = Dp[1], d02 = Dp[2], d11 = Dp[3], d12 = Dp[4], d22 = Dp[5];
-    double W[18];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        const double h0 = Ha[3 * i], h1 = Ha[3 * i + 1], h2 = Ha[3 * i + 2];
-        W[3 * i + 0] = h0 * d00 + h1 * d01 + h2 * d02;
-        W[3 * i + 1] = h0 * d01 + h1 * d11 + h2 * d12;
-        W[3 * i + 2] = h0 * d02 + h1 * d12 + h2 * d22;
+    for (int i = 0; i < 2; ++i) {
+        const double j0 = JXa[3 * i] * wa, j1 = JXa[3 * i + 1] * wa, j2 = JXa[3 * i + 2] * wa;
+        E[3 * i] = j0 * d00 + j1 * d01 + j2 * d02;
+        E[3 * i + 1] = j0 * d01 + j1 * d11 + j2 * d12;
+        E[3 * i + 2] = j0 * d02 + j1 * d12 + j2 * d22;
     }
+    if constexpr (RowA<T, CM>::normalised) {
+        double xc, yc, zc;
+        transform(Rf, tf, in.x, in.y, in.z, xc, yc, zc);
+        const double iz = recip<double>(zc);
+        wb[0] = xc * iz; wb[1] = yc * iz; wb[2] = iz;
+        wb[3] = in.x; wb[4] = in.y; wb[5] = in.z;
 #pragma unroll
-    for (int e = 0; e < 18; ++e) wb[e] = W[e];
-    wb[18] = in.x; wb[19] = in.y; wb[20] = in.z;
+        for (int j = 0; j < 3; ++j) {
+            wb[6 + j] = E[j] * P.fx;
+            wb[9 + j] = E[3 + j] * P.fy;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 6; ++j) wb[j] = E[j];
+        wb[6] = in.x; wb[7] = in.y; wb[8] = in.z;
+        T* xi = reinterpret_cast<T*>(wb + 9);
+        int q = 0;
+#pragma unroll
+        for (int j = 0; j < 12; ++j)
+            if (!zx || (j != 4 && j != 9)) xi[q++] = La.Jxi[j];
+    }
     if (g0) {
-        // Dinv bl of the point (the right-hand side's point term)
-        const double b0 = hp[6], b1 = hp[7], b2 = hp[8];
-        const double q0 = d00 * b0 + d01 * b1 + d02 * b2;
-        const double q1 = d01 * b0 + d11 * b1 + d12 * b2;
-        const double q2 = d02 * b0 + d12 * b1 + d22 * b2;
+        double A0[6], A1[6], C[4], M0[6], M1[6];
 #pragma unroll
-        for (int i = 0; i < 6; ++i)
-            coef[i] = fma(Ha[3 * i + 2], q2, fma(Ha[3 * i + 1], q1, fma(Ha[3 * i], q0, coef[i])));
+        for (int c = 0; c < 6; ++c) { A0[c] = (double)La.Jxi[c]; A1[c] = (double)La.Jxi[6 + c]; }
+        const double q0 = E[0] * hp[6] + E[1] * hp[7] + E[2] * hp[8];  // E bl of the point
+        const double q1 = E[3] * hp[6] + E[4] * hp[7] + E[5] * hp[8];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            if (zx && i == 4) coef[i] = fma(A1[i], q1, coef[i]);
+            else if (zx && i == 3) coef[i] = fma(A0[i], q0, coef[i]);
+            else coef[i] = fma(A1[i], q1, fma(A0[i], q0, coef[i]));
+        }
+        mul_et(E, JXa, C);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) C[q] *= wa;
+        mul_xi_c<CM>(A0, A1, C, M0, M1);
         int q = 0;
 #pragma unroll
         for (int i = 0; i < 6; ++i)
 #pragma unroll
-            for (int c = i; c < 6; ++c, ++q)
-                dsum[q] = fma(W[3 * i + 2], Ha[3 * c + 2], fma(W[3 * i + 1], Ha[3 * c + 1], fma(W[3 * i], Ha[3 * c], dsum[q])));
+            for (int c = i; c < 6; ++c, ++q) {
+                if (zx && c == 4) dsum[q] = fma(M1[i], A1[c], dsum[q]);
+                else if (zx && c == 3) dsum[q] = fma(M0[i], A0[c], dsum[q]);
+                else dsum[q] = fma(M1[i], A1[c], fma(M0[i], A0[c], dsum[q]));
+            }
     }
 }
 
@@ -168,6 +260,56 @@ __device__ __forceinline__ void pair_add(double sacc[36], const double M0[6], co
         }
 }
 
+// One pair's factors: J_xi,a^T (E_a (w_b J_X,b)^T) = [M0 M1] (6x2) and J_xi,b =
+// [B0; B1] (2x6), from a's row wb and b's Jacobians at the point stored there.
+template <typename T, int CM>
+__device__ __forceinline__ void pair_factors(const DevProblem& P, const double* wb, double wgt, const double Rb[9],
+                                             const double tb[3], double M0[6], double M1[6], double B0[6],
+                                             double B1[6]) {
+    double A0[6], A1[6], C[4];
+    if constexpr (RowA<T, CM>::normalised) {
+        double xc, yc, zc;
+        transform(Rb, tb, wb[3], wb[4], wb[5], xc, yc, zc);
+        const double iz = recip<double>(zc);
+        const double a = xc * iz, b = yc * iz;
+        // J_X,b over its focal length and 1 / z; these and b's Huber weight scale C
+        double J[6], E[6];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            J[c] = fma(a, Rb[6 + c], -Rb[c]);
+            J[3 + c] = fma(b, Rb[6 + c], -Rb[3 + c]);
+        }
+#pragma unroll
+        for (int q = 0; q < 6; ++q) E[q] = wb[6 + q];
+        mul_et(E, J, C);
+        const double wz = wgt * iz, s0 = wz * (P.fx * P.fx), s1 = wz * (P.fy * P.fy);
+        C[0] *= s0; C[2] *= s0;
+        C[1] *= s1; C[3] *= s1;
+        unit_xi(wb[0], wb[1], wb[2], A0, A1);
+        unit_xi(a, b, iz, B0, B1);
+    } else {
+        EdgeLin<T> Lb;
+        edge_linearize_m<CM>(P, Rb, tb, wb[6], wb[7], wb[8], 0.0, 0.0, Lb);
+        double JXb[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) JXb[q] = wgt * (double)Lb.JX[q];  // the Huber weight of b folded in
+        mul_et(wb, JXb, C);
+        const T* xi = reinterpret_cast<const T*>(wb + 9);
+        int q = 0;
+#pragma unroll
+        for (int j = 0; j < 12; ++j) {
+            const bool zero = CamTraits<CM>::xi_zeros && (j == 4 || j == 9);
+            const double v = zero ? 0.0 : (double)xi[q];
+            if (!zero) ++q;
+            if (j < 6) A0[j] = v;
+            else A1[j - 6] = v;
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) { B0[c] = (double)Lb.Jxi[c]; B1[c] = (double)Lb.Jxi[6 + c]; }
+    }
+    mul_xi_c<CM>(A0, A1, C, M0, M1);
+}
+
 // Phase B: the lane's pairs (entry rows of stride kWave from pl, nrow rows; e0,
 // e1 and the weight w0 of e0 already loaded) into sacc, with the camera (R, t).
 // Each load has a pair's work to land: at pair j the weight of entry j + 1
@@ -179,73 +321,11 @@ __device__ __forceinline__ void schur_pairs(const DevProblem& P, const T* __rest
     for (int j = 0; j < nrow && e0.x >= 0; ++j) {
         const double w1 = P.robust ? (double)w[e1.x >= 0 ? e1.x : 0] : 1.0;
         const int2 e2 = j + 2 < nrow ? pl[(size_t)(j + 2) * kWave] : int2{-1, 0};
-        const double* wb = wbuf + e0.y * kWbuf;
-        EdgeLin<T> Lb;
-        edge_linearize_m<CM>(P, Rb, tb, wb[18], wb[19], wb[20], 0.0, 0.0, Lb);
-        // the Huber weight of b folded into J_X,b: W_a (w_b J_X,b)^T J_xi,b
-        double JXb[6];
-#pragma unroll
-        for (int q = 0; q < 6; ++q) JXb[q] = w0 * (double)Lb.JX[q];
-        double M0[6], M1[6];
-#pragma unroll
-        for (int rr = 0; rr < 6; ++rr) {
-            const double v0 = wb[3 * rr], v1 = wb[3 * rr + 1], v2 = wb[3 * rr + 2];
-            M0[rr] = v0 * JXb[0] + v1 * JXb[1] + v2 * JXb[2];
-            M1[rr] = v0 * JXb[3] + v1 * JXb[4] + v2 * JXb[5];
-        }
-        double B0[6], B1[6];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) { B0[c] = (double)Lb.Jxi[c]; B1[c] = (double)Lb.Jxi[6 + c]; }
+        double M0[6], M1[6], B0[6], B1[6];
+        pair_factors<T, CM>(P, wbuf + e0.y * RowA<T, CM>::stride, w0, Rb, tb, M0, M1, B0, B1);
         pair_add<CM>(sacc, M0, M1, B0, B1);
         e0 = e1; w0 = w1;
         e1 = e2;
-    }
-}
-
-// One pair's factors: W_a (w_b J_X,b)^T = [M0 M1] (6x2) and J_xi,b = [B0; B1]
-// (2x6), with b's Jacobians at the point stored in a's W row wb.
-template <typename T, int CM>
-__device__ __forceinline__ void pair_factors(const DevProblem& P, const double* wb, double wgt, const double Rb[9],
-                                             const double tb[3], double M0[6], double M1[6], double B0[6],
-                                             double B1[6]) {
-    EdgeLin<T> Lb;
-    edge_linearize_m<CM>(P, Rb, tb, wb[18], wb[19], wb[20], 0.0, 0.0, Lb);
-    double JXb[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) JXb[q] = wgt * (double)Lb.JX[q];
-#pragma unroll
-    for (int rr = 0; rr < 6; ++rr) {
-        const double v0 = wb[3 * rr], v1 = wb[3 * rr + 1], v2 = wb[3 * rr + 2];
-        M0[rr] = v0 * JXb[0] + v1 * JXb[1] + v2 * JXb[2];
-        M1[rr] = v0 * JXb[3] + v1 * JXb[4] + v2 * JXb[5];
-    }
-#pragma unroll
-    for (int c = 0; c < 6; ++c) { B0[c] = (double)Lb.Jxi[c]; B1[c] = (double)Lb.Jxi[6 + c]; }
-}
-
-// Phase B two pairs at a time (the same sums, in the same order, as
-// schur_pairs): the two pairs' Jacobians and products are independent, so
-// their latencies overlap.  e[0..3] are the lane's first four entries (or
-// {-1, 0} past its share) and wa, wb the weights of the first two.  Each
-// step issues the weights of the next two entries and the entries two steps
-// ahead.
-template <typename T, int CM>
-__device__ __forceinline__ void schur_pairs2(const DevProblem& P, const T* __restrict__ w, const double* wbuf,
-                                             const int2* pl, int nrow, int2 eA, int2 eB, int2 eC, int2 eD,
-                                             double wA, double wB, const double Rb[9], const double tb[3],
-                                             double sacc[36]) {
-    for (int j = 0; j < nrow && eA.x >= 0; j += 2) {
-        const double wC = P.robust ? (double)w[eC.x >= 0 ? eC.x : 0] : 1.0;
-        const double wD = P.robust ? (double)w[eD.x >= 0 ? eD.x : 0] : 1.0;
-        const int2 eE = j + 4 < nrow ? pl[(size_t)(j + 4) * kWave] : int2{-1, 0};
-        const int2 eF = j + 5 < nrow ? pl[(size_t)(j + 5) * kWave] : int2{-1, 0};
-        double MA0[6], MA1[6], BA0[6], BA1[6], MB0[6], MB1[6], BB0[6], BB1[6];
-        pair_factors<T, CM>(P, wbuf + eA.y * kWbuf, wA, Rb, tb, MA0, MA1, BA0, BA1);
-        pair_factors<T, CM>(P, wbuf + eB.y * kWbuf, wB, Rb, tb, MB0, MB1, BB0, BB1);
-        pair_add<CM>(sacc, MA0, MA1, BA0, BA1);
-        if (eB.x >= 0) pair_add<CM>(sacc, MB0, MB1, BB0, BB1);
-        eA = eC; eB = eD; wA = wC; wB = wD;
-        eC = eE; eD = eF;
     }
 }
 
@@ -297,12 +377,13 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
     if (!running(lm, win)) return;
     const double lambda = lm[win].lambda;
     const bool g0 = (g == 0);
-    const SchurLayout L(ns);
+    const SchurLayout<T, CM> L(ns);
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
     double* acc = reinterpret_cast<double*>(smem + L.acc);
     double* wbuf = reinterpret_cast<double*>(smem + L.wbuf);
     int* lslot = reinterpret_cast<int*>(smem + L.lslot);
+    int* lcam = reinterpret_cast<int*>(smem + L.lcam);
     int* lfirst = reinterpret_cast<int*>(smem + L.lrange);
     int* lcount = lfirst + ns;
     double* red = reinterpret_cast<double*>(smem + L.red);
@@ -316,6 +397,8 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
 #pragma unroll
     for (int k = 0; k < 21; ++k) dsum[k] = 0.0;
 
+    for (int s = tid; s < ns; s += kBlock) lcam[s] = P.free_cam[P.colcam[col0 + s]];
+    __syncthreads();
     const int rnd0 = P.sitem_rnd0[it];
     const int nrounds = (a1 - a0 + kBlock - 1) / kBlock;
     for (int r = 0; r < nrounds; ++r) {
@@ -332,7 +415,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
         double w0 = 1.0;
         double Rb[9], tb[3];
         if (busy) {
-            load_cam(cam, P.free_cam[P.colcam[col0 + sl]], Rb, tb);
+            load_cam(cam, lcam[sl], Rb, tb);
             e0 = pl[0];
             if (nrow > 1) e1 = pl[kWave];
             if (P.robust && e0.x >= 0) w0 = (double)w[e0.x];
@@ -344,7 +427,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
             load_cam(cam, cf, Rf, tf);
             PaLazy in;
             pa_load_lazy(P, X, Hl, k, P.c_pt[k], in);
-            schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + tid * kWbuf, coef, dsum);
+            schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + tid * RowA<T, CM>::stride, coef, dsum);
         }
         lslot[tid] = sl;
         for (int s = tid; s < ns; s += kBlock) lcount[s] = 0;
@@ -407,7 +490,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
 
 // ---- Producer/consumer variant: the item's lanes split by role, slots bound per item.
 // Waves 0-1 (producers) run phase A on rounds of kPcRound observations, one
-// per lane, into one of two W buffers; waves 2-3 (consumers) are bound to one
+// per lane, into one of two row buffers; waves 2-3 (consumers) are bound to one
 // slot each for the whole item and sum the pairs of the previous round from
 // the other buffer, so the two phases overlap and one barrier per round
 // separates them.  Each consumer lane keeps its slot's sum in registers
@@ -417,23 +500,24 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
 // producers' registers the same way (staged rows, then fixed partial sums).
 // Host tables: rnd_lane_slot is [items][kPcCons], rnd_rows.x / .y are the
 // pair rows of the two consumer waves.
+template <typename T, int CM>
 struct PcLayout {
+    static constexpr int rows = RowA<T, CM>::stride * 2 * kPcRound, staged = kPcCons * kStageStride;
     size_t wbuf, lslot, lrange, red, total;
     __host__ __device__ PcLayout(int ns) {
         size_t o = 0;
-        wbuf = o;   o += sizeof(double) * kWbuf * 2 * kPcRound;       // two W buffers; staging at the end
+        wbuf = o;   o += sizeof(double) * (rows > staged ? rows : staged);  // two row buffers; staging at the end
         lslot = o;  o += sizeof(int) * kPcCons;
         lrange = o; o += sizeof(int) * 2 * (size_t)ns;                // first consumer lane, end lane per slot
         red = o;    o += sizeof(double) * 4 * 27;                     // diagonal + coefficient, 4 partial sums
         total = (o + 15) & ~(size_t)15;
     }
 };
-static_assert(kPcCons * kStageStride <= kWbuf * 2 * kPcRound, "consumer rows fit in the W buffers");
-static_assert(kPcRound * 27 <= kWbuf * 2 * kPcRound, "producer rows fit in the W buffers");
+static_assert(kPcRound * 27 <= kPcCons * kStageStride, "the producers' rows fit in the staging");
 static_assert(kPcRound + kPcCons == kBlock && kPcRound == 2 * kWave, "two producer and two consumer waves");
 
 template <typename T, int CM>
-__global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const CamRT* __restrict__ cam,
+__global__ __launch_bounds__(kBlock, CM == kCamPinhole ? 3 : 2) void k_schur_row_pc(DevProblem P, const CamRT* __restrict__ cam,
                                                          const T* __restrict__ w,
                                                          const double* __restrict__ Hl, const LMDev* lm,
                                                          double* __restrict__ spart) {
@@ -447,7 +531,8 @@ __global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const Cam
     if (!running(lm, win)) return;
     const double lambda = lm[win].lambda;
     const bool g0 = (g == 0);
-    const PcLayout L(ns);
+    constexpr int ws = RowA<T, CM>::stride;
+    const PcLayout<T, CM> L(ns);
     const int tid = threadIdx.x, lane = tid % kWave;
     double* wbuf = reinterpret_cast<double*>(smem + L.wbuf);
     int* lslot = reinterpret_cast<int*>(smem + L.lslot);
@@ -476,13 +561,13 @@ __global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const Cam
         PaIn in;
         pa_load(P, X, Hl, a0 + tid, point_of(0), in);
         int p_next = point_of(1);
-        schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + tid * kWbuf, coef, dsum);
+        schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + tid * ws, coef, dsum);
         pa_load(P, X, Hl, a0 + kPcRound + tid, p_next, in);
         p_next = point_of(2);
         __syncthreads();
         for (int r = 0; r < nrounds; ++r) {
             // in: round r + 1; p_next: round r + 2
-            schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + (((r + 1) & 1) * kPcRound + tid) * kWbuf, coef,
+            schur_phase_a<T, CM>(P, Rf, tf, in, lambda, g0, wbuf + (((r + 1) & 1) * kPcRound + tid) * ws, coef,
                                  dsum);
             pa_load(P, X, Hl, a0 + (r + 2) * kPcRound + tid, p_next, in);
             p_next = point_of(r + 3);
@@ -521,36 +606,29 @@ __global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const Cam
 #pragma unroll
         for (int e = 0; e < 36; ++e) sacc[e] = 0.0;
         if (sl != 255) load_cam(cam, P.free_cam[P.colcam[col0 + sl]], Rb, tb);
-        // round r's pair rows, first four entries and first two weights; the
-        // next round's entries are loaded at the start of a round and their
-        // weights at its end, so both land while the round runs
+        // round r's pair rows, first two entries and first weight; the next
+        // round's entries are loaded at the start of a round and their weight
+        // at its end, so both land while the round runs
         int nrow = 0, nrow_n = 0;
         const int2* pl = nullptr;
         const int2* pl_n = nullptr;
-        int2 e[4], n[4];
-        double wa = 1.0, wb = 1.0, wa_n = 1.0, wb_n = 1.0;
+        int2 e0, e1, n0, n1;
+        double wa = 1.0, wa_n = 1.0;
         auto fetch_entries = [&](int rnd) {
             const int4 rows = P.rnd_rows[rnd];
             nrow_n = cw == 0 ? rows.x : rows.y;
             pl_n = P.pairs + (size_t)P.rnd_pair0[rnd] + (size_t)(cw == 0 ? 0 : rows.x) * kWave + lane;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) n[q] = (sl != 255 && q < nrow_n) ? pl_n[q * kWave] : int2{-1, 0};
+            n0 = (sl != 255 && nrow_n > 0) ? pl_n[0] : int2{-1, 0};
+            n1 = (sl != 255 && nrow_n > 1) ? pl_n[kWave] : int2{-1, 0};
         };
-        auto fetch_weights = [&]() {
-            wa_n = 1.0; wb_n = 1.0;
-            if (P.robust && sl != 255 && nrow_n > 0) {
-                wa_n = (double)w[n[0].x >= 0 ? n[0].x : 0];
-                wb_n = (double)w[n[1].x >= 0 ? n[1].x : 0];
-            }
-        };
+        auto fetch_weight = [&]() { wa_n = P.robust && n0.x >= 0 ? (double)w[n0.x] : 1.0; };
         auto advance = [&]() {
             nrow = nrow_n; pl = pl_n;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) e[q] = n[q];
-            wa = wa_n; wb = wb_n;
+            e0 = n0; e1 = n1;
+            wa = wa_n;
         };
         fetch_entries(rnd0);
-        fetch_weights();
+        fetch_weight();
         __syncthreads();
         // slots' consumer lanes are contiguous: each slot's first and end lane
         if (sl != 255) {
@@ -560,17 +638,9 @@ __global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const Cam
         for (int r = 0; r < nrounds; ++r) {
             advance();
             if (r + 1 < nrounds) fetch_entries(rnd0 + r + 1);
-            // two pairs per step for the pinhole; the fisheye Jacobians leave no
-            // registers for a second pair in flight
-            if (sl != 255) {
-                if constexpr (CamTraits<CM>::xi_zeros)
-                    schur_pairs2<T, CM>(P, w, wbuf + (size_t)(r & 1) * kPcRound * kWbuf, pl, nrow, e[0], e[1], e[2],
-                                        e[3], wa, wb, Rb, tb, sacc);
-                else
-                    schur_pairs<T, CM>(P, w, wbuf + (size_t)(r & 1) * kPcRound * kWbuf, pl, nrow, e[0], e[1], wa, Rb,
-                                       tb, sacc);
-            }
-            if (r + 1 < nrounds) fetch_weights();
+            if (sl != 255)
+                schur_pairs<T, CM>(P, w, wbuf + (size_t)(r & 1) * kPcRound * ws, pl, nrow, e0, e1, wa, Rb, tb, sacc);
+            if (r + 1 < nrounds) fetch_weight();
             __syncthreads();
         }
         if (g0) {
@@ -608,13 +678,16 @@ __global__ __launch_bounds__(kBlock) void k_schur_row_pc(DevProblem P, const Cam
     if (g0 && tid < 6) out[36 * ns + tid] = (red[21 + tid] + red[48 + tid]) + (red[75 + tid] + red[102 + tid]);
 }
 
+template <typename T>
 size_t schur_row_smem(const DevProblem& P) {
-    return P.schur_pc ? PcLayout(P.max_ns).total : SchurLayout(P.max_ns).total;
+    if (P.cam_model == kCamKB8)
+        return P.schur_pc ? PcLayout<T, kCamKB8>(P.max_ns).total : SchurLayout<T, kCamKB8>(P.max_ns).total;
+    return P.schur_pc ? PcLayout<T, kCamPinhole>(P.max_ns).total : SchurLayout<T, kCamPinhole>(P.max_ns).total;
 }
 
 template <typename T>
 int prepare_schur_row(const DevProblem& P) {
-    const size_t bytes = schur_row_smem(P);
+    const size_t bytes = schur_row_smem<T>(P);
     if (bytes > 160 * 1024) return -1;
     const bool kb = P.cam_model == kCamKB8;
     const void* fn = P.schur_pc ? (kb ? (const void*)k_schur_row_pc<T, kCamKB8> : (const void*)k_schur_row_pc<T, kCamPinhole>)
@@ -629,7 +702,7 @@ void launch_schur_row(const DevProblem& P, const DevState& s, const DevWork& W, 
     const bool kb = P.cam_model == kCamKB8;
     auto fn = P.schur_pc ? (kb ? k_schur_row_pc<T, kCamKB8> : k_schur_row_pc<T, kCamPinhole>)
                          : (kb ? k_schur_row<T, kCamKB8> : k_schur_row<T, kCamPinhole>);
-    hipLaunchKernelGGL(fn, dim3(P.n_sitems), dim3(kBlock), schur_row_smem(P), st, P, s.cam, (const T*)W.w,
+    hipLaunchKernelGGL(fn, dim3(P.n_sitems), dim3(kBlock), schur_row_smem<T>(P), st, P, s.cam, (const T*)W.w,
                        (const double*)W.Hl, (const LMDev*)W.lm, W.spart);
 }
 
