@@ -2,18 +2,23 @@
 //
 // Hand-written adjoint of C = sum rho(|z - pi_d(T X)|^2) for a batch of
 // problems sharing one pinhole + radial-tangential camera.  The observation
-// structure is uploaded once (point-major order, tiles of whole points that
-// never span two problems, camera-major index lists); each evaluation runs
-//   k_cg_obs    one lane per observation: cost term and its adjoint; the
-//               point gradient is summed per point from LDS in fixed order,
-//               cost and intrinsic gradients per tile, and the pose gradient
-//               term of each observation goes to a buffer;
-//   k_cg_cam    one workgroup per camera: its observations' pose terms in
-//               camera-major order (fixed order);
-//   k_cg_final  per-problem costs and the intrinsic gradient over the tiles.
-// The forward (cost only) skips the adjoint and the second kernel.
+// structure is uploaded once, in two orders: point-major, in tiles of whole
+// points and groups of consecutive tiles that never span two problems, and
+// camera-major, in chunks of one camera's observations.  Each evaluation runs
+//   k_cg_obs    one workgroup per group: cost terms and their adjoint, a lane
+//               per observation of a tile; the point gradient is summed per
+//               point from LDS in fixed order, cost and intrinsic gradients per
+//               group; in the same launch one workgroup per camera chunk: its
+//               pose gradient, from the terms formed again in camera-major
+//               order; and zeros for the points without observations;
+//   k_cg_final  per-problem costs, the total and the intrinsic gradient over the
+//               groups, the pose gradients over the chunks (fixed order).
+// The forward (cost only) runs the groups without the adjoint.
 // T = double or float: the projection and residual are FP64 either way, the
-// adjoint runs in T; tile partials and the final sums are FP64.
+// adjoint runs in T; partial and final sums are FP64.
+// Forming an observation's terms twice costs less than one pass that writes six
+// pose terms per observation (72 MB at 3 M observations, float) for a second one
+// to gather.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,23 +37,35 @@ using navba::wave_sum;
 
 constexpr int kTileObs = 256;  // observations per tile (whole points; one larger point has a tile of its own)
 constexpr int kThreads = 256;
+// Groups and chunks are as long as still leaves kGroups and kChunks of them (eight
+// and four workgroups per CU), so that their sums over the workgroup come once in
+// many observations, and at most kGroupTiles tiles, kChunkMax observations.
+constexpr int kXcds = 8;
+constexpr int kGroups = 2048;
+constexpr int kChunks = 1024;
+constexpr int kGroupTiles = 8;
+constexpr int kChunkMax = 4096;
 constexpr int kPoseThreads = 64;  // one pose per thread: a wave per workgroup spreads few poses over the CUs
 
 struct CostProblem {
-    int n_obs, n_tiles, n_cam, n_pt, n_prob;
+    int n_obs, n_groups, n_chunks, n_unseen, n_cam, n_pt, n_prob;
     int robust;
     double delta;
     const int* o_cam;      // point-major, caller (global) camera index
     const int* o_pt;       // point-major, caller (global) point index
-    const double* uv_d;    // 2 per observation (FP64 for both compute types: the residual is FP64)
+    const double2* uv;     // point-major (FP64 for both compute types: the residual is FP64)
     const int* pt_list;    // unique points with observations, ascending
     const int* pt_ptr;     // [n_pts_used + 1]
     const int* tile_obs;   // [n_tiles + 1]
     const int* tile_pt;    // [n_tiles + 1] range in pt_list
-    const int* tile_prob;  // [n_tiles]
-    const int* prob_tile0; // [n_prob + 1]
-    const int* cam_ptr;    // [n_cam + 1] camera-major lists
-    const int* cam_obs;    // positions in point-major order
+    const int* group_tile; // [n_groups + 1]
+    const int* prob_group0; // [n_prob + 1]
+    const int* c_pt;       // camera-major, caller (global) point index
+    const double2* c_uv;   // camera-major
+    const int* chunk_cam;  // [n_chunks]
+    const int* chunk_ptr;  // [n_chunks + 1] range of camera-major observations
+    const int* cam_chunk0; // [n_cam + 1]
+    const int* unseen;     // [n_unseen] points without observations
 };
 
 template <typename T>
@@ -62,13 +79,17 @@ struct ObsGrad {
 template <typename T>
 __device__ __forceinline__ T sqrt_t(T v) { return sqrt(v); }
 
-// Cost term of one observation and, if kGrad, its adjoint.  The projection
+// What of an observation's terms a caller wants: the cost, with the gradients
+// to point and intrinsics, or the gradient to the pose alone.
+enum Want { kCost = 0, kPointSide = 1, kPoseSide = 2 };
+
+// Cost term of one observation and, unless kCost, its adjoint.  The projection
 // and residual are formed in FP64 whatever T is: the residual is a difference
 // of two pixel coordinates of a few hundred pixels, and in FP32 that
 // cancellation alone left the cost of an FP32 problem 6.6e-4 off its FP64
 // value (FP64 issues at the FP32 rate on gfx950 without packed math, so the
 // forward costs the same).  The adjoint then runs in T.
-template <typename T, bool kGrad>
+template <typename T, Want kWant>
 __device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __restrict__ X, const T in[8], double u,
                                          double v, int robust, double delta, ObsGrad<T>& g) {
     const double R0 = Tcw[0], R1 = Tcw[1], R2 = Tcw[2], R3 = Tcw[3], R4 = Tcw[4], R5 = Tcw[5];
@@ -77,7 +98,7 @@ __device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __r
     const double Xc0 = R0 * x0 + R1 * x1 + R2 * x2 + (double)Tcw[9];
     const double Xc1 = R3 * x0 + R4 * x1 + R5 * x2 + (double)Tcw[10];
     const double Xc2 = R6 * x0 + R7 * x1 + R8 * x2 + (double)Tcw[11];
-    const double iz = 1.0 / Xc2;
+    const double iz = navba::recip<double>(Xc2);
     const double x = Xc0 * iz, y = Xc1 * iz;
     const double fx = in[0], fy = in[1], cx = in[2], cy = in[3], k1 = in[4], k2 = in[5], p1 = in[6], p2 = in[7];
     const double r2 = x * x + y * y;
@@ -98,7 +119,7 @@ __device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __r
         g.cost = 2.0 * delta * r - d2;
         w = delta / r;
     }
-    if (!kGrad) return;
+    if (kWant == kCost) return;
     // the adjoint in T from the FP64 forward values
     const T tx = (T)x, ty = (T)y, tr2 = (T)r2, trad = (T)rad, txy = (T)xy, tiz = (T)iz;
     const T tk1 = in[4], tk2 = in[5], tp1 = in[6], tp2 = in[7], tfx = in[0], tfy = in[1];
@@ -134,126 +155,215 @@ __device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __r
     g.gpose[5] = gc2;
 }
 
-// One workgroup per tile.  part[t] = {cost, d/d intrinsics (8)} of the tile (FP64).
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+// Sum over the two (four) lanes that differ in bit 4 (and 5) of their index, in each of them.
+__device__ __forceinline__ double sum_quarters(double v) {
+    const long long b = __double_as_longlong(v);
+    const auto l1 = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+    const auto h1 = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    const double s = __longlong_as_double(((long long)h1[0] << 32) | l1[0]) +
+                     __longlong_as_double(((long long)h1[1] << 32) | l1[1]);
+    const long long c = __double_as_longlong(s);
+    const auto l2 = __builtin_amdgcn_permlane32_swap((unsigned)c, (unsigned)c, false, false);
+    const auto h2 = __builtin_amdgcn_permlane32_swap((unsigned)(c >> 32), (unsigned)(c >> 32), false, false);
+    return __longlong_as_double(((long long)h2[0] << 32) | l2[0]) +
+           __longlong_as_double(((long long)h2[1] << 32) | l2[1]);
+}
+
+// Sums of N values per lane over the workgroup, in a fixed order: value q in
+// thread q < N.  A wave's 64 lanes are added by a matrix instruction with a
+// second operand of ones (16 row sums of four lanes each, four to a lane), then
+// within lanes and over the lanes' quarters: half the instructions of a sum by
+// lane moves.
+template <int N>
+__device__ __forceinline__ double block_sums(const double v[N], double (*red)[N]) {
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        const dbl4 r = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q], 1.0, dbl4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+        const double s = sum_quarters((r[0] + r[1]) + (r[2] + r[3]));
+        if (lane == 0) red[wid][q] = s;
+    }
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x < N)
+        for (int i = 0; i < kThreads / kWave; ++i) s += red[i][threadIdx.x];
+    return s;
+}
+
+// Item of workgroup b of n: workgroups b = x (mod kXcds) run on one XCD and take
+// consecutive items, so the points and poses that these share stay in its L2.
+__device__ __forceinline__ int xcd_band(int b, int n) {
+    const int x = b % kXcds, lo = n / kXcds, more = n % kXcds;
+    return x * lo + min(x, more) + b / kXcds;
+}
+
+// Workgroups 0 .. n_groups - 1: part[q n_groups + group] = {cost, d / d intrinsics
+// (8)}[q] (FP64); with kGrad the next n_chunks (if gpart): gpart[6 chunk + j]; then those that
+// clear the unseen points' gradients.  Bound by the FP64 operations of the terms
+// and by memory together: 24 bytes per observation in one order and 20 in the
+// other.  64 scenes of 5 000 points (3.16 M observations, float): 67 us for a
+// gradient and 20 for the cost alone (3.8 TB/s), with the sums over groups and
+// chunks in 4; before, 77 us, 60 in a gather of the pose terms and 59 in one
+// workgroup's sums over all tiles.  One scene of 700 points: 6 us and 2.4,
+// before 28 in all.
 template <typename T, bool kGrad>
-__global__ __launch_bounds__(kThreads) void k_cg_obs(CostProblem P, const T* __restrict__ Tcw,
+__global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const T* __restrict__ Tcw,
                                                      const T* __restrict__ X, const T* __restrict__ intr,
-                                                     T* __restrict__ gpo, T* __restrict__ gX,
-                                                     double* __restrict__ part) {
-    __shared__ T sh[3][kTileObs];
-    __shared__ double red[kThreads / kWave];
-    __shared__ T redp[kThreads / kWave][3];
-    const int t = blockIdx.x;
-    const int o0 = P.tile_obs[t], o1 = P.tile_obs[t + 1];
-    const int q0 = P.tile_pt[t], q1 = P.tile_pt[t + 1];
+                                                     T* __restrict__ gX, double* __restrict__ part,
+                                                     double* __restrict__ gpart) {
+    constexpr int kSums = kGrad ? 9 : 1;
+    __shared__ T sh[2][3][kTileObs];
+    __shared__ double red[kThreads / kWave][kSums];
+    __shared__ double redc[kThreads / kWave][6];
+    const int tid = threadIdx.x;
     T in[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) in[k] = intr[k];
-    double cost = 0.0, gi[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    T gp[3] = {T(0), T(0), T(0)};
-    for (int a = o0 + (int)threadIdx.x; a < o1; a += kThreads) {
-        const int c = P.o_cam[a], q = P.o_pt[a];
-        const double* uv = P.uv_d + 2 * (size_t)a;
-        ObsGrad<T> g;
-        obs_term<T, kGrad>(Tcw + 12 * (size_t)c, X + 3 * (size_t)q, in, uv[0], uv[1], P.robust, P.delta, g);
-        cost += g.cost;
-        if (kGrad) {
+    int b = blockIdx.x;
+    if (b < P.n_groups) {
+        b = xcd_band(b, P.n_groups);
+        double acc[kSums];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) gi[k] += (double)g.gintr[k];
+        for (int k = 0; k < kSums; ++k) acc[k] = 0.0;
+        const int t0 = P.group_tile[b], t1 = P.group_tile[b + 1];
+        int o0 = P.tile_obs[t0], c = 0, q = 0;
+        double2 uv;
+        // the lane's first observation of tile t, loaded while the tile before is worked on
+        auto load = [&](int a, int o1) {
+            if (a < o1) {
+                c = P.o_cam[a];
+                q = P.o_pt[a];
+                uv = P.uv[a];
+            }
+        };
+        load(o0 + tid, P.tile_obs[t0 + 1]);
+        for (int t = t0; t < t1; ++t) {
+            const int o1 = P.tile_obs[t + 1];
+            const bool one = o1 - o0 > kTileObs;  // one point with more than kTileObs observations
+            // the point that this thread sums, loaded before the terms are formed
+            int q0 = 0, n_sum = 0, pt = 0, a0 = 0, a1 = 0;
+            auto point = [&](int p) {
+                pt = P.pt_list[p];
+                a0 = P.pt_ptr[p];
+                a1 = P.pt_ptr[p + 1];
+            };
+            if (kGrad && gX) {
+                q0 = P.tile_pt[t];
+                n_sum = 3 * (P.tile_pt[t + 1] - q0);
+                if (tid < n_sum) point(q0 + tid / 3);
+            }
+            T gp[3] = {T(0), T(0), T(0)};
+            for (int a = o0 + tid; a < o1; a += kThreads) {
+                const T* Tc = Tcw + 12 * (size_t)c;
+                const T* Xq = X + 3 * (size_t)q;
+                const double u = uv.x, v = uv.y;
+                if (a + kThreads < o1) load(a + kThreads, o1);
+                ObsGrad<T> g;
+                obs_term<T, kGrad ? kPointSide : kCost>(Tc, Xq, in, u, v, P.robust, P.delta, g);
+                acc[0] += g.cost;
+                if constexpr (kGrad) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) gpo[6 * (size_t)a + k] = g.gpose[k];
-            gp[0] += g.gX[0]; gp[1] += g.gX[1]; gp[2] += g.gX[2];
-        }
-    }
-    if (kGrad && gX) {  // uniform: gX is a kernel argument
-        if (o1 - o0 <= kTileObs) {
-            // one observation per lane: per-point sums in fixed order from LDS
-            sh[0][threadIdx.x] = gp[0]; sh[1][threadIdx.x] = gp[1]; sh[2][threadIdx.x] = gp[2];
-            __syncthreads();
-            for (int i = q0 + (int)threadIdx.x; i < q1; i += kThreads) {
-                T s0 = T(0), s1 = T(0), s2 = T(0);
-                for (int a = P.pt_ptr[i]; a < P.pt_ptr[i + 1]; ++a) {
-                    s0 += sh[0][a - o0]; s1 += sh[1][a - o0]; s2 += sh[2][a - o0];
+                    for (int k = 0; k < 8; ++k) acc[1 + k] += (double)g.gintr[k];
+                    gp[0] += g.gX[0]; gp[1] += g.gX[1]; gp[2] += g.gX[2];
                 }
-                const int q = P.pt_list[i];
-                gX[3 * (size_t)q] = s0; gX[3 * (size_t)q + 1] = s1; gX[3 * (size_t)q + 2] = s2;
             }
-        } else {
-            // one point with more than kTileObs observations
-            const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+            if (t + 1 < t1) load(o1 + tid, P.tile_obs[t + 2]);
+            if (kGrad && gX) {  // uniform: gX is a kernel argument
+                T (*st)[kTileObs] = sh[(t - t0) & 1];  // written again two tiles, hence a barrier, later
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const T v = wave_sum(gp[k]);
-                if (lane == 0) redp[wid][k] = v;
+                for (int k = 0; k < 3; ++k) st[k][tid] = gp[k];
+                __syncthreads();
+                // per-point sums in fixed order, a thread per point and component
+                for (int i = tid; i < n_sum; i += kThreads) {
+                    if (i != tid) point(q0 + i / 3);
+                    const T* v = st[i % 3];
+                    int a = one ? 0 : a0 - o0;
+                    const int e = one ? kThreads : a1 - o0;
+                    T s = T(0);
+                    for (; a + 4 <= e; a += 4) {
+                        const T v0 = v[a], v1 = v[a + 1], v2 = v[a + 2], v3 = v[a + 3];
+                        s = (((s + v0) + v1) + v2) + v3;
+                    }
+                    for (; a < e; ++a) s += v[a];
+                    gX[3 * (size_t)pt + i % 3] = s;
+                }
             }
-            __syncthreads();
-            if (threadIdx.x < 3) {
-                T s = T(0);
-                for (int i = 0; i < kThreads / kWave; ++i) s += redp[i][threadIdx.x];
-                gX[3 * (size_t)P.pt_list[q0] + threadIdx.x] = s;
-            }
+            o0 = o1;
         }
-    }
-    const double cs = block_sum<double, kThreads>(cost, red);
-    if (threadIdx.x == 0) part[9 * (size_t)t] = cs;
-    if (kGrad) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            __syncthreads();
-            const double v = block_sum<double, kThreads>(gi[k], red);
-            if (threadIdx.x == 0) part[9 * (size_t)t + 1 + k] = v;
-        }
-    }
-}
-
-// One workgroup per camera: d C / d xi in fixed order over its observations.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_cg_cam(CostProblem P, const T* __restrict__ gpo, T* __restrict__ gpose) {
-    __shared__ double red[kThreads / kWave];
-    const int c = blockIdx.x;
-    double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = P.cam_ptr[c] + (int)threadIdx.x; k < P.cam_ptr[c + 1]; k += kThreads) {
-        const int a = P.cam_obs[k];
-#pragma unroll
-        for (int j = 0; j < 6; ++j) acc[j] += (double)gpo[6 * (size_t)a + j];
-    }
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        __syncthreads();
-        const double v = block_sum<double, kThreads>(acc[j], red);
-        if (threadIdx.x == 0) gpose[6 * (size_t)c + j] = (T)v;
-    }
-}
-
-// Workgroup p < n_prob: cost of problem p over its tiles; workgroup n_prob:
-// the total cost and the intrinsic gradient over all tiles (fixed order).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_cg_final(CostProblem P, const double* __restrict__ part, int grad,
-                                                       T* __restrict__ cost, T* __restrict__ total,
-                                                       T* __restrict__ gintr) {
-    __shared__ double red[kThreads / kWave];
-    const int pr = blockIdx.x;
-    if (pr < P.n_prob) {
-        double s = 0.0;
-        for (int t = P.prob_tile0[pr] + (int)threadIdx.x; t < P.prob_tile0[pr + 1]; t += kThreads)
-            s += part[9 * (size_t)t];
-        const double v = block_sum<double, kThreads>(s, red);
-        if (threadIdx.x == 0) cost[pr] = (T)v;
+        const double s = block_sums<kSums>(acc, red);
+        if (tid < kSums) part[(size_t)tid * P.n_groups + b] = s;
         return;
     }
-    if (total) {
-        double s = 0.0;
-        for (int t = threadIdx.x; t < P.n_tiles; t += kThreads) s += part[9 * (size_t)t];
-        const double v = block_sum<double, kThreads>(s, red);
-        if (threadIdx.x == 0) *total = (T)v;
+    if constexpr (kGrad) {
+        b -= P.n_groups;
+        if (gpart) {
+            if (b < P.n_chunks) {
+                b = xcd_band(b, P.n_chunks);
+                double acc[6] = {0, 0, 0, 0, 0, 0};
+                const T* Tc = Tcw + 12 * (size_t)P.chunk_cam[b];
+                const int k1 = P.chunk_ptr[b + 1];
+                int k = P.chunk_ptr[b] + tid, q = 0;
+                double2 uv;
+                if (k < k1) {
+                    q = P.c_pt[k];
+                    uv = P.c_uv[k];
+                }
+                for (; k < k1; k += kThreads) {
+                    const T* Xq = X + 3 * (size_t)q;
+                    const double u = uv.x, v = uv.y;
+                    if (k + kThreads < k1) {
+                        q = P.c_pt[k + kThreads];
+                        uv = P.c_uv[k + kThreads];
+                    }
+                    ObsGrad<T> g;
+                    obs_term<T, kPoseSide>(Tc, Xq, in, u, v, P.robust, P.delta, g);
+#pragma unroll
+                    for (int j = 0; j < 6; ++j) acc[j] += (double)g.gpose[j];
+                }
+                const double s = block_sums<6>(acc, redc);
+                if (tid < 6) gpart[6 * (size_t)b + tid] = s;
+                return;
+            }
+            b -= P.n_chunks;
+        }
+        const int i = b * kThreads + tid;
+        if (gX && i < P.n_unseen)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) gX[3 * (size_t)P.unseen[i] + k] = T(0);
     }
-    if (!grad || !gintr) return;
-    for (int k = 0; k < 8; ++k) {
+}
+
+// Workgroup p < n_prob: cost of problem p over its groups; the next n_sums: the
+// total (sum 0) and the intrinsic gradient (1..8) over all groups; the others:
+// pose gradients over the cameras' chunks, a thread per entry (all in a fixed order).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_cg_final(CostProblem P, const double* __restrict__ part, int n_sums,
+                                                       T* __restrict__ cost, T* __restrict__ total,
+                                                       T* __restrict__ gintr, const double* __restrict__ gpart,
+                                                       T* __restrict__ gpose) {
+    __shared__ double red[kThreads / kWave];
+    const int pr = blockIdx.x;
+    if (pr < P.n_prob + n_sums) {
+        const int q = pr < P.n_prob ? 0 : pr - P.n_prob;
+        const int g0 = pr < P.n_prob ? P.prob_group0[pr] : 0, g1 = pr < P.n_prob ? P.prob_group0[pr + 1] : P.n_groups;
         double s = 0.0;
-        for (int t = threadIdx.x; t < P.n_tiles; t += kThreads) s += part[9 * (size_t)t + 1 + k];
+        for (int g = g0 + (int)threadIdx.x; g < g1; g += kThreads) s += part[(size_t)q * P.n_groups + g];
         const double v = block_sum<double, kThreads>(s, red);
-        if (threadIdx.x == 0) gintr[k] = (T)v;
+        if (threadIdx.x == 0) {
+            if (pr < P.n_prob) cost[pr] = (T)v;
+            else if (q > 0 && gintr) gintr[q - 1] = (T)v;
+            else if (q == 0 && total) *total = (T)v;
+        }
+        return;
     }
+    const int i = (pr - P.n_prob - n_sums) * kThreads + (int)threadIdx.x;
+    if (i >= 6 * P.n_cam) return;
+    const int c = i / 6, j = i % 6;
+    double s = 0.0;
+    for (int k = P.cam_chunk0[c]; k < P.cam_chunk0[c + 1]; ++k) s += gpart[6 * (size_t)k + j];
+    gpose[i] = (T)s;
 }
 
 // ---- pose tangents ----------------------------------------------------------
@@ -308,9 +418,8 @@ __device__ __forceinline__ void rot3(const double w[3], double p, double q, cons
 // T = exp(xi) T_cw, one pose per thread.  Launch bound: a few hundred
 // operations and at most 144 bytes per pose.  As torch operations the map and
 // its derivative were about 230 launches of a gradient step; with these two
-// kernels a step of BACost takes 260 us instead of 1970 on 64 scenes of
-// 5 000 points (1 280 poses, float) and 168 instead of 1800 on one of 700
-// (double).
+// kernels a step of BACost (64 scenes of 5 000 points, 1 280 poses, float) went
+// from 1970 us to 260, on one scene of 700 (double) from 1800 to 168.
 template <typename T>
 __global__ void k_se3_left(int n, const T* __restrict__ xi, const T* __restrict__ Tcw, T* __restrict__ out) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -373,11 +482,6 @@ __global__ void k_tangent_grad(int n, const T* __restrict__ xi, const T* __restr
     }
 }
 
-template <typename T>
-__global__ void k_zero(T* p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = T(0);
-}
-
 }  // namespace navcost
 
 using namespace navcost;
@@ -388,9 +492,8 @@ struct nav_ba_cost_handle {
     bool prepared = false;
     CostProblem P{};
     std::vector<void*> bufs;
-    void* gpo = nullptr;
-    size_t gpo_bytes = 0;
-    double* part = nullptr;
+    double* part = nullptr;   // [9][n_groups]
+    double* gpart = nullptr;  // [n_chunks][6]
 };
 
 namespace {
@@ -398,10 +501,7 @@ namespace {
 void free_all(nav_ba_cost_handle* h) {
     for (void* p : h->bufs) (void)hipFree(p);
     h->bufs.clear();
-    if (h->gpo) (void)hipFree(h->gpo);
-    h->gpo = nullptr;
-    h->gpo_bytes = 0;
-    h->part = nullptr;
+    h->part = h->gpart = nullptr;
 }
 
 template <class V>
@@ -431,20 +531,20 @@ int32_t eval_t(nav_ba_cost_handle* h, const T* Tcw, const T* X, const T* intr, T
                T* gintr, hipStream_t s) {
     const CostProblem& P = h->P;
     const bool grad = gpose || gX || gintr;
-    T* gpo = (T*)h->gpo;
-    if (grad && gX) hipLaunchKernelGGL(k_zero<T>, dim3(256), dim3(256), 0, s, gX, (size_t)3 * P.n_pt);
-    if (P.n_tiles > 0) {
-        if (grad)  // gX may be null: the per-point sums are then skipped
-            hipLaunchKernelGGL((k_cg_obs<T, true>), dim3(P.n_tiles), dim3(kThreads), 0, s, P, Tcw, X, intr, gpo, gX,
-                               h->part);
+    const int unseen = gX ? (P.n_unseen + kThreads - 1) / kThreads : 0;
+    const int blocks = P.n_groups + (gpose ? P.n_chunks : 0) + unseen;
+    if (blocks > 0) {
+        if (grad)  // a null gX or gpose skips its part
+            hipLaunchKernelGGL((k_cg_obs<T, true>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, gX, h->part,
+                               gpose ? h->gpart : nullptr);
         else
-            hipLaunchKernelGGL((k_cg_obs<T, false>), dim3(P.n_tiles), dim3(kThreads), 0, s, P, Tcw, X, intr,
-                               (T*)nullptr, (T*)nullptr, h->part);
+            hipLaunchKernelGGL((k_cg_obs<T, false>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, (T*)nullptr,
+                               h->part, (double*)nullptr);
     }
-    if (grad && gpose && P.n_cam > 0)
-        hipLaunchKernelGGL(k_cg_cam<T>, dim3(P.n_cam), dim3(kThreads), 0, s, P, (const T*)gpo, gpose);
-    hipLaunchKernelGGL(k_cg_final<T>, dim3(P.n_prob + 1), dim3(kThreads), 0, s, P, (const double*)h->part,
-                       grad ? 1 : 0, cost, total, gintr);
+    const int n_sums = gintr ? 9 : total ? 1 : 0;
+    const int cam_blocks = gpose ? (6 * P.n_cam + kThreads - 1) / kThreads : 0;
+    hipLaunchKernelGGL(k_cg_final<T>, dim3(P.n_prob + n_sums + cam_blocks), dim3(kThreads), 0, s, P,
+                       (const double*)h->part, n_sums, cost, total, gintr, (const double*)h->gpart, gpose);
     return launch_status(h);
 }
 
@@ -547,14 +647,14 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
         for (size_t k = 0; k < no; ++k) { const int i = byc[k]; ord[poff[gpt[i]]++] = i; }
     }
     std::vector<int> o_cam(no), o_pt(no);
-    std::vector<double> uv_d(2 * no);
+    std::vector<double2> uv(no);
     for (size_t k = 0; k < no; ++k) {
         const int i = ord[k];
         o_cam[k] = gcam[i]; o_pt[k] = gpt[i];
-        uv_d[2 * k] = guv[2 * (size_t)i]; uv_d[2 * k + 1] = guv[2 * (size_t)i + 1];
+        uv[k] = double2{guv[2 * (size_t)i], guv[2 * (size_t)i + 1]};
     }
     // unique points, tiles of whole points per problem
-    std::vector<int> pt_list, pt_ptr{0}, tile_obs{0}, tile_pt{0}, tile_prob, prob_tile0{0};
+    std::vector<int> pt_list, pt_ptr{0}, tile_obs{0}, tile_pt{0}, prob_tile0{0};
     {
         size_t k = 0;
         for (int p = 0; p < n_probs; ++p) {  // a problem's points, hence observations, are contiguous
@@ -576,40 +676,75 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
                 if (j == i) j = i + 1;
                 tile_obs.push_back(pt_ptr[j]);
                 tile_pt.push_back(j);
-                tile_prob.push_back(p);
                 i = j;
             }
-            prob_tile0.push_back((int)tile_prob.size());
+            prob_tile0.push_back((int)tile_pt.size() - 1);
         }
     }
-    std::vector<int> cam_ptr(nc + 1, 0), cam_obs(no);
+    // groups of consecutive tiles of one problem
+    const int n_tiles = prob_tile0.back();
+    const int per_group = std::min(kGroupTiles, std::max(1, n_tiles / kGroups));
+    std::vector<int> group_tile{0}, prob_group0{0};
+    for (int p = 0; p < n_probs; ++p) {
+        for (int t = prob_tile0[p]; t < prob_tile0[p + 1];) {
+            t = std::min(t + per_group, prob_tile0[p + 1]);
+            group_tile.push_back(t);
+        }
+        prob_group0.push_back((int)group_tile.size() - 1);
+    }
+    // camera-major order and its chunks
+    std::vector<int> cam_ptr(nc + 1, 0), c_pt(no);
+    std::vector<double2> c_uv(no);
     for (size_t k = 0; k < no; ++k) cam_ptr[o_cam[k] + 1]++;
     for (int c = 0; c < nc; ++c) cam_ptr[c + 1] += cam_ptr[c];
     {
         std::vector<int> pos(cam_ptr.begin(), cam_ptr.end() - 1);
-        for (size_t k = 0; k < no; ++k) cam_obs[pos[o_cam[k]]++] = (int)k;
+        for (size_t k = 0; k < no; ++k) {
+            const int at = pos[o_cam[k]]++;
+            c_pt[at] = o_pt[k];
+            c_uv[at] = uv[k];
+        }
+    }
+    const int chunk = std::min<int>(kChunkMax, std::max<int>(1, (int)(no / ((size_t)kChunks * kThreads))) * kThreads);
+    std::vector<int> chunk_cam, chunk_ptr{0}, cam_chunk0{0};
+    for (int c = 0; c < nc; ++c) {
+        for (int k = cam_ptr[c]; k < cam_ptr[c + 1];) {
+            k = std::min(cam_ptr[c + 1] - k, chunk) + k;
+            chunk_cam.push_back(c);
+            chunk_ptr.push_back(k);
+        }
+        cam_chunk0.push_back((int)chunk_cam.size());
+    }
+    std::vector<int> unseen;
+    for (int q = 0, i = 0; q < np; ++q) {
+        if (i < (int)pt_list.size() && pt_list[i] == q) ++i;
+        else unseen.push_back(q);
     }
     CostProblem& P = h->P;
     P = CostProblem{};
-    P.n_obs = (int)no; P.n_tiles = (int)tile_prob.size(); P.n_cam = nc; P.n_pt = np; P.n_prob = n_probs;
+    P.n_obs = (int)no; P.n_groups = prob_group0.back(); P.n_chunks = (int)chunk_cam.size();
+    P.n_unseen = (int)unseen.size();
+    P.n_cam = nc; P.n_pt = np; P.n_prob = n_probs;
     P.robust = robust ? 1 : 0;
     P.delta = huber_delta;
     int st;
-    if ((st = up(h, o_cam, &P.o_cam)) || (st = up(h, o_pt, &P.o_pt)) || (st = up(h, uv_d, &P.uv_d)) ||
+    if ((st = up(h, o_cam, &P.o_cam)) || (st = up(h, o_pt, &P.o_pt)) || (st = up(h, uv, &P.uv)) ||
         (st = up(h, pt_list, &P.pt_list)) || (st = up(h, pt_ptr, &P.pt_ptr)) ||
         (st = up(h, tile_obs, &P.tile_obs)) || (st = up(h, tile_pt, &P.tile_pt)) ||
-        (st = up(h, tile_prob, &P.tile_prob)) || (st = up(h, prob_tile0, &P.prob_tile0)) ||
-        (st = up(h, cam_ptr, &P.cam_ptr)) || (st = up(h, cam_obs, &P.cam_obs)))
+        (st = up(h, group_tile, &P.group_tile)) || (st = up(h, prob_group0, &P.prob_group0)) ||
+        (st = up(h, c_pt, &P.c_pt)) || (st = up(h, c_uv, &P.c_uv)) || (st = up(h, chunk_cam, &P.chunk_cam)) ||
+        (st = up(h, chunk_ptr, &P.chunk_ptr)) || (st = up(h, cam_chunk0, &P.cam_chunk0)) ||
+        (st = up(h, unseen, &P.unseen)))
         return st;
     void* part = nullptr;
-    if (hipMalloc(&part, sizeof(double) * 9 * std::max<size_t>(tile_prob.size(), 1)) != hipSuccess) {
+    const size_t n_part = 9 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks;
+    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_part + n_gpart, 1)) != hipSuccess) {
         h->err = "hipMalloc part";
         return NAV_BA_HIP_ERROR;
     }
     h->bufs.push_back(part);
     h->part = (double*)part;
-    h->gpo_bytes = sizeof(double) * 6 * std::max<size_t>(no, 1);
-    if (hipMalloc(&h->gpo, h->gpo_bytes) != hipSuccess) { h->err = "hipMalloc gpo"; return NAV_BA_HIP_ERROR; }
+    h->gpart = h->part + n_part;
     h->prepared = true;
     return NAV_BA_OK;
 }
