@@ -4,7 +4,7 @@
 // cameras, points and observations of window w occupy contiguous ranges, and
 // every kernel covers all windows in one launch.  A single problem is the
 // one-window case.  Each window carries its own LM state on the device, and
-// the accept kernel runs g2o's trial loop per window, so one replayed graph
+// the accept kernel runs g2o's trial loop per window, so one step
 // (linearise if needed, one trial, decide) advances every window at once.
 #pragma once
 
@@ -185,7 +185,6 @@ struct DevWork {
     double* red_aux;    // [n_cblk] outlier counts
     uint8_t* outlier;   // [n_obs] caller order
     double* hist;       // [n_win * (n_iter + 1)] chi2 before / after each iteration
-    double* final;      // [n_win * 2] FP64 final cost, outlier count
     int* done_count;    // windows finished
     LMDev* lm;          // [n_win]
     double* pcg;        // conjugate gradients (one problem): 36 per camera block, x r z p q, partial sums
@@ -202,6 +201,19 @@ struct ResultPlaces {
         X = T + sizeof(double) * 12 * cams;
         flags = (X + sizeof(double) * 3 * pts + 15) & ~(size_t)15;
         total = flags + ((obs + 15) & ~(size_t)15);
+    }
+};
+
+// Offsets in bytes of what the host reads of a run, in one pinned buffer: the count
+// of finished windows (int, at 0), LM states [n_win], costs [n_win][n_iter + 1] and
+// final cost and flag count [n_win][2].
+struct ReportPlaces {
+    size_t lm, hist, final, total;
+    ReportPlaces(size_t n_win, size_t n_iter) {
+        lm = 16;
+        hist = lm + sizeof(LMDev) * n_win;
+        final = hist + sizeof(double) * n_win * (n_iter + 1);
+        total = final + sizeof(double) * 2 * n_win;
     }
 };
 
@@ -278,7 +290,7 @@ __device__ __forceinline__ double camera_candidate(const CamIn& ci, double lambd
 // Launchers.  T = double (FP64 path) or float (mixed path).
 template <typename T> int prepare_schur_row(const DevProblem& P);  // LDS attribute; < 0 if too large
 void launch_cam_rt(const DevProblem& P, const DevState& s, hipStream_t st);
-void launch_lm_reset(const DevProblem& P, const DevWork& W, hipStream_t st);
+void launch_run_start(const DevProblem& P, const DevState& init, const DevState& cur, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lin_pt(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lin_cam(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lambda_init(const DevProblem& P, const DevWork& W, hipStream_t st);
@@ -323,7 +335,8 @@ void launch_lm_accept(const DevProblem& P, const DevState& cur, const DevState& 
 void launch_lm_set_chi(const DevProblem& P, const DevWork& W, hipStream_t st);
 void launch_commit(const DevProblem& P, const DevState& cur, const DevState& cand, const DevWork& W, hipStream_t st);
 void launch_flags(const DevProblem& P, const DevState& s, const DevWork& W, double thr, hipStream_t st);
-void launch_final(const DevProblem& P, const DevWork& W, hipStream_t st);
+void launch_report(const DevProblem& P, const DevWork& W, const ReportPlaces& at, bool state, bool final, char* out,
+                   hipStream_t st);
 // The results in caller order into `out` (device-visible host memory): pt_src
 // the local point of each caller point, or -1 (then the caller's own, from x_in);
 // compat rounds the points to float.

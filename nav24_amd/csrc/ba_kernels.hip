@@ -43,20 +43,38 @@ void launch_cam_rt(const DevProblem& P, const DevState& s, hipStream_t st) {
     hipLaunchKernelGGL(k_cam_rt, dim3((P.n_cam + 255) / 256), dim3(256), 0, st, P.n_cam, s.pose, s.cam);
 }
 
-__global__ void k_lm_reset(int n_win, int n_iter, double lambda0, LMDev* lm, int* done_count) {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w == 0) *done_count = n_iter > 0 ? 0 : n_win;
-    if (w >= n_win) return;
-    LMDev L{};
-    L.lambda = lambda0;
-    L.nu = 2.0;
-    L.phase = n_iter > 0 ? kPhaseLin : kPhaseDone;
-    lm[w] = L;
+// A run's start in one launch: poses and points from the prepared state, the
+// cameras' R|t, and every window's LM state.  (Two copies, two launches and
+// their gaps before it, about 10 us of a run.)
+__global__ __launch_bounds__(256) void k_run_start(DevProblem P, const PoseQT* __restrict__ pose0,
+                                                   const D4* __restrict__ X0, PoseQT* __restrict__ pose,
+                                                   CamRT* __restrict__ cam, D4* __restrict__ X, double lambda0,
+                                                   LMDev* lm, int* done_count) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < P.n_pt) X[i] = X0[i];
+    if (i < P.n_cam) {
+        const PoseQT p = pose0[i];
+        pose[i] = p;
+        CamRT o;
+        quat_to_R(p.q, o.R);
+        o.t[0] = p.t[0]; o.t[1] = p.t[1]; o.t[2] = p.t[2];
+        cam[i] = o;
+    }
+    if (i == 0) *done_count = P.n_iter > 0 ? 0 : P.n_win;
+    if (i < P.n_win) {
+        LMDev L{};
+        L.lambda = lambda0;
+        L.nu = 2.0;
+        L.phase = P.n_iter > 0 ? kPhaseLin : kPhaseDone;
+        lm[i] = L;
+    }
 }
 
-void launch_lm_reset(const DevProblem& P, const DevWork& W, hipStream_t st) {
-    hipLaunchKernelGGL(k_lm_reset, dim3((P.n_win + 255) / 256), dim3(256), 0, st, P.n_win, P.n_iter,
-                       P.auto_lambda ? 0.0 : P.lambda0, W.lm, W.done_count);
+void launch_run_start(const DevProblem& P, const DevState& init, const DevState& cur, const DevWork& W, hipStream_t st) {
+    const int n = std::max(std::max(P.n_pt, P.n_cam), std::max(P.n_win, 1));
+    hipLaunchKernelGGL(k_run_start, dim3((n + 255) / 256), dim3(256), 0, st, P, (const PoseQT*)init.pose,
+                       (const D4*)init.X, cur.pose, cur.cam, cur.X, P.auto_lambda ? 0.0 : P.lambda0, W.lm,
+                       W.done_count);
 }
 
 // ---------------------------------------------------------------- lin_pt
@@ -970,19 +988,40 @@ void launch_flags(const DevProblem& P, const DevState& s, const DevWork& W, doub
                        st, P, s.cam, (const LMDev*)W.lm, thr, W.outlier, W.red_cost, W.red_aux);
 }
 
-__global__ __launch_bounds__(256) void k_final(DevProblem P, const double* __restrict__ red_cost,
-                                               const double* __restrict__ red_cnt, double* __restrict__ out) {
+// What the host reads of a run, into pinned memory: the count of finished
+// windows; with `state` each window's LM state and costs, and with `final` the
+// final cost and the flag count (over the blocks of k_flags).  One workgroup per window.
+__global__ __launch_bounds__(256) void k_report(DevProblem P, const double* __restrict__ red_cost,
+                                                const double* __restrict__ red_cnt, const LMDev* __restrict__ lm,
+                                                const double* __restrict__ hist, const int* __restrict__ done_count,
+                                                ReportPlaces at, int state, int final, char* __restrict__ out) {
     __shared__ double sh[4];
     const int win = blockIdx.x;
+    if (win == 0 && threadIdx.x == 0) *reinterpret_cast<int*>(out) = *done_count;
+    if (!state) return;
+    static_assert(sizeof(LMDev) % sizeof(double) == 0, "copied by doubles");
+    constexpr int kLm = sizeof(LMDev) / sizeof(double);
+    const double* l = reinterpret_cast<const double*>(lm + win);
+    const int nh = P.n_iter + 1;
+    if (threadIdx.x < kLm) reinterpret_cast<double*>(out + at.lm)[(size_t)kLm * win + threadIdx.x] = l[threadIdx.x];
+    for (int i = threadIdx.x; i < nh; i += 256)
+        reinterpret_cast<double*>(out + at.hist)[(size_t)nh * win + i] = hist[(size_t)nh * win + i];
+    if (!final) return;
     const double c = sum_range(red_cost, P.win_cblk0[win], P.win_cblk0[win + 1], sh);
     __syncthreads();
     const double n = sum_range(red_cnt, P.win_cblk0[win], P.win_cblk0[win + 1], sh);
-    if (threadIdx.x == 0) { out[2 * win] = c; out[2 * win + 1] = n; }
+    if (threadIdx.x == 0) {
+        double* o = reinterpret_cast<double*>(out + at.final) + 2 * (size_t)win;
+        o[0] = c;
+        o[1] = n;
+    }
 }
 
-void launch_final(const DevProblem& P, const DevWork& W, hipStream_t st) {
-    hipLaunchKernelGGL(k_final, dim3(P.n_win), dim3(256), 0, st, P, (const double*)W.red_cost,
-                       (const double*)W.red_aux, W.final);
+void launch_report(const DevProblem& P, const DevWork& W, const ReportPlaces& at, bool state, bool final, char* out,
+                   hipStream_t st) {
+    hipLaunchKernelGGL(k_report, dim3(state ? P.n_win : 1), dim3(256), 0, st, P, (const double*)W.red_cost,
+                       (const double*)W.red_aux, (const LMDev*)W.lm, (const double*)W.hist, (const int*)W.done_count,
+                       at, state ? 1 : 0, final ? 1 : 0, out);
 }
 
 // ---------------------------------------------------------------- results

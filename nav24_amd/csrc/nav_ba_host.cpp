@@ -6,7 +6,7 @@
 //              observations ordered by (point, camera, input order), camera-major
 //              index lists, linearisation tiles, Schur work items, co-visibility.
 //   run      = optimizer.optimize(nIterations) (:66-68) on the device.  One
-//              replayed hipGraph advances every window by one LM trial (gated
+//              step's launches advance every window by one LM trial (gated
 //              linearisation, trial, accept/reject, next phase); the host only
 //              watches a small status.
 //   fetch    = recoverPose / recoverMapPoints (:213-244) plus the outlier flags.
@@ -187,8 +187,6 @@ struct nav_ba_handle {
     DevWork W{};
     std::vector<DevBuf> bufs;
     int nbuf = 0;
-    hipGraphExec_t step = nullptr;   // one LM step
-    hipGraphExec_t step0 = nullptr;  // the first step of a solve
     bool timing = false;
     bool timing_active = false;
     int solver_mode = 0;  // 0 auto, 1 tiles, 2 blocks, 3 in-LDS per window, 4 conjugate gradients
@@ -200,8 +198,8 @@ struct nav_ba_handle {
     int schur_kernel = 0;  // Schur row kernel: 0 = default or tuned, 1 = rounds of kBlock, 2 = producer/consumer
     bool schur_pc_used = false;
     StageTimer timer;
-    int* hdone = nullptr;      // pinned: windows finished
-    LMDev* hlm = nullptr;      // pinned: the LM state of up to kBurstWindows windows, between bursts
+    char* report = nullptr;    // pinned: what the host reads of a run (ReportPlaces)
+    size_t report_cap = 0;
     char* stage = nullptr;     // pinned staging of a prepare's uploads (grown on demand)
     size_t stage_cap = 0;
     char* stage_s = nullptr;   // pinned staging of the Schur work items (the tuner re-uploads them)
@@ -406,32 +404,15 @@ void enqueue_step(nav_ba_handle* h, bool first) {
     });
 }
 
+// The launches of a step, one by one: a step's kernels take 5 us and more each, a
+// launch 3 us of the host, so the queue stays ahead of the GPU.  A graph per step
+// cost 8 us between steps and, for a new structure, 100 us of capture at prepare.
 int launch_step(nav_ba_handle* h, bool first) {
-    if (!h->timing && !h->P.use_pcg) {
-        HIPTRY(h, hipGraphLaunch(first ? h->step0 : h->step, h->stream));
-        return NAV_BA_OK;
-    }
-    // stage timing, or conjugate gradients: the step's launches one by one
     h->timing_active = h->timing;
     h->pcg_err = NAV_BA_OK;
     if (mixed(h)) enqueue_step<float>(h, first); else enqueue_step<double>(h, first);
     h->timing_active = false;
     if (h->pcg_err != NAV_BA_OK) return fail(h, h->pcg_err, h->err);
-    return NAV_BA_OK;
-}
-
-// Two graphs: the first step of a solve (with the lambda initialisation) and every later one.
-int capture_step(nav_ba_handle* h) {
-    for (int first = 0; first < 2; ++first) {
-        hipGraph_t g = nullptr;
-        HIPTRY(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        if (mixed(h)) enqueue_step<float>(h, first); else enqueue_step<double>(h, first);
-        HIPTRY(h, hipStreamEndCapture(h->stream, &g));
-        hipError_t e = hipGraphInstantiate(first ? &h->step0 : &h->step, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess)
-            return fail(h, NAV_BA_HIP_ERROR, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-    }
     return NAV_BA_OK;
 }
 
@@ -1315,8 +1296,7 @@ std::string check_layout(const HostLayout& L, const SchurItems& S) {
 
 // Build the device structure of n_win windows laid end to end (see ba_kernels.h).
 // Everything a prepare's structure depends on: sizes, observation indices,
-// fixed flags, the camera, the options (they are baked into the captured step
-// graphs) and the handle's forced settings.  Poses, points and measurements
+// fixed flags, the camera, the options and the handle's forced settings.  Poses, points and measurements
 // are not part of it.
 void make_prep_key(const nav_ba_handle* h, const nav_ba_problem* probs, int n_win, const nav_ba_options* o,
                    bool batched, std::vector<char>& key) {
@@ -1344,7 +1324,7 @@ void make_prep_key(const nav_ba_handle* h, const nav_ba_problem* probs, int n_wi
 }
 
 // A prepare whose key equals the last one's: the host layout, work items,
-// tuned choices and step graphs stay; the new initial poses, points and
+// and tuned choices stay; the new initial poses, points and
 // measurements (in the orders prepare chose) go to the device.
 int refresh_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, const nav_ba_options* o) {
     HostLayout& L = h->layout;
@@ -1432,8 +1412,6 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     h->schur_chunk_used = 0;
     HIPTRY(h, hipSetDevice(h->device));
     HIPTRY(h, hipStreamSynchronize(h->stream));
-    if (h->step) { (void)hipGraphExecDestroy(h->step); h->step = nullptr; }
-    if (h->step0) { (void)hipGraphExecDestroy(h->step0); h->step0 = nullptr; }
     h->opt = *o;
     if (h->opt.max_trials <= 0) h->opt.max_trials = 10;
     h->batched = batched;
@@ -1542,7 +1520,6 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     AL(W.red_aux, sizeof(double) * std::max(P.n_cblk, 1));
     AL(W.outlier, std::max<size_t>(no, 1));
     AL(W.hist, sizeof(double) * (size_t)n_win * (o->n_iter + 1));
-    AL(W.final, sizeof(double) * 2 * (size_t)n_win);
     AL(W.done_count, sizeof(int));
     AL(W.lm, sizeof(LMDev) * n_win);
     AL(W.pcg, sizeof(double) * (P.use_pcg ? pcg_work_doubles(P.n) : (size_t)1));
@@ -1565,7 +1542,6 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
         if ((st = tune_schur_items(h, G, schur_mark, h->schur_kernel, h->schur_chunk, SI)) != NAV_BA_OK) return st;
         remember_choice(key, TuneChoice{SI.chunk, SI.pc});
     }
-    if (!P.use_pcg && (st = capture_step(h)) != NAV_BA_OK) return st;
     h->prepared = true;
     h->prep_key.swap(pkey);
     return NAV_BA_OK;
@@ -1628,6 +1604,7 @@ int fetch_all(nav_ba_handle* h, nav_ba_result* results, int n) {
         HIPTRY(h, hipHostMalloc((void**)&h->rbuf, at.total, hipHostMallocDefault));
         h->rbuf_cap = at.total;
     }
+    (void)hipGetLastError();  // an error that an earlier call of the program left is not this one's
     launch_results(h->P, h->cur, h->W, h->pt_src, h->x_in, at, h->opt.compat_fp32_io != 0, h->rbuf, h->stream);
     HIPTRY(h, hipGetLastError());
     HIPTRY(h, hipStreamSynchronize(h->stream));
@@ -1678,8 +1655,6 @@ int32_t nav_ba_create(nav_ba_handle** out, int32_t device) {
     h->device = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess ||
-        hipHostMalloc((void**)&h->hdone, sizeof(int), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&h->hlm, sizeof(LMDev) * kBurstWindows, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&h->hpcg, sizeof(PcgState), hipHostMallocDefault) != hipSuccess) {
         nav_ba_destroy(h);
         return NAV_BA_HIP_ERROR;
@@ -1692,12 +1667,9 @@ void nav_ba_destroy(nav_ba_handle* h) {
     if (!h) return;
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    if (h->step) (void)hipGraphExecDestroy(h->step);
-    if (h->step0) (void)hipGraphExecDestroy(h->step0);
     for (auto& b : h->bufs)
         if (b.p) (void)hipFree(b.p);
-    if (h->hdone) (void)hipHostFree(h->hdone);
-    if (h->hlm) (void)hipHostFree(h->hlm);
+    if (h->report) (void)hipHostFree(h->report);
     if (h->hpcg) (void)hipHostFree(h->hpcg);
     if (h->stage) (void)hipHostFree(h->stage);
     if (h->stage_s) (void)hipHostFree(h->stage_s);
@@ -1732,11 +1704,17 @@ int32_t nav_ba_run(nav_ba_handle* h) {
     hipStream_t s = h->stream;
     const DevProblem& P = h->P;
     const bool m = mixed(h);
+    const ReportPlaces at((size_t)P.n_win, (size_t)P.n_iter);
+    if (h->report_cap < at.total) {
+        if (h->report) (void)hipHostFree(h->report);
+        h->report = nullptr;
+        h->report_cap = 0;
+        HIPTRY(h, hipHostMalloc((void**)&h->report, at.total, hipHostMallocDefault));
+        h->report_cap = at.total;
+    }
+    (void)hipGetLastError();  // an error that an earlier call of the program left is not this run's
     HIPTRY(h, hipEventRecord(h->ev0, s));
-    HIPTRY(h, hipMemcpyAsync(h->cur.pose, h->init.pose, sizeof(PoseQT) * P.n_cam, hipMemcpyDeviceToDevice, s));
-    HIPTRY(h, hipMemcpyAsync(h->cur.X, h->init.X, sizeof(D4) * P.n_pt, hipMemcpyDeviceToDevice, s));
-    launch_lm_reset(P, h->W, s);
-    launch_cam_rt(P, h->cur, s);
+    launch_run_start(P, h->init, h->cur, h->W, s);
     if (m) launch_cost<float>(P, h->cur, h->W, 0, s); else launch_cost<double>(P, h->cur, h->W, 0, s);
     launch_lm_set_chi(P, h->W, s);
     // every window needs at most n_iter * max_trials steps.  Steps are
@@ -1745,42 +1723,53 @@ int32_t nav_ba_run(nav_ba_handle* h) {
     // the most iterations a running window still has (a step past a window's
     // end returns at once from every kernel, and costs about as much GPU time
     // as the host's check costs idle time), else 2.  The host checks the
-    // count of finished windows after each burst.
+    // count of finished windows after each burst.  For few windows, which most
+    // often end with the first burst, the outlier flags and the FP64 cost at the
+    // final state go with every burst, so that a run has one wait; otherwise
+    // they follow the last one.
     const long long max_steps = (long long)P.n_iter * P.max_trials;
     long long steps = 0;
     int st;
     long long burst = std::max(1, P.n_iter);
     const bool few = P.n_win <= kBurstWindows;
-    while (steps < max_steps) {
-        for (long long i = 0; i < burst && steps < max_steps; ++i, ++steps)
+    bool final = few && !h->timing, finished = false;
+    while (true) {
+        for (long long i = 0; i < burst && steps < max_steps && !finished; ++i, ++steps)
             if ((st = launch_step(h, steps == 0)) != NAV_BA_OK) return st;
-        HIPTRY(h, hipMemcpyAsync(h->hdone, h->W.done_count, sizeof(int), hipMemcpyDeviceToHost, s));
-        if (few) HIPTRY(h, hipMemcpyAsync(h->hlm, h->W.lm, sizeof(LMDev) * P.n_win, hipMemcpyDeviceToHost, s));
+        if (final) {
+            h->timing_active = h->timing;
+            stage(h, NAV_BA_ST_FLAGS, [&] {
+                launch_flags(P, h->cur, h->W, h->opt.outlier_chi2, s);
+                launch_report(P, h->W, at, true, true, h->report, s);
+            });
+            h->timing_active = false;
+            HIPTRY(h, hipEventRecord(h->ev1, s));
+        } else {
+            launch_report(P, h->W, at, few, false, h->report, s);
+        }
+        HIPTRY(h, hipGetLastError());
         HIPTRY(h, hipStreamSynchronize(s));
-        if (*h->hdone >= P.n_win) break;
+        finished = finished || steps >= max_steps || *(const int*)h->report >= P.n_win;
+        if (finished) {
+            if (final) break;
+            final = true;
+            continue;
+        }
         burst = 2;
         if (few) {
+            const LMDev* lm = (const LMDev*)(h->report + at.lm);
             int rem = 0;
             for (int w = 0; w < P.n_win; ++w)
-                if (h->hlm[w].phase != kPhaseDone) rem = std::max(rem, P.n_iter - h->hlm[w].iter);
+                if (lm[w].phase != kPhaseDone) rem = std::max(rem, P.n_iter - lm[w].iter);
             burst = std::max<long long>(2, rem + (rem + 1) / 2);
         }
     }
-    // outlier flags and the FP64 cost at the final state
-    h->timing_active = h->timing;
-    stage(h, NAV_BA_ST_FLAGS, [&] {
-        launch_flags(P, h->cur, h->W, h->opt.outlier_chi2, s);
-        launch_final(P, h->W, s);
-    });
-    h->timing_active = false;
-    HIPTRY(h, hipEventRecord(h->ev1, s));
-    h->lm_out.resize(P.n_win);
-    h->hist_out.resize((size_t)P.n_win * (P.n_iter + 1));
-    h->final_out.resize(2 * (size_t)P.n_win);
-    HIPTRY(h, hipMemcpyAsync(h->lm_out.data(), h->W.lm, sizeof(LMDev) * P.n_win, hipMemcpyDeviceToHost, s));
-    HIPTRY(h, hipMemcpyAsync(h->hist_out.data(), h->W.hist, sizeof(double) * h->hist_out.size(), hipMemcpyDeviceToHost, s));
-    HIPTRY(h, hipMemcpyAsync(h->final_out.data(), h->W.final, sizeof(double) * h->final_out.size(), hipMemcpyDeviceToHost, s));
-    HIPTRY(h, hipStreamSynchronize(s));
+    const LMDev* lm = (const LMDev*)(h->report + at.lm);
+    const double* hist = (const double*)(h->report + at.hist);
+    const double* fin = (const double*)(h->report + at.final);
+    h->lm_out.assign(lm, lm + P.n_win);
+    h->hist_out.assign(hist, hist + (size_t)P.n_win * (P.n_iter + 1));
+    h->final_out.assign(fin, fin + 2 * (size_t)P.n_win);
     float ms = 0.f;
     HIPTRY(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
     h->solve_ms = ms;

@@ -1,0 +1,42 @@
+"""A run's bursts and what the host reads of them, against the FP64 oracle: no,
+one and several iterations, on either side of the window count up to which the
+final flags go with every burst, with trials that are rejected."""
+import numpy as np
+import pytest
+
+from nav24_amd import problems
+from nav24_amd.abi import NAV_BA_FP64, workload_options
+from oracle import oracle
+from parity_util import say
+
+pytestmark = pytest.mark.gpu
+
+
+def window(seed, far):
+    # far: a start from which some trials fail (a tenth of a radian, a metre)
+    return problems.workload(3, seed=seed, n_cam=4, n_pt=60, obs_min=3, rot_sigma=0.1 if far else 0.005,
+                             trans_sigma=1.0 if far else 0.01, point_sigma=0.3 if far else 0.02)
+
+
+@pytest.mark.parametrize("n_win", [1, 2, 64, 65])
+@pytest.mark.parametrize("n_iter", [0, 1, 6])
+def test_bursts_match_oracle(n_win, n_iter):
+    """The same counts, and costs to the repository's parity bar (1e-9) while the
+    paths agree; three distinct windows, so that the oracle solves three."""
+    from nav24_amd.ba import GraphOptimHip
+    kinds = [window(1, False), window(2, True), window(3, False)]
+    o = workload_options(3)
+    o.precision, o.n_iter, o.lambda_init = NAV_BA_FP64, n_iter, 1e-4
+    refs = [oracle.solve(p, o) for p in kinds]
+    s = GraphOptimHip(0)
+    rs = s.solve_batched([kinds[k % 3] for k in range(n_win)], o)
+    again = s.solve_batched([kinds[k % 3] for k in range(n_win)], o)
+    s.close()
+    say(f"{n_win} windows, {n_iter} iterations: trials {[r.trials for r in refs]}")
+    for k, (r, a) in enumerate(zip(rs, again)):
+        ref = refs[k % 3]
+        assert (r.iterations, r.trials, r.stop_reason) == (ref.iterations, ref.trials, ref.stop_reason)
+        assert np.abs(r.cost_history - ref.cost_history).max() <= 1e-9 * ref.cost_history.max()
+        assert abs(r.final_cost - ref.final_cost) <= 1e-9 * ref.cost_history.max()
+        assert np.array_equal(r.outlier, ref.outlier) and r.n_outliers == ref.n_outliers
+        assert np.array_equal(r.T_cw, a.T_cw) and np.array_equal(r.cost_history, a.cost_history)
