@@ -54,6 +54,16 @@ struct PcgState {
     int iter, done, fail, pad;
 };
 
+// One Schur work item, in dispatch order: what its workgroup reads first, in one
+// aligned record (a chain of loads through the item's tables cost each workgroup
+// four more round trips before its first useful load).
+struct alignas(16) SchurDesc {
+    int it, f, cam, win;       // item, S row (free camera), its camera, its window
+    int a0, a1, g, ns;         // camera-major observations, column group, slots
+    int col0, rnd0;            // first entry of colcam / colcamera, first round
+    long long pofs;            // its partial blocks in spart
+};
+
 struct DevProblem {
     int n_cam, n_pt, n_obs, n_fc;
     int robust;
@@ -92,18 +102,13 @@ struct DevProblem {
     int n_hitems;
     // Schur work items (free camera, column group, chunk), group-major per camera;
     // each item is taken in rounds of kBlock observations
-    const int* sitem_f;
-    const int* sitem_a0;
-    const int* sitem_a1;
-    const int* sitem_g;
     const int* sitem_nslots;
     const long long* sitem_pofs;
-    const int* sitem_rnd0;     // [n_sitems] first round of the item
     const int* row_sitem_ptr;  // [n_fc + 1]
     const int* row_nchunks;    // [n_fc]
     const long long* row_pofs0; // [n_fc] partial-sum offset of each row's first item (the items of a row
                                 //   of one column group lie back to back)
-    const int* sitem_order;    // [n_sitems] dispatch order: estimated work, heaviest first
+    const SchurDesc* sdesc;    // [n_sitems] the items in dispatch order: estimated work, heaviest first
     int schur_pc;              // 0: rounds of kBlock, lanes bound per round; 1: producer/consumer rounds
     const uint8_t* rnd_lane_slot;  // slot of each lane (slots' lanes contiguous), 255 idle: [rounds][kBlock],
                                    // or (producer/consumer) [items][kPcCons] for the consumer lanes
@@ -117,6 +122,7 @@ struct DevProblem {
     // column blocks of each S row: free indices >= row (same window), first is the row itself
     const int* colptr;         // [n_fc + 1]
     const int* colcam;
+    const int* colcamera;      // the column blocks' cameras: free_cam[colcam]
     const int* zcolptr;        // [n_fc + 1] per S row: the blocks g > f with no co-visibility
     const int* zcolcam;        //   (written as zeros by the reduction every trial)
     // windows

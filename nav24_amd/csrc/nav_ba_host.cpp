@@ -722,13 +722,18 @@ bool build_schur_items(const SchurGraph& G, int chunk, bool pc, SchurItems& S) {
 int upload_schur_items(nav_ba_handle* h, const SchurItems& S) {
     DevProblem& P = h->P;
     int st;
+    const HostLayout& L = h->layout;
+    std::vector<SchurDesc> desc(S.sf.size());
+    for (size_t b = 0; b < desc.size(); ++b) {
+        const int it = S.sorder[b], f = S.sf[it], cam = L.free_cam[f];
+        desc[b] = SchurDesc{it, f, cam, L.cam_win[cam], S.sa0[it], S.sa1[it], S.sg[it], S.sns[it],
+                            L.colptr[f] + S.sg[it] * kMaxSlots, S.srnd0[it], S.spofs[it]};
+    }
     // staging: prepare synchronises the stream before the tuner, and the tuner after every timing
     Packer pk(&h->stage_s, &h->stage_s_cap);
 #define UP(dst, vec) pk.add(&(dst), (vec))
-    UP(P.sitem_f, S.sf); UP(P.sitem_a0, S.sa0); UP(P.sitem_a1, S.sa1); UP(P.sitem_g, S.sg); UP(P.sitem_nslots, S.sns);
-    UP(P.sitem_pofs, S.spofs); UP(P.row_sitem_ptr, S.row_sitem_ptr); UP(P.row_nchunks, S.row_nch);
+    UP(P.sdesc, desc); UP(P.sitem_nslots, S.sns); UP(P.sitem_pofs, S.spofs); UP(P.row_sitem_ptr, S.row_sitem_ptr); UP(P.row_nchunks, S.row_nch);
     UP(P.row_pofs0, S.row_pofs0);
-    UP(P.sitem_order, S.sorder); UP(P.sitem_rnd0, S.srnd0);
     UP(P.rnd_lane_slot, S.lane_slot); UP(P.rnd_pair0, S.rnd_pair0); UP(P.rnd_rows, S.rnd_rows);
     UP(P.rnd_group, S.rnd_group); UP(P.pairs, S.pairs);
 #undef UP
@@ -1460,7 +1465,9 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     UP(P.c_pt, L.c_pt); UP(P.c_uv, L.c_uv);
     UP(P.tile_obs, L.tile_obs); UP(P.tile_pt, L.tile_pt); UP(P.tile_win, L.tile_win);
     UP(P.hitem_f, L.hf); UP(P.hitem_a0, L.ha0); UP(P.hitem_a1, L.ha1); UP(P.cam_hitem_ptr, L.cam_hitem_ptr);
-    UP(P.colptr, L.colptr); UP(P.colcam, L.colcam); UP(P.zcolptr, L.zcolptr); UP(P.zcolcam, L.zcolcam);
+    std::vector<int> colcamera(L.colcam.size());
+    for (size_t k = 0; k < colcamera.size(); ++k) colcamera[k] = L.free_cam[L.colcam[k]];
+    UP(P.colptr, L.colptr); UP(P.colcam, L.colcam); UP(P.colcamera, colcamera); UP(P.zcolptr, L.zcolptr); UP(P.zcolcam, L.zcolcam);
     UP(P.cam_win, L.cam_win); UP(P.pt_win, L.pt_win); UP(P.win_cam0, L.win_cam0); UP(P.win_fc0, L.win_fc0);
     UP(P.win_pt0, L.win_pt0); UP(P.win_S, L.win_S); UP(P.win_lda, L.win_lda);
     UP(P.cblk_o0, L.cblk_o0); UP(P.cblk_win, L.cblk_win); UP(P.win_cblk0, L.win_cblk0);

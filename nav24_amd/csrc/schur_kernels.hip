@@ -33,7 +33,8 @@
 // instead of 11 16-byte words, and the producer/consumer kernel fits three
 // workgroups on a CU: 512 windows 352 -> 280 us per launch, 24 windows 28 -> 24
 // (FP32 Jacobians), 300-keyframe loop 212 -> 197, 60 keyframes 145 -> 137 (per round
-// form, limited by its registers to two workgroups).  Two pairs per step in the
+// form, limited by its registers to two workgroups).  With an item's record in one
+// load (SchurDesc) 269, 23.5, 194 and 134.6; one 30-camera window 14.2 -> 13.0.  Two pairs per step in the
 // consumers, which needs 200 registers, was slower than the third workgroup.
 // A round is 256 observations for the whole workgroup: its 256 lanes share
 // the slots (balance over many lanes), with workgroup barriers between the
@@ -368,15 +369,12 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
                                                       const double* __restrict__ Hl, const LMDev* lm,
                                                       double* __restrict__ spart) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int it = P.sitem_order[blockIdx.x];
-    const int f = P.sitem_f[it], a0 = P.sitem_a0[it], a1 = P.sitem_a1[it];
-    const int g = P.sitem_g[it], ns = P.sitem_nslots[it];
-    const int cf = P.free_cam[f];
-    const int win = P.cam_win[cf];
+    const SchurDesc d = P.sdesc[blockIdx.x];
+    const int a0 = d.a0, a1 = d.a1, ns = d.ns, cf = d.cam, win = d.win;
     const D4* __restrict__ X = x_cur(P, lm, win);  // the window's current points
     if (!running(lm, win)) return;
     const double lambda = lm[win].lambda;
-    const bool g0 = (g == 0);
+    const bool g0 = (d.g == 0);
     const SchurLayout<T, CM> L(ns);
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -388,7 +386,6 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
     int* lcount = lfirst + ns;
     double* red = reinterpret_cast<double*>(smem + L.red);
 
-    const int col0 = P.colptr[f] + g * kMaxSlots;
     for (int i = tid; i < ns * 36; i += kBlock) acc[i] = 0.0;
 
     double coef[6], dsum[21];
@@ -397,9 +394,9 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
 #pragma unroll
     for (int k = 0; k < 21; ++k) dsum[k] = 0.0;
 
-    for (int s = tid; s < ns; s += kBlock) lcam[s] = P.free_cam[P.colcam[col0 + s]];
+    for (int s = tid; s < ns; s += kBlock) lcam[s] = P.colcamera[d.col0 + s];
     __syncthreads();
-    const int rnd0 = P.sitem_rnd0[it];
+    const int rnd0 = d.rnd0;
     const int nrounds = (a1 - a0 + kBlock - 1) / kBlock;
     for (int r = 0; r < nrounds; ++r) {
         const int rnd = rnd0 + r;
@@ -469,7 +466,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_schur_row(DevProblem P, const Cam
         if ((lane & 1) == 0 && k27 >= 0) red[wid * 27 + k27] = v;
     }
     __syncthreads();
-    double* out = spart + P.sitem_pofs[it];
+    double* out = spart + d.pofs;
     if (g0 && tid < 27) {
         double s = red[tid];
 #pragma unroll
@@ -522,15 +519,12 @@ __global__ __launch_bounds__(kBlock, CM == kCamPinhole ? 3 : 2) void k_schur_row
                                                          const double* __restrict__ Hl, const LMDev* lm,
                                                          double* __restrict__ spart) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int it = P.sitem_order[blockIdx.x];
-    const int f = P.sitem_f[it], a0 = P.sitem_a0[it], a1 = P.sitem_a1[it];
-    const int g = P.sitem_g[it], ns = P.sitem_nslots[it];
-    const int cf = P.free_cam[f];
-    const int win = P.cam_win[cf];
+    const SchurDesc d = P.sdesc[blockIdx.x];
+    const int a0 = d.a0, a1 = d.a1, ns = d.ns, cf = d.cam, win = d.win;
     const D4* __restrict__ X = x_cur(P, lm, win);  // the window's current points
     if (!running(lm, win)) return;
     const double lambda = lm[win].lambda;
-    const bool g0 = (g == 0);
+    const bool g0 = (d.g == 0);
     constexpr int ws = RowA<T, CM>::stride;
     const PcLayout<T, CM> L(ns);
     const int tid = threadIdx.x, lane = tid % kWave;
@@ -539,8 +533,7 @@ __global__ __launch_bounds__(kBlock, CM == kCamPinhole ? 3 : 2) void k_schur_row
     int* lfirst = reinterpret_cast<int*>(smem + L.lrange);
     int* lend = lfirst + ns;
     double* red = reinterpret_cast<double*>(smem + L.red);
-    const int col0 = P.colptr[f] + g * kMaxSlots;
-    const int rnd0 = P.sitem_rnd0[it];
+    const int rnd0 = d.rnd0;
     const int nrounds = (a1 - a0 + kPcRound - 1) / kPcRound;
     for (int s = tid; s < ns; s += kBlock) { lfirst[s] = 0; lend[s] = 0; }
 
@@ -600,12 +593,12 @@ __global__ __launch_bounds__(kBlock, CM == kCamPinhole ? 3 : 2) void k_schur_row
     } else {
         // ---- consumers: bound to one slot for the item; pairs of round r
         const int c = tid - kPcRound, cw = c / kWave;
-        const int sl = P.rnd_lane_slot[(size_t)it * kPcCons + c];
+        const int sl = P.rnd_lane_slot[(size_t)d.it * kPcCons + c];
         lslot[c] = sl;
         double sacc[36], Rb[9], tb[3];
 #pragma unroll
         for (int e = 0; e < 36; ++e) sacc[e] = 0.0;
-        if (sl != 255) load_cam(cam, P.free_cam[P.colcam[col0 + sl]], Rb, tb);
+        if (sl != 255) load_cam(cam, P.colcamera[d.col0 + sl], Rb, tb);
         // round r's pair rows, first two entries and first weight; the next
         // round's entries are loaded at the start of a round and their weight
         // at its end, so both land while the round runs
@@ -652,7 +645,7 @@ __global__ __launch_bounds__(kBlock, CM == kCamPinhole ? 3 : 2) void k_schur_row
         __syncthreads();
     }
     // ---- each (slot, entry) adds its slot's staged consumer rows in lane order
-    double* out = spart + P.sitem_pofs[it];
+    double* out = spart + d.pofs;
     for (int task = tid; task < ns * 36; task += kBlock) {
         const int s = task / 36, e = task % 36;
         const int l0 = lfirst[s], n = lend[s] - l0;
