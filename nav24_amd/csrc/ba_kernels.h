@@ -29,6 +29,11 @@ constexpr int kBlocksMaxFc = 128;  // one problem: the single-workgroup block Ch
                                    // possible up to this size (chosen only on request)
 constexpr int kCostObs = 1024;     // observations per cost / flag block
 constexpr int kXcds = 8;           // XCDs of one MI355X: workgroup i of a launch runs on XCD i % 8
+// Tiles and camera items up to which the linearisation's two sides go in one launch,
+// pinhole and fisheye: four and two workgroups per CU (their registers), all of
+// them resident at once.  An 8-camera window: 13.4 us in three launches, 5.7 in one;
+// 30 cameras 14.9 and 6.0; 15 fisheye cameras 16.6 and 8.2.
+constexpr int kLinTogether[2] = {1024, 512};
 constexpr int kBurstWindows = 64;  // up to this many windows the host reads their LM state between bursts
 constexpr int kCommitInAcceptCams = 1024;  // windows up to this many cameras commit them inside the LM decision
 
@@ -100,6 +105,7 @@ struct DevProblem {
     const int* hitem_a1;
     const int* cam_hitem_ptr;  // [n_fc + 1]
     int n_hitems;
+    int one_hitem;             // 1: every free camera has exactly one item
     // Schur work items (free camera, column group, chunk), group-major per camera;
     // each item is taken in rounds of kBlock observations
     const int* sitem_nslots;
@@ -299,6 +305,7 @@ void launch_cam_rt(const DevProblem& P, const DevState& s, hipStream_t st);
 void launch_run_start(const DevProblem& P, const DevState& init, const DevState& cur, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lin_pt(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lin_cam(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
+template <typename T> void launch_lin(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
 template <typename T> void launch_lambda_init(const DevProblem& P, const DevWork& W, hipStream_t st);
 template <typename T> void launch_schur_row(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st);
 void launch_fill_system(const DevProblem& P, const DevWork& W, hipStream_t st);  // once per prepare

@@ -85,15 +85,18 @@ void launch_run_start(const DevProblem& P, const DevState& init, const DevState&
 // Registers capped at 72 for the pinhole (7 waves per SIMD instead of 6): the
 // kernel waits on its gathers, and the extra wave gave 6 % at 3 M
 // observations.  The fisheye model's transcendental functions need more.
-template <typename T, int CM>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CM == kCamPinhole ? 7 : 1, 8))) void k_lin_pt(DevProblem P, const CamRT* __restrict__ cam,
-                                                   const LMDev* lm,
-                                                   T* __restrict__ w_out, double* __restrict__ Hl) {
+struct LinPtLds {
     // rows padded by one double: the 9 sums of one point read one column, which
     // an unpadded 2 KB row stride would put in a single LDS bank
-    __shared__ double sh[9][kTile + 1];
-    __shared__ double red[kBlock / kWave][9];
-    const int t = blockIdx.x;
+    double sh[9][kTile + 1];
+    double red[kBlock / kWave][9];
+};
+
+template <typename T, int CM>
+__device__ __forceinline__ void lin_pt_tile(const DevProblem& P, const CamRT* __restrict__ cam, const LMDev* lm,
+                                            T* __restrict__ w_out, double* __restrict__ Hl, int t, LinPtLds& lds) {
+    auto& sh = lds.sh;
+    auto& red = lds.red;
     const D4* __restrict__ X = x_cur(P, lm, P.tile_win[t]);  // its selector loaded beside the LM state
     if (!needs_lin(lm, P.tile_win[t])) return;
     const int o0 = P.tile_obs[t], o1 = P.tile_obs[t + 1];
@@ -168,6 +171,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CM == kC
     }
 }
 
+template <typename T, int CM>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CM == kCamPinhole ? 7 : 1, 8))) void k_lin_pt(
+    DevProblem P, const CamRT* __restrict__ cam, const LMDev* lm, T* __restrict__ w_out, double* __restrict__ Hl) {
+    __shared__ LinPtLds lds;
+    lin_pt_tile<T, CM>(P, cam, lm, w_out, Hl, blockIdx.x, lds);
+}
+
 template <typename T>
 void launch_lin_pt(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st) {
     if (P.n_tiles == 0) return;
@@ -180,13 +190,15 @@ void launch_lin_pt(const DevProblem& P, const DevState& s, const DevWork& W, hip
 // One workgroup per (free camera, chunk of its observations): Hpp (21 packed)
 // and bp (6) from T Jacobians, formed in FP64 and reduced per wave by a
 // reduce-scatter of the 27 sums, then over the waves in order; then one
-// workgroup per camera sums the chunks.  Inputs are read in camera-major
-// order (c_pt, c_uv), so the per-observation reads are contiguous.
+// workgroup per camera sums the chunks (k_cam_reduce), except where every camera
+// is one chunk: it then writes the camera's sums itself.  Inputs are read in
+// camera-major order (c_pt, c_uv), so the per-observation reads are contiguous.
+typedef double LinCamLds[kBlock / kWave][27];
+
 template <typename T, int CM>
-__global__ __launch_bounds__(kBlock) void k_lin_cam(DevProblem P, const CamRT* __restrict__ cam,
-                                                    const LMDev* lm, double* __restrict__ hpart) {
-    __shared__ double red[kBlock / kWave][27];
-    const int it = blockIdx.x;
+__device__ __forceinline__ void lin_cam_item(const DevProblem& P, const CamRT* __restrict__ cam, const LMDev* lm,
+                                             double* __restrict__ hpart, double* __restrict__ Hc, int it,
+                                             LinCamLds& red) {
     const int f = P.hitem_f[it], a0 = P.hitem_a0[it], a1 = P.hitem_a1[it];
     const int cf = P.free_cam[f];
     const D4* __restrict__ X = x_cur(P, lm, P.cam_win[cf]);  // its selector loaded beside the LM state
@@ -250,8 +262,36 @@ __global__ __launch_bounds__(kBlock) void k_lin_cam(DevProblem P, const CamRT* _
     if (threadIdx.x < 27) {
         double s = 0.0;
         for (int i = 0; i < kBlock / kWave; ++i) s += red[i][threadIdx.x];
-        hpart[27 * (size_t)it + threadIdx.x] = s;
+        if (P.one_hitem) Hc[28 * (size_t)f + threadIdx.x] = s;
+        else hpart[27 * (size_t)it + threadIdx.x] = s;
+    } else if (threadIdx.x == 27 && P.one_hitem) {
+        Hc[28 * (size_t)f + 27] = 0.0;  // as k_cam_reduce leaves the last place
     }
+}
+
+template <typename T, int CM>
+__global__ __launch_bounds__(kBlock) void k_lin_cam(DevProblem P, const CamRT* __restrict__ cam, const LMDev* lm,
+                                                    double* __restrict__ hpart, double* __restrict__ Hc) {
+    __shared__ LinCamLds red;
+    lin_cam_item<T, CM>(P, cam, lm, hpart, Hc, blockIdx.x, red);
+}
+
+// Both in one launch for small problems, cameras first: neither reads what the
+// other writes.  A window's linearisation is launch and load latency; one 8-camera
+// window took 4.7 + 2.7 + 6.0 us in three launches.  A large problem keeps the
+// two apart: the camera side's registers would cost the point side waves, and
+// its gathers need them.
+template <typename T, int CM>
+__global__ __launch_bounds__(kBlock) void k_lin(DevProblem P, const CamRT* __restrict__ cam, const LMDev* lm,
+                                                T* __restrict__ w_out, double* __restrict__ Hl,
+                                                double* __restrict__ hpart, double* __restrict__ Hc) {
+    __shared__ union {
+        LinPtLds pt;
+        LinCamLds cam;
+    } lds;
+    const int b = blockIdx.x;
+    if (b < P.n_hitems) lin_cam_item<T, CM>(P, cam, lm, hpart, Hc, b, lds.cam);
+    else lin_pt_tile<T, CM>(P, cam, lm, w_out, Hl, b - P.n_hitems, lds.pt);
 }
 
 __global__ void k_cam_reduce(DevProblem P, const double* __restrict__ hpart, const LMDev* lm, double* __restrict__ Hc) {
@@ -276,14 +316,27 @@ __global__ void k_cam_reduce(DevProblem P, const double* __restrict__ hpart, con
     }
 }
 
+static void launch_cam_reduce(const DevProblem& P, const DevWork& W, hipStream_t st) {
+    if (P.one_hitem) return;  // written by the camera side
+    hipLaunchKernelGGL(k_cam_reduce, dim3(P.n_fc), dim3(64), 0, st, P, (const double*)W.hpart, (const LMDev*)W.lm, W.Hc);
+}
+
 template <typename T>
 void launch_lin_cam(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st) {
     if (P.n_fc == 0) return;
     if (P.n_hitems > 0) {
         const auto fn = P.cam_model == kCamKB8 ? k_lin_cam<T, kCamKB8> : k_lin_cam<T, kCamPinhole>;
-        hipLaunchKernelGGL(fn, dim3(P.n_hitems), dim3(kBlock), 0, st, P, s.cam, (const LMDev*)W.lm, W.hpart);
+        hipLaunchKernelGGL(fn, dim3(P.n_hitems), dim3(kBlock), 0, st, P, s.cam, (const LMDev*)W.lm, W.hpart, W.Hc);
     }
-    hipLaunchKernelGGL(k_cam_reduce, dim3(P.n_fc), dim3(64), 0, st, P, (const double*)W.hpart, (const LMDev*)W.lm, W.Hc);
+    launch_cam_reduce(P, W, st);
+}
+
+template <typename T>
+void launch_lin(const DevProblem& P, const DevState& s, const DevWork& W, hipStream_t st) {
+    const auto fn = P.cam_model == kCamKB8 ? k_lin<T, kCamKB8> : k_lin<T, kCamPinhole>;
+    hipLaunchKernelGGL(fn, dim3(P.n_hitems + P.n_tiles), dim3(kBlock), 0, st, P, s.cam, (const LMDev*)W.lm, (T*)W.w,
+                       W.Hl, W.hpart, W.Hc);
+    launch_cam_reduce(P, W, st);
 }
 
 // ---------------------------------------------------------------- lambda init
@@ -1107,6 +1160,7 @@ void launch_results(const DevProblem& P, const DevState& cur, const DevWork& W, 
 #define NAVBA_INST(T)                                                                                         \
     template void launch_lin_pt<T>(const DevProblem&, const DevState&, const DevWork&, hipStream_t);         \
     template void launch_lin_cam<T>(const DevProblem&, const DevState&, const DevWork&, hipStream_t);        \
+    template void launch_lin<T>(const DevProblem&, const DevState&, const DevWork&, hipStream_t);            \
     template void launch_lambda_init<T>(const DevProblem&, const DevWork&, hipStream_t);                     \
     template void launch_schur_reduce<T>(const DevProblem&, const DevWork&, hipStream_t);                    \
     template void launch_backsub<T>(const DevProblem&, const DevState&, const DevState&, const DevWork&,     \

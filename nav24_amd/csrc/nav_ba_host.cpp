@@ -345,8 +345,13 @@ void stage(nav_ba_handle* h, int cat, F&& f) {
 // The first step of a solve (every window at iteration 0) also sets lambda.
 template <typename T>
 void enqueue_lin(nav_ba_handle* h, bool first) {
-    stage(h, NAV_BA_ST_LIN_PT, [&] { launch_lin_pt<T>(h->P, h->cur, h->W, h->stream); });
-    stage(h, NAV_BA_ST_LIN_CAM, [&] { launch_lin_cam<T>(h->P, h->cur, h->W, h->stream); });
+    const DevProblem& P = h->P;
+    if (!h->timing_active && P.n_fc > 0 && P.n_hitems > 0 && P.n_tiles > 0 && P.n_hitems + P.n_tiles <= kLinTogether[P.cam_model == kCamKB8]) {
+        launch_lin<T>(P, h->cur, h->W, h->stream);
+    } else {
+        stage(h, NAV_BA_ST_LIN_PT, [&] { launch_lin_pt<T>(P, h->cur, h->W, h->stream); });
+        stage(h, NAV_BA_ST_LIN_CAM, [&] { launch_lin_cam<T>(P, h->cur, h->W, h->stream); });
+    }
     if (first && h->P.auto_lambda) stage(h, NAV_BA_ST_LAMBDA, [&] { launch_lambda_init<T>(h->P, h->W, h->stream); });
 }
 
@@ -1481,6 +1486,9 @@ int prepare_windows(nav_ba_handle* h, const nav_ba_problem* probs, int n_win, co
     h->x_in = const_cast<double*>(xin_dev);
     P.n_tiles = (int)L.tile_win.size();
     P.n_hitems = (int)L.hf.size();
+    P.one_hitem = 1;
+    for (int f = 0; f < nfc; ++f)
+        if (L.cam_hitem_ptr[f + 1] - L.cam_hitem_ptr[f] != 1) P.one_hitem = 0;
     P.n_win = n_win;
     P.max_win_fc = 0;
     for (int w = 0; w < n_win; ++w) P.max_win_fc = std::max(P.max_win_fc, L.win_fc0[w + 1] - L.win_fc0[w]);

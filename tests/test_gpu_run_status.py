@@ -1,11 +1,12 @@
-"""A run's bursts and what the host reads of them, against the FP64 oracle: no,
+"""A run's launches: the linearisation's two sides in one launch or apart (as stage
+timing runs them), and its bursts and what the host reads of them, against the FP64 oracle: no,
 one and several iterations, on either side of the window count up to which the
 final flags go with every burst, with trials that are rejected."""
 import numpy as np
 import pytest
 
 from nav24_amd import problems
-from nav24_amd.abi import NAV_BA_FP64, workload_options
+from nav24_amd.abi import NAV_BA_FP64, NAV_BA_MIXED, workload_options
 from oracle import oracle
 from parity_util import say
 
@@ -40,3 +41,22 @@ def test_bursts_match_oracle(n_win, n_iter):
         assert abs(r.final_cost - ref.final_cost) <= 1e-9 * ref.cost_history.max()
         assert np.array_equal(r.outlier, ref.outlier) and r.n_outliers == ref.n_outliers
         assert np.array_equal(r.T_cw, a.T_cw) and np.array_equal(r.cost_history, a.cost_history)
+
+
+@pytest.mark.parametrize("fisheye", [False, True])
+@pytest.mark.parametrize("precision", [NAV_BA_FP64, NAV_BA_MIXED])
+@pytest.mark.parametrize("n_pt", [40, 1500])  # a camera in one item, in several
+def test_linearisation_together_or_apart(fisheye, precision, n_pt):
+    from nav24_amd.ba import GraphOptimHip
+    p = problems.workload(3, seed=n_pt, n_cam=6, n_pt=n_pt, obs_min=3, rot_sigma=0.005, trans_sigma=0.01)
+    if fisheye:
+        p = problems.with_kb8(p, seed=1)
+    o = workload_options(3)
+    o.precision, o.n_iter = precision, 3
+    s = GraphOptimHip(0)
+    one = s.solve(p, o)
+    s.set_timing(True)
+    apart = s.solve(p, o)
+    s.close()
+    assert np.array_equal(one.T_cw, apart.T_cw) and np.array_equal(one.X, apart.X)
+    assert np.array_equal(one.cost_history, apart.cost_history) and one.trials == apart.trials
