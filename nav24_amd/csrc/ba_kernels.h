@@ -190,7 +190,7 @@ struct DevWork {
     double* dp;
     double* Lm;         // one problem: Cholesky factor (tiled: n_pad^2; blocks: packed 6x6 blocks)
     double* Li;         // tiled path: inverses of the diagonal factor tiles [nt][kInvTile]
-    double* fpart;      // tiled path: forward-step products L_ij y_j [nt][nt][64]
+    double* fsum;       // tiled path: forward sums sum_k L_ik y_k of each tile row [nt][64]
     double* red_cost;   // [n_cblk] the cost at the current state (start of a solve, flags)
     double* red_tcost;  // [n_tiles] the trial cost at the candidate state, per linearisation tile
     double* red_scale;  // [n_win + n_tiles]: per-window camera part, then per-tile point parts

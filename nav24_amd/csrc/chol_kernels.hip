@@ -20,8 +20,8 @@
 // the diagonal factors L_kk themselves are never stored (only M_k is used).
 // All products run on FP64 MFMA (v_mfma_f64_16x16x4).
 // Measured (rocprofv3, average per launch, launch included): 28 tiles, step
-// 23.8 -> 16.8 us, first tile 18 -> 12.9 us, backward 28 launches of 4.2 -> 7 of
-// 9.5 us; 6 tiles, step 21.6 -> 14.6 us, against a factorisation of the diagonal
+// 23.8 -> 15.6 us, first tile 18 -> 12.6 us, backward 28 launches of 4.2 -> 7 of
+// 9.5 us; 6 tiles, step 21.6 -> 14.2 us, against a factorisation of the diagonal
 // tile by pivots (31 k cycles of the step's 55 k; square roots, a column per
 // pivot through LDS), operands staged through LDS and a launch per tile in the
 // backward step.  A step's floor is its launch (about 2 us), one round trip to
@@ -221,17 +221,20 @@ __device__ __forceinline__ void inv_store(double* __restrict__ Li, int b, int c,
 
 // a: the calling wave's blocks; D.g is written (a barrier follows before it is
 // read); nst: stages that hold rows of the system.  Li and y receive the
-// tile's inverse and forward result.  Returns false in the wave that met a
+// tile's inverse and forward result.  idle(h), h = 0, 1: other work for one wave
+// each, called where the chain does not wait for that wave.  Returns false in the wave that met a
 // pivot which is not positive and finite.
+template <class Idle>
 __device__ __forceinline__ bool diag_factor(dbl4 a[4], DiagLds& D, int nst, double* __restrict__ Li,
-                                            double* __restrict__ y) {
+                                            double* __restrict__ y, Idle idle) {
     const int lane = threadIdx.x & 63, w = wave_id(), r16 = lane & 15, kq = lane >> 4;
     const dbl4 zero = {0.0, 0.0, 0.0, 0.0};
     bool good = true;
     dbl4 m[4], gt[4], zs = zero;  // m[i]: block (i, w) of the unit inverse, result layout
-    for (int b = 0; b < w; ++b)  // the blocks above the diagonal
+    auto clear = [&](int b, int c) {  // a block above the diagonal
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Li[(16 * b + 4 * v + kq) * 64 + 16 * w + r16] = 0.0;
+        for (int v = 0; v < 4; ++v) Li[(16 * b + 4 * v + kq) * 64 + 16 * c + r16] = 0.0;
+    };
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         dbl4 R = zero;
@@ -260,6 +263,14 @@ __device__ __forceinline__ bool diag_factor(dbl4 a[4], DiagLds& D, int nst, doub
                     for (int p = 0; p < 4; ++p)
                         R = mfma16x16x4(W[64 * p + lane] * D.dinv[16 * k + 4 * p + kq], m[k][p], R);
                 }
+        }
+        if (s == 1 && w == 0) idle(0);
+        if (s == 2 && w == 1) idle(1);
+        if (s == 3 && w < 2) {
+            clear(w, 1 + w);
+            clear(w, 2 + w);
+            if (w == 0) clear(0, 3);
+            else clear(2, 3);
         }
         if (w == 0 && s > 0) {
             if (r16 == 0)
@@ -333,7 +344,7 @@ __global__ __launch_bounds__(256) void k_chol_first(const double* __restrict__ S
             for (int p = 0; p < 4; ++p) a[j][p] = S[(size_t)(16 * w + r16) * lda + 16 * j + 4 * p + kq];
     if (threadIdx.x < 64) D.g[threadIdx.x] = g[threadIdx.x];
     if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished
-    if (!diag_factor(a, D, tile_stages(n, 0), Li, y) && lane == 0) atomicOr(&lm->fail, 1);
+    if (!diag_factor(a, D, tile_stages(n, 0), Li, y, [](int) {}) && lane == 0) atomicOr(&lm->fail, 1);
 }
 
 // Four consecutive doubles of a row.
@@ -365,23 +376,26 @@ __device__ __forceinline__ void panel_rows(const double va[16], const double vm[
 // the rows 16 w.. of the tile.  Operands come from memory straight into
 // registers in the order the matrix instructions take them, L_ik stays there
 // (panel_rows), and only L_jk, which every wave needs, goes through LDS: one
-// barrier.  Workgroup (k+1, k+1) goes on to factor its tile, its wave 0 as soon
-// as it has the first block; it is the launch's critical path, so its waves take
-// priority over those that share its compute unit.
+// barrier.  (M_k through LDS too, loaded once instead of by each wave, cost a
+// second barrier and 2 k cycles.)  Workgroup (k+1, k+1) goes on to factor its tile
+// and is the launch's critical path: wave 0 starts the first block's
+// factorisation while the others still update theirs, L is stored by waves that
+// the chain does not wait for, and its waves take priority over those that share
+// its compute unit.
 __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, double* __restrict__ Lm,
                                                       double* __restrict__ Li, int lda, int n, int k,
                                                       const double* __restrict__ g, double* __restrict__ y,
-                                                      double* __restrict__ fpart, int nt, LMDev* lm) {
+                                                      double* __restrict__ fsum, LMDev* lm) {
     __shared__ double Wj[4][16][64];  // [rows 16 b][element][lane]
     __shared__ double ys[64];
     __shared__ DiagLds D;
     const int idx = blockIdx.x;
-    int ii = (int)((sqrt(8.0 * idx + 1.0) - 1.0) * 0.5);
+    int ii = (int)((sqrtf(8.0f * idx + 1.0f) - 1.0f) * 0.5f);  // to one; then exactly
     while ((ii + 1) * (ii + 2) / 2 <= idx) ++ii;
     while (ii * (ii + 1) / 2 > idx) --ii;
     const int jj = idx - ii * (ii + 1) / 2;
     const int i = k + 1 + ii, j = k + 1 + jj;
-    const bool same = (i == j), diag = idx == 0;
+    const bool same = (i == j), diag = idx == 0, panel = j == k + 1;
     if (diag) __builtin_amdgcn_s_setprio(3);
     // every global load of the launch in flight at once (no other workgroup
     // writes any of them)
@@ -399,7 +413,6 @@ __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, do
         for (int q = 0; q < 4; ++q) load4(vj + 4 * q, Aj + 16 * q);
     }
     dbl4 cur[4];
-    const double yk = j == k + 1 && w == 1 ? y[64 * k + lane] : 0.0;
     double* Aij = S + (size_t)(64 * i + 16 * w) * lda + 64 * j;
     if (diag) {
 #pragma unroll
@@ -413,20 +426,30 @@ __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, do
 #pragma unroll
             for (int v = 0; v < 4; ++v) cur[b][v] = Aij[(size_t)(4 * v + kq) * lda + 16 * b + r16];
     }
+    // the forward step: y_k, and sum_{t<k} L_it y_t of the earlier launches (one
+    // workgroup per launch adds its term, so the order is fixed)
+    const double yk = panel && w == 0 ? y[64 * k + lane] : 0.0;
+    double f0 = 0.0;
+    if (panel && k > 0) f0 = diag ? (w == 1 ? fsum[64 * i + lane] : 0.0) : (kq == 0 ? fsum[64 * i + 16 * w + r16] : 0.0);
+    const double gi = diag && w == 1 ? g[64 * i + lane] : 0.0;
     if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished (loads in flight meanwhile)
-    dbl4 Wi[4], Wr[4];
+    if (w == 0) ys[lane] = yk;
+    auto share = [&](const dbl4 W[4]) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Wj[w][4 * b + v][lane] = W[b][v];
+    };
+    dbl4 Wi[4];
     panel_rows(vi, vm, Wi);  // L_ik
-    if (same) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) Wr[b] = Wi[b];
-    } else {
+    __builtin_amdgcn_sched_barrier(0);  // what follows would lengthen the operands' lives
+    if (!same) {
+        dbl4 Wr[4];
         panel_rows(vj, vm, Wr);  // L_jk
+        share(Wr);
+    } else {
+        share(Wi);
     }
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Wj[w][4 * b + v][lane] = Wr[b][v];
-    if (w == 1) ys[lane] = yk;
     __syncthreads();
     if (diag) {
 #pragma unroll
@@ -434,41 +457,34 @@ __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, do
             if (b <= w)
 #pragma unroll
                 for (int p = 0; p < 16; ++p) cur[b] = mfma16x16x4(-Wj[b][p][lane], Wi[p >> 2][p & 3], cur[b]);
-    }
-    if (diag) {
-        // right-hand side of the tile, by wave 1, a row per lane: the terms
-        // L_it y_t of the earlier launches and this one's L_ik y_k
         if (w == 1) {
-            const double* fp = fpart + (size_t)i * nt * 64 + lane;
-            double f[4] = {g[64 * i + lane], 0.0, 0.0, 0.0};
-            int t = 0;
-            for (; t + 4 <= k; t += 4)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) f[u] -= fp[64 * (t + u)];
-            for (; t < k; ++t) f[0] -= fp[64 * t];
+            // the tile's right-hand side, a row per lane
+            double f[4] = {gi - f0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int p = 0; p < 16; ++p)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) f[q] = fma(-Wj[kq][p][r16 + 16 * q], ys[4 * p + q], f[q]);
             D.g[lane] = (f[0] + f[1]) + (f[2] + f[3]);
         }
-    } else if (j == k + 1) {
-        // L_ik y_k, for the forward step of tile i
-        double f = 0.0;
+        // two waves store L_ik while the chain goes on without them
+        auto store_l = [&](int half) {
+            double* L = Lm + (size_t)(64 * i + 32 * half + r16) * lda + 64 * k + kq;
+#pragma unroll
+            for (int p = 0; p < 32; ++p) L[(size_t)(16 * (p >> 4)) * lda + 4 * (p & 15)] = Wj[2 * half + (p >> 4)][p & 15][lane];
+        };
+        if (!diag_factor(cur, D, tile_stages(n, i), Li + (size_t)kInvTile * i, y + 64 * i, store_l) && lane == 0)
+            atomicOr(&lm->fail, 1);
+        return;
+    }
+    if (panel) {
+        double f = f0;  // + L_ik y_k
 #pragma unroll
         for (int p = 0; p < 16; ++p) f = fma(Wi[p >> 2][p & 3], ys[4 * p + kq], f);
         f = sum_over_k(f);
-        if (kq == 0) fpart[((size_t)i * nt + k) * 64 + 16 * w + r16] = f;
-    }
-    if (j == k + 1) {
+        if (kq == 0) fsum[64 * i + 16 * w + r16] = f;
         double* L = Lm + (size_t)(64 * i + 16 * w + r16) * lda + 64 * k + kq;
 #pragma unroll
         for (int p = 0; p < 16; ++p) L[4 * p] = Wi[p >> 2][p & 3];
-    }
-    if (diag) {
-        if (!diag_factor(cur, D, tile_stages(n, i), Li + (size_t)kInvTile * i, y + 64 * i) && lane == 0)
-            atomicOr(&lm->fail, 1);
-        return;
     }
 #pragma unroll
     for (int b = 0; b < 4; ++b)
@@ -1488,7 +1504,7 @@ void launch_cholesky_solve(const DevProblem& P, const DevState& cur, const DevSt
     for (int k = 0; k + 1 < nt; ++k) {
         const int rem = nt - k - 1;
         hipLaunchKernelGGL(k_chol_step, dim3(rem * (rem + 1) / 2), dim3(256), 0, st, W.S, W.Lm, W.Li, lda, P.n, k,
-                           (const double*)W.g, W.y, W.fpart, nt, W.lm);
+                           (const double*)W.g, W.y, W.fsum, W.lm);
     }
     if (nt <= kBackSingleMax) {
         const int np = std::max(1, (64 * (nt - 1) + 127) / 128);
