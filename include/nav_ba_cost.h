@@ -81,6 +81,16 @@ int32_t nav_ba_cost_eval_tangent(nav_ba_cost_handle* h, int32_t dtype, const voi
 int32_t nav_ba_cost_tangent_grad(int32_t device, int32_t dtype, int32_t n, const void* xi, const void* g_pose,
                                  void* g_xi, void* stream);
 
+/*
+ * The gradients of a cost times the incoming gradient *g (device, dtype), in one
+ * launch on `stream`: out_xi [n_cam][6] = *g J_l(xi)^T g_pose, out_X [n_pt][3] =
+ * *g g_X, out_intr [8] = *g g_intr, the inputs as nav_ba_cost_eval_tangent took
+ * and returned them.  Null outputs are skipped.  Needs no handle.
+ */
+int32_t nav_ba_cost_backward(int32_t device, int32_t dtype, int32_t n_cam, int32_t n_pt, const void* xi,
+                             const void* g_pose, const void* g_X, const void* g_intr, const void* g, void* out_xi,
+                             void* out_X, void* out_intr, void* stream);
+
 /* Sizes of the prepared batch. */
 int32_t nav_ba_cost_sizes(const nav_ba_cost_handle* h, int32_t* n_cam, int32_t* n_pt, int32_t* n_obs,
                           int32_t* n_problems);

@@ -451,10 +451,10 @@ __global__ void k_se3_left(int n, const T* __restrict__ xi, const T* __restrict_
 //   g_upsilon -> V^T g_u
 //   g_omega   -> V^T (g_w - p x g_u) + grad_omega (g_u . V u),
 // the last term from V u = u + b w x u + c (w (w.u) - |w|^2 u).
+// The result is rounded to T and then multiplied by scale.
 template <typename T>
-__global__ void k_tangent_grad(int n, const T* __restrict__ xi, const T* __restrict__ g, T* __restrict__ out) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
+__device__ __forceinline__ void tangent_grad_row(int c, const T* __restrict__ xi, const T* __restrict__ g, T scale,
+                                                 T* __restrict__ out) {
     double w[3], u[3], gw[3], gu[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -477,9 +477,45 @@ __global__ void k_tangent_grad(int n, const T* __restrict__ xi, const T* __restr
     const double s = k.db * wug + k.dc * (gw0 * wu - t2 * gu0) - 2.0 * k.c * gu0;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        out[6 * (size_t)c + i] = (T)(rw[i] + k.b * ug[i] + k.c * (gu[i] * wu + u[i] * gw0) + s * w[i]);
-        out[6 * (size_t)c + 3 + i] = (T)ru[i];
+        out[6 * (size_t)c + i] = (T)(rw[i] + k.b * ug[i] + k.c * (gu[i] * wu + u[i] * gw0) + s * w[i]) * scale;
+        out[6 * (size_t)c + 3 + i] = (T)ru[i] * scale;
     }
+}
+
+template <typename T>
+__global__ void k_tangent_grad(int n, const T* __restrict__ xi, const T* __restrict__ g, T* __restrict__ out) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < n) tangent_grad_row<T>(c, xi, g, T(1), out);
+}
+
+// The three gradients of a cost times the incoming gradient: poses (b_pose
+// workgroups), points (four entries per thread), intrinsics.  Launch bound; as a
+// kernel for the poses and three products it was four launches, 20 us of a
+// step's host time.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_backward(int n, long long nx, const T* __restrict__ xi,
+                                                       const T* __restrict__ gp, const T* __restrict__ gX,
+                                                       const T* __restrict__ gi, const T* __restrict__ scale,
+                                                       T* __restrict__ out_xi, T* __restrict__ out_X,
+                                                       T* __restrict__ out_i, int b_pose, int b_pt) {
+    const T s = *scale;
+    int b = blockIdx.x;
+    if (b < b_pose) {
+        const int c = b * kThreads + threadIdx.x;
+        if (c < n) tangent_grad_row<T>(c, xi, gp, s, out_xi);
+        return;
+    }
+    b -= b_pose;
+    if (b < b_pt) {
+        const long long i0 = 4LL * kThreads * b + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const long long i = i0 + q * kThreads;
+            if (i < nx) out_X[i] = gX[i] * s;
+        }
+        return;
+    }
+    if (threadIdx.x < 8) out_i[threadIdx.x] = gi[threadIdx.x] * s;
 }
 
 }  // namespace navcost
@@ -563,6 +599,19 @@ template <typename T>
 int32_t tangent_grad_t(int n, const T* xi, const T* g, T* out, hipStream_t s) {
     hipLaunchKernelGGL(k_tangent_grad<T>, dim3((n + kPoseThreads - 1) / kPoseThreads), dim3(kPoseThreads), 0, s, n, xi, g,
                        out);
+    return hipGetLastError() == hipSuccess ? NAV_BA_OK : NAV_BA_HIP_ERROR;
+}
+
+// Null outputs are skipped.
+template <typename T>
+int32_t backward_t(int n, long long nx, const T* xi, const T* gp, const T* gX, const T* gi, const T* scale, T* out_xi,
+                   T* out_X, T* out_i, hipStream_t s) {
+    const int b_pose = out_xi ? (n + kThreads - 1) / kThreads : 0;
+    const int b_pt = out_X ? (int)((nx + 4 * kThreads - 1) / (4 * kThreads)) : 0;
+    const int blocks = b_pose + b_pt + (out_i ? 1 : 0);
+    if (blocks == 0) return NAV_BA_OK;
+    hipLaunchKernelGGL(k_backward<T>, dim3(blocks), dim3(kThreads), 0, s, n, nx, xi, gp, gX, gi, scale, out_xi, out_X,
+                       out_i, b_pose, b_pt);
     return hipGetLastError() == hipSuccess ? NAV_BA_OK : NAV_BA_HIP_ERROR;
 }
 
@@ -811,6 +860,28 @@ int32_t nav_ba_cost_tangent_grad(int32_t device, int32_t dtype, int32_t n, const
     const int32_t st = dtype == NAV_BA_COST_F64
                            ? tangent_grad_t<double>(n, (const double*)xi, (const double*)g_pose, (double*)g_xi, s)
                            : tangent_grad_t<float>(n, (const float*)xi, (const float*)g_pose, (float*)g_xi, s);
+    if (was != device && hipSetDevice(was) != hipSuccess) return NAV_BA_HIP_ERROR;
+    return st;
+}
+
+int32_t nav_ba_cost_backward(int32_t device, int32_t dtype, int32_t n_cam, int32_t n_pt, const void* xi,
+                             const void* g_pose, const void* g_X, const void* g_intr, const void* g, void* out_xi,
+                             void* out_X, void* out_intr, void* stream) {
+    if (n_cam < 0 || n_pt < 0 || !g || (dtype != NAV_BA_COST_F64 && dtype != NAV_BA_COST_F32)) return NAV_BA_BAD_ARG;
+    if ((out_xi && n_cam > 0 && (!xi || !g_pose)) || (out_X && n_pt > 0 && !g_X) || (out_intr && !g_intr))
+        return NAV_BA_BAD_ARG;
+    int was = 0;
+    if (hipGetDevice(&was) != hipSuccess) return NAV_BA_HIP_ERROR;
+    if (was != device && hipSetDevice(device) != hipSuccess) return NAV_BA_HIP_ERROR;
+    hipStream_t s = (hipStream_t)stream;
+    const long long nx = 3LL * n_pt;
+    const int32_t st =
+        dtype == NAV_BA_COST_F64
+            ? backward_t<double>(n_cam, nx, (const double*)xi, (const double*)g_pose, (const double*)g_X,
+                                 (const double*)g_intr, (const double*)g, (double*)out_xi, (double*)out_X,
+                                 (double*)out_intr, s)
+            : backward_t<float>(n_cam, nx, (const float*)xi, (const float*)g_pose, (const float*)g_X,
+                                (const float*)g_intr, (const float*)g, (float*)out_xi, (float*)out_X, (float*)out_intr, s);
     if (was != device && hipSetDevice(was) != hipSuccess) return NAV_BA_HIP_ERROR;
     return st;
 }

@@ -53,6 +53,8 @@ def lib() -> C.CDLL:
         L.nav_ba_cost_eval_tangent.restype = C.c_int32
         L.nav_ba_cost_tangent_grad.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp]
         L.nav_ba_cost_tangent_grad.restype = C.c_int32
+        L.nav_ba_cost_backward.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32] + [vp] * 9
+        L.nav_ba_cost_backward.restype = C.c_int32
         L.nav_ba_cost_sizes.argtypes = [H, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32),
                                         C.POINTER(C.c_int32)]
         L.nav_ba_cost_sizes.restype = C.c_int32
@@ -174,6 +176,31 @@ def _tangent_grad(xi, g_pose):
     return out
 
 
+def _scaled_gradients(g, xi, gp, gx, gi, need):
+    """(g J_l(xi)^T gp, g gx, g gi) in one kernel, None where not needed, for
+    tensors that `_one_kernel` accepts."""
+    import torch
+    out = [torch.empty_like(t) if n else None for t, n in zip((gp, gx, gi), need)]
+    st = lib().nav_ba_cost_backward(
+        xi.device.index, NAV_BA_COST_F64 if xi.dtype == torch.float64 else NAV_BA_COST_F32, xi.shape[0], gx.shape[0],
+        xi.data_ptr(), gp.data_ptr(), gx.data_ptr(), gi.data_ptr(), g.data_ptr(),
+        *[None if t is None else t.data_ptr() for t in out], torch.cuda.current_stream(xi.device).cuda_stream)
+    if st != NAV_BA_OK:
+        raise CostError(st, "nav_ba_cost_backward")
+    return out
+
+
+def _one_kernel(g, *saved) -> bool:
+    """Whether the gradients can be formed in one kernel: no graph of the backward
+    is asked for, and the incoming gradient and the saved tensors (a hook may have
+    moved or converted them) are plain device tensors of one type and device."""
+    import torch
+    dt, dev = g.dtype, g.device
+    return (not torch.is_grad_enabled() and g.is_cuda and g.dim() == 0 and dt in (torch.float64, torch.float32)
+            and all(type(t) is torch.Tensor and t.dtype == dt and t.device == dev and t.is_contiguous()
+                    for t in (g, *saved)))
+
+
 def se3_left(xi, T_cw):
     """exp(xi) T_cw for every pose row [R (9) | t (3)], xi = (omega, upsilon), in torch.
     Below theta^2 = 1e-6 the Rodrigues and V coefficients are their series to
@@ -247,6 +274,8 @@ try:
         @staticmethod
         def backward(ctx, g):
             gp, gx, gi, xi, T_cw, T = ctx.saved_tensors
+            if ctx.kernels and _one_kernel(g, gp, gx, gi, xi):
+                return (*_scaled_gradients(g, xi, gp, gx, gi, ctx.needs_input_grad[:3]), None, None)
             g_xi = None
             if ctx.needs_input_grad[0]:
                 # d cost / d xi = J_l(xi)^T gp, gp the left-tangent gradient at T

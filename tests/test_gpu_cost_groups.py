@@ -83,3 +83,31 @@ def test_layouts_match_oracle(name, idle_cam):
         assert all(bool((t == -1.0).all()) for j, t in enumerate(got) if j != k)
     assert torch.equal(b.eval(dT, dX, dI, grad=False).cost, r.cost)
     b.close()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n_cam,n_pt", [(2, 1), (4, 341), (4, 342), (257, 400)])  # 1 024 point entries per workgroup
+def test_scaled_gradients_in_one_kernel(dtype, n_cam, n_pt):
+    """The backward's one kernel against the product with the pose kernel's result
+    and the saved gradients: the same operations, so the same bits; with a graph
+    of the backward the products are differentiable in the incoming gradient."""
+    from nav24_amd.diffcost import BACost, CostBatch, _tangent_grad
+    p = counted(1, [3] * n_pt, n_cam=n_cam)
+    T = torch.tensor(p.T_cw, device="cuda", dtype=dtype)
+    gen = torch.Generator().manual_seed(n_cam)
+    leaves = [(0.05 * torch.randn(n_cam, 6, generator=gen)).to("cuda", dtype), torch.tensor(p.X, device="cuda", dtype=dtype),
+              torch.tensor([p.fx, p.fy, p.cx, p.cy, *p.dist], device="cuda", dtype=dtype)]
+    b = CostBatch([p])
+    r = b._eval_tangent(*leaves, T, True)[2]
+    g = torch.tensor(0.37, device="cuda", dtype=dtype)
+    want = [g * _tangent_grad(leaves[0], r.g_pose), g * r.g_X, g * r.g_intr]
+    leaves = [t.requires_grad_(True) for t in leaves]
+    got = torch.autograd.grad(BACost.apply(*leaves, T, b), leaves, g)
+    assert all(torch.equal(a, w) for a, w in zip(got, want))
+    (one,) = torch.autograd.grad(BACost.apply(leaves[0].detach(), leaves[1], leaves[2].detach(), T, b), leaves[1], g)
+    assert torch.equal(one, want[1])
+    gr = g.clone().requires_grad_(True)
+    again = torch.autograd.grad(BACost.apply(*leaves, T, b), leaves, gr, create_graph=True)
+    (dg,) = torch.autograd.grad(again[2].sum(), gr)
+    assert all(torch.equal(a, w) for a, w in zip(again, want)) and torch.allclose(dg, r.g_intr.sum())
+    b.close()
