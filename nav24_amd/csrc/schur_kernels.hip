@@ -283,7 +283,8 @@ __device__ __forceinline__ void pair_factors(const DevProblem& P, const double* 
 #pragma unroll
         for (int q = 0; q < 6; ++q) E[q] = wb[6 + q];
         mul_et(E, J, C);
-        const double wz = wgt * iz, s0 = wz * (P.fx * P.fx), s1 = wz * (P.fy * P.fy);
+        // (the weight last: its load has the longest to land)
+        const double s0 = wgt * (iz * (P.fx * P.fx)), s1 = wgt * (iz * (P.fy * P.fy));
         C[0] *= s0; C[2] *= s0;
         C[1] *= s1; C[3] *= s1;
         unit_xi(wb[0], wb[1], wb[2], A0, A1);
