@@ -196,9 +196,15 @@ def _one_kernel(g, *saved) -> bool:
     moved or converted them) are plain device tensors of one type and device."""
     import torch
     dt, dev = g.dtype, g.device
-    return (not torch.is_grad_enabled() and g.is_cuda and g.dim() == 0 and dt in (torch.float64, torch.float32)
-            and all(type(t) is torch.Tensor and t.dtype == dt and t.device == dev and t.is_contiguous()
-                    for t in (g, *saved)))
+    if (torch.is_grad_enabled() or not g.is_cuda or g.dim() != 0 or dt not in (torch.float64, torch.float32)
+            or any(type(t) is not torch.Tensor or t.dtype != dt or t.device != dev or not t.is_contiguous()
+                   for t in (g, *saved))):
+        return False
+    try:
+        g.data_ptr()  # a batch of incoming gradients (is_grads_batched) has no memory of its own
+    except RuntimeError:
+        return False
+    return True
 
 
 def se3_left(xi, T_cw):

@@ -111,3 +111,21 @@ def test_scaled_gradients_in_one_kernel(dtype, n_cam, n_pt):
     (dg,) = torch.autograd.grad(again[2].sum(), gr)
     assert all(torch.equal(a, w) for a, w in zip(again, want)) and torch.allclose(dg, r.g_intr.sum())
     b.close()
+
+
+def test_batch_of_incoming_gradients():
+    """torch.autograd.grad's is_grads_batched runs the backward on a batch at once."""
+    from nav24_amd.diffcost import BACost, CostBatch
+    p = counted(2, [4] * 20, n_cam=4)
+    T = torch.tensor(p.T_cw, device="cuda")
+    leaves = [torch.full((4, 6), 0.01, device="cuda", dtype=torch.float64), torch.tensor(p.X, device="cuda"),
+              torch.tensor([p.fx, p.fy, p.cx, p.cy, *p.dist], device="cuda")]
+    leaves = [t.requires_grad_(True) for t in leaves]
+    b = CostBatch([p])
+    gs = torch.tensor([1.0, -0.5, 3.0], device="cuda", dtype=torch.float64)
+    cost = BACost.apply(*leaves, T, b)
+    many = torch.autograd.grad(cost, leaves, gs, is_grads_batched=True, retain_graph=True)
+    for k, g in enumerate(gs):
+        one = torch.autograd.grad(cost, leaves, g, retain_graph=True)
+        assert all(torch.equal(m[k], o) for m, o in zip(many, one))
+    b.close()
