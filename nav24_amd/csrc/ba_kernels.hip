@@ -342,7 +342,7 @@ void launch_lin(const DevProblem& P, const DevState& s, const DevWork& W, hipStr
 // ---------------------------------------------------------------- lambda init
 // g2o computeLambdaInit with no user lambda: tau * max |H_jj| over the free
 // vertices of the window, tau = 1e-5.  Launched in the first step only, where
-// every window is at iteration 0 and its lambda slot holds 0 (k_lm_reset).
+// every window is at iteration 0 and its lambda slot holds 0 (k_run_start).
 // k_diag_max: one thread per free vertex (free cameras, then points); the
 // maximum goes into the window's lambda slot by an integer atomic max on the
 // bit pattern, which orders non-negative doubles as their values (NaN

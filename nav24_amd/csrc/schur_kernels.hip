@@ -55,18 +55,24 @@ namespace navba {
 constexpr int kStageStride = 37; // odd stride of the staged rows (one per lane group, 36 entries)
 
 // An observation a's row in LDS: what a pair (a, b) needs of a.
-//   E_a (6 doubles), the point (3) and the entries of J_xi,a (type T; a pinhole's
-//   two structural zeros left out); or, for the FP64 pinhole, the normalised
-//   image point (x / z, y / z) and 1 / z in place of J_xi,a, whose entries are
-//   products of these, with the focal lengths folded into E_a: 12 doubles.
+//   Pinhole, FP64: the normalised image point (x / z, y / z) and 1 / z, of which
+//   J_xi,a's entries are products, the point (3) and E_a with the focal lengths
+//   folded in (6): 12 doubles.
+//   Pinhole, mixed: E_a, the point and the entries of J_xi,a but for the two
+//   structural zeros (10 floats).
+//   Fisheye: W_a = J_xi,a^T E_a (18 doubles) and the point.  Without the zeros a
+//   pair costs the same 36 multiply-adds through E_a or W_a, and J_xi,a next to b's
+//   Jacobians spills more registers: with E_a the rounds kernel spilled 105
+//   instead of 81 (mixed 109 instead of 53) and took 272 us against 257 on 60
+//   keyframes and 565 000 observations.
 // A row is a whole number of 16-byte reads, and its stride in banks is 4 times an
 // odd number, so that the lanes' rows start in all sixteen 16-byte columns.
 template <typename T, int CM>
 struct RowA {
     static constexpr bool normalised = CM == kCamPinhole && sizeof(T) == 8;
-    static constexpr int stride = normalised || CM == kCamPinhole ? 14 : sizeof(T) == 8 ? 22 : 18;
-    static constexpr int n_xi = CM == kCamPinhole ? 10 : 12;
-    static_assert(normalised || 9 * sizeof(double) + n_xi * sizeof(T) <= stride * sizeof(double), "row size");
+    static constexpr bool whole = CM != kCamPinhole;  // the row holds W_a
+    static constexpr int stride = whole ? 22 : 14;
+    static_assert(normalised || whole || 9 * sizeof(double) + 10 * sizeof(T) <= stride * sizeof(double), "row size");
     static_assert(stride % 2 == 0 && (stride / 2) % 2 == 1, "row stride");
 };
 
@@ -207,6 +213,12 @@ __device__ __forceinline__ void schur_phase_a(const DevProblem& P, const double 
             wb[6 + j] = E[j] * P.fx;
             wb[9 + j] = E[3 + j] * P.fy;
         }
+    } else if constexpr (RowA<T, CM>::whole) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) wb[3 * i + j] = (double)La.Jxi[i] * E[j] + (double)La.Jxi[6 + i] * E[3 + j];
+        wb[18] = in.x; wb[19] = in.y; wb[20] = in.z;
     } else {
 #pragma unroll
         for (int j = 0; j < 6; ++j) wb[j] = E[j];
@@ -215,7 +227,7 @@ __device__ __forceinline__ void schur_phase_a(const DevProblem& P, const double 
         int q = 0;
 #pragma unroll
         for (int j = 0; j < 12; ++j)
-            if (!zx || (j != 4 && j != 9)) xi[q++] = La.Jxi[j];
+            if (j != 4 && j != 9) xi[q++] = La.Jxi[j];
     }
     if (g0) {
         double A0[6], A1[6], C[4], M0[6], M1[6];
@@ -267,8 +279,8 @@ template <typename T, int CM>
 __device__ __forceinline__ void pair_factors(const DevProblem& P, const double* wb, double wgt, const double Rb[9],
                                              const double tb[3], double M0[6], double M1[6], double B0[6],
                                              double B1[6]) {
-    double A0[6], A1[6], C[4];
     if constexpr (RowA<T, CM>::normalised) {
+        double A0[6], A1[6], C[4];
         double xc, yc, zc;
         transform(Rb, tb, wb[3], wb[4], wb[5], xc, yc, zc);
         const double iz = recip<double>(zc);
@@ -289,27 +301,37 @@ __device__ __forceinline__ void pair_factors(const DevProblem& P, const double* 
         C[1] *= s1; C[3] *= s1;
         unit_xi(wb[0], wb[1], wb[2], A0, A1);
         unit_xi(a, b, iz, B0, B1);
+        mul_xi_c<CM>(A0, A1, C, M0, M1);
     } else {
+        constexpr int pt = RowA<T, CM>::whole ? 18 : 6;
         EdgeLin<T> Lb;
-        edge_linearize_m<CM>(P, Rb, tb, wb[6], wb[7], wb[8], 0.0, 0.0, Lb);
+        edge_linearize_m<CM>(P, Rb, tb, wb[pt], wb[pt + 1], wb[pt + 2], 0.0, 0.0, Lb);
         double JXb[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) JXb[q] = wgt * (double)Lb.JX[q];  // the Huber weight of b folded in
-        mul_et(wb, JXb, C);
-        const T* xi = reinterpret_cast<const T*>(wb + 9);
-        int q = 0;
+        if constexpr (RowA<T, CM>::whole) {
 #pragma unroll
-        for (int j = 0; j < 12; ++j) {
-            const bool zero = CamTraits<CM>::xi_zeros && (j == 4 || j == 9);
-            const double v = zero ? 0.0 : (double)xi[q];
-            if (!zero) ++q;
-            if (j < 6) A0[j] = v;
-            else A1[j - 6] = v;
+            for (int r = 0; r < 6; ++r) {
+                const double v0 = wb[3 * r], v1 = wb[3 * r + 1], v2 = wb[3 * r + 2];
+                M0[r] = v0 * JXb[0] + v1 * JXb[1] + v2 * JXb[2];
+                M1[r] = v0 * JXb[3] + v1 * JXb[4] + v2 * JXb[5];
+            }
+        } else {
+            double A0[6], A1[6], C[4];
+            mul_et(wb, JXb, C);
+            const T* xi = reinterpret_cast<const T*>(wb + 9);
+            int q = 0;
+#pragma unroll
+            for (int j = 0; j < 12; ++j) {
+                const double v = j == 4 || j == 9 ? 0.0 : (double)xi[q++];
+                if (j < 6) A0[j] = v;
+                else A1[j - 6] = v;
+            }
+            mul_xi_c<CM>(A0, A1, C, M0, M1);
         }
 #pragma unroll
         for (int c = 0; c < 6; ++c) { B0[c] = (double)Lb.Jxi[c]; B1[c] = (double)Lb.Jxi[6 + c]; }
     }
-    mul_xi_c<CM>(A0, A1, C, M0, M1);
 }
 
 // Phase B: the lane's pairs (entry rows of stride kWave from pl, nrow rows; e0,
