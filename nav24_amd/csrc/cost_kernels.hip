@@ -37,9 +37,13 @@ using navba::wave_sum;
 
 constexpr int kTileObs = 256;  // observations per tile (whole points; one larger point has a tile of its own)
 constexpr int kThreads = 256;
-// Groups and chunks are as long as still leaves kGroups and kChunks of them (eight
-// and four workgroups per CU), so that their sums over the workgroup come once in
-// many observations, and at most kGroupTiles tiles, kChunkMax observations.
+// Sums over the workgroup come once per group or chunk, so these are long where
+// there are many observations.  Groups are as short as keeps them to kGroups (eight
+// workgroups per CU, resident together for the cost alone), up to kGroupTiles tiles:
+// one round of workgroups and a little more is the worst case (gradients of 0.8, 1.0
+// and 3.2 M observations: 26.7, 31.0 and 63 us; with at least kGroups of them, 31.8,
+// 37.4 and 64; with twice as many, 31.8, 37.1 and 66.5).  Chunks are as long as
+// leaves kChunks of them, up to kChunkMax observations.
 constexpr int kXcds = 8;
 constexpr int kGroups = 2048;
 constexpr int kChunks = 1024;
@@ -731,8 +735,13 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
         }
     }
     // groups of consecutive tiles of one problem
-    const int n_tiles = prob_tile0.back();
-    const int per_group = std::min(kGroupTiles, std::max(1, n_tiles / kGroups));
+    auto groups_of = [&](int per) {
+        long long n = 0;
+        for (int p = 0; p < n_probs; ++p) n += (prob_tile0[p + 1] - prob_tile0[p] + per - 1) / per;
+        return n;
+    };
+    int per_group = 1;
+    while (per_group < kGroupTiles && groups_of(per_group) > kGroups) ++per_group;
     std::vector<int> group_tile{0}, prob_group0{0};
     for (int p = 0; p < n_probs; ++p) {
         for (int t = prob_tile0[p]; t < prob_tile0[p + 1];) {

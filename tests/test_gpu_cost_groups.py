@@ -49,6 +49,9 @@ CASES = {
     "a point of several rounds": [[3, 700, 0, 5]],
     "many small points": [[4] * 200],
     "an empty problem between": [[5, 0, 7], [0, 0], [130, 130, 2]],
+    "as many tiles as groups": [[256] * 2048],
+    "one tile more": [[256] * 2049],
+    "groups of three, two problems": [[256] * 2049, [256] * 2050],
 }
 
 
