@@ -388,6 +388,7 @@ __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, do
                                                       double* __restrict__ fsum, LMDev* lm) {
     __shared__ double Wj[4][16][64];  // [rows 16 b][element][lane]
     __shared__ double ys[64];
+    __shared__ int nz[4];
     __shared__ DiagLds D;
     const int idx = blockIdx.x;
     int ii = (int)((sqrtf(8.0f * idx + 1.0f) - 1.0f) * 0.5f);  // to one; then exactly
@@ -433,6 +434,31 @@ __global__ __launch_bounds__(256, 2) void k_chol_step(double* __restrict__ S, do
     if (panel && k > 0) f0 = diag ? (w == 1 ? fsum[64 * i + lane] : 0.0) : (kq == 0 ? fsum[64 * i + 16 * w + r16] : 0.0);
     const double gi = diag && w == 1 ? g[64 * i + lane] : 0.0;
     if (lm->phase == kPhaseDone) return;  // a step launched after the solve has finished (loads in flight meanwhile)
+    if (!diag) {
+        // A zero A_ik or A_jk (cameras that share no points, and no fill) leaves the
+        // tile as it is: the workgroup ends here and leaves the matrix cores to the
+        // others.  28 tiles of a 300-camera loop, where 55 of the 378 tiles take part
+        // in the first step: 422 -> 412 us for the 27 steps, the same bits.
+        bool zi = true, zj = true;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            zi = zi && vi[q] == 0.0;
+            zj = zj && (same || vj[q] == 0.0);
+        }
+        const int some = (__any(!zi) ? 1 : 0) | (__any(same ? !zi : !zj) ? 2 : 0);
+        if (lane == 0) nz[w] = some;
+        __syncthreads();
+        const int all = nz[0] | nz[1] | nz[2] | nz[3];
+        if (!(all & 1) || (!panel && !(all & 2))) {
+            if (panel) {  // L_ik = 0; its term of the forward sum too
+                if (k == 0 && kq == 0) fsum[64 * i + 16 * w + r16] = 0.0;
+                double* L = Lm + (size_t)(64 * i + 16 * w + r16) * lda + 64 * k + kq;
+#pragma unroll
+                for (int p = 0; p < 16; ++p) L[4 * p] = 0.0;
+            }
+            return;
+        }
+    }
     if (w == 0) ys[lane] = yk;
     auto share = [&](const dbl4 W[4]) {
 #pragma unroll

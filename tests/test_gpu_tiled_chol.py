@@ -38,3 +38,31 @@ def test_tiled_sizes_match_oracle(n_free):
     say(f"free cameras {n_free}: cost {rel:.1e}, pose {dT:.1e}")
     assert rel <= 1e-9 and dT <= 1e-6
     assert np.array_equal(r.T_cw, again.T_cw)
+
+
+# A loop, where cameras on opposite sides share no points: 7, 12 and 14 tiles with
+# whole tiles of zeros that the factorisation skips, in the first column too.
+@pytest.mark.parametrize("n_cam,n_pt", [(72, 2000), (130, 3000), (150, 4000)])
+def test_zero_tiles_match_oracle(n_cam, n_pt):
+    """Three LM iterations, a few mrad and cm from the solution: the bars of the
+    test above.  The second solve of the handle, whose factors hold the first
+    one's, gives the same bits."""
+    from nav24_amd.ba import GraphOptimHip
+    p = problems.workload(2, seed=1, n_cam=n_cam, n_pt=n_pt, rot_sigma=0.005, trans_sigma=0.01, point_sigma=0.02)
+    seen = np.zeros((n_pt, n_cam), int)
+    seen[p.obs_pt, p.obs_cam] = 1
+    shared = (seen.T @ seen)[2:, 2:] > 0  # the free cameras
+    assert not shared[:11, n_cam // 2 - 11:n_cam // 2 + 11].any()  # more than a tile's 64 unknowns either way
+    o = workload_options(2)
+    o.precision, o.n_iter = NAV_BA_FP64, 3
+    ref = oracle.solve(p, o)
+    s = GraphOptimHip(0)
+    s.set_solver(1)
+    r, again = s.solve(p, o), s.solve(p, o)
+    s.close()
+    assert (r.iterations, r.trials, r.stop_reason) == (ref.iterations, ref.trials, ref.stop_reason)
+    rel = np.abs(r.cost_history - ref.cost_history).max() / ref.cost_history.max()
+    dT = np.abs(r.T_cw - ref.T_cw).max()
+    say(f"loop of {n_cam}: cost {rel:.1e}, pose {dT:.1e}")
+    assert rel <= 1e-9 and dT <= 1e-6
+    assert np.array_equal(r.T_cw, again.T_cw)
