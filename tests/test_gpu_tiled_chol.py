@@ -41,8 +41,10 @@ def test_tiled_sizes_match_oracle(n_free):
 
 
 # A loop, where cameras on opposite sides share no points: 7, 12 and 14 tiles with
-# whole tiles of zeros that the factorisation skips, in the first column too.
-@pytest.mark.parametrize("n_cam,n_pt", [(72, 2000), (130, 3000), (150, 4000)])
+# whole tiles of zeros that the factorisation skips, in the first column too; 25
+# and 34 tiles, whose first steps have 300 and 561 workgroups (the critical one is
+# placed by their number: up to 256, below 512, more).
+@pytest.mark.parametrize("n_cam,n_pt", [(72, 2000), (130, 3000), (150, 4000), (262, 7000), (362, 9000)])
 def test_zero_tiles_match_oracle(n_cam, n_pt):
     """Three LM iterations, a few mrad and cm from the solution: the bars of the
     test above.  The second solve of the handle, whose factors hold the first
