@@ -20,7 +20,7 @@
 // the diagonal factors L_kk themselves are never stored (only M_k is used).
 // All products run on FP64 MFMA (v_mfma_f64_16x16x4).
 // Measured (rocprofv3, average per launch, launch included): 28 tiles, step
-// 23.8 -> 15.6 us, first tile 18 -> 12.6 us, backward 28 launches of 4.2 -> 7 of
+// 23.8 -> 15.6 us (14.9 without the zero tiles), first tile 18 -> 12.6 us, backward 28 launches of 4.2 -> 7 of
 // 9.5 us; 6 tiles, step 21.6 -> 14.2 us, against a factorisation of the diagonal
 // tile by pivots (31 k cycles of the step's 55 k; square roots, a column per
 // pivot through LDS), operands staged through LDS and a launch per tile in the
