@@ -67,7 +67,8 @@ int32_t nav_ba_cost_eval(nav_ba_cost_handle* h, int32_t dtype, const void* T_cw,
 
 /* The same evaluation at the poses T = exp(xi) T_cw, xi [n_cam][6] pose
  * tangents (omega, upsilon):
- *   T       [n_cam][12]  out: the poses the cost was evaluated at
+ *   T       [n_cam][12]  out: the poses the cost was evaluated at, rounded to
+ *                        dtype (they are formed and used in FP64 for both types)
  *   total   [1]          out: the sum of the problems' costs (FP64 sum, rounded once)
  * and the rest as nav_ba_cost_eval (g_pose is the left-tangent gradient at T). */
 int32_t nav_ba_cost_eval_tangent(nav_ba_cost_handle* h, int32_t dtype, const void* xi, const void* T_cw,

@@ -92,9 +92,12 @@ enum Want { kCost = 0, kPointSide = 1, kPoseSide = 2 };
 // of two pixel coordinates of a few hundred pixels, and in FP32 that
 // cancellation alone left the cost of an FP32 problem 6.6e-4 off its FP64
 // value (FP64 issues at the FP32 rate on gfx950 without packed math, so the
-// forward costs the same).  The adjoint then runs in T.
-template <typename T, Want kWant>
-__device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __restrict__ X, const T in[8], double u,
+// forward costs the same).  The adjoint then runs in T.  TP is the type of the
+// poses: T where they are the caller's, FP64 where they come from k_se3_left (a
+// pose of ~10 m rounded to float is half a micrometre off, which near a camera's
+// plane is the whole error of the gradients).
+template <typename T, Want kWant, typename TP>
+__device__ __forceinline__ void obs_term(const TP* __restrict__ Tcw, const T* __restrict__ X, const T in[8], double u,
                                          double v, int robust, double delta, ObsGrad<T>& g) {
     const double R0 = Tcw[0], R1 = Tcw[1], R2 = Tcw[2], R3 = Tcw[3], R4 = Tcw[4], R5 = Tcw[5];
     const double R6 = Tcw[6], R7 = Tcw[7], R8 = Tcw[8];
@@ -146,9 +149,9 @@ __device__ __forceinline__ void obs_term(const T* __restrict__ Tcw, const T* __r
     const T gy = gxd * dxdy + gyd * dydy;
     const T gc0 = gx * tiz, gc1 = gy * tiz, gc2 = -(gx * tx + gy * ty) * tiz;  // d C / d Xc
     // world point: R^T gc
-    g.gX[0] = Tcw[0] * gc0 + Tcw[3] * gc1 + Tcw[6] * gc2;
-    g.gX[1] = Tcw[1] * gc0 + Tcw[4] * gc1 + Tcw[7] * gc2;
-    g.gX[2] = Tcw[2] * gc0 + Tcw[5] * gc1 + Tcw[8] * gc2;
+    g.gX[0] = (T)R0 * gc0 + (T)R3 * gc1 + (T)R6 * gc2;
+    g.gX[1] = (T)R1 * gc0 + (T)R4 * gc1 + (T)R7 * gc2;
+    g.gX[2] = (T)R2 * gc0 + (T)R5 * gc1 + (T)R8 * gc2;
     // pose, left perturbation: d Xc / d omega = -[Xc]x, d Xc / d upsilon = I
     const T tc0 = (T)Xc0, tc1 = (T)Xc1, tc2 = (T)Xc2;
     g.gpose[0] = tc1 * gc2 - tc2 * gc1;
@@ -212,11 +215,11 @@ __device__ __forceinline__ int xcd_band(int b, int n) {
 // chunks in 4; before, 77 us, 60 in a gather of the pose terms and 59 in one
 // workgroup's sums over all tiles.  One scene of 700 points: 6 us and 2.4,
 // before 28 in all.
-template <typename T, bool kGrad>
-__global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const T* __restrict__ Tcw,
-                                                     const T* __restrict__ X, const T* __restrict__ intr,
-                                                     T* __restrict__ gX, double* __restrict__ part,
-                                                     double* __restrict__ gpart) {
+template <typename T, bool kGrad, typename TP>
+__global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP* __restrict__ Tcw,
+                                                        const T* __restrict__ X, const T* __restrict__ intr,
+                                                        T* __restrict__ gX, double* __restrict__ part,
+                                                        double* __restrict__ gpart) {
     constexpr int kSums = kGrad ? 9 : 1;
     __shared__ T sh[2][3][kTileObs];
     __shared__ double red[kThreads / kWave][kSums];
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const T* 
             }
             T gp[3] = {T(0), T(0), T(0)};
             for (int a = o0 + tid; a < o1; a += kThreads) {
-                const T* Tc = Tcw + 12 * (size_t)c;
+                const TP* Tc = Tcw + 12 * (size_t)c;
                 const T* Xq = X + 3 * (size_t)q;
                 const double u = uv.x, v = uv.y;
                 if (a + kThreads < o1) load(a + kThreads, o1);
@@ -306,7 +309,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const T* 
             if (b < P.n_chunks) {
                 b = xcd_band(b, P.n_chunks);
                 double acc[6] = {0, 0, 0, 0, 0, 0};
-                const T* Tc = Tcw + 12 * (size_t)P.chunk_cam[b];
+                const TP* Tc = Tcw + 12 * (size_t)P.chunk_cam[b];
                 const int k1 = P.chunk_ptr[b + 1];
                 int k = P.chunk_ptr[b] + tid, q = 0;
                 double2 uv;
@@ -419,16 +422,22 @@ __device__ __forceinline__ void rot3(const double w[3], double p, double q, cons
     for (int i = 0; i < 3; ++i) r[i] = v[i] + p * wv[i] + q * wwv[i];
 }
 
-// T = exp(xi) T_cw, one pose per thread.  Launch bound: a few hundred
-// operations and at most 144 bytes per pose.  As torch operations the map and
+// T = exp(xi) T_cw, one pose per thread; out64: the same before its rounding to
+// T, for the cost to be evaluated at (null where T is FP64: out serves).  Launch
+// bound: a few hundred operations and at most 240 bytes per pose.  As torch operations the map and
 // its derivative were about 230 launches of a gradient step; with these two
 // kernels a step of BACost (64 scenes of 5 000 points, 1 280 poses, float) went
 // from 1970 us to 260, on one scene of 700 (double) from 1800 to 168.
 template <typename T>
-__global__ void k_se3_left(int n, const T* __restrict__ xi, const T* __restrict__ Tcw, T* __restrict__ out) {
+__global__ void k_se3_left(int n, const T* __restrict__ xi, const T* __restrict__ Tcw, T* __restrict__ out,
+                           double* __restrict__ out64) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= n) return;
     double w[3], u[3], t[3], col[3], r[3], v[3];
+    auto put = [&](int e, double x) {
+        out[12 * (size_t)c + e] = (T)x;
+        if (out64) out64[12 * (size_t)c + e] = x;
+    };
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         w[i] = (double)xi[6 * (size_t)c + i];
@@ -442,12 +451,12 @@ __global__ void k_se3_left(int n, const T* __restrict__ xi, const T* __restrict_
         for (int i = 0; i < 3; ++i) col[i] = (double)Tcw[12 * (size_t)c + 3 * i + j];
         rot3(w, k.a, k.b, col, r);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) out[12 * (size_t)c + 3 * i + j] = (T)r[i];
+        for (int i = 0; i < 3; ++i) put(3 * i + j, r[i]);
     }
     rot3(w, k.a, k.b, t, r);
     rot3(w, k.b, k.c, u, v);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) out[12 * (size_t)c + 9 + i] = (T)(r[i] + v[i]);
+    for (int i = 0; i < 3; ++i) put(9 + i, r[i] + v[i]);
 }
 
 // g_xi = J_l(xi)^T g.  With p = V u, a step d of omega turns T by J d (J = V)
@@ -534,6 +543,7 @@ struct nav_ba_cost_handle {
     std::vector<void*> bufs;
     double* part = nullptr;   // [9][n_groups]
     double* gpart = nullptr;  // [n_chunks][6]
+    double* pose = nullptr;   // [n_cam][12] exp(xi) T_cw in FP64, where the caller's type is float
 };
 
 namespace {
@@ -541,7 +551,7 @@ namespace {
 void free_all(nav_ba_cost_handle* h) {
     for (void* p : h->bufs) (void)hipFree(p);
     h->bufs.clear();
-    h->part = h->gpart = nullptr;
+    h->part = h->gpart = h->pose = nullptr;
 }
 
 template <class V>
@@ -566,8 +576,8 @@ int32_t launch_status(nav_ba_cost_handle* h) {
     return NAV_BA_HIP_ERROR;
 }
 
-template <typename T>
-int32_t eval_t(nav_ba_cost_handle* h, const T* Tcw, const T* X, const T* intr, T* total, T* cost, T* gpose, T* gX,
+template <typename T, typename TP>
+int32_t eval_t(nav_ba_cost_handle* h, const TP* Tcw, const T* X, const T* intr, T* total, T* cost, T* gpose, T* gX,
                T* gintr, hipStream_t s) {
     const CostProblem& P = h->P;
     const bool grad = gpose || gX || gintr;
@@ -575,10 +585,10 @@ int32_t eval_t(nav_ba_cost_handle* h, const T* Tcw, const T* X, const T* intr, T
     const int blocks = P.n_groups + (gpose ? P.n_chunks : 0) + unseen;
     if (blocks > 0) {
         if (grad)  // a null gX or gpose skips its part
-            hipLaunchKernelGGL((k_cg_obs<T, true>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, gX, h->part,
+            hipLaunchKernelGGL((k_cg_obs<T, true, TP>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, gX, h->part,
                                gpose ? h->gpart : nullptr);
         else
-            hipLaunchKernelGGL((k_cg_obs<T, false>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, (T*)nullptr,
+            hipLaunchKernelGGL((k_cg_obs<T, false, TP>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, (T*)nullptr,
                                h->part, (double*)nullptr);
     }
     const int n_sums = gintr ? 9 : total ? 1 : 0;
@@ -588,15 +598,17 @@ int32_t eval_t(nav_ba_cost_handle* h, const T* Tcw, const T* X, const T* intr, T
     return launch_status(h);
 }
 
-// T = exp(xi) T_cw, then the evaluation there.
+// T = exp(xi) T_cw, then the evaluation there, at the poses before their rounding to T.
 template <typename T>
 int32_t eval_tangent_t(nav_ba_cost_handle* h, const T* xi, const T* Tcw, const T* X, const T* intr, T* Tout, T* total,
                        T* cost, T* gpose, T* gX, T* gintr, hipStream_t s) {
     const int n = h->P.n_cam;
+    double* pose = sizeof(T) < sizeof(double) ? h->pose : nullptr;
     if (n > 0)
         hipLaunchKernelGGL(k_se3_left<T>, dim3((n + kPoseThreads - 1) / kPoseThreads), dim3(kPoseThreads), 0, s, n, xi,
-                           Tcw, Tout);
-    return eval_t<T>(h, Tout, X, intr, total, cost, gpose, gX, gintr, s);
+                           Tcw, Tout, pose);
+    if (pose) return eval_t<T, double>(h, pose, X, intr, total, cost, gpose, gX, gintr, s);
+    return eval_t<T, T>(h, Tout, X, intr, total, cost, gpose, gX, gintr, s);
 }
 
 template <typename T>
@@ -795,14 +807,15 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
         (st = up(h, unseen, &P.unseen)))
         return st;
     void* part = nullptr;
-    const size_t n_part = 9 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks;
-    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_part + n_gpart, 1)) != hipSuccess) {
+    const size_t n_part = 9 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks, n_pose = 12 * (size_t)nc;
+    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_part + n_gpart + n_pose, 1)) != hipSuccess) {
         h->err = "hipMalloc part";
         return NAV_BA_HIP_ERROR;
     }
     h->bufs.push_back(part);
     h->part = (double*)part;
     h->gpart = h->part + n_part;
+    h->pose = h->gpart + n_gpart;
     h->prepared = true;
     return NAV_BA_OK;
 }
@@ -825,10 +838,10 @@ int32_t nav_ba_cost_eval(nav_ba_cost_handle* h, int32_t dtype, const void* T_cw,
     if (hipSetDevice(h->device) != hipSuccess) { h->err = "hipSetDevice"; return NAV_BA_HIP_ERROR; }
     hipStream_t s = (hipStream_t)stream;
     if (dtype == NAV_BA_COST_F64)
-        return eval_t<double>(h, (const double*)T_cw, (const double*)X, (const double*)intr, nullptr, (double*)cost,
+        return eval_t<double, double>(h, (const double*)T_cw, (const double*)X, (const double*)intr, nullptr, (double*)cost,
                               (double*)g_pose, (double*)g_X, (double*)g_intr, s);
     if (dtype == NAV_BA_COST_F32)
-        return eval_t<float>(h, (const float*)T_cw, (const float*)X, (const float*)intr, nullptr, (float*)cost,
+        return eval_t<float, float>(h, (const float*)T_cw, (const float*)X, (const float*)intr, nullptr, (float*)cost,
                              (float*)g_pose, (float*)g_X, (float*)g_intr, s);
     h->err = "unknown dtype";
     return NAV_BA_BAD_ARG;

@@ -1,0 +1,87 @@
+"""BACost's value and gradients against FP64 from the tangents: the poses
+exp(xi) T_cw are formed in double from the inputs, whatever type these have."""
+import numpy as np
+import pytest
+
+from nav24_amd import problems
+from oracle import cost_oracle as co
+from parity_util import say
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def scenes(seed, dtype):
+    """One or two scenes, and xi, X, intrinsics and poses as values of `dtype` (FP64 tensors)."""
+    probs = []
+    for k in range(1 + seed % 2):
+        g = problems.params_for(4, 7 * seed + k)
+        g.n_pt, g.n_cam = 60 + 37 * (seed % 7), 3 + seed % 6
+        probs.append(problems.make(g))
+    q = probs[0]
+    T = np.concatenate([p.T_cw for p in probs])
+    xi = np.random.default_rng(seed).normal(0.0, 0.01, (len(T), 6))
+    intr = np.array([q.fx, q.fy, q.cx, q.cy, *q.dist])
+    return probs, [torch.tensor(a).to(dtype).double() for a in (xi, np.concatenate([p.X for p in probs]), intr, T)]
+
+
+def reference(probs, xi, X, intr, T_cw):
+    """Total cost and the gradients to xi, X and the intrinsics, in FP64 on the CPU."""
+    from nav24_amd.diffcost import se3_left, tangent_to_entry_grad
+    x = xi.clone().requires_grad_(True)
+    T = se3_left(x, T_cw)
+    cost, gp, gx, gi, c0, p0 = 0.0, [], [], np.zeros(8), 0, 0
+    for p in probs:
+        r = co.cost_and_grad(T.detach().numpy()[c0:c0 + p.n_cam], X.numpy()[p0:p0 + p.n_pt], p.obs_cam, p.obs_pt,
+                             p.obs_uv, intr.numpy(), True)
+        cost, gi = cost + r[0], gi + r[3]
+        gp.append(r[1])
+        gx.append(r[2])
+        c0, p0 = c0 + p.n_cam, p0 + p.n_pt
+    (g_xi,) = torch.autograd.grad(T, x, tangent_to_entry_grad(torch.tensor(np.concatenate(gp)), T.detach()))
+    return cost, g_xi.numpy(), np.concatenate(gx), gi
+
+
+def test_fp32_gradients_match_fp64_from_the_tangents():
+    """48 batches of small scenes.  The adjoint's terms take some twenty float
+    operations in a row, 2^-24 each at most and independent over the entries:
+    about 2e-7 of a gradient's norm, so 1e-6.  Poses rounded to float before the
+    cost is formed are off by up to half a micrometre, which near a camera's plane
+    is 1e-5 of the point gradients."""
+    from nav24_amd.diffcost import BACost, CostBatch
+    worst = np.zeros(4)
+    for seed in range(48):
+        probs, inputs = scenes(seed, torch.float32)
+        want = reference(probs, *inputs)
+        leaves = [t.float().cuda().requires_grad_(True) for t in inputs[:3]]
+        b = CostBatch(probs)
+        cost = BACost.apply(*leaves, inputs[3].float().cuda(), b)
+        got = [cost.detach(), *torch.autograd.grad(cost, leaves)]
+        worst = np.maximum(worst, [np.linalg.norm(g.double().cpu().numpy() - w) / np.linalg.norm(w)
+                                   for g, w in zip(got, want)])
+        with torch.no_grad():  # the value alone: the same poses, the same bits
+            assert torch.equal(BACost.apply(*leaves, inputs[3].float().cuda(), b), got[0])
+        b.close()
+    say("fp32 cost, xi, X, intrinsics: " + " ".join(f"{v:.1e}" for v in worst))
+    assert (worst <= 1e-6).all()
+
+
+@pytest.mark.parametrize("n_cam", [2, 65])
+def test_float_poses_are_rounded_once(n_cam):
+    """Each entry of the returned float poses is the FP64 one to half a unit in its
+    last place (2^-24 of it), and the FP64 value to a few dozen operations."""
+    from nav24_amd.diffcost import CostBatch, se3_left
+    g = problems.params_for(4, 3)
+    g.n_pt, g.n_cam = 60, n_cam
+    p = problems.make(g)
+    xi = (0.3 * torch.randn(n_cam, 6, generator=torch.Generator().manual_seed(n_cam))).float()
+    intr = torch.tensor([p.fx, p.fy, p.cx, p.cy, *p.dist])
+    args = [a.float().cuda() for a in (xi, torch.tensor(p.X), intr, torch.tensor(p.T_cw))]
+    b = CostBatch([p])
+    T = b._eval_tangent(*args, False)[1].double().cpu()
+    b.close()
+    ref = se3_left(xi.double(), torch.tensor(p.T_cw).float().double())
+    for part in (slice(0, 9), slice(9, 12)):
+        t, r = T[:, part], ref[:, part]
+        assert ((t - r).abs() <= 2.0 ** -24 * r.abs() + 1e-13 * r.abs().max()).all()
