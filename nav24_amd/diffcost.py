@@ -135,7 +135,8 @@ class CostBatch:
         `_poses_on_device` accepts, on torch's current stream."""
         import torch
         dt, dev = xi.dtype, xi.device
-        xi, X, intr, T_cw = (t.contiguous() for t in (xi, X, intr, T_cw))
+        # (memory of a lazily negated tensor holds the values before the sign)
+        xi, X, intr, T_cw = (t.resolve_neg().contiguous() for t in (xi, X, intr, T_cw))
         T = torch.empty_like(T_cw)
         total = torch.empty((), dtype=dt, device=dev)
         cost = torch.empty(self.n_problems, dtype=dt, device=dev)
@@ -166,7 +167,7 @@ def _tangent_grad(xi, g_pose):
     """J_l(xi)^T g_pose in one kernel, for xi and g_pose as `_eval_tangent` took
     and returned them."""
     import torch
-    xi = xi.contiguous()
+    xi, g_pose = xi.resolve_neg().contiguous(), g_pose.resolve_neg().contiguous()
     out = torch.empty_like(g_pose)
     st = lib().nav_ba_cost_tangent_grad(
         xi.device.index, NAV_BA_COST_F64 if xi.dtype == torch.float64 else NAV_BA_COST_F32, xi.shape[0], xi.data_ptr(),
@@ -193,11 +194,12 @@ def _scaled_gradients(g, xi, gp, gx, gi, need):
 def _one_kernel(g, *saved) -> bool:
     """Whether the gradients can be formed in one kernel: no graph of the backward
     is asked for, and the incoming gradient and the saved tensors (a hook may have
-    moved or converted them) are plain device tensors of one type and device."""
+    moved or converted them) are plain device tensors of one type and device, with
+    their values in memory (no lazy negation)."""
     import torch
     dt, dev = g.dtype, g.device
     if (torch.is_grad_enabled() or not g.is_cuda or g.dim() != 0 or dt not in (torch.float64, torch.float32)
-            or any(type(t) is not torch.Tensor or t.dtype != dt or t.device != dev or not t.is_contiguous()
+            or any(type(t) is not torch.Tensor or t.dtype != dt or t.device != dev or not t.is_contiguous() or t.is_neg()
                    for t in (g, *saved))):
         return False
     try:
@@ -287,7 +289,7 @@ try:
                 # d cost / d xi = J_l(xi)^T gp, gp the left-tangent gradient at T
                 # (a saved-tensor hook may have moved or converted them)
                 if ctx.kernels and xi.is_cuda and (gp.device, gp.dtype) == (xi.device, xi.dtype):
-                    g_xi = _tangent_grad(xi, gp.contiguous())
+                    g_xi = _tangent_grad(xi, gp)
                 else:
                     # (d T / d xi)^T G_T, G_T the entry gradient of gp at T
                     with torch.enable_grad():
