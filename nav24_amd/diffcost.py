@@ -150,14 +150,18 @@ class CostBatch:
         return total, T, CostResult(cost, gp, gx, gi)
 
 
+_EVAL = CostBatch.eval
+
+
 def _poses_on_device(batch, xi, X, intr, T_cw) -> bool:
     """Whether the pose map and its adjoint can run in the device kernels: one
     type and one device for all four tensors, and the batch's shapes.  Anything
-    else (mixed types, broadcast poses, another evaluator) goes through
+    else (mixed types, broadcast poses, another evaluator: a class of its own, or
+    an `eval` put in place of this one on the class or the batch) goes through
     `se3_left` and the batch's `eval`."""
     import torch
     dt, dev = xi.dtype, xi.device
-    return (getattr(type(batch), "eval", None) is CostBatch.eval and dt in (torch.float64, torch.float32) and xi.is_cuda
+    return (getattr(batch.eval, "__func__", None) is _EVAL and dt in (torch.float64, torch.float32) and xi.is_cuda
             and all(t.dtype == dt and t.device == dev for t in (X, intr, T_cw))
             and tuple(xi.shape) == (batch.n_cam, 6) and tuple(T_cw.shape) == (batch.n_cam, 12)
             and tuple(X.shape) == (batch.n_pt, 3) and tuple(intr.shape) == (8,))

@@ -117,3 +117,28 @@ def test_lazily_negated_tensors(dtype):
                 assert all(torch.equal(a, w) for a, w in zip(step(inputs, g, **kw), want))
     assert torch.equal(_tangent_grad(lazy[0], lazy[0]), _tangent_grad(t[0], t[0]))
     b.close()
+
+
+@pytest.mark.parametrize("where", ["batch", "class", "subclass"])
+def test_another_evaluator_is_called(where, monkeypatch):
+    """BACost evaluates through the batch's `eval`, whoever provides it."""
+    from nav24_amd import diffcost
+    b, t = small()
+    calls, plain = [], diffcost.CostBatch.eval
+
+    def watched(self, *a, **kw):
+        calls.append(1)
+        return plain(self, *a, **kw)
+
+    want = diffcost.BACost.apply(*t, b)
+    assert not calls
+    if where == "batch":
+        b.eval = watched.__get__(b)
+    elif where == "class":
+        monkeypatch.setattr(diffcost.CostBatch, "eval", watched)
+    else:
+        b.__class__ = type("Watched", (diffcost.CostBatch,), dict(eval=watched))
+    got = diffcost.BACost.apply(*t, b)
+    assert len(calls) == 1
+    assert abs(got.item() - want.item()) <= 1e-12 * want.item()
+    b.close()
