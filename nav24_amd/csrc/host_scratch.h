@@ -83,14 +83,22 @@ inline char* host_stage_get(HostScratch& s, size_t bytes) {
 // one copy brings the inputs in and one the outputs back.
 //   HostCall c;  auto a = c.in(src, bytes);  auto t = c.tmp(bytes);  auto r = c.out(dst, bytes);
 //   if (!c.begin(hs)) ...;  launch with c.ptr<T>(a), ...;  if (!c.finish()) ...
-// in, then tmp, then out; the caller holds the scratch's mutex.
+// in, then tmp, then out; the caller holds the scratch's mutex.  begin fails for
+// a null array of some bytes, as a copy from or to it would.
 class HostCall {
 public:
-    int in(const void* src, size_t bytes) { return add(src, nullptr, bytes, &in_end_); }
+    int in(const void* src, size_t bytes) {
+        null_ = null_ || (!src && bytes > 0);
+        return add(src, nullptr, bytes, &in_end_);
+    }
     int tmp(size_t bytes) { return add(nullptr, nullptr, bytes, &out_beg_); }
-    int out(void* dst, size_t bytes) { return add(nullptr, dst, bytes, nullptr); }
+    int out(void* dst, size_t bytes) {
+        null_ = null_ || (!dst && bytes > 0);
+        return add(nullptr, dst, bytes, nullptr);
+    }
 
     bool begin(HostScratch& hs) {
+        if (null_) return false;
         if (out_beg_ < in_end_) out_beg_ = in_end_;
         d_ = (char*)host_scratch_get(hs, total_);
         if (!d_) return false;
@@ -147,6 +155,7 @@ private:
     }
     Array a_[kMaxArrays];
     int n_ = 0;
+    bool null_ = false;
     size_t total_ = 0, in_end_ = 0, out_beg_ = 0;
     char* d_ = nullptr;
     char* pin_ = nullptr;

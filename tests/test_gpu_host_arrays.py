@@ -75,3 +75,27 @@ def test_calls_from_several_threads(scene):
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_null_key_points_are_refused():
+    """A count of key points without the array is an error, also where no match
+    reads them (n = 0), and 0 key points need none."""
+    import ctypes as C
+    from nav24_amd import twoview
+    L = twoview.lib()
+    kp, best, score = (C.c_float * 4)(), C.c_int32(), C.c_float()
+    K = (C.c_float * 9)(1, 0, 0, 0, 1, 0, 0, 0, 1)
+    t = (C.c_float * 3)()
+    ng, par, cs, p3, gd = C.c_int32(), C.c_float(), C.c_float(), (C.c_float * 6)(), (C.c_uint8 * 2)()
+
+    def scored(k1, n1):
+        return L.nav_tv_score_homography_host(k1, n1, kp, 2, None, 0, None, None, 0, 1.0, 5.991, None, C.byref(best),
+                                              C.byref(score), None, 0)
+
+    def checked(k1, n1):
+        return L.nav_tv_check_rt_host(k1, n1, kp, 2, None, None, 0, K, K, t, 1, 4.0, 0.99998, 50, C.byref(ng),
+                                      C.byref(par), C.byref(cs), p3, gd, 0)
+
+    for f in (scored, checked):
+        assert f(kp, 2) == 0 and f(None, 0) == 0
+        assert f(None, 2) != 0
