@@ -7,13 +7,15 @@
 // camera-major, in chunks of one camera's observations.  Each evaluation runs
 //   k_cg_obs    one workgroup per group: cost terms and their adjoint, a lane
 //               per observation of a tile; the point gradient is summed per
-//               point from LDS in fixed order, cost and intrinsic gradients per
-//               group; in the same launch one workgroup per camera chunk: its
-//               pose gradient, from the terms formed again in camera-major
-//               order; and zeros for the points without observations;
-//   k_cg_final  per-problem costs, the total and the intrinsic gradient over the
-//               groups, the pose gradients over the chunks (fixed order).
-// The forward (cost only) runs the groups without the adjoint.
+//               point from LDS in fixed order, the cost per tile, the intrinsic
+//               gradients per group; in the same launch one workgroup per camera
+//               chunk: its pose gradient, from the terms formed again in
+//               camera-major order; and zeros for the points without observations;
+//   k_cg_final  per-problem costs and the total over the tiles, the intrinsic
+//               gradient over the groups, the pose gradients over the chunks
+//               (fixed order).
+// The forward (cost only) is k_cg_cost, one workgroup per tile: the same sums per
+// tile, so the same costs.
 // T = double or float: the projection and residual are FP64 either way, the
 // adjoint runs in T; partial and final sums are FP64.
 // Forming an observation's terms twice costs less than one pass that writes six
@@ -38,11 +40,10 @@ using navba::wave_sum;
 constexpr int kTileObs = 256;  // observations per tile (whole points; one larger point has a tile of its own)
 constexpr int kThreads = 256;
 // Sums over the workgroup come once per group or chunk, so these are long where
-// there are many observations.  Groups are as short as keeps them to kGroups (eight
-// workgroups per CU, resident together for the cost alone), up to kGroupTiles tiles:
-// one round of workgroups and a little more is the worst case (gradients of 0.8, 1.0
-// and 3.2 M observations: 26.7, 31.0 and 63 us; with at least kGroups of them, 31.8,
-// 37.4 and 64; with twice as many, 31.8, 37.1 and 66.5).  Chunks are as long as
+// there are many observations.  Groups are as short as keeps them to kGroups, up to
+// kGroupTiles tiles (gradients of 0.8, 1.0 and 3.2 M observations: 26.7, 31.0 and
+// 63 us; with at least kGroups of them, 31.8, 37.4 and 64; with twice as many, 31.8,
+// 37.1 and 66.5).  Chunks are as long as
 // leaves kChunks of them, up to kChunkMax observations.
 constexpr int kXcds = 8;
 constexpr int kGroups = 2048;
@@ -52,7 +53,7 @@ constexpr int kChunkMax = 4096;
 constexpr int kPoseThreads = 64;  // one pose per thread: a wave per workgroup spreads few poses over the CUs
 
 struct CostProblem {
-    int n_obs, n_groups, n_chunks, n_unseen, n_cam, n_pt, n_prob;
+    int n_obs, n_tiles, n_groups, n_chunks, n_unseen, n_cam, n_pt, n_prob;
     int robust;
     double delta;
     const int* o_cam;      // point-major, caller (global) camera index
@@ -63,7 +64,7 @@ struct CostProblem {
     const int* tile_obs;   // [n_tiles + 1]
     const int* tile_pt;    // [n_tiles + 1] range in pt_list
     const int* group_tile; // [n_groups + 1]
-    const int* prob_group0; // [n_prob + 1]
+    const int* prob_tile0; // [n_prob + 1]
     const int* c_pt;       // camera-major, caller (global) point index
     const double2* c_uv;   // camera-major
     const int* chunk_cam;  // [n_chunks]
@@ -178,18 +179,23 @@ __device__ __forceinline__ double sum_quarters(double v) {
            __longlong_as_double(((long long)h2[1] << 32) | l2[1]);
 }
 
-// Sums of N values per lane over the workgroup, in a fixed order: value q in
-// thread q < N.  A wave's 64 lanes are added by a matrix instruction with a
-// second operand of ones (16 row sums of four lanes each, four to a lane), then
-// within lanes and over the lanes' quarters: half the instructions of a sum by
+// Sum of a value per lane over the wave, in every lane: a matrix instruction with
+// a second operand of ones (16 row sums of four lanes each, four to a lane), then
+// within lanes and over the lanes' quarters, half the instructions of a sum by
 // lane moves.
+__device__ __forceinline__ double wave_total(double v) {
+    const dbl4 r = __builtin_amdgcn_mfma_f64_16x16x4f64(v, 1.0, dbl4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+    return sum_quarters((r[0] + r[1]) + (r[2] + r[3]));
+}
+
+// Sums of N values per lane over the workgroup, in a fixed order: value q in
+// thread q < N.
 template <int N>
 __device__ __forceinline__ double block_sums(const double v[N], double (*red)[N]) {
     const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
 #pragma unroll
     for (int q = 0; q < N; ++q) {
-        const dbl4 r = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q], 1.0, dbl4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
-        const double s = sum_quarters((r[0] + r[1]) + (r[2] + r[3]));
+        const double s = wave_total(v[q]);
         if (lane == 0) red[wid][q] = s;
     }
     __syncthreads();
@@ -206,23 +212,57 @@ __device__ __forceinline__ int xcd_band(int b, int n) {
     return x * lo + min(x, more) + b / kXcds;
 }
 
-// Workgroups 0 .. n_groups - 1: part[q n_groups + group] = {cost, d / d intrinsics
-// (8)}[q] (FP64); with kGrad the next n_chunks (if gpart): gpart[6 chunk + j]; then those that
-// clear the unseen points' gradients.  Bound by the FP64 operations of the terms
-// and by memory together: 24 bytes per observation in one order and 20 in the
-// other.  64 scenes of 5 000 points (3.16 M observations, float): 67 us for a
-// gradient and 20 for the cost alone (3.8 TB/s), with the sums over groups and
-// chunks in 4; before, 77 us, 60 in a gather of the pose terms and 59 in one
-// workgroup's sums over all tiles.  One scene of 700 points: 6 us and 2.4,
-// before 28 in all.
-template <typename T, bool kGrad, typename TP>
+// A tile's cost from its lanes' in LDS, by one wave; both kernels form it so.
+__device__ __forceinline__ double tile_total(const double c[kThreads]) {
+    static_assert(kThreads == 4 * kWave, "four values a lane");
+    const int l = threadIdx.x % kWave;
+    return wave_total((c[l] + c[l + kWave]) + (c[l + 2 * kWave] + c[l + 3 * kWave]));
+}
+
+// The cost alone: one workgroup per tile, its cost to tile_cost; eight workgroups
+// per CU.  Bound by memory and the FP64 operations of the terms.  64 scenes of
+// 5 000 points (3.16 M observations), with the final sums: 25.2 us in FP64 and 21.3
+// in FP32; one workgroup per group of tiles 28.5 and 25.2, and without the bound on
+// registers 25.4 and 23.8.
+template <typename T, typename TP>
+__global__ __launch_bounds__(kThreads, 8) void k_cg_cost(CostProblem P, const TP* __restrict__ Tcw,
+                                                      const T* __restrict__ X, const T* __restrict__ intr,
+                                                      double* __restrict__ tile_cost) {
+    __shared__ double lane_cost[kThreads];
+    const int tid = threadIdx.x, t = xcd_band(blockIdx.x, P.n_tiles);
+    T in[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) in[k] = intr[k];
+    const int o1 = P.tile_obs[t + 1];
+    double cost = 0.0;
+    for (int a = P.tile_obs[t] + tid; a < o1; a += kThreads) {
+        const double2 uv = P.uv[a];
+        ObsGrad<T> g;
+        obs_term<T, kCost>(Tcw + 12 * (size_t)P.o_cam[a], X + 3 * (size_t)P.o_pt[a], in, uv.x, uv.y, P.robust, P.delta, g);
+        cost += g.cost;
+    }
+    lane_cost[tid] = cost;
+    __syncthreads();
+    if (tid >= kWave) return;
+    const double s = tile_total(lane_cost);
+    if (tid == 0) tile_cost[t] = s;
+}
+
+// Workgroups 0 .. n_groups - 1: the tiles' costs to tile_cost, part[q n_groups +
+// group] = d / d intrinsics[q] (FP64); the next n_chunks (if gpart): gpart[6 chunk
+// + j]; then those that clear the unseen points' gradients.  Bound by the FP64
+// operations of the terms and by memory together: 24 bytes per observation in one
+// order and 20 in the other.  64 scenes of 5 000 points, with the final sums: 67 us
+// in FP64 and 63 in FP32, before 220 and 191 (a gather of six stored pose terms per
+// observation, and one workgroup's sums over all tiles).
+template <typename T, typename TP>
 __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP* __restrict__ Tcw,
                                                         const T* __restrict__ X, const T* __restrict__ intr,
-                                                        T* __restrict__ gX, double* __restrict__ part,
-                                                        double* __restrict__ gpart) {
-    constexpr int kSums = kGrad ? 9 : 1;
+                                                        T* __restrict__ gX, double* __restrict__ tile_cost,
+                                                        double* __restrict__ part, double* __restrict__ gpart) {
     __shared__ T sh[2][3][kTileObs];
-    __shared__ double red[kThreads / kWave][kSums];
+    __shared__ double lane_cost[kGroupTiles][kThreads];
+    __shared__ double red[kThreads / kWave][8];
     __shared__ double redc[kThreads / kWave][6];
     const int tid = threadIdx.x;
     T in[8];
@@ -231,9 +271,9 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP*
     int b = blockIdx.x;
     if (b < P.n_groups) {
         b = xcd_band(b, P.n_groups);
-        double acc[kSums];
+        double acc[8];
 #pragma unroll
-        for (int k = 0; k < kSums; ++k) acc[k] = 0.0;
+        for (int k = 0; k < 8; ++k) acc[k] = 0.0;
         const int t0 = P.group_tile[b], t1 = P.group_tile[b + 1];
         int o0 = P.tile_obs[t0], c = 0, q = 0;
         double2 uv;
@@ -256,11 +296,12 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP*
                 a0 = P.pt_ptr[p];
                 a1 = P.pt_ptr[p + 1];
             };
-            if (kGrad && gX) {
+            if (gX) {
                 q0 = P.tile_pt[t];
                 n_sum = 3 * (P.tile_pt[t + 1] - q0);
                 if (tid < n_sum) point(q0 + tid / 3);
             }
+            double cost = 0.0;
             T gp[3] = {T(0), T(0), T(0)};
             for (int a = o0 + tid; a < o1; a += kThreads) {
                 const TP* Tc = Tcw + 12 * (size_t)c;
@@ -268,104 +309,119 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP*
                 const double u = uv.x, v = uv.y;
                 if (a + kThreads < o1) load(a + kThreads, o1);
                 ObsGrad<T> g;
-                obs_term<T, kGrad ? kPointSide : kCost>(Tc, Xq, in, u, v, P.robust, P.delta, g);
-                acc[0] += g.cost;
-                if constexpr (kGrad) {
+                obs_term<T, kPointSide>(Tc, Xq, in, u, v, P.robust, P.delta, g);
+                cost += g.cost;
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) acc[1 + k] += (double)g.gintr[k];
-                    gp[0] += g.gX[0]; gp[1] += g.gX[1]; gp[2] += g.gX[2];
-                }
+                for (int k = 0; k < 8; ++k) acc[k] += (double)g.gintr[k];
+                gp[0] += g.gX[0]; gp[1] += g.gX[1]; gp[2] += g.gX[2];
             }
             if (t + 1 < t1) load(o1 + tid, P.tile_obs[t + 2]);
-            if (kGrad && gX) {  // uniform: gX is a kernel argument
-                T (*st)[kTileObs] = sh[(t - t0) & 1];  // written again two tiles, hence a barrier, later
+            lane_cost[t - t0][tid] = cost;
+            T (*st)[kTileObs] = sh[(t - t0) & 1];  // written again two tiles, hence a barrier, later
+            if (gX) {  // uniform: gX is a kernel argument
 #pragma unroll
                 for (int k = 0; k < 3; ++k) st[k][tid] = gp[k];
                 __syncthreads();
-                // per-point sums in fixed order, a thread per point and component
-                for (int i = tid; i < n_sum; i += kThreads) {
-                    if (i != tid) point(q0 + i / 3);
-                    const T* v = st[i % 3];
-                    int a = one ? 0 : a0 - o0;
-                    const int e = one ? kThreads : a1 - o0;
-                    T s = T(0);
-                    for (; a + 4 <= e; a += 4) {
-                        const T v0 = v[a], v1 = v[a + 1], v2 = v[a + 2], v3 = v[a + 3];
-                        s = (((s + v0) + v1) + v2) + v3;
-                    }
-                    for (; a < e; ++a) s += v[a];
-                    gX[3 * (size_t)pt + i % 3] = s;
+            }
+            // per-point sums in fixed order, a thread per point and component
+            for (int i = tid; i < n_sum; i += kThreads) {
+                if (i != tid) point(q0 + i / 3);
+                const T* v = st[i % 3];
+                int a = one ? 0 : a0 - o0;
+                const int e = one ? kThreads : a1 - o0;
+                T s = T(0);
+                for (; a + 4 <= e; a += 4) {
+                    const T v0 = v[a], v1 = v[a + 1], v2 = v[a + 2], v3 = v[a + 3];
+                    s = (((s + v0) + v1) + v2) + v3;
                 }
+                for (; a < e; ++a) s += v[a];
+                gX[3 * (size_t)pt + i % 3] = s;
             }
             o0 = o1;
         }
-        const double s = block_sums<kSums>(acc, red);
-        if (tid < kSums) part[(size_t)tid * P.n_groups + b] = s;
+        if (!gX) __syncthreads();
+        // after the last tile: a sum per tile within the loop cost 4 % of a gradient
+        for (int t = t0 + tid / kWave; t < t1; t += kThreads / kWave) {
+            const double s = tile_total(lane_cost[t - t0]);
+            if (tid % kWave == 0) tile_cost[t] = s;
+        }
+        const double s = block_sums<8>(acc, red);
+        if (tid < 8) part[(size_t)tid * P.n_groups + b] = s;
         return;
     }
-    if constexpr (kGrad) {
-        b -= P.n_groups;
-        if (gpart) {
-            if (b < P.n_chunks) {
-                b = xcd_band(b, P.n_chunks);
-                double acc[6] = {0, 0, 0, 0, 0, 0};
-                const TP* Tc = Tcw + 12 * (size_t)P.chunk_cam[b];
-                const int k1 = P.chunk_ptr[b + 1];
-                int k = P.chunk_ptr[b] + tid, q = 0;
-                double2 uv;
-                if (k < k1) {
-                    q = P.c_pt[k];
-                    uv = P.c_uv[k];
-                }
-                for (; k < k1; k += kThreads) {
-                    const T* Xq = X + 3 * (size_t)q;
-                    const double u = uv.x, v = uv.y;
-                    if (k + kThreads < k1) {
-                        q = P.c_pt[k + kThreads];
-                        uv = P.c_uv[k + kThreads];
-                    }
-                    ObsGrad<T> g;
-                    obs_term<T, kPoseSide>(Tc, Xq, in, u, v, P.robust, P.delta, g);
-#pragma unroll
-                    for (int j = 0; j < 6; ++j) acc[j] += (double)g.gpose[j];
-                }
-                const double s = block_sums<6>(acc, redc);
-                if (tid < 6) gpart[6 * (size_t)b + tid] = s;
-                return;
+    b -= P.n_groups;
+    if (gpart) {
+        if (b < P.n_chunks) {
+            b = xcd_band(b, P.n_chunks);
+            double acc[6] = {0, 0, 0, 0, 0, 0};
+            const TP* Tc = Tcw + 12 * (size_t)P.chunk_cam[b];
+            const int k1 = P.chunk_ptr[b + 1];
+            int k = P.chunk_ptr[b] + tid, q = 0;
+            double2 uv;
+            if (k < k1) {
+                q = P.c_pt[k];
+                uv = P.c_uv[k];
             }
-            b -= P.n_chunks;
-        }
-        const int i = b * kThreads + tid;
-        if (gX && i < P.n_unseen)
+            for (; k < k1; k += kThreads) {
+                const T* Xq = X + 3 * (size_t)q;
+                const double u = uv.x, v = uv.y;
+                if (k + kThreads < k1) {
+                    q = P.c_pt[k + kThreads];
+                    uv = P.c_uv[k + kThreads];
+                }
+                ObsGrad<T> g;
+                obs_term<T, kPoseSide>(Tc, Xq, in, u, v, P.robust, P.delta, g);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) gX[3 * (size_t)P.unseen[i] + k] = T(0);
+                for (int j = 0; j < 6; ++j) acc[j] += (double)g.gpose[j];
+            }
+            const double s = block_sums<6>(acc, redc);
+            if (tid < 6) gpart[6 * (size_t)b + tid] = s;
+            return;
+        }
+        b -= P.n_chunks;
     }
+    const int i = b * kThreads + tid;
+    if (gX && i < P.n_unseen)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gX[3 * (size_t)P.unseen[i] + k] = T(0);
 }
 
-// Workgroup p < n_prob: cost of problem p over its groups; the next n_sums: the
-// total (sum 0) and the intrinsic gradient (1..8) over all groups; the others:
-// pose gradients over the cameras' chunks, a thread per entry (all in a fixed order).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_cg_final(CostProblem P, const double* __restrict__ part, int n_sums,
-                                                       T* __restrict__ cost, T* __restrict__ total,
-                                                       T* __restrict__ gintr, const double* __restrict__ gpart,
-                                                       T* __restrict__ gpose) {
-    __shared__ double red[kThreads / kWave];
-    const int pr = blockIdx.x;
-    if (pr < P.n_prob + n_sums) {
-        const int q = pr < P.n_prob ? 0 : pr - P.n_prob;
-        const int g0 = pr < P.n_prob ? P.prob_group0[pr] : 0, g1 = pr < P.n_prob ? P.prob_group0[pr + 1] : P.n_groups;
-        double s = 0.0;
-        for (int g = g0 + (int)threadIdx.x; g < g1; g += kThreads) s += part[(size_t)q * P.n_groups + g];
-        const double v = block_sum<double, kThreads>(s, red);
-        if (threadIdx.x == 0) {
-            if (pr < P.n_prob) cost[pr] = (T)v;
-            else if (q > 0 && gintr) gintr[q - 1] = (T)v;
-            else if (q == 0 && total) *total = (T)v;
-        }
-        return;
+// This thread's share of a sum over v[i0 .. i1), sixteen loads in flight: the
+// partial sums come from other XCDs, a microsecond away.
+__device__ __forceinline__ double strided_sum(const double* __restrict__ v, int i0, int i1) {
+    constexpr int kLoads = 16;
+    double s = 0.0;
+    for (int i = i0 + (int)threadIdx.x; i < i1; i += kLoads * kThreads) {
+        double x[kLoads];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) x[k] = v[min(i + k * kThreads, i1 - 1)];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) s += i + k * kThreads < i1 ? x[k] : 0.0;
     }
-    const int i = (pr - P.n_prob - n_sums) * kThreads + (int)threadIdx.x;
+    return s;
+}
+
+// Workgroup p < n_prob: cost of problem p over its tiles; then one for the total
+// over all tiles (if asked for), eight for the intrinsic gradient over the groups
+// (likewise); the others: pose gradients over the cameras' chunks, a thread per
+// entry (all in a fixed order).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_cg_final(CostProblem P, const double* __restrict__ tile_cost,
+                                                       const double* __restrict__ part, T* __restrict__ cost,
+                                                       T* __restrict__ total, T* __restrict__ gintr,
+                                                       const double* __restrict__ gpart, T* __restrict__ gpose) {
+    __shared__ double red[kThreads / kWave];
+    int b = blockIdx.x;
+    auto sum = [&](const double* v, int i0, int i1, T* out) {
+        const double s = block_sum<double, kThreads>(strided_sum(v, i0, i1), red);
+        if (threadIdx.x == 0) *out = (T)s;
+    };
+    if (b < P.n_prob) return sum(tile_cost, P.prob_tile0[b], P.prob_tile0[b + 1], cost + b);
+    b -= P.n_prob;
+    if (total && b-- == 0) return sum(tile_cost, 0, P.n_tiles, total);
+    if (gintr && b < 8) return sum(part + (size_t)b * P.n_groups, 0, P.n_groups, gintr + b);
+    if (gintr) b -= 8;
+    const int i = b * kThreads + (int)threadIdx.x;
     if (i >= 6 * P.n_cam) return;
     const int c = i / 6, j = i % 6;
     double s = 0.0;
@@ -541,7 +597,8 @@ struct nav_ba_cost_handle {
     bool prepared = false;
     CostProblem P{};
     std::vector<void*> bufs;
-    double* part = nullptr;   // [9][n_groups]
+    double* tile_cost = nullptr;  // [n_tiles]
+    double* part = nullptr;   // [8][n_groups]
     double* gpart = nullptr;  // [n_chunks][6]
     double* pose = nullptr;   // [n_cam][12] exp(xi) T_cw in FP64, where the caller's type is float
 };
@@ -551,7 +608,7 @@ namespace {
 void free_all(nav_ba_cost_handle* h) {
     for (void* p : h->bufs) (void)hipFree(p);
     h->bufs.clear();
-    h->part = h->gpart = h->pose = nullptr;
+    h->tile_cost = h->part = h->gpart = h->pose = nullptr;
 }
 
 template <class V>
@@ -583,18 +640,14 @@ int32_t eval_t(nav_ba_cost_handle* h, const TP* Tcw, const T* X, const T* intr, 
     const bool grad = gpose || gX || gintr;
     const int unseen = gX ? (P.n_unseen + kThreads - 1) / kThreads : 0;
     const int blocks = P.n_groups + (gpose ? P.n_chunks : 0) + unseen;
-    if (blocks > 0) {
-        if (grad)  // a null gX or gpose skips its part
-            hipLaunchKernelGGL((k_cg_obs<T, true, TP>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, gX, h->part,
-                               gpose ? h->gpart : nullptr);
-        else
-            hipLaunchKernelGGL((k_cg_obs<T, false, TP>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, (T*)nullptr,
-                               h->part, (double*)nullptr);
-    }
-    const int n_sums = gintr ? 9 : total ? 1 : 0;
-    const int cam_blocks = gpose ? (6 * P.n_cam + kThreads - 1) / kThreads : 0;
-    hipLaunchKernelGGL(k_cg_final<T>, dim3(P.n_prob + n_sums + cam_blocks), dim3(kThreads), 0, s, P,
-                       (const double*)h->part, n_sums, cost, total, gintr, (const double*)h->gpart, gpose);
+    if (grad && blocks > 0)  // a null gX or gpose skips its part
+        hipLaunchKernelGGL((k_cg_obs<T, TP>), dim3(blocks), dim3(kThreads), 0, s, P, Tcw, X, intr, gX, h->tile_cost,
+                           h->part, gpose ? h->gpart : nullptr);
+    if (!grad && P.n_tiles > 0)
+        hipLaunchKernelGGL((k_cg_cost<T, TP>), dim3(P.n_tiles), dim3(kThreads), 0, s, P, Tcw, X, intr, h->tile_cost);
+    const int finals = P.n_prob + (total ? 1 : 0) + (gintr ? 8 : 0) + (gpose ? (6 * P.n_cam + kThreads - 1) / kThreads : 0);
+    hipLaunchKernelGGL(k_cg_final<T>, dim3(finals), dim3(kThreads), 0, s, P, (const double*)h->tile_cost,
+                       (const double*)h->part, cost, total, gintr, (const double*)h->gpart, gpose);
     return launch_status(h);
 }
 
@@ -754,13 +807,12 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
     };
     int per_group = 1;
     while (per_group < kGroupTiles && groups_of(per_group) > kGroups) ++per_group;
-    std::vector<int> group_tile{0}, prob_group0{0};
+    std::vector<int> group_tile{0};
     for (int p = 0; p < n_probs; ++p) {
         for (int t = prob_tile0[p]; t < prob_tile0[p + 1];) {
             t = std::min(t + per_group, prob_tile0[p + 1]);
             group_tile.push_back(t);
         }
-        prob_group0.push_back((int)group_tile.size() - 1);
     }
     // camera-major order and its chunks
     std::vector<int> cam_ptr(nc + 1, 0), c_pt(no);
@@ -792,7 +844,7 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
     }
     CostProblem& P = h->P;
     P = CostProblem{};
-    P.n_obs = (int)no; P.n_groups = prob_group0.back(); P.n_chunks = (int)chunk_cam.size();
+    P.n_obs = (int)no; P.n_tiles = prob_tile0.back(); P.n_groups = (int)group_tile.size() - 1; P.n_chunks = (int)chunk_cam.size();
     P.n_unseen = (int)unseen.size();
     P.n_cam = nc; P.n_pt = np; P.n_prob = n_probs;
     P.robust = robust ? 1 : 0;
@@ -801,19 +853,20 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
     if ((st = up(h, o_cam, &P.o_cam)) || (st = up(h, o_pt, &P.o_pt)) || (st = up(h, uv, &P.uv)) ||
         (st = up(h, pt_list, &P.pt_list)) || (st = up(h, pt_ptr, &P.pt_ptr)) ||
         (st = up(h, tile_obs, &P.tile_obs)) || (st = up(h, tile_pt, &P.tile_pt)) ||
-        (st = up(h, group_tile, &P.group_tile)) || (st = up(h, prob_group0, &P.prob_group0)) ||
+        (st = up(h, group_tile, &P.group_tile)) || (st = up(h, prob_tile0, &P.prob_tile0)) ||
         (st = up(h, c_pt, &P.c_pt)) || (st = up(h, c_uv, &P.c_uv)) || (st = up(h, chunk_cam, &P.chunk_cam)) ||
         (st = up(h, chunk_ptr, &P.chunk_ptr)) || (st = up(h, cam_chunk0, &P.cam_chunk0)) ||
         (st = up(h, unseen, &P.unseen)))
         return st;
     void* part = nullptr;
-    const size_t n_part = 9 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks, n_pose = 12 * (size_t)nc;
-    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_part + n_gpart + n_pose, 1)) != hipSuccess) {
+    const size_t n_tile = (size_t)P.n_tiles, n_part = 8 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks, n_pose = 12 * (size_t)nc;
+    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_tile + n_part + n_gpart + n_pose, 1)) != hipSuccess) {
         h->err = "hipMalloc part";
         return NAV_BA_HIP_ERROR;
     }
     h->bufs.push_back(part);
-    h->part = (double*)part;
+    h->tile_cost = (double*)part;
+    h->part = h->tile_cost + n_tile;
     h->gpart = h->part + n_part;
     h->pose = h->gpart + n_gpart;
     h->prepared = true;
