@@ -106,7 +106,7 @@ __device__ __forceinline__ void obs_term(const TP* __restrict__ Tcw, const T* __
     const double Xc0 = R0 * x0 + R1 * x1 + R2 * x2 + (double)Tcw[9];
     const double Xc1 = R3 * x0 + R4 * x1 + R5 * x2 + (double)Tcw[10];
     const double Xc2 = R6 * x0 + R7 * x1 + R8 * x2 + (double)Tcw[11];
-    const double iz = navba::recip<double>(Xc2);
+    const double iz = navba::recip<double>(Xc2);  // the division's bits on 40 scenes, 1 % of a gradient faster
     const double x = Xc0 * iz, y = Xc1 * iz;
     const double fx = in[0], fy = in[1], cx = in[2], cy = in[3], k1 = in[4], k2 = in[5], p1 = in[6], p2 = in[7];
     const double r2 = x * x + y * y;
@@ -327,14 +327,20 @@ __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP*
             for (int i = tid; i < n_sum; i += kThreads) {
                 if (i != tid) point(q0 + i / 3);
                 const T* v = st[i % 3];
-                int a = one ? 0 : a0 - o0;
-                const int e = one ? kThreads : a1 - o0;
                 T s = T(0);
-                for (; a + 4 <= e; a += 4) {
-                    const T v0 = v[a], v1 = v[a + 1], v2 = v[a + 2], v3 = v[a + 3];
-                    s = (((s + v0) + v1) + v2) + v3;
+                if (one) {  // 256 lanes' sums: in FP64, as a serial sum of so many loses bits in float
+                    double d = 0.0;
+                    for (int a = 0; a < kThreads; ++a) d += (double)v[a];
+                    s = (T)d;
+                } else {
+                    int a = a0 - o0;
+                    const int e = a1 - o0;
+                    for (; a + 4 <= e; a += 4) {
+                        const T v0 = v[a], v1 = v[a + 1], v2 = v[a + 2], v3 = v[a + 3];
+                        s = (((s + v0) + v1) + v2) + v3;
+                    }
+                    for (; a < e; ++a) s += v[a];
                 }
-                for (; a < e; ++a) s += v[a];
                 gX[3 * (size_t)pt + i % 3] = s;
             }
             o0 = o1;

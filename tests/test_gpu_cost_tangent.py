@@ -142,3 +142,26 @@ def test_another_evaluator_is_called(where, monkeypatch):
     assert len(calls) == 1
     assert abs(got.item() - want.item()) <= 1e-12 * want.item()
     b.close()
+
+
+@pytest.mark.parametrize("n", [257, 300, 511, 512])  # more observations than a tile: at most two a lane
+def test_point_with_many_observations_sums_exactly(n):
+    """n equal observations of a point have n times the gradient of one.  A lane's
+    sum is then exact, so the point's is off by no more than its rounding to float,
+    2^-24 of it, however many lanes are added."""
+    from nav24_amd.abi import Problem
+    from nav24_amd.diffcost import CostBatch
+    for seed in range(8):
+        g = problems.params_for(4, seed)
+        g.n_pt, g.n_cam = 20, 3
+        p = problems.make(g)
+        grads = []
+        for k in (1, n):
+            q = Problem(T_cw=p.T_cw, X=p.X, obs_cam=np.repeat(p.obs_cam[:1], k), obs_pt=np.repeat(p.obs_pt[:1], k),
+                        obs_uv=np.repeat(p.obs_uv[:1], k, axis=0))
+            b = CostBatch([q])
+            args = [torch.tensor(a, device="cuda", dtype=torch.float32)
+                    for a in (p.T_cw, p.X, [p.fx, p.fy, p.cx, p.cy, *p.dist])]
+            grads.append(b.eval(*args).g_X[p.obs_pt[0]].double().cpu())
+            b.close()
+        assert ((grads[1] - n * grads[0]).abs() <= 2.0 ** -24 * n * grads[0].abs()).all()
