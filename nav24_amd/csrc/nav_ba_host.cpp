@@ -334,6 +334,21 @@ inline double rf32(double v) { return (double)(float)v; }
 
 bool mixed(const nav_ba_handle* h) { return h->opt.precision == NAV_BA_MIXED; }
 
+// The launches after this was made: an error that was pending before them (an
+// earlier call of the program left it) stays where it is, for its owner.
+class LaunchErrors {
+public:
+    int check(nav_ba_handle* h) const {
+        const hipError_t e = hipPeekAtLastError();
+        if (e == before_) return NAV_BA_OK;
+        if (before_ == hipSuccess) (void)hipGetLastError();
+        return fail(h, NAV_BA_HIP_ERROR, std::string("launch: ") + hipGetErrorString(e));
+    }
+
+private:
+    hipError_t before_ = hipPeekAtLastError();
+};
+
 // Enqueue one stage; with timing active it is bracketed by HIP events.
 template <class F>
 void stage(nav_ba_handle* h, int cat, F&& f) {
@@ -1619,9 +1634,9 @@ int fetch_all(nav_ba_handle* h, nav_ba_result* results, int n) {
         HIPTRY(h, hipHostMalloc((void**)&h->rbuf, at.total, hipHostMallocDefault));
         h->rbuf_cap = at.total;
     }
-    (void)hipGetLastError();  // an error that an earlier call of the program left is not this one's
+    const LaunchErrors errors;
     launch_results(h->P, h->cur, h->W, h->pt_src, h->x_in, at, h->opt.compat_fp32_io != 0, h->rbuf, h->stream);
-    HIPTRY(h, hipGetLastError());
+    if (errors.check(h) != NAV_BA_OK) return NAV_BA_HIP_ERROR;
     HIPTRY(h, hipStreamSynchronize(h->stream));
     // the copies to the caller's arrays fault their pages in: a few threads where
     // that is megabytes
@@ -1727,7 +1742,7 @@ int32_t nav_ba_run(nav_ba_handle* h) {
         HIPTRY(h, hipHostMalloc((void**)&h->report, at.total, hipHostMallocDefault));
         h->report_cap = at.total;
     }
-    (void)hipGetLastError();  // an error that an earlier call of the program left is not this run's
+    const LaunchErrors errors;
     HIPTRY(h, hipEventRecord(h->ev0, s));
     launch_run_start(P, h->init, h->cur, h->W, s);
     if (m) launch_cost<float>(P, h->cur, h->W, 0, s); else launch_cost<double>(P, h->cur, h->W, 0, s);
@@ -1762,7 +1777,7 @@ int32_t nav_ba_run(nav_ba_handle* h) {
         } else {
             launch_report(P, h->W, at, few, false, h->report, s);
         }
-        HIPTRY(h, hipGetLastError());
+        if (errors.check(h) != NAV_BA_OK) return NAV_BA_HIP_ERROR;
         HIPTRY(h, hipStreamSynchronize(s));
         finished = finished || steps >= max_steps || *(const int*)h->report >= P.n_win;
         if (finished) {

@@ -60,3 +60,27 @@ def test_linearisation_together_or_apart(fisheye, precision, n_pt):
     s.close()
     assert np.array_equal(one.T_cw, apart.T_cw) and np.array_equal(one.X, apart.X)
     assert np.array_equal(one.cost_history, apart.cost_history) and one.trials == apart.trials
+
+
+def test_pending_error_of_the_program_stays():
+    """An error that the program's own HIP call left is neither taken by a run and a
+    fetch nor taken for theirs."""
+    import ctypes as C
+    from nav24_amd.ba import GraphOptimHip, lib
+    hip = lib()  # the runtime that the library is linked to
+    o = workload_options(3)
+    o.precision, o.n_iter = NAV_BA_FP64, 2
+    s = GraphOptimHip(0)
+    s.prepare(window(1, False), o)
+    s.run()
+    want = s.fetch()
+    hip.hipGetLastError()
+    assert hip.hipMemcpy(None, None, C.c_size_t(8), C.c_int(2)) != 0  # null arrays: refused on the host
+    left = hip.hipPeekAtLastError()
+    assert left != 0
+    s.run()
+    got = s.fetch()
+    assert hip.hipPeekAtLastError() == left
+    hip.hipGetLastError()
+    s.close()
+    assert np.array_equal(got.T_cw, want.T_cw) and np.array_equal(got.X, want.X)
