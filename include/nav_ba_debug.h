@@ -102,6 +102,11 @@ int32_t nav_ba_debug_set_schur_kernel(nav_ba_handle* h, int32_t kernel);
  * when the problem had nothing to optimise). */
 int32_t nav_ba_debug_get_schur_kernel(const nav_ba_handle* h, int32_t* kernel);
 
+/* Whether later runs and fetches on this handle may have their results written to
+ * pinned memory (the default), or take the way through pageable memory that they
+ * fall back to where it cannot be pinned: the same bits. */
+int32_t nav_ba_debug_set_pinned(nav_ba_handle* h, int32_t enable);
+
 /* After a prepare (one problem or a batch): linearise every window at its
  * initial state, damping lambda, and time the Schur-row kernel over all
  * windows: one warm-up launch, then `reps` launches back to back between two

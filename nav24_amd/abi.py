@@ -225,7 +225,8 @@ _RESULT_RECORD = np.dtype({
 
 class BatchResultBuffers:
     """Output arrays for the nav_ba_results of a batch: one allocation per kind
-    of output, of which every window's result holds its part."""
+    of output, of which every window's result is a view.  A result that is kept
+    keeps the batch's arrays: copy its arrays to keep one window of many."""
 
     def __init__(self, windows, n_iter: int):
         n = len(windows)

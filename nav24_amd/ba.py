@@ -28,7 +28,7 @@ EXPORTED = [
     "nav_ba_prepare_batched", "nav_ba_fetch_batched", "nav_ba_solve_batched",
     "nav_ba_debug_reduced_system", "nav_ba_set_timing", "nav_ba_get_timing", "nav_ba_debug_set_solver",
     "nav_ba_debug_set_schur_chunk", "nav_ba_debug_get_schur_chunk", "nav_ba_debug_check_layout",
-    "nav_ba_debug_time_schur_rows", "nav_ba_debug_time_stage", "nav_ba_debug_pcg_stats", "nav_ba_debug_set_schur_kernel", "nav_ba_debug_get_schur_kernel",
+    "nav_ba_debug_time_schur_rows", "nav_ba_debug_time_stage", "nav_ba_debug_pcg_stats", "nav_ba_debug_set_pinned", "nav_ba_debug_set_schur_kernel", "nav_ba_debug_get_schur_kernel",
     "nav_ba_debug_prepare_cached",
 ]
 
@@ -86,6 +86,8 @@ def lib() -> C.CDLL:
         L.nav_ba_debug_get_schur_chunk.restype = C.c_int32
         L.nav_ba_debug_prepare_cached.argtypes = [H, C.POINTER(C.c_int32)]
         L.nav_ba_debug_prepare_cached.restype = C.c_int32
+        L.nav_ba_debug_set_pinned.argtypes = [H, C.c_int32]
+        L.nav_ba_debug_set_pinned.restype = C.c_int32
         L.nav_ba_debug_set_schur_kernel.argtypes = [H, C.c_int32]
         L.nav_ba_debug_set_schur_kernel.restype = C.c_int32
         L.nav_ba_debug_get_schur_kernel.argtypes = [H, C.POINTER(C.c_int32)]
@@ -178,7 +180,9 @@ class GraphOptimHip:
         return arr, opts.c_struct()
 
     def solve_batched(self, windows: Sequence[Problem], opts: Options) -> List[Result]:
-        """One GraphOptim::solve per window, all windows in one device solve."""
+        """One GraphOptim::solve per window, all windows in one device solve.
+        The results' arrays are views of the batch's, as those of fetch_batched:
+        copy them to keep one window of many."""
         arr, os_ = self._batch(windows, opts)
         bufs = BatchResultBuffers(windows, opts.n_iter)
         st = lib().nav_ba_solve_batched(self._h, arr, len(windows), C.byref(os_), bufs.c)

@@ -66,6 +66,57 @@ struct DevBuf {
     size_t cap = 0;
 };
 
+// A buffer that a kernel writes and the host reads after the stream's next wait,
+// grown to the largest use: pinned memory that the kernel writes itself, or, where
+// that much cannot be pinned, device memory copied to pageable memory.
+struct HostOut {
+    char* pin = nullptr;
+    size_t pin_cap = 0;
+    char* dev = nullptr;
+    size_t dev_cap = 0;
+    std::vector<char> page;
+    bool pinned = false;  // the buffer of the last begin
+
+    hipError_t begin(size_t bytes, bool may_pin) {
+        pinned = may_pin && grow_pinned(bytes);
+        if (pinned) return hipSuccess;
+        if (page.size() < bytes) page.resize(bytes);
+        if (dev_cap >= bytes) return hipSuccess;
+        if (dev) (void)hipFree(dev);
+        dev = nullptr;
+        dev_cap = 0;
+        const hipError_t e = hipMalloc((void**)&dev, bytes);
+        if (e == hipSuccess) dev_cap = bytes;
+        return e;
+    }
+    char* target() const { return pinned ? pin : dev; }           // for the kernel
+    const char* data() const { return pinned ? pin : page.data(); }  // after finish and the wait
+    hipError_t finish(size_t bytes, hipStream_t s) {
+        return pinned ? hipSuccess : hipMemcpyAsync(page.data(), dev, bytes, hipMemcpyDeviceToHost, s);
+    }
+    void release() {
+        if (pin) (void)hipHostFree(pin);
+        if (dev) (void)hipFree(dev);
+        *this = HostOut{};
+    }
+
+private:
+    bool grow_pinned(size_t bytes) {
+        if (pin_cap >= bytes) return true;
+        if (pin) (void)hipHostFree(pin);
+        pin = nullptr;
+        pin_cap = 0;
+        const hipError_t before = hipPeekAtLastError();
+        if (hipHostMalloc((void**)&pin, bytes, hipHostMallocDefault) != hipSuccess) {
+            if (before == hipSuccess) (void)hipGetLastError();
+            pin = nullptr;
+            return false;
+        }
+        pin_cap = bytes;
+        return true;
+    }
+};
+
 // HIP event pairs around stage launches; read back after a stream sync.
 struct StageTimer {
     std::vector<hipEvent_t> ev;
@@ -198,8 +249,8 @@ struct nav_ba_handle {
     int schur_kernel = 0;  // Schur row kernel: 0 = default or tuned, 1 = rounds of kBlock, 2 = producer/consumer
     bool schur_pc_used = false;
     StageTimer timer;
-    char* report = nullptr;    // pinned: what the host reads of a run (ReportPlaces)
-    size_t report_cap = 0;
+    HostOut report;            // what the host reads of a run (ReportPlaces)
+    bool may_pin = true;       // whether report and results may be pinned memory
     char* stage = nullptr;     // pinned staging of a prepare's uploads (grown on demand)
     size_t stage_cap = 0;
     char* stage_s = nullptr;   // pinned staging of the Schur work items (the tuner re-uploads them)
@@ -209,11 +260,10 @@ struct nav_ba_handle {
     std::vector<char> prep_key;
     bool prep_cached = false;  // the last prepare took the cached index
     // results: the points' sources and, where some have no observation, the
-    // caller's points; a pinned buffer that fetch's kernel writes in caller order
+    // caller's points; the buffer that fetch's kernel writes in caller order
     const int* pt_src = nullptr;
     double* x_in = nullptr;
-    char* rbuf = nullptr;
-    size_t rbuf_cap = 0;
+    HostOut results;
     // results of the last run
     bool ran = false;
     std::vector<LMDev> lm_out;
@@ -1603,13 +1653,14 @@ int fetch_window(nav_ba_handle* h, int w, nav_ba_result* r) {
     return NAV_BA_OK;
 }
 
-// Window w's poses, points and flags from the pinned result buffer.
+// Window w's poses, points and flags from the result buffer.
 void copy_window(const nav_ba_handle* h, int w, const ResultPlaces& at, const nav_ba_result& r) {
     const WinHost& wh = h->layout.win[w];
     if (wh.empty) return;
-    if (r.T_cw) std::memcpy(r.T_cw, (const double*)(h->rbuf + at.T) + 12 * (size_t)wh.cam0, sizeof(double) * 12 * wh.n_cam);
-    if (r.X) std::memcpy(r.X, (const double*)(h->rbuf + at.X) + 3 * wh.pt0, sizeof(double) * 3 * (size_t)wh.n_pt);
-    if (r.outlier && wh.n_obs > 0) std::memcpy(r.outlier, h->rbuf + at.flags + wh.obs0, (size_t)wh.n_obs);
+    const char* buf = h->results.data();
+    if (r.T_cw) std::memcpy(r.T_cw, (const double*)(buf + at.T) + 12 * (size_t)wh.cam0, sizeof(double) * 12 * wh.n_cam);
+    if (r.X) std::memcpy(r.X, (const double*)(buf + at.X) + 3 * wh.pt0, sizeof(double) * 3 * (size_t)wh.n_pt);
+    if (r.outlier && wh.n_obs > 0) std::memcpy(r.outlier, buf + at.flags + wh.obs0, (size_t)wh.n_obs);
 }
 
 int fetch_all(nav_ba_handle* h, nav_ba_result* results, int n) {
@@ -1624,19 +1675,16 @@ int fetch_all(nav_ba_handle* h, nav_ba_result* results, int n) {
     if (h->all_empty) return worst;
     // poses, points and flags in caller order, written by one kernel straight into
     // pinned memory: no copies in device order (each through a staging buffer of
-    // the runtime) and no reordering on the host
+    // the runtime) and no reordering on the host.  The handle keeps the buffer, as
+    // large as its largest result (40 MB for 512 windows)
     HIPTRY(h, hipSetDevice(h->device));
     const ResultPlaces at(h->P.n_cam, h->layout.pt_src.size(), h->P.n_obs);
-    if (h->rbuf_cap < at.total) {
-        if (h->rbuf) (void)hipHostFree(h->rbuf);
-        h->rbuf = nullptr;
-        h->rbuf_cap = 0;
-        HIPTRY(h, hipHostMalloc((void**)&h->rbuf, at.total, hipHostMallocDefault));
-        h->rbuf_cap = at.total;
-    }
+    HIPTRY(h, h->results.begin(at.total, h->may_pin));
     const LaunchErrors errors;
-    launch_results(h->P, h->cur, h->W, h->pt_src, h->x_in, at, h->opt.compat_fp32_io != 0, h->rbuf, h->stream);
+    launch_results(h->P, h->cur, h->W, h->pt_src, h->x_in, at, h->opt.compat_fp32_io != 0,
+                   h->results.target(), h->stream);
     if (errors.check(h) != NAV_BA_OK) return NAV_BA_HIP_ERROR;
+    HIPTRY(h, h->results.finish(at.total, h->stream));
     HIPTRY(h, hipStreamSynchronize(h->stream));
     // the copies to the caller's arrays fault their pages in: a few threads where
     // that is megabytes
@@ -1699,11 +1747,11 @@ void nav_ba_destroy(nav_ba_handle* h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (auto& b : h->bufs)
         if (b.p) (void)hipFree(b.p);
-    if (h->report) (void)hipHostFree(h->report);
+    h->report.release();
+    h->results.release();
     if (h->hpcg) (void)hipHostFree(h->hpcg);
     if (h->stage) (void)hipHostFree(h->stage);
     if (h->stage_s) (void)hipHostFree(h->stage_s);
-    if (h->rbuf) (void)hipHostFree(h->rbuf);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1735,13 +1783,7 @@ int32_t nav_ba_run(nav_ba_handle* h) {
     const DevProblem& P = h->P;
     const bool m = mixed(h);
     const ReportPlaces at((size_t)P.n_win, (size_t)P.n_iter);
-    if (h->report_cap < at.total) {
-        if (h->report) (void)hipHostFree(h->report);
-        h->report = nullptr;
-        h->report_cap = 0;
-        HIPTRY(h, hipHostMalloc((void**)&h->report, at.total, hipHostMallocDefault));
-        h->report_cap = at.total;
-    }
+    HIPTRY(h, h->report.begin(at.total, h->may_pin));
     const LaunchErrors errors;
     HIPTRY(h, hipEventRecord(h->ev0, s));
     launch_run_start(P, h->init, h->cur, h->W, s);
@@ -1770,16 +1812,17 @@ int32_t nav_ba_run(nav_ba_handle* h) {
             h->timing_active = h->timing;
             stage(h, NAV_BA_ST_FLAGS, [&] {
                 launch_flags(P, h->cur, h->W, h->opt.outlier_chi2, s);
-                launch_report(P, h->W, at, true, true, h->report, s);
+                launch_report(P, h->W, at, true, true, h->report.target(), s);
             });
             h->timing_active = false;
             HIPTRY(h, hipEventRecord(h->ev1, s));
         } else {
-            launch_report(P, h->W, at, few, false, h->report, s);
+            launch_report(P, h->W, at, few, false, h->report.target(), s);
         }
         if (errors.check(h) != NAV_BA_OK) return NAV_BA_HIP_ERROR;
+        HIPTRY(h, h->report.finish(at.total, s));
         HIPTRY(h, hipStreamSynchronize(s));
-        finished = finished || steps >= max_steps || *(const int*)h->report >= P.n_win;
+        finished = finished || steps >= max_steps || *(const int*)h->report.data() >= P.n_win;
         if (finished) {
             if (final) break;
             final = true;
@@ -1787,16 +1830,16 @@ int32_t nav_ba_run(nav_ba_handle* h) {
         }
         burst = 2;
         if (few) {
-            const LMDev* lm = (const LMDev*)(h->report + at.lm);
+            const LMDev* lm = (const LMDev*)(h->report.data() + at.lm);
             int rem = 0;
             for (int w = 0; w < P.n_win; ++w)
                 if (lm[w].phase != kPhaseDone) rem = std::max(rem, P.n_iter - lm[w].iter);
             burst = std::max<long long>(2, rem + (rem + 1) / 2);
         }
     }
-    const LMDev* lm = (const LMDev*)(h->report + at.lm);
-    const double* hist = (const double*)(h->report + at.hist);
-    const double* fin = (const double*)(h->report + at.final);
+    const LMDev* lm = (const LMDev*)(h->report.data() + at.lm);
+    const double* hist = (const double*)(h->report.data() + at.hist);
+    const double* fin = (const double*)(h->report.data() + at.final);
     h->lm_out.assign(lm, lm + P.n_win);
     h->hist_out.assign(hist, hist + (size_t)P.n_win * (P.n_iter + 1));
     h->final_out.assign(fin, fin + 2 * (size_t)P.n_win);
@@ -1867,6 +1910,12 @@ int32_t nav_ba_debug_get_schur_chunk(const nav_ba_handle* h, int32_t* chunk) {
 int32_t nav_ba_debug_prepare_cached(const nav_ba_handle* h, int32_t* cached) {
     if (!h || !cached) return NAV_BA_BAD_ARG;
     *cached = h->prep_cached ? 1 : 0;
+    return NAV_BA_OK;
+}
+
+int32_t nav_ba_debug_set_pinned(nav_ba_handle* h, int32_t enable) {
+    if (!h) return NAV_BA_BAD_ARG;
+    h->may_pin = enable != 0;
     return NAV_BA_OK;
 }
 

@@ -70,3 +70,24 @@ def test_batch_equals_single_and_empty_windows_are_returned():
         for k in ("T_cw", "X", "outlier", "cost_history"):
             assert np.array_equal(getattr(g, k), getattr(r, k)), k
     s.close()
+
+
+@pytest.mark.parametrize("n_win", [1, 3, 65])  # a window, few of them, more than the host reads between bursts
+def test_results_without_pinned_memory(n_win):
+    """Where the results' buffer cannot be pinned, they come through pageable memory."""
+    from nav24_amd.ba import GraphOptimHip, lib
+    o = options()
+    wins = [window(1 + k % 3, 399 + k % 3, 5 * (k % 2)) for k in range(n_win)]
+    s = GraphOptimHip(0)
+    s.prepare_batched(wins, o)
+    got = []
+    for pinned in (1, 0, 1):
+        assert lib().nav_ba_debug_set_pinned(s._h, pinned) == 0
+        s.run()
+        got.append(s.fetch_batched())
+    s.close()
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            for k in ("T_cw", "X", "outlier", "cost_history"):
+                assert np.array_equal(getattr(a, k), getattr(b, k)), k
+            assert (a.iterations, a.trials, a.n_outliers, a.final_cost) == (b.iterations, b.trials, b.n_outliers, b.final_cost)
