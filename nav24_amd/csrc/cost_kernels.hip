@@ -617,20 +617,48 @@ void free_all(nav_ba_cost_handle* h) {
     h->tile_cost = h->part = h->gpart = h->pose = nullptr;
 }
 
-template <class V>
-int up(nav_ba_cost_handle* h, const V& v, const typename V::value_type** out) {
-    void* p = nullptr;
-    const size_t bytes = std::max<size_t>(sizeof(typename V::value_type) * v.size(), 256);
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) { h->err = std::string("hipMalloc: ") + hipGetErrorString(e); return NAV_BA_HIP_ERROR; }
-    h->bufs.push_back(p);
-    if (!v.empty() && hipMemcpy(p, v.data(), sizeof(typename V::value_type) * v.size(), hipMemcpyHostToDevice) != hipSuccess) {
-        h->err = "hipMemcpy failed";
-        return NAV_BA_HIP_ERROR;
+// A prepare's arrays and scratch in one allocation; arrays up to kPackBytes go in
+// one copy (a copy of its own costs the host 18 us whatever its size up to there).
+class Upload {
+public:
+    template <class V>
+    void add(const V& v, const typename V::value_type** out) {
+        a_.push_back(Array{v.data(), sizeof(typename V::value_type) * v.size(), reinterpret_cast<const void**>(out)});
     }
-    *out = (const typename V::value_type*)p;
-    return NAV_BA_OK;
-}
+    void scratch(size_t bytes, double** out) {
+        a_.push_back(Array{nullptr, bytes, reinterpret_cast<const void**>(const_cast<const double**>(out))});
+    }
+    int flush(nav_ba_cost_handle* h) {
+        constexpr size_t kPackBytes = 64 << 10;
+        std::stable_partition(a_.begin(), a_.end(), [](const Array& a) { return a.src && a.bytes <= kPackBytes; });
+        std::vector<size_t> at(a_.size());
+        size_t total = 0, packed = 0;
+        for (size_t k = 0; k < a_.size(); ++k) {
+            at[k] = total;
+            total += (std::max<size_t>(a_[k].bytes, 1) + 255) & ~size_t(255);
+            if (a_[k].src && a_[k].bytes <= kPackBytes) packed = total;
+        }
+        void* d = nullptr;
+        const hipError_t e = hipMalloc(&d, std::max<size_t>(total, 256));
+        if (e != hipSuccess) { h->err = std::string("hipMalloc: ") + hipGetErrorString(e); return NAV_BA_HIP_ERROR; }
+        h->bufs.push_back(d);
+        std::vector<char> pack(packed);
+        bool ok = true;
+        for (size_t k = 0; k < a_.size(); ++k) {
+            *a_[k].dst = static_cast<char*>(d) + at[k];
+            if (!a_[k].src || a_[k].bytes == 0) continue;
+            if (at[k] < packed) std::memcpy(pack.data() + at[k], a_[k].src, a_[k].bytes);
+            else ok = ok && hipMemcpy(static_cast<char*>(d) + at[k], a_[k].src, a_[k].bytes, hipMemcpyHostToDevice) == hipSuccess;
+        }
+        if (packed > 0) ok = ok && hipMemcpy(d, pack.data(), packed, hipMemcpyHostToDevice) == hipSuccess;
+        if (!ok) { h->err = "hipMemcpy failed"; return NAV_BA_HIP_ERROR; }
+        return NAV_BA_OK;
+    }
+
+private:
+    struct Array { const void* src; size_t bytes; const void** dst; };  // src null: scratch
+    std::vector<Array> a_;
+};
 
 int32_t launch_status(nav_ba_cost_handle* h) {
     const hipError_t e = hipGetLastError();
@@ -746,36 +774,43 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
     }
     if (no > (size_t)0x7fffffff) { h->err = "too many observations"; return NAV_BA_TOO_LARGE; }
     const int nc = cam_off[n_probs], np = pt_off[n_probs];
-    std::vector<int> gcam(no), gpt(no);
-    std::vector<double> guv(2 * no);
+    // Both orders, a problem at a time (its cameras and points are contiguous, and
+    // its part of every array stays in the cache): point-major (point, camera, input
+    // order) by two stable counting sorts, camera-major from it by a third.
+    std::vector<int> o_cam(no), o_pt(no), c_pt(no), cam_ptr(nc + 1, 0);
+    std::vector<double2> uv(no), c_uv(no);
     {
-        size_t k = 0;
-        for (int p = 0; p < n_probs; ++p)
-            for (int i = 0; i < probs[p].n_obs; ++i, ++k) {
-                gcam[k] = cam_off[p] + probs[p].obs_cam[i];
-                gpt[k] = pt_off[p] + probs[p].obs_pt[i];
-                guv[2 * k] = probs[p].obs_uv[2 * (size_t)i];
-                guv[2 * k + 1] = probs[p].obs_uv[2 * (size_t)i + 1];
+        std::vector<int> byc, off, poff;
+        size_t o0 = 0;
+        for (int p = 0; p < n_probs; ++p) {
+            const nav_ba_problem& q = probs[p];
+            const int m = q.n_obs, c0 = cam_off[p], p0 = pt_off[p];
+            off.assign(q.n_cam + 1, 0);
+            poff.assign(q.n_pt + 1, 0);
+            for (int i = 0; i < m; ++i) {
+                off[q.obs_cam[i] + 1]++;
+                poff[q.obs_pt[i] + 1]++;
             }
-    }
-    // point-major order (point, camera, input order): two stable counting sorts
-    std::vector<int> byc(no), ord(no);
-    {
-        std::vector<int> off(nc + 1, 0);
-        for (size_t i = 0; i < no; ++i) off[gcam[i] + 1]++;
-        for (int c = 0; c < nc; ++c) off[c + 1] += off[c];
-        for (size_t i = 0; i < no; ++i) byc[off[gcam[i]]++] = (int)i;
-        std::vector<int> poff(np + 1, 0);
-        for (size_t i = 0; i < no; ++i) poff[gpt[i] + 1]++;
-        for (int q = 0; q < np; ++q) poff[q + 1] += poff[q];
-        for (size_t k = 0; k < no; ++k) { const int i = byc[k]; ord[poff[gpt[i]]++] = i; }
-    }
-    std::vector<int> o_cam(no), o_pt(no);
-    std::vector<double2> uv(no);
-    for (size_t k = 0; k < no; ++k) {
-        const int i = ord[k];
-        o_cam[k] = gcam[i]; o_pt[k] = gpt[i];
-        uv[k] = double2{guv[2 * (size_t)i], guv[2 * (size_t)i + 1]};
+            for (int c = 0; c < q.n_cam; ++c) off[c + 1] += off[c];
+            for (int c = 0; c < q.n_pt; ++c) poff[c + 1] += poff[c];
+            for (int c = 0; c < q.n_cam; ++c) cam_ptr[c0 + c + 1] = (int)o0 + off[c + 1];
+            byc.resize(m);
+            for (int i = 0; i < m; ++i) byc[off[q.obs_cam[i]]++] = i;
+            for (int k = 0; k < m; ++k) {
+                const int i = byc[k];
+                const size_t at = o0 + poff[q.obs_pt[i]]++;
+                o_cam[at] = c0 + q.obs_cam[i];
+                o_pt[at] = p0 + q.obs_pt[i];
+                uv[at] = double2{q.obs_uv[2 * (size_t)i], q.obs_uv[2 * (size_t)i + 1]};
+            }
+            for (int c = 0; c < q.n_cam; ++c) off[c] = cam_ptr[c0 + c];
+            for (size_t k = o0; k < o0 + m; ++k) {
+                const int at = off[o_cam[k] - c0]++;
+                c_pt[at] = o_pt[k];
+                c_uv[at] = uv[k];
+            }
+            o0 += m;
+        }
     }
     // unique points, tiles of whole points per problem
     std::vector<int> pt_list, pt_ptr{0}, tile_obs{0}, tile_pt{0}, prob_tile0{0};
@@ -820,19 +855,7 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
             group_tile.push_back(t);
         }
     }
-    // camera-major order and its chunks
-    std::vector<int> cam_ptr(nc + 1, 0), c_pt(no);
-    std::vector<double2> c_uv(no);
-    for (size_t k = 0; k < no; ++k) cam_ptr[o_cam[k] + 1]++;
-    for (int c = 0; c < nc; ++c) cam_ptr[c + 1] += cam_ptr[c];
-    {
-        std::vector<int> pos(cam_ptr.begin(), cam_ptr.end() - 1);
-        for (size_t k = 0; k < no; ++k) {
-            const int at = pos[o_cam[k]]++;
-            c_pt[at] = o_pt[k];
-            c_uv[at] = uv[k];
-        }
-    }
+    // chunks of the camera-major order
     const int chunk = std::min<int>(kChunkMax, std::max<int>(1, (int)(no / ((size_t)kChunks * kThreads))) * kThreads);
     std::vector<int> chunk_cam, chunk_ptr{0}, cam_chunk0{0};
     for (int c = 0; c < nc; ++c) {
@@ -855,26 +878,19 @@ int32_t nav_ba_cost_prepare(nav_ba_cost_handle* h, const nav_ba_problem* probs, 
     P.n_cam = nc; P.n_pt = np; P.n_prob = n_probs;
     P.robust = robust ? 1 : 0;
     P.delta = huber_delta;
-    int st;
-    if ((st = up(h, o_cam, &P.o_cam)) || (st = up(h, o_pt, &P.o_pt)) || (st = up(h, uv, &P.uv)) ||
-        (st = up(h, pt_list, &P.pt_list)) || (st = up(h, pt_ptr, &P.pt_ptr)) ||
-        (st = up(h, tile_obs, &P.tile_obs)) || (st = up(h, tile_pt, &P.tile_pt)) ||
-        (st = up(h, group_tile, &P.group_tile)) || (st = up(h, prob_tile0, &P.prob_tile0)) ||
-        (st = up(h, c_pt, &P.c_pt)) || (st = up(h, c_uv, &P.c_uv)) || (st = up(h, chunk_cam, &P.chunk_cam)) ||
-        (st = up(h, chunk_ptr, &P.chunk_ptr)) || (st = up(h, cam_chunk0, &P.cam_chunk0)) ||
-        (st = up(h, unseen, &P.unseen)))
-        return st;
-    void* part = nullptr;
-    const size_t n_tile = (size_t)P.n_tiles, n_part = 8 * (size_t)P.n_groups, n_gpart = 6 * (size_t)P.n_chunks, n_pose = 12 * (size_t)nc;
-    if (hipMalloc(&part, sizeof(double) * std::max<size_t>(n_tile + n_part + n_gpart + n_pose, 1)) != hipSuccess) {
-        h->err = "hipMalloc part";
-        return NAV_BA_HIP_ERROR;
-    }
-    h->bufs.push_back(part);
-    h->tile_cost = (double*)part;
-    h->part = h->tile_cost + n_tile;
-    h->gpart = h->part + n_part;
-    h->pose = h->gpart + n_gpart;
+    Upload u;
+    u.add(o_cam, &P.o_cam); u.add(o_pt, &P.o_pt); u.add(uv, &P.uv);
+    u.add(pt_list, &P.pt_list); u.add(pt_ptr, &P.pt_ptr); u.add(tile_obs, &P.tile_obs); u.add(tile_pt, &P.tile_pt);
+    u.add(group_tile, &P.group_tile); u.add(prob_tile0, &P.prob_tile0);
+    u.add(c_pt, &P.c_pt); u.add(c_uv, &P.c_uv);
+    u.add(chunk_cam, &P.chunk_cam); u.add(chunk_ptr, &P.chunk_ptr); u.add(cam_chunk0, &P.cam_chunk0);
+    u.add(unseen, &P.unseen);
+    u.scratch(sizeof(double) * P.n_tiles, &h->tile_cost);
+    u.scratch(sizeof(double) * 8 * P.n_groups, &h->part);
+    u.scratch(sizeof(double) * 6 * P.n_chunks, &h->gpart);
+    u.scratch(sizeof(double) * 12 * nc, &h->pose);
+    const int st = u.flush(h);
+    if (st != NAV_BA_OK) return st;
     h->prepared = true;
     return NAV_BA_OK;
 }
