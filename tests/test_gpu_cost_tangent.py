@@ -165,3 +165,49 @@ def test_point_with_many_observations_sums_exactly(n):
             grads.append(b.eval(*args).g_X[p.obs_pt[0]].double().cpu())
             b.close()
         assert ((grads[1] - n * grads[0]).abs() <= 2.0 ** -24 * n * grads[0].abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("name", ["one observation", "one short, then over", "a point of several rounds",
+                                  "an empty problem between", "one tile more"])
+def test_outputs_stay_within_their_buffers(name, dtype):
+    """Every output lies one element off an aligned address between guard elements,
+    which all calls leave as they are, at the layouts' remainders."""
+    from nav24_amd import diffcost
+    from test_gpu_cost_groups import CASES, counted
+    probs = [counted(3 + k, c, idle_cam=True) for k, c in enumerate(CASES[name])]
+    q, guard, pad = probs[0], -7.25, 65
+    args = [torch.tensor(np.asarray(a), device="cuda", dtype=dtype)
+            for a in (np.concatenate([p.T_cw for p in probs]), np.concatenate([p.X for p in probs]),
+                      [q.fx, q.fy, q.cx, q.cy, *q.dist])]
+    b = diffcost.CostBatch(probs)
+    xi = torch.full((b.n_cam, 6), 0.01, device="cuda", dtype=dtype)
+    want = b.eval(*args)
+    lib, stream = diffcost.lib(), torch.cuda.current_stream().cuda_stream
+    code = diffcost.NAV_BA_COST_F64 if dtype == torch.float64 else diffcost.NAV_BA_COST_F32
+    guarded = []
+
+    def out(n):
+        t = torch.full((n + 2 * pad,), guard, device="cuda", dtype=dtype)
+        guarded.append((t, n))
+        return t[pad:pad + n]
+
+    sizes = (6 * b.n_cam, 3 * b.n_pt, 8)
+    cost, grads = out(b.n_problems), [out(n) for n in sizes]
+    b._check(lib.nav_ba_cost_eval(b._h, code, *(a.data_ptr() for a in args), cost.data_ptr(),
+                                  *(g.data_ptr() for g in grads), stream))
+    for g, w in zip((cost, *grads), (want.cost, want.g_pose, want.g_X, want.g_intr)):
+        assert torch.equal(g, w.flatten())
+    T, total, cost, grads = out(12 * b.n_cam), out(1), out(b.n_problems), [out(n) for n in sizes]
+    b._check(lib.nav_ba_cost_eval_tangent(b._h, code, xi.data_ptr(), *(a.data_ptr() for a in args), T.data_ptr(),
+                                          total.data_ptr(), cost.data_ptr(), *(g.data_ptr() for g in grads), stream))
+    back = [out(n) for n in sizes]
+    one = torch.ones((), device="cuda", dtype=dtype)
+    assert lib.nav_ba_cost_backward(0, code, b.n_cam, b.n_pt, xi.data_ptr(), *(g.data_ptr() for g in grads),
+                                    one.data_ptr(), *(g.data_ptr() for g in back), stream) == 0
+    assert torch.equal(back[1], grads[1]) and torch.equal(back[2], grads[2])
+    torch.cuda.synchronize()
+    for t, n in guarded:
+        assert not bool((t[pad:pad + n] == guard).any())  # every element of an output is written
+        assert bool((t[:pad] == guard).all()) and bool((t[pad + n:] == guard).all())
+    b.close()
