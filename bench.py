@@ -212,7 +212,7 @@ def headline_leg(n_windows, steps, warmup, with_cpu):
     plain = []
     for w in wins:
         s.prepare(w, o64)
-        s.run()  # warm-up of this window's graph
+        s.run()  # warm-up of this window
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         s.run()
@@ -656,8 +656,8 @@ def window_leg(n_windows, reps, with_cpu):
     the LM solve, results back to the host) for windows 0..n_windows-1 of the
     uneven-window generator, `reps` calls each, with the prepare / run / fetch
     split of the same calls.  Two cases: a new structure every call (another
-    window solved on the handle in between: host ordering, work items and
-    graph capture each time), and the same structure with new poses, points
+    window solved on the handle in between: host ordering and work items
+    each time), and the same structure with new poses, points
     and measurements (the cached index: only the state is uploaded).  The FP64
     oracle on window 0 is the CPU baseline."""
     import torch

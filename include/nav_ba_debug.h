@@ -44,10 +44,10 @@ typedef struct nav_ba_timing {
     int32_t launches[16];  /* timed launches per stage */
 } nav_ba_timing;
 
-/* enable != 0: later nav_ba_run calls launch the stages one by one (no
- * graphs) with HIP events on the handle's stream around each stage, and
- * accumulate the times; enable == 0 returns to graph replay.  Enabling
- * clears the accumulators. */
+/* enable != 0: later nav_ba_run calls put HIP events on the handle's stream
+ * around each stage's launches and accumulate the times (and launch the two
+ * sides of a small problem's linearisation apart); enable == 0 returns to runs
+ * without them.  Enabling clears the accumulators. */
 int32_t nav_ba_set_timing(nav_ba_handle* h, int32_t enable);
 int32_t nav_ba_get_timing(const nav_ba_handle* h, nav_ba_timing* out);
 

@@ -203,7 +203,7 @@ class GraphOptimHip:
         return bufs.results()
 
     def set_timing(self, enable: bool) -> None:
-        """Stage-by-stage launches with HIP events around each stage (no graphs)."""
+        """HIP events around each stage's launches in later runs."""
         self._check(lib().nav_ba_set_timing(self._h, int(bool(enable))))
 
     def timing(self) -> dict:

@@ -1,6 +1,6 @@
 // ba_kernels.hip — gfx950 kernels of the BA Levenberg-Marquardt solve.
 //
-// One replay of the step graph advances every window by one LM trial (g2o
+// One step's launches advance every window by one LM trial (g2o
 // OptimizationAlgorithmLevenberg::solve, the optimizer nav24 runs at
 // core/backEnd/BE_GraphOptim.cpp:66-68):
 //   lin_pt     windows starting an iteration: one lane per observation in

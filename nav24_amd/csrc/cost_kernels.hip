@@ -35,7 +35,6 @@ namespace navcost {
 
 using navba::block_sum;
 using navba::kWave;
-using navba::wave_sum;
 
 constexpr int kTileObs = 256;  // observations per tile (whole points; one larger point has a tile of its own)
 constexpr int kThreads = 256;
@@ -80,9 +79,6 @@ struct ObsGrad {
     T gpose[6];
     T gintr[8];
 };
-
-template <typename T>
-__device__ __forceinline__ T sqrt_t(T v) { return sqrt(v); }
 
 // What of an observation's terms a caller wants: the cost, with the gradients
 // to point and intrinsics, or the gradient to the pose alone.
@@ -253,8 +249,8 @@ __global__ __launch_bounds__(kThreads, 8) void k_cg_cost(CostProblem P, const TP
 // + j]; then those that clear the unseen points' gradients.  Bound by the FP64
 // operations of the terms and by memory together: 24 bytes per observation in one
 // order and 20 in the other.  64 scenes of 5 000 points, with the final sums: 67 us
-// in FP64 and 63 in FP32, before 220 and 191 (a gather of six stored pose terms per
-// observation, and one workgroup's sums over all tiles).
+// in FP64 and 63 in FP32 (68 at FP64 poses), before 220 and 191 (a gather of six
+// stored pose terms per observation, and one workgroup's sums over all tiles).
 template <typename T, typename TP>
 __global__ __launch_bounds__(kThreads, 4) void k_cg_obs(CostProblem P, const TP* __restrict__ Tcw,
                                                         const T* __restrict__ X, const T* __restrict__ intr,
@@ -439,7 +435,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_final(CostProblem P, const doub
 // Coefficients of exp on SE3 at th2 = |omega|^2 and their derivatives:
 //   a = sin t / t, b = (1 - cos t) / t^2, c = (t - sin t) / t^3,
 //   db = b'(t) / t = (a - 2 b) / t^2,  dc = c'(t) / t = (b - 3 c) / t^2.
-// Below th2 = 0.25 their Taylor series (seven terms, truncation below 1e-17):
+// Below th2 = 0.25 their Taylor series (seven terms, truncation below 5e-17):
 // the closed forms cancel there.  FP64 for both compute types.
 struct ExpCoef { double a, b, c, db, dc; };
 

@@ -295,7 +295,9 @@ __device__ __forceinline__ void pair_factors(const DevProblem& P, const double* 
 #pragma unroll
         for (int q = 0; q < 6; ++q) E[q] = wb[6 + q];
         mul_et(E, J, C);
-        // (the weight last: its load has the longest to land)
+        // (the weight last, as its load has the longest to land: 1 % of the rounds
+        // kernel on 60 keyframes, 156.2 against 158.1 us, and within 1 % either way
+        // on 512 windows and a 300-keyframe loop)
         const double s0 = wgt * (iz * (P.fx * P.fx)), s1 = wgt * (iz * (P.fy * P.fy));
         C[0] *= s0; C[2] *= s0;
         C[1] *= s1; C[3] *= s1;

@@ -41,8 +41,8 @@ struct KpParams {
 
 // 1 / d, correctly rounded: the steps of the compiler's division without its
 // scalings, which for a numerator of 1 change nothing unless d or the result is
-// subnormal (d here is 1 plus something, so 0 or at least 2^-53, and far below
-// 2^1022 for any float input), and with its fix-up of 0, infinities and NaN.  8
+// subnormal (d here is 1 plus something, so 0 or at least 2^-53, and for a point
+// anywhere near an image far below 2^1022), and with its fix-up of 0, infinities and NaN.  8
 // instructions instead of 11.
 __device__ __forceinline__ double reciprocal(double d) {
     double r = __builtin_amdgcn_rcp(d);
