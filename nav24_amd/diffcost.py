@@ -13,9 +13,10 @@ OptimizableTypes.hpp:221-227), X [n_pt, 3] the points and intr [8] =
 (fx, fy, cx, cy, k1, k2, p1, p2).  The device kernel returns the
 left-tangent gradient g at T = exp(xi) T_cw (the gradient for a perturbation
 exp(d) T); backward maps it to d cost / d xi = J_l(xi)^T g, J_l the SE3 left
-Jacobian, by the chain rule through `se3_left`, so the two agree only at
-xi = 0 and every xi gets its true gradient.  There is no CPU fallback:
-without the built library or a gfx950 device the calls raise.
+Jacobian, so the two agree only at xi = 0 and every xi gets its true gradient.
+Where all four tensors share a type the poses exp(xi) T_cw are formed and used
+in FP64, whichever it is.  There is no CPU fallback: without the built library
+or a gfx950 device the calls raise.
 """
 from __future__ import annotations
 
